@@ -589,8 +589,11 @@ static void elph_cache(ElphHandle* H, const double* U1, int nb1, const double* k
       for (int i = 0; i < H->nRp; ++i) pp[i] = make_double2(1. / hDegP[i], 0.);
       h2d(H->phP1, pp, s);
     }
-    H->sPhE.reserve(size_t(H->nRe));
-    launch_phase_table(1, H->nRe, H->sK.p, H->Re.p, H->invE.p, 1.0, H->sPhE.p, s);
+    H->sPhE.reserve(cache_phase_size(H->nRe));
+    if (H->precision == PHX_FP64)
+      launch_phase_cols<double>(1, H->nRe, H->sK.p, H->Re.p, H->invE.p, H->sPhE.p, s);
+    else
+      launch_phase_cols<float>(1, H->nRe, H->sK.p, H->Re.p, H->invE.p, H->sPhE.p, s);
     CacheParams cp{};
     cp.nRe = H->nRe;
     cp.nRp = H->nRp;
@@ -1635,7 +1638,7 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
     if (L->precision == PHX_FP64) L->TgD.reserve(nA * L->nGe * N);
     else L->TgF.reserve(nA * L->nGe * N);
   } else {
-    L->phE.reserve(size_t(nkk) * L->nRe);
+    L->phE.reserve(cache_phase_size(L->nRe));
   }
   b.nLinesB = nLinesB;
   L->phP.reserve(size_t(nkk) * L->nRp);
@@ -1725,7 +1728,12 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
   const int* dPGS = dPB1 + nPanels;
   const int* dPGZ = dPGS + nPanels;
   // phases: e^{ik1.Re}/de (GEMM form), e^{-ik1.Rp}/dp
-  if (!line) launch_phase_table(nkk, L->nRe, b.k1.p, L->Re.p, L->invDegE.p, 1.0, L->phE.p, s);
+  if (!line) {
+    if (L->precision == PHX_FP64)
+      launch_phase_cols<double>(nkk, L->nRe, b.k1.p, L->Re.p, L->invDegE.p, L->phE.p, s);
+    else
+      launch_phase_cols<float>(nkk, L->nRe, b.k1.p, L->Re.p, L->invDegE.p, L->phE.p, s);
+  }
   launch_phase_table(nkk, L->nRp, b.k1.p, L->Rp.p, L->invDegP.p, -1.0, L->phP.p, s);
   if (L->timing) PHX_HIP(hipEventRecord(L->ev[0], s));
   // cacheElPh for the whole batch
@@ -2373,7 +2381,7 @@ static void phel_setup(PhelHandle* P, const phx_problem& p, ElphHandle* H, const
     for (int k = 0; k < kCacheNKK; ++k)
       for (int i = 0; i < H->nRp; ++i) pp[size_t(k) * H->nRp + i] = make_double2(1. / degP[i], 0.);
     h2d(P->phP, pp, s);
-    P->phE.alloc(size_t(kCacheNKK) * H->nRe);
+    P->phE.alloc(cache_phase_size(H->nRe));
     P->kb.alloc(3 * size_t(kCacheNKK));
     P->cmeta.alloc(3 * size_t(kCacheNKK));
     P->pmeta.alloc(size_t(kCacheNKK) * (1 + 2 * P->nb1max));
@@ -2467,7 +2475,8 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
   PHX_HIP(hipMemcpyAsync(P->pmeta.p, pm.data(), pm.size() * sizeof(int), hipMemcpyHostToDevice, s));
   PHX_HIP(hipMemcpyAsync(P->F1.p, F.data(), F.size() * sizeof(double), hipMemcpyHostToDevice, s));
   rec(0);
-  launch_phase_table(n, H->nRe, P->kb.p, H->Re.p, P->invE.p, 1.0, P->phE.p, s);
+  if (f64) launch_phase_cols<double>(n, H->nRe, P->kb.p, H->Re.p, P->invE.p, P->phE.p, s);
+  else launch_phase_cols<float>(n, H->nRe, P->kb.p, H->Re.p, P->invE.p, P->phE.p, s);
   CacheParams cp{};
   cp.nRe = H->nRe;
   cp.nRp = H->nRp;

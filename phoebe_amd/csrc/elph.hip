@@ -22,6 +22,7 @@
 //            including the b1 degenerate-group average of symmetrizeCoupling.
 #include <algorithm>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "elph_params.hpp"
@@ -135,6 +136,38 @@ void launch_phase_table(int rows, int nR, const double* kc, const double* R, con
   PHX_HIP(hipGetLastError());
 }
 
+// The same table transposed for k_cache, in the GEMM's precision: out(r, i) with
+// `cols` points per row (points beyond `rows` zero) and nR rounded up to whole
+// quads (rows beyond nR zero).
+template <typename T>
+__global__ void k_phase_cols(int rows, int cols, int nR, const double* __restrict__ kc,
+                             const double* __restrict__ R, const double* __restrict__ scale, T* __restrict__ out) {
+  const int n = (nR + 3) / 4 * 4 * cols;
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
+    const int r = t / cols, i = t - r * cols;
+    double s = 0., c = 0.;
+    if (r < nR && i < rows) {
+      sincos(kc[3 * i] * R[3 * r] + kc[3 * i + 1] * R[3 * r + 1] + kc[3 * i + 2] * R[3 * r + 2], &s, &c);
+      s *= scale[r];
+      c *= scale[r];
+    }
+    out[2 * size_t(t)] = T(c);
+    out[2 * size_t(t) + 1] = T(s);
+  }
+}
+
+template <typename T>
+void launch_phase_cols(int rows, int nR, const double* kc, const double* R, const double* scale, void* out,
+                       hipStream_t s) {
+  if (rows <= 0) return;
+  const int cols = cache_phase_cols(rows);
+  hipLaunchKernelGGL(k_phase_cols<T>, dim3(ceil_div(ceil_div(nR, 4) * 4 * cols, 256)), dim3(256), 0, s, rows, cols,
+                     nR, kc, R, scale, static_cast<T*>(out));
+  PHX_HIP(hipGetLastError());
+}
+template void launch_phase_cols<double>(int, int, const double*, const double*, const double*, void*, hipStream_t);
+template void launch_phase_cols<float>(int, int, const double*, const double*, const double*, void*, hipStream_t);
+
 // GEMM A operand: rows of e^{ik.Rp} (no degeneracy factor), interleaved (re, im)
 // over Kp >= 2 nRp columns (zero padded), for rowsPad rows (rows >= nrows zero).
 template <typename T>
@@ -229,14 +262,14 @@ void launch_transpose_e3(int nk, int nm, const double2* ev, void* out, bool fp32
 }
 
 // ------------------------------------------------------------------ cacheElPh
-// g1(k1; Rp,nu,w1,w2) = sum_Re P(k1,Re) gW(Re,Rp,nu,w1,w2) as a real MFMA GEMM.
-// Output rows m < NKK hold Re(g1) of outer point m, rows NKK+m hold Im(g1);
-// the K dimension walks R_e in chunks of 8 vectors, ordered so that lane
-// group g of k-step ks reads (Re, Im) of gW at R_e = re0 + g + 4*(ks/2) with
-// one 2-element load serving k-steps 2q (Re part) and 2q+1 (Im part):
-//   A'(m, k) = [ Pr | -Pi ] for m < NKK,  [ Pi | Pr ] for m >= NKK.
-// One workgroup owns one (Rp, nu) block of nw^2 columns (256 per pass), so the
-// U1 rotation and the e^{-ik1.Rp}/dp factor run as its epilogue.
+// g1(k1; Rp,nu,w1,w2) = sum_Re P(k1,Re) gW(Re,Rp,nu,w1,w2) as a real MFMA GEMM:
+// M = the outer points (tiles of 16, real and imaginary parts of g1 in
+// accumulators of their own), N = gW columns, K = R_e in quads.  Lane (lr, lg)
+// loads P(R_e = 4q + lg, point lr) and gW(R_e, column lr) as complex numbers,
+// and four products per tile pair and quad take their components:
+//   Re += Pr x, Im += Pi x;  Re += (-Pi) y, Im += Pr y     (gW = x + i y).
+// A workgroup owns whole (Rp, nu) blocks of nw^2 columns, so the U1 rotation
+// and the e^{-ik1.Rp}/dp factor run as its epilogue.
 
 template <typename T> struct Vec2;
 template <> struct Vec2<double> { typedef double2 type; };
@@ -262,15 +295,14 @@ template <> struct MfmaC<float> {
 __host__ __device__ inline int cache_pass_cols(int nw) { return (256 / nw) * nw; }
 
 // Panel epilogue shared by the cacheElPh kernels.  Cb holds g1 of up to 16
-// outer points (kbase .. min(kbase+16, kend)-1) for the columns c0 .. c0+255 of block (rp, nu),
-// of which the pass owns c0 .. c0 + cache_pass_cols(nw) - 1 (whole w1 blocks):
-// real parts in rows 0..15, imaginary parts in rows 16..31.  Applies the U1
-// rotation over the w1 range of those columns and the factor s(k1, Rp), and
-// writes (c0 == 0) or adds (later column passes) the panel entries.  Each
-// output (outer point, b1, w2) is owned by the same thread in every pass (the
-// thread-to-output map does not depend on c0).
+// outer points (kbase .. min(kbase+16, kend)-1) for the columns (w1, w2),
+// w1lo <= w1 < w1hi, of block (rp, nu): real parts in rows 0..15, imaginary
+// parts in rows 16..31, CW elements per row.  Applies the U1 rotation over that
+// w1 range and the factor s(k1, Rp), and writes (w1lo == 0) or adds (later
+// passes) the panel entries.  Each output (outer point, b1, w2) is owned by the
+// same thread in every pass (the thread-to-output map does not depend on w1lo).
 template <typename T, typename OutT>
-__device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const T* Cb, int c0,
+__device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const T* Cb, int CW, int w1lo, int w1hi,
                                                      int kbase, int rp, int nu, int kend) {
   const int t = threadIdx.x, nw = p.nw;
   OutT* Bout = static_cast<OutT*>(p.B);
@@ -281,8 +313,6 @@ __device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const
   for (int kl = 0; kl < nkl; ++kl) nbm = max(nbm, p.nb1[kbase + kl]);
   nbm = __builtin_amdgcn_readfirstlane(nbm);
   const int per = nbm * nw;
-  // columns of this pass: w1 in [c0/nw, (c0 + pass)/nw), all w2
-  const int w1lo = c0 / nw, w1hi = min(nw, (c0 + cache_pass_cols(nw)) / nw);
   for (int idx = t; idx < nkl * per; idx += 256) {
     const int kl = idx / per, rem = idx - kl * per, b1 = rem / nw, w2 = rem - b1 * nw;
     const int kk = kbase + kl;
@@ -291,8 +321,8 @@ __device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const
     const double2 s = p.phP[size_t(kk) * p.nRp + rp];
     double2 v = make_double2(0., 0.);
     for (int w1 = w1lo; w1 < w1hi; ++w1) {
-      const int cl = w1 * nw + w2 - c0;
-      const double ar = double(Cb[kl * 256 + cl]), ai = double(Cb[(16 + kl) * 256 + cl]);
+      const int cl = (w1 - w1lo) * nw + w2;
+      const double ar = double(Cb[kl * CW + cl]), ai = double(Cb[(16 + kl) * CW + cl]);
       const double2 u = U1[w1 + nw * b1];
       v.x += ar * u.x - ai * u.y;
       v.y += ar * u.y + ai * u.x;
@@ -300,7 +330,7 @@ __device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const
     const double2 c = make_double2(v.x * s.x - v.y * s.y, v.x * s.y + v.y * s.x);
     OutT* panel = Bout + size_t(p.panelBase[kk] + b1) * p.panelStride;
     const size_t col = 2 * (size_t(nu) * nw + w2);
-    if (c0 == 0) {
+    if (w1lo == 0) {
       panel[size_t(2 * rp) * p.ldb + col] = OutT(c.x);
       panel[size_t(2 * rp) * p.ldb + col + 1] = OutT(c.y);
       panel[size_t(2 * rp + 1) * p.ldb + col] = OutT(-c.y);
@@ -314,105 +344,179 @@ __device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const
   }
 }
 
-template <typename T, typename OutT>
+// How k_cache cuts the gW columns: a workgroup takes `blocks` whole (Rp, nu)
+// blocks of nw^2 columns in `passes` passes of `w1Rows` rows of nw columns, as
+// ntw tiles of 16 columns per wave on wc waves; 4 / wc waves share the R_e sum.
+struct CacheTiling {
+  int blocks, passes, w1Rows, wc, ntw;
+};
+inline CacheTiling cache_tiling(int nw) {
+  CacheTiling t{};
+  const int E = nw * nw;
+  t.blocks = E <= 32 ? 64 / E : 1;
+  t.passes = t.blocks > 1 ? 1 : (nw + 256 / nw - 1) / (256 / nw);
+  t.w1Rows = (nw + t.passes - 1) / t.passes;
+  const int cols = t.blocks > 1 ? t.blocks * E : t.w1Rows * nw;
+  const int tiles = (cols + 15) / 16;
+  t.wc = tiles <= 4 ? 1 : tiles <= 8 ? 2 : 4;
+  t.ntw = (tiles + t.wc - 1) / t.wc;
+  return t;
+}
+// LDS row of the epilogue (elements): every column of the pass, padded so that
+// the four row groups of an accumulator tile fall into different banks.
+__host__ __device__ inline int cache_row(int wc, int ntw) { return 16 * wc * ntw + 4; }
+
+// Bound by HBM and the matrix cores alike at a batch of 32 points (16 bytes and
+// 256 FLOP per gW element in FP64), by HBM at a few points.  The main loop has
+// no barrier: a wave reads its A fragment (the phases, transposed so that 16
+// lanes read consecutive points; a table of some 100 KB that stays in L2) and
+// its gW columns straight into registers, two R_e quads at a time.  With few
+// columns per block (nw <= 11) two or all four waves of a workgroup share the
+// block and split the R_e sum, which LDS adds up in wave order; with all four on
+// columns, three of them had none at nw = 8.  A batch of up to 16 points runs
+// one tile of points instead of two.
+// nw = 8, 6 modes, R on WS(7^3) x WS(6^3) (0.73 GB of gW in FP64), against a
+// version with the phases staged in LDS between barriers and all waves on
+// columns: 32 points 0.98 -> 0.22 ms in FP64 (52 TFLOP/s) and 0.55 -> 0.145 ms
+// in FP32; one point 0.89 -> 0.16 ms (4.6 TB/s, the copy rate).
+template <typename T, typename OutT, int MH, int NTW>
 __global__ void __launch_bounds__(256, 2) k_cache(CacheParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NKK = kCacheNKK, MR = 2 * NKK, MTc = MR / 16, LDA = 17;
   typedef typename Vec2<T>::type T2;
   typedef typename MfmaC<T>::acc_t acc_t;
-  const int rp = blockIdx.x / p.nm, nu = blockIdx.x % p.nm;
-  const int E = p.nw * p.nw;
+  constexpr int D = 2;  // 3 and 4 cost FP32 registers and time
+  const int E = p.nw * p.nw, nBlocks = p.nRp * p.nm;
+  const int blk0 = blockIdx.x * p.blocks, nblk = min(p.blocks, nBlocks - blk0);
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lr = lane & 15, lg = lane >> 4;
-  const size_t strideRe = size_t(p.nRp) * p.nm * E;
-  const T2* G = static_cast<const T2*>(p.gW) + (size_t(rp) * p.nm + nu) * E;
-  T* As = reinterpret_cast<T*>(smem);               // MR x LDA
-  T* Cb = reinterpret_cast<T*>(smem);               // epilogue: 2 x 16 x 256
-  const int nchunk = (p.nRe + 7) / 8;
+  const int WC = p.wc, WK = 4 / WC, wc = wave % WC, wk = wave / WC;
+  const int CW = cache_row(WC, NTW);
+  T* Cb = reinterpret_cast<T*>(smem);  // (WK, 32, CW): real parts of 16 points, then imaginary
+  const size_t stride = size_t(nBlocks) * E;
+  const T2* G = static_cast<const T2*>(p.gW) + size_t(blk0) * E;
+  const T2* ph = static_cast<const T2*>(p.phE);
+  const int nq = p.nRe / 4, q0 = nq * wk / WK, q1 = nq * (wk + 1) / WK;
 
-  for (int c0 = 0; c0 < E; c0 += cache_pass_cols(p.nw)) {
-    acc_t acc[MTc][4];
+  for (int w1lo = 0; w1lo < p.nw; w1lo += p.w1Rows) {
+    const int w1hi = min(p.nw, w1lo + p.w1Rows);
+    const int cols = p.blocks > 1 ? nblk * E : (w1hi - w1lo) * p.nw;
+    const T2* Gc[NTW];  // columns beyond the pass read its last one; nothing uses their sums
 #pragma unroll
-    for (int m = 0; m < MTc; ++m)
+    for (int j = 0; j < NTW; ++j) Gc[j] = G + size_t(w1lo) * p.nw + min((wc * NTW + j) * 16 + lr, cols - 1);
+    acc_t accr[MH][NTW], acci[MH][NTW];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+    for (int m = 0; m < MH; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[m][j][i] = 0;
-    T2 bq[2][4], bn[2][4];
-    auto load_b = [&](T2(&b)[2][4], int re0) {
+      for (int j = 0; j < NTW; ++j)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = c0 + (wave * 4 + j) * 16 + lr;
+        for (int i = 0; i < 4; ++i) accr[m][j][i] = acci[m][j][i] = 0;
+    // A ring of D quads.  The loop's loads are unconditional (quads beyond the
+    // wave's last read valid rows again and are not used): a load under a branch
+    // makes the compiler wait for every load in flight.
+    T2 b[D][NTW], a[D][MH];
+    auto load = [&](T2(&bb)[NTW], T2(&aa)[MH], int q) {
+      const int re = 4 * q + lg;
+      const size_t row = size_t(min(re, p.nRe - 1)) * stride;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int re = re0 + lg + 4 * h;
-          b[h][j] = (re < p.nRe && col < E) ? G[size_t(re) * strideRe + col] : T2{T(0), T(0)};
-        }
-      }
+      for (int j = 0; j < NTW; ++j) bb[j] = Gc[j][row];
+#pragma unroll
+      for (int m = 0; m < MH; ++m) aa[m] = ph[size_t(re) * (16 * MH) + 16 * m + lr];
     };
-    load_b(bq, 0);
-    for (int ch = 0; ch < nchunk; ++ch) {
-      const int re0 = ch * 8;
-      __syncthreads();
-      for (int i = t; i < MR * 16; i += 256) {
-        const int m = i / 16, k = i % 16, ks = k / 4, g = k % 4;
-        const int re = re0 + g + 4 * (ks >> 1), s = ks & 1, kk = m % NKK;
-        const double2 P = (kk < p.nkk && re < p.nRe) ? p.phE[size_t(kk) * p.nRe + re] : make_double2(0., 0.);
-        const double v = (m < NKK) ? (s ? -P.y : P.x) : (s ? P.x : P.y);
-        As[m * LDA + k] = T(v);
-      }
-      __syncthreads();
-      if (ch + 1 < nchunk) load_b(bn, re0 + 8);
+    auto product = [&](const T2(&bb)[NTW], const T2(&aa)[MH]) {
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        T a[MTc];
+      for (int j = 0; j < NTW; ++j)
 #pragma unroll
-        for (int m = 0; m < MTc; ++m) a[m] = As[(16 * m + lr) * LDA + 4 * ks + lg];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const T b = (ks & 1) ? bq[ks >> 1][j].y : bq[ks >> 1][j].x;
-#pragma unroll
-          for (int m = 0; m < MTc; ++m) acc[m][j] = MfmaC<T>::mac(a[m], b, acc[m][j]);
+        for (int m = 0; m < MH; ++m) {
+          accr[m][j] = MfmaC<T>::mac(aa[m].x, bb[j].x, accr[m][j]);
+          acci[m][j] = MfmaC<T>::mac(aa[m].y, bb[j].x, acci[m][j]);
         }
+#pragma unroll
+      for (int j = 0; j < NTW; ++j)
+#pragma unroll
+        for (int m = 0; m < MH; ++m) {
+          accr[m][j] = MfmaC<T>::mac(-aa[m].y, bb[j].y, accr[m][j]);
+          acci[m][j] = MfmaC<T>::mac(aa[m].x, bb[j].y, acci[m][j]);
+        }
+    };
+    const int n = q1 - q0, qLast = max(nq - 1, 0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(b[d], a[d], min(q0 + d, qLast));
+    int i = 0;
+    for (; i + D <= n; i += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        product(b[d], a[d]);
+        load(b[d], a[d], min(q0 + i + d + D, qLast));
       }
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bq[h][j] = bn[h][j];
     }
-    // epilogue in passes of 16 outer points: real tile q and imaginary tile MTc/2 + q
 #pragma unroll
-    for (int q = 0; q < MTc / 2; ++q) {
-      __syncthreads();
+    for (int d = 0; d < D - 1; ++d)
+      if (i + d < n) product(b[d], a[d]);
+    if ((p.nRe & 3) && wk == WK - 1) {  // the last R_e, less than a quad: rows beyond them are zero
+      load(b[0], a[0], nq);
+      if (4 * nq + lg >= p.nRe)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int cl = (wave * 4 + j) * 16 + lr;
+        for (int j = 0; j < NTW; ++j) b[0][j] = T2{T(0), T(0)};
+      product(b[0], a[0]);
+    }
+    // panel epilogue in passes of 16 outer points
+#pragma unroll
+    for (int m = 0; m < MH; ++m) {
+      if (16 * m >= p.nkk) break;
+      __syncthreads();  // the previous pass has read Cb
+      T* Cw = Cb + size_t(wk) * 32 * CW;
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) {
+        const int cl = (wc * NTW + j) * 16 + lr;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = MfmaC<T>::row(lg, i);
-          Cb[r * 256 + cl] = acc[q][j][i];
-          Cb[(16 + r) * 256 + cl] = acc[MTc / 2 + q][j][i];
+          Cw[r * CW + cl] = accr[m][j][i];
+          Cw[(16 + r) * CW + cl] = acci[m][j][i];
         }
       }
       __syncthreads();
-      cache_panel_epilogue<T, OutT>(p, Cb, c0, 16 * q, rp, nu, p.nkk);
+      if (WK > 1) {
+        for (int i = t; i < 32 * CW; i += 256) {
+          T v = Cb[i];
+          for (int k = 1; k < WK; ++k) v += Cb[size_t(k) * 32 * CW + i];
+          Cb[i] = v;
+        }
+        __syncthreads();
+      }
+      for (int bl = 0; bl < nblk; ++bl)
+        cache_panel_epilogue<T, OutT>(p, Cb + bl * E, CW, w1lo, w1hi, 16 * m, (blk0 + bl) / p.nm,
+                                      (blk0 + bl) % p.nm, p.nkk);
     }
   }
 }
 
-inline size_t cache_lds_bytes(int elem) {
-  return std::max(size_t(2 * kCacheNKK) * 17 * elem, size_t(2) * 16 * 256 * elem);
-}
-
 template <typename T, typename OutT>
-void launch_cache(const CacheParams& p, hipStream_t s) {
+void launch_cache(const CacheParams& p0, hipStream_t s) {
+  CacheParams p = p0;
   PHX_REQUIRE(p.nw <= 32, "cacheElPh kernel supports nw <= 32");
   PHX_REQUIRE(p.nkk <= kCacheNKK, "cacheElPh kernel: too many outer points per launch");
   if (p.nkk <= 0) return;
-  const size_t lds = cache_lds_bytes(sizeof(T));
-  auto kern = k_cache<T, OutT>;
-  PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-  hipLaunchKernelGGL(kern, dim3(p.nRp * p.nm), dim3(256), lds, s, p);
+  const CacheTiling c = cache_tiling(p.nw);
+  p.blocks = c.blocks;
+  p.w1Rows = c.w1Rows;
+  p.wc = c.wc;
+  const size_t lds = size_t(4 / c.wc) * 32 * cache_row(c.wc, c.ntw) * sizeof(T);
+  auto go = [&](auto kern) {
+    PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    hipLaunchKernelGGL(kern, dim3(ceil_div(p.nRp * p.nm, c.blocks)), dim3(256), lds, s, p);
+  };
+  auto ntw = [&](auto mh) {
+    constexpr int MH = decltype(mh)::value;
+    switch (c.ntw) {
+      case 1: go(k_cache<T, OutT, MH, 1>); break;
+      case 2: go(k_cache<T, OutT, MH, 2>); break;
+      case 3: go(k_cache<T, OutT, MH, 3>); break;
+      default: go(k_cache<T, OutT, MH, 4>);
+    }
+  };
+  if (cache_phase_cols(p.nkk) == 16) ntw(std::integral_constant<int, 1>{});
+  else ntw(std::integral_constant<int, 2>{});
   PHX_HIP(hipGetLastError());
 }
 template void launch_cache<double, double>(const CacheParams&, hipStream_t);
@@ -637,7 +741,8 @@ __global__ void __launch_bounds__(256) k_cache_line_b(CacheParams p) {
           Cb[(16 + kl) * 256 + t] = acci[kl];
         }
         __syncthreads();
-        cache_panel_epilogue<T, OutT>(p, Cb, c0, kbase, rp, nu, kend);
+        cache_panel_epilogue<T, OutT>(p, Cb, 256, c0 / p.nw, min(p.nw, (c0 + cache_pass_cols(p.nw)) / p.nw), kbase, rp,
+                                      nu, kend);
       }
     }
   }

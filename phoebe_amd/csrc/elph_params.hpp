@@ -20,12 +20,20 @@ inline int line_count_padded(int n) {
   return n <= 4 ? n : n <= 6 ? 6 : n <= 8 ? 8 : n <= 12 ? 12 : 16;
 }
 
+// Outer points per row of the GEMM form's phase table: the batch rounded up to
+// k_cache's 16-point tiles.
+inline int cache_phase_cols(int nkk) { return nkk <= 16 ? 16 : kCacheNKK; }
+// Complex FP64 values that hold the table of any batch, in either precision.
+inline size_t cache_phase_size(int nRe) { return size_t(kCacheNKK) * ((nRe + 3) / 4 * 4); }
+
 // g1(k1; Rp,nu,w1,w2) = sum_Re e^{ik1.Re}/de gW(Re,Rp,nu,w1,w2), rotated by U1
 // and scaled by s(k1, Rp) into one real panel per (k1, b1).
 struct CacheParams {
   int nRe, nRp, nm, nw, nkk;
   const void* gW;         // (nRe, nRp, nm, nw, nw) complex, element type T
-  const double2* phE;     // (nkk, nRe): e^{ik1.Re}/de (GEMM form)
+  const void* phE;        // (nRe rounded up to quads, cache_phase_cols(nkk)): e^{ik1.Re}/de, complex T,
+                          // zero in the padding (GEMM form)
+  int blocks, w1Rows, wc; // k_cache's column tiling (set by its launcher)
   const double2* phP;     // (nkk, nRp): e^{-ik1.Rp}/dp or 1/dp
   const double2* U1pool;  // per kk: (nw, nb1) column-major
   const int* U1off;       // complex offset per kk
@@ -62,6 +70,9 @@ struct CollectParams {
 };
 
 template <typename T, typename OutT> void launch_cache(const CacheParams& p, hipStream_t s);
+template <typename T>
+void launch_phase_cols(int rows, int nR, const double* kc, const double* R, const double* scale, void* out,
+                       hipStream_t s);
 template <typename T, typename OutT> void launch_cache_line(const CacheParams& p, hipStream_t s);
 void launch_collect(const CollectParams& p, hipStream_t s);
 
