@@ -606,6 +606,7 @@ static void elph_cache(ElphHandle* H, const double* U1, int nb1, const double* k
     cp.U1pool = H->U1.p;
     cp.U1off = H->meta.p + 0;
     cp.nb1 = H->meta.p + 1;
+    cp.nb1Max = nb1;
     cp.panelBase = H->meta.p + 2;
     cp.panelStride = pstride;
     cp.ldb = H->ldb;
@@ -720,13 +721,16 @@ struct BatchMeta {
   double flops = 0.;  // algorithmic FLOPs of the coupling stage (timing)
   // [U1off nkk][nb1 nkk][panelBase nkk][kkMesh nkk][kkStateOff nkk][panelKK P][panelB1 P][panelGStart P][panelGSize P]
   std::vector<int> hmeta, hLineKK;
+  std::vector<int4> hJobs;
   std::vector<double> hk1;
   std::vector<double2> hwLine, hphLine;
-  std::vector<float2> hphLineF;
-  DevBuf<int> meta, lineKK;
+  std::vector<float2> hwLineF, hphLineF;
+  int nJobs = 0, jobTiles = 0;
+  DevBuf<int> meta;
+  DevBuf<int4> jobs;
   DevBuf<double> k1;
-  DevBuf<double2> wLine, phLineD;
-  DevBuf<float2> phLineF;
+  DevBuf<double2> wLineD, phLineD;
+  DevBuf<float2> wLineF, phLineF;
 };
 
 struct LwHandle {
@@ -1608,18 +1612,37 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
             make_double2((ty.x * tz.x - ty.y * tz.y) * d, (ty.x * tz.y + ty.y * tz.x) * d);
       }
     }
-    b.hwLine.resize(size_t(nkk) * L->nGe);
-    for (int i = 0; i < nkk; ++i) {
-      int x, y, z;
-      mesh_coords(L->active[k1s[i]], m0, m1, x, y, z);
-      for (int g = 0; g < L->nGe; ++g)
-        b.hwLine[size_t(i) * L->nGe + g] = twiddle((long long)x * L->grpF0e[g], m0);
+    // stage b: the points of each line in jobs of whole 16-point tiles
+    b.hJobs.clear();
+    b.jobTiles = 1;
+    for (int l = 0; l < nLinesB; ++l) {
+      const int n = lk[l + 1] - lk[l], tiles = ceil_div(n, 16), per = ceil_div(tiles, ceil_div(tiles, kJobTiles));
+      b.jobTiles = std::max(b.jobTiles, per);
+      for (int i = 0; i < n; i += 16 * per) b.hJobs.push_back(make_int4(lk[l] + i, std::min(16 * per, n - i), l, 0));
     }
-    b.lineKK.reserve(lk.size());
-    PHX_HIP(hipMemcpyAsync(b.lineKK.p, lk.data(), lk.size() * sizeof(int), hipMemcpyHostToDevice, s));
-    b.wLine.reserve(b.hwLine.size());
-    PHX_HIP(hipMemcpyAsync(b.wLine.p, b.hwLine.data(), b.hwLine.size() * sizeof(double2),
-                           hipMemcpyHostToDevice, s));
+    b.nJobs = int(b.hJobs.size());
+    const int cols = 16 * b.jobTiles;
+    const size_t gPad = size_t(L->nGe + 3) / 4 * 4;
+    b.hwLine.assign(b.hJobs.size() * gPad * cols, make_double2(0., 0.));
+    for (size_t j = 0; j < b.hJobs.size(); ++j)
+      for (int i = 0; i < b.hJobs[j].y; ++i) {
+        int x, y, z;
+        mesh_coords(L->active[k1s[b.hJobs[j].x + i]], m0, m1, x, y, z);
+        for (int g = 0; g < L->nGe; ++g)
+          b.hwLine[(j * gPad + g) * cols + i] = twiddle((long long)x * L->grpF0e[g], m0);
+      }
+    b.jobs.reserve(b.hJobs.size());
+    PHX_HIP(hipMemcpyAsync(b.jobs.p, b.hJobs.data(), b.hJobs.size() * sizeof(int4), hipMemcpyHostToDevice, s));
+    const size_t nwl = b.hwLine.size();
+    if (L->precision == PHX_FP64) {
+      b.wLineD.reserve(nwl);
+      PHX_HIP(hipMemcpyAsync(b.wLineD.p, b.hwLine.data(), nwl * sizeof(double2), hipMemcpyHostToDevice, s));
+    } else {
+      b.hwLineF.resize(nwl);
+      for (size_t i = 0; i < nwl; ++i) b.hwLineF[i] = make_float2(float(b.hwLine[i].x), float(b.hwLine[i].y));
+      b.wLineF.reserve(nwl);
+      PHX_HIP(hipMemcpyAsync(b.wLineF.p, b.hwLineF.data(), nwl * sizeof(float2), hipMemcpyHostToDevice, s));
+    }
     const size_t nph = b.hphLine.size();
     if (L->precision == PHX_FP64) {
       b.phLineD.reserve(nph);
@@ -1749,6 +1772,8 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
   cp.U1pool = L->U2pool.p;
   cp.U1off = dU1off;
   cp.nb1 = dNb1;
+  cp.nb1Max = b.nb1Max;
+  cp.evenRows = L->transform == PHX_TRANSFORM_SEPARABLE;
   cp.panelBase = dPbase;
   cp.panelStride = pstride;
   cp.ldb = L->ldb;
@@ -1762,8 +1787,10 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     cp.reBlkEnd = L->reBlkEndD.p;
     cp.nLinesB = nLinesB;
     cp.nLinesA = line_count_padded(nLinesB);
-    cp.lineKK = b.lineKK.p;
-    cp.wLine = b.wLine.p;
+    cp.jobs = b.jobs.p;
+    cp.nJobs = b.nJobs;
+    cp.jobTiles = b.jobTiles;
+    cp.phE = L->precision == PHX_FP64 ? static_cast<const void*>(b.wLineD.p) : static_cast<const void*>(b.wLineF.p);
   }
   if (L->precision == PHX_FP64) {
     cp.B = L->Bd.p;
@@ -2489,6 +2516,7 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
   cp.U1pool = P->U1d.p;
   cp.U1off = P->cmeta.p;
   cp.nb1 = P->cmeta.p + K;
+  cp.nb1Max = P->nb1max;
   cp.panelBase = P->cmeta.p + 2 * K;
   cp.panelStride = P->pstride;
   cp.ldb = H->ldb;

@@ -291,55 +291,46 @@ template <> struct MfmaC<float> {
   __device__ static int row(int lk, int i) { return 4 * lk + i; }
 };
 
-// Column passes of the cacheElPh kernels cover whole w1 blocks: (256 / nw) * nw columns.
-__host__ __device__ inline int cache_pass_cols(int nw) { return (256 / nw) * nw; }
-
-// Panel epilogue shared by the cacheElPh kernels.  Cb holds g1 of up to 16
-// outer points (kbase .. min(kbase+16, kend)-1) for the columns (w1, w2),
-// w1lo <= w1 < w1hi, of block (rp, nu): real parts in rows 0..15, imaginary
-// parts in rows 16..31, CW elements per row.  Applies the U1 rotation over that
-// w1 range and the factor s(k1, Rp), and writes (w1lo == 0) or adds (later
-// passes) the panel entries.  Each output (outer point, b1, w2) is owned by the
-// same thread in every pass (the thread-to-output map does not depend on w1lo).
+// Panel epilogue of k_cache.  Cb holds g1 of up to 16 outer points (in rows
+// 0..15 the real parts, in rows 16..31 the imaginary parts, CW elements per row)
+// for the columns (w1, w2), w1lo <= w1 < w1hi, of block (rp, nu); pan[0 .. np - 1]
+// are those points' panels: (row in Cb | point << 4, offset of its U1 column).
+// Applies the U1 rotation over that w1 range and the factor s(k1, Rp), and
+// writes (w1lo == 0) or adds (later passes) the panel entries.  Each output
+// (panel, w2) is owned by the same thread in every pass (the thread-to-output
+// map does not depend on w1lo).
 template <typename T, typename OutT>
 __device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const T* Cb, int CW, int w1lo, int w1hi,
-                                                     int kbase, int rp, int nu, int kend) {
-  const int t = threadIdx.x, nw = p.nw;
-  OutT* Bout = static_cast<OutT*>(p.B);
-  const int nkl = min(16, kend - kbase);
-  // one thread per (outer point, b1, w2) of the batch: the band count of the
-  // batch's widest point bounds b1, so all 256 threads share the work
-  int nbm = 0;
-  for (int kl = 0; kl < nkl; ++kl) nbm = max(nbm, p.nb1[kbase + kl]);
-  nbm = __builtin_amdgcn_readfirstlane(nbm);
-  const int per = nbm * nw;
-  for (int idx = t; idx < nkl * per; idx += 256) {
-    const int kl = idx / per, rem = idx - kl * per, b1 = rem / nw, w2 = rem - b1 * nw;
-    const int kk = kbase + kl;
-    if (b1 >= p.nb1[kk]) continue;
-    const double2* U1 = p.U1pool + p.U1off[kk];
-    const double2 s = p.phP[size_t(kk) * p.nRp + rp];
+                                                     const int2* pan, int pan0, int np, int rp, int nu) {
+  typedef typename Vec2<OutT>::type O2;
+  const int nw = p.nw;
+  for (int idx = threadIdx.x; idx < np * nw; idx += 256) {
+    const int e = idx / nw, w2 = idx - e * nw;
+    const int2 m = pan[e];
+    const int kl = m.x & 15;
+    const double2 s = p.phP[size_t(m.x >> 4) * p.nRp + rp];
+    const double2* U1 = p.U1pool + m.y;
+    const T* xr = Cb + kl * CW + w2 - w1lo * nw;
+    const T* xi = xr + 16 * CW;
     double2 v = make_double2(0., 0.);
+#pragma unroll 8
     for (int w1 = w1lo; w1 < w1hi; ++w1) {
-      const int cl = (w1 - w1lo) * nw + w2;
-      const double ar = double(Cb[kl * CW + cl]), ai = double(Cb[(16 + kl) * CW + cl]);
-      const double2 u = U1[w1 + nw * b1];
+      const double ar = double(xr[w1 * nw]), ai = double(xi[w1 * nw]);
+      const double2 u = U1[w1];
       v.x += ar * u.x - ai * u.y;
       v.y += ar * u.y + ai * u.x;
     }
     const double2 c = make_double2(v.x * s.x - v.y * s.y, v.x * s.y + v.y * s.x);
-    OutT* panel = Bout + size_t(p.panelBase[kk] + b1) * p.panelStride;
-    const size_t col = 2 * (size_t(nu) * nw + w2);
+    // rows 2 rp (C) and 2 rp + 1 (i C) of the panel, whose rows are whole 16-element blocks
+    O2* row = reinterpret_cast<O2*>(static_cast<OutT*>(p.B) + size_t(pan0 + e) * p.panelStride +
+                                    size_t(2 * rp) * p.ldb) + size_t(nu) * nw + w2;
+    O2* rowI = row + p.ldb / 2;
     if (w1lo == 0) {
-      panel[size_t(2 * rp) * p.ldb + col] = OutT(c.x);
-      panel[size_t(2 * rp) * p.ldb + col + 1] = OutT(c.y);
-      panel[size_t(2 * rp + 1) * p.ldb + col] = OutT(-c.y);
-      panel[size_t(2 * rp + 1) * p.ldb + col + 1] = OutT(c.x);
+      row[0] = O2{OutT(c.x), OutT(c.y)};
+      if (!p.evenRows) rowI[0] = O2{OutT(-c.y), OutT(c.x)};
     } else {  // later column passes add their w1 range
-      panel[size_t(2 * rp) * p.ldb + col] += OutT(c.x);
-      panel[size_t(2 * rp) * p.ldb + col + 1] += OutT(c.y);
-      panel[size_t(2 * rp + 1) * p.ldb + col] += OutT(-c.y);
-      panel[size_t(2 * rp + 1) * p.ldb + col + 1] += OutT(c.x);
+      row[0] = O2{row[0].x + OutT(c.x), row[0].y + OutT(c.y)};
+      if (!p.evenRows) rowI[0] = O2{rowI[0].x + OutT(-c.y), rowI[0].y + OutT(c.x)};
     }
   }
 }
@@ -380,7 +371,7 @@ __host__ __device__ inline int cache_row(int wc, int ntw) { return 16 * wc * ntw
 // columns: 32 points 0.98 -> 0.22 ms in FP64 (52 TFLOP/s) and 0.55 -> 0.145 ms
 // in FP32; one point 0.89 -> 0.16 ms (4.6 TB/s, the copy rate).
 template <typename T, typename OutT, int MH, int NTW>
-__global__ void __launch_bounds__(256, 2) k_cache(CacheParams p) {
+__global__ void __launch_bounds__(256, MH * sizeof(T) > 16 ? 1 : 2) k_cache(CacheParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   typedef typename Vec2<T>::type T2;
   typedef typename MfmaC<T>::acc_t acc_t;
@@ -391,10 +382,23 @@ __global__ void __launch_bounds__(256, 2) k_cache(CacheParams p) {
   const int WC = p.wc, WK = 4 / WC, wc = wave % WC, wk = wave / WC;
   const int CW = cache_row(WC, NTW);
   T* Cb = reinterpret_cast<T*>(smem);  // (WK, 32, CW): real parts of 16 points, then imaginary
+  int2* sPan = reinterpret_cast<int2*>(Cb + size_t(WK) * 32 * CW);  // the job's panels
   const size_t stride = size_t(nBlocks) * E;
-  const T2* G = static_cast<const T2*>(p.gW) + size_t(blk0) * E;
-  const T2* ph = static_cast<const T2*>(p.phE);
-  const int nq = p.nRe / 4, q0 = nq * wk / WK, q1 = nq * (wk + 1) / WK;
+  // the job: rows summed over (R_e of gW, or the groups of a line's Tg), their
+  // phase table and the outer points kk0 .. kk0 + nk - 1
+  const int4 jb = p.jobs ? p.jobs[blockIdx.y] : make_int4(0, p.nkk, 0, 0);
+  const int kk0 = jb.x, nk = jb.y, nRows = p.jobs ? p.nGe : p.nRe;
+  const T2* G = (p.jobs ? static_cast<const T2*>(p.Tg) + size_t(jb.z) * nRows * stride : static_cast<const T2*>(p.gW)) +
+                size_t(blk0) * E;
+  const T2* ph = static_cast<const T2*>(p.phE) + size_t(blockIdx.y) * ((nRows + 3) / 4 * 4) * (16 * MH);
+  // the panels' metadata goes to LDS while the main loop runs: read in the
+  // epilogue, its chain of loads took longer there than the products
+  const int pan0 = p.panelBase[kk0];
+  for (int i = t; i < nk * p.nb1Max; i += 256) {
+    const int kl = i / p.nb1Max, b1 = i - kl * p.nb1Max, kk = kk0 + kl;
+    if (b1 < p.nb1[kk]) sPan[p.panelBase[kk] - pan0 + b1] = make_int2(kk << 4 | (kl & 15), p.U1off[kk] + p.nw * b1);
+  }
+  const int nq = nRows / 4, q0 = nq * wk / WK, q1 = nq * (wk + 1) / WK;
 
   for (int w1lo = 0; w1lo < p.nw; w1lo += p.w1Rows) {
     const int w1hi = min(p.nw, w1lo + p.w1Rows);
@@ -415,7 +419,7 @@ __global__ void __launch_bounds__(256, 2) k_cache(CacheParams p) {
     T2 b[D][NTW], a[D][MH];
     auto load = [&](T2(&bb)[NTW], T2(&aa)[MH], int q) {
       const int re = 4 * q + lg;
-      const size_t row = size_t(min(re, p.nRe - 1)) * stride;
+      const size_t row = size_t(min(re, nRows - 1)) * stride;
 #pragma unroll
       for (int j = 0; j < NTW; ++j) bb[j] = Gc[j][row];
 #pragma unroll
@@ -451,9 +455,9 @@ __global__ void __launch_bounds__(256, 2) k_cache(CacheParams p) {
 #pragma unroll
     for (int d = 0; d < D - 1; ++d)
       if (i + d < n) product(b[d], a[d]);
-    if ((p.nRe & 3) && wk == WK - 1) {  // the last R_e, less than a quad: rows beyond them are zero
+    if ((nRows & 3) && wk == WK - 1) {  // the last R_e, less than a quad: rows beyond them are zero
       load(b[0], a[0], nq);
-      if (4 * nq + lg >= p.nRe)
+      if (4 * nq + lg >= nRows)
 #pragma unroll
         for (int j = 0; j < NTW; ++j) b[0][j] = T2{T(0), T(0)};
       product(b[0], a[0]);
@@ -461,7 +465,7 @@ __global__ void __launch_bounds__(256, 2) k_cache(CacheParams p) {
     // panel epilogue in passes of 16 outer points
 #pragma unroll
     for (int m = 0; m < MH; ++m) {
-      if (16 * m >= p.nkk) break;
+      if (16 * m >= nk) break;
       __syncthreads();  // the previous pass has read Cb
       T* Cw = Cb + size_t(wk) * 32 * CW;
 #pragma unroll
@@ -483,28 +487,29 @@ __global__ void __launch_bounds__(256, 2) k_cache(CacheParams p) {
         }
         __syncthreads();
       }
+      const int kl1 = min(16 * m + 16, nk) - 1;
+      const int e0 = p.panelBase[kk0 + 16 * m] - pan0, e1 = p.panelBase[kk0 + kl1] + p.nb1[kk0 + kl1] - pan0;
       for (int bl = 0; bl < nblk; ++bl)
-        cache_panel_epilogue<T, OutT>(p, Cb + bl * E, CW, w1lo, w1hi, 16 * m, (blk0 + bl) / p.nm,
-                                      (blk0 + bl) % p.nm, p.nkk);
+        cache_panel_epilogue<T, OutT>(p, Cb + bl * E, CW, w1lo, w1hi, sPan + e0, pan0 + e0, e1 - e0,
+                                      (blk0 + bl) / p.nm, (blk0 + bl) % p.nm);
     }
   }
 }
 
+// tiles: 16-point tiles of the phase table's rows; nJobs: grid rows.
 template <typename T, typename OutT>
-void launch_cache(const CacheParams& p0, hipStream_t s) {
-  CacheParams p = p0;
-  PHX_REQUIRE(p.nw <= 32, "cacheElPh kernel supports nw <= 32");
-  PHX_REQUIRE(p.nkk <= kCacheNKK, "cacheElPh kernel: too many outer points per launch");
-  if (p.nkk <= 0) return;
+static void launch_cache_gemm(CacheParams p, int tiles, int nJobs, hipStream_t s) {
   const CacheTiling c = cache_tiling(p.nw);
   p.blocks = c.blocks;
   p.w1Rows = c.w1Rows;
   p.wc = c.wc;
-  const size_t lds = size_t(4 / c.wc) * 32 * cache_row(c.wc, c.ntw) * sizeof(T);
+  PHX_REQUIRE(p.nb1Max >= 1 && p.nb1Max <= p.nw && p.ldb % 2 == 0, "cacheElPh kernel: bad band count or panel row");
+  const size_t lds = size_t(4 / c.wc) * 32 * cache_row(c.wc, c.ntw) * sizeof(T) +
+                     size_t(16) * tiles * p.nb1Max * sizeof(int2);
   auto go = [&](auto kern) {
     PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL(kern, dim3(ceil_div(p.nRp * p.nm, c.blocks)), dim3(256), lds, s, p);
+    hipLaunchKernelGGL(kern, dim3(ceil_div(p.nRp * p.nm, c.blocks), nJobs), dim3(256), lds, s, p);
   };
   auto ntw = [&](auto mh) {
     constexpr int MH = decltype(mh)::value;
@@ -515,9 +520,19 @@ void launch_cache(const CacheParams& p0, hipStream_t s) {
       default: go(k_cache<T, OutT, MH, 4>);
     }
   };
-  if (cache_phase_cols(p.nkk) == 16) ntw(std::integral_constant<int, 1>{});
-  else ntw(std::integral_constant<int, 2>{});
+  if (tiles == 1) ntw(std::integral_constant<int, 1>{});
+  else if (tiles == 2) ntw(std::integral_constant<int, 2>{});
+  else ntw(std::integral_constant<int, 3>{});
   PHX_HIP(hipGetLastError());
+}
+
+template <typename T, typename OutT>
+void launch_cache(const CacheParams& p, hipStream_t s) {
+  PHX_REQUIRE(p.nw <= 32, "cacheElPh kernel supports nw <= 32");
+  PHX_REQUIRE(p.nkk <= kCacheNKK, "cacheElPh kernel: too many outer points per launch");
+  PHX_REQUIRE(!p.jobs, "cacheElPh kernel: jobs belong to the line form");
+  if (p.nkk <= 0) return;
+  launch_cache_gemm<T, OutT>(p, cache_phase_cols(p.nkk) / 16, 1, s);
 }
 template void launch_cache<double, double>(const CacheParams&, hipStream_t);
 template void launch_cache<float, float>(const CacheParams&, hipStream_t);
@@ -529,8 +544,12 @@ template void launch_cache<float, float>(const CacheParams&, hipStream_t);
 // Stage a (one HBM stream over gW for up to kLinesPerBatch = 16 lines):
 //   Tg(l, g, c) = sum_{R_e in group g} e^{2 pi i (j1 n1/m1 + j2 n2/m2)}/de gW(R_e, c)
 // with groups of equal n0 mod m0 (about 2 * 10 + 1 of them for a 10^3 R_e grid).
-// Stage b (per outer point): g1(k1, c) = sum_g e^{2 pi i j0 n0(g)/m0} Tg(l(k1), g, c),
-// then the same U1 / s(k1, Rp) panel epilogue as k_cache.
+// Stage b (per outer point): g1(k1, c) = sum_g e^{2 pi i j0 n0(g)/m0} Tg(l(k1), g, c):
+// k_cache with the groups in the place of R_e and a job per up to 48 points of a
+// line, so its products run on the matrix cores too.  A line's 40 points take
+// three tiles in one job and Tg is read once; FMAs with the partial sums of all
+// groups in registers took 7.7 ms where this takes 5.6 (16 bands, 12 modes, 640 points,
+// 21 groups, FP32: 7.1 GB read); what is left is the rotation epilogue.
 constexpr int kLineDepth = 4;  // gW rows in flight per thread (16 bytes each)
 
 // NL lines, CPT adjacent columns per thread (one 16-byte load per R_e for
@@ -669,85 +688,6 @@ __global__ void __launch_bounds__(256, 4) k_cache_line_am(CacheParams p) {
   }
 }
 
-// One workgroup per (Rp, nu) block of nw^2 columns, in passes of 256 columns
-// and, per line, of 16 outer points.  With at most kLineGe R_e groups, a
-// thread's partial sums of the line (one per group) are loaded once, all at
-// once, into registers and serve every batch of 16 outer points; the batch's
-// factors e^{2 pi i j0 n0 / m0} are staged in LDS.
-constexpr int kLineGe = 32;
-
-template <typename T, typename OutT>
-__global__ void __launch_bounds__(256) k_cache_line_b(CacheParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  typedef typename Vec2<T>::type T2;
-  const int rp = blockIdx.x / p.nm, nu = blockIdx.x % p.nm;
-  const int E = p.nw * p.nw, t = threadIdx.x;
-  T* Cb = reinterpret_cast<T*>(smem);                                        // 2 x 16 x 256
-  T2* sw = reinterpret_cast<T2*>(smem + size_t(2) * 16 * 256 * sizeof(T));  // 16 x kLineGe
-  const T2* Tg = static_cast<const T2*>(p.Tg);
-  const bool inReg = p.nGe <= kLineGe;
-  for (int c0 = 0; c0 < E; c0 += cache_pass_cols(p.nw)) {
-    const int cl = c0 + t;
-    const bool ok = cl < E;
-    const size_t colg = (size_t(rp) * p.nm + nu) * E + cl;
-    for (int l = 0; l < p.nLinesB; ++l) {
-      const int kend = p.lineKK[l + 1];
-      T2 v[kLineGe];
-      if (inReg) {
-#pragma unroll
-        for (int g = 0; g < kLineGe; ++g)
-          v[g] = (ok && g < p.nGe) ? Tg[(size_t(l) * p.nGe + g) * p.N + colg] : T2{T(0), T(0)};
-      }
-      for (int kbase = p.lineKK[l]; kbase < kend; kbase += 16) {
-        T accr[16], acci[16];
-#pragma unroll
-        for (int kl = 0; kl < 16; ++kl) accr[kl] = acci[kl] = T(0);
-        if (inReg) {
-          __syncthreads();  // the previous batch's readers of sw are done
-          for (int i = t; i < 16 * p.nGe; i += 256) {
-            const int kl = i / p.nGe, g = i % p.nGe;
-            const double2 w = p.wLine[size_t(min(kbase + kl, kend - 1)) * p.nGe + g];
-            sw[kl * kLineGe + g] = T2{T(w.x), T(w.y)};
-          }
-          __syncthreads();
-#pragma unroll
-          for (int g = 0; g < kLineGe; ++g) {
-            if (g < p.nGe) {
-#pragma unroll
-              for (int kl = 0; kl < 16; ++kl) {
-                const T2 w = sw[kl * kLineGe + g];
-                accr[kl] += w.x * v[g].x - w.y * v[g].y;
-                acci[kl] += w.x * v[g].y + w.y * v[g].x;
-              }
-            }
-          }
-        } else {
-          for (int g = 0; g < p.nGe; ++g) {
-            const T2 vg = ok ? Tg[(size_t(l) * p.nGe + g) * p.N + colg] : T2{T(0), T(0)};
-#pragma unroll
-            for (int kl = 0; kl < 16; ++kl) {
-              const int kk = min(kbase + kl, kend - 1);
-              const double2 w = p.wLine[size_t(kk) * p.nGe + g];
-              const T wr = T(w.x), wi = T(w.y);
-              accr[kl] += wr * vg.x - wi * vg.y;
-              acci[kl] += wr * vg.y + wi * vg.x;
-            }
-          }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kl = 0; kl < 16; ++kl) {
-          Cb[kl * 256 + t] = accr[kl];
-          Cb[(16 + kl) * 256 + t] = acci[kl];
-        }
-        __syncthreads();
-        cache_panel_epilogue<T, OutT>(p, Cb, 256, c0 / p.nw, min(p.nw, (c0 + cache_pass_cols(p.nw)) / p.nw), kbase, rp,
-                                      nu, kend);
-      }
-    }
-  }
-}
-
 template <typename T, int NL>
 static void launch_line_a(const CacheParams& p, hipStream_t s) {
   if constexpr (sizeof(T) == 4 && NL == 16) {
@@ -782,6 +722,8 @@ void launch_cache_line(const CacheParams& p, hipStream_t s) {
   PHX_REQUIRE(p.nGe >= 1 && p.N == size_t(p.nRp) * p.nm * p.nw * p.nw, "cacheElPh line: bad sizes");
   PHX_REQUIRE(p.nLinesB >= 1 && p.nLinesB <= kLinesPerBatch && p.nLinesA == line_count_padded(p.nLinesB),
               "cacheElPh line: 1 to 16 lines per batch");
+  PHX_REQUIRE(p.jobs && p.nJobs >= 1 && p.jobTiles >= 1 && p.jobTiles <= kJobTiles,
+              "cacheElPh line: bad stage b jobs");
   if (p.nkk <= 0) return;
   switch (p.nLinesA) {
     case 1: launch_line_a<T, 1>(p, s); break;
@@ -793,12 +735,7 @@ void launch_cache_line(const CacheParams& p, hipStream_t s) {
     case 12: launch_line_a<T, 12>(p, s); break;
     default: launch_line_a<T, 16>(p, s); break;
   }
-  const size_t lds = size_t(2) * 16 * 256 * sizeof(T) + size_t(16) * kLineGe * 2 * sizeof(T);
-  auto kb = k_cache_line_b<T, OutT>;
-  PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kb),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-  hipLaunchKernelGGL(kb, dim3(p.nRp * p.nm), dim3(256), lds, s, p);
-  PHX_HIP(hipGetLastError());
+  launch_cache_gemm<T, OutT>(p, p.jobTiles, p.nJobs, s);  // stage b
 }
 template void launch_cache_line<double, double>(const CacheParams&, hipStream_t);
 template void launch_cache_line<float, float>(const CacheParams&, hipStream_t);

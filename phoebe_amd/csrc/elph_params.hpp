@@ -13,6 +13,7 @@ constexpr int kCMax = 4;       // largest number of (T, mu) calculations
 constexpr int kCacheNKK = 32;  // outer points per GEMM cacheElPh launch
 constexpr int kLinesPerBatch = 16;   // mesh lines per line-form cacheElPh launch
 constexpr int kLinePointsMax = 1024; // outer points per line-form batch
+constexpr int kJobTiles = 3;         // 16-point tiles per job of the line form's second stage
 
 // Line counts k_cache_line_a is instantiated for; a batch's count is rounded
 // up to the next one (the extra lines have zero phases and are never read).
@@ -38,10 +39,12 @@ struct CacheParams {
   const double2* U1pool;  // per kk: (nw, nb1) column-major
   const int* U1off;       // complex offset per kk
   const int* nb1;         // per kk
-  const int* panelBase;   // first panel of kk
+  int nb1Max;             // largest nb1 of the batch
+  const int* panelBase;   // first panel of kk; the panels of consecutive points follow each other
   void* B;                // panels
   size_t panelStride;     // elements
-  int ldb;                // elements per panel row
+  int ldb;                // elements per panel row (a multiple of 16)
+  int evenRows;           // write the panels' rows 2 Rp (C) only: the mesh-separable transform reads no others
   // outer points on one mesh line (k_cache_line_a / k_cache_line_b)
   size_t N;               // gW columns: nRp * nm * nw^2
   int nGe;                // R_e groups: distinct n0(R_e) mod m0
@@ -53,10 +56,13 @@ struct CacheParams {
   const int* reBlkEnd;    // nRePad / 4: group index if the 4-entry block ends its group, else -1
   int nLinesB;            // lines of the batch (<= kLinesPerBatch)
   int nLinesA;            // lines stage a computes: line_count_padded(nLinesB), rows of phLine and Tg
-  const int* lineKK;      // nLinesB + 1: first outer point of each line (points grouped by line)
   const void* phLine;     // (nRe, nLinesA) complex T: e^{2 pi i (j1 n1/m1 + j2 n2/m2)} / de
   void* Tg;               // (nLinesA, nGe, N) complex T: partial sums of the lines
-  const double2* wLine;   // (nkk, nGe): e^{2 pi i j0(kk) n0(g) / m0}
+  // stage b: job j sums the nGe groups of line jobs[j].z for the outer points jobs[j].x ..
+  // jobs[j].x + jobs[j].y - 1 (at most 16 jobTiles of one line), with phE as the
+  // (job, nGe rounded up to quads, 16 jobTiles) table of e^{2 pi i j0(kk) n0(g) / m0}
+  const int4* jobs;
+  int nJobs, jobTiles;
 };
 
 // Deterministic sum of the per-tile partial linewidths of one batch.

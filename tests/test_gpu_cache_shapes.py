@@ -52,3 +52,19 @@ def test_batches_equal_single_points(nw, count, precision, tol):
     m = a != 0
     assert m.any() and np.array_equal(m, b != 0)
     assert np.abs(b[m] / a[m] - 1).max() <= tol
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("fp32", 2e-6)])
+@pytest.mark.parametrize("mesh,nw", [((16, 2, 2), 9), ((17, 2, 2), 6), ((33, 2, 2), 6), ((52, 2, 1), 6), ((20, 2, 2), 17)])
+def test_line_jobs_equal_gemm_batches(mesh, nw, precision, tol):
+    """Mesh lines of 16 to 52 points: one, two or three tiles per job, several jobs per line."""
+    prob = synth.make_problem(1, nw, 3, 3, mesh, seed=80 + nw, window_ev=3.0)
+    gemm = P.ElectronLinewidths(prob, precision=precision, transform="separable" if nw < 17 else "direct")
+    gemm.run()
+    line = P.ElectronLinewidths(prob, precision=precision, transform="separable" if nw < 17 else "direct")
+    line.set_line_batching(1)
+    line.run()
+    a, b = gemm.linewidths(average=False), line.linewidths(average=False)
+    m = a != 0
+    assert m.any() and np.array_equal(m, b != 0)
+    assert np.abs(b[m] / a[m] - 1).max() <= tol
