@@ -119,14 +119,16 @@ def roofline(res, form, workload):
             pairs = st["rows"] / nb1 / n
             # with the y-stage inside the x-stage kernel (k_sep_yx) it reads T1 instead of the slabs
             xk = "k_sep_yx" if sp.get("fused_y") else "k_sep_xg"
+            # the committed traffic figures are of the FP32 kernels
+            traffic = lambda k: traffic_per_dispatch(k, workload) if precision == "fp32" else None
             xg = {"kernel": xk, "avg_launch_ms": round(t_xg * 1e3, 4), "bytes_per_launch": xg_bytes,
                   "achieved_GBps": round(xg_bytes / t_xg / 1e9, 1),
                   "frac": round(xg_bytes / t_xg / 1e9 / HBM_PEAK_GBS, 4),
-                  "traffic": traffic_per_dispatch(xk, workload),
+                  "traffic": traffic(xk),
                   "mfma_TFLOPs": round(st["flops"] / n / t_xg / 1e12, 3)}
             ep = {"kernel": "k_sep_ep2", "avg_launch_ms": round(t_ep * 1e3, 4), "bytes_per_launch": g3,
                   "achieved_GBps": round(g3 / t_ep / 1e9, 1), "frac": round(g3 / t_ep / 1e9 / HBM_PEAK_GBS, 4),
-                  "traffic": traffic_per_dispatch("k_sep_ep2", workload),
+                  "traffic": traffic("k_sep_ep2"),
                   "pair_bytes": round(pair_bytes, 1), "pairs_per_launch": pairs,
                   "frac_pair_bytes": round(pair_bytes * pairs / t_ep / 1e9 / HBM_PEAK_GBS, 4)}
             dom = xg if t_xg >= t_ep else ep

@@ -457,22 +457,21 @@ int phx_lw_set_line_batching(phx_lw* h, int min_points);
 int phx_lw_set_panel_chunk(phx_lw* h, int panels);
 /* Last stage of the separable transform as two kernels (on, the default) or
  * one fused kernel (off).  Split: an x-stage kernel writes the kept rows' g3
- * to device memory, (panel chunk) x (y, z lines) x m0 x nm nw complex FP32,
+ * to device memory, (panel chunk) x (y, z lines) x m0 x nm nw complex,
  * and an epilogue kernel reads them; both use far fewer registers and LDS
  * than the fused kernel, so more workgroups hide the memory latency.  Applies
- * to PHX_FP32 with nm, nw <= 16, nm nw <= 192, an x mesh <= 64 and at most 24
- * x-groups; elsewhere the fused kernel runs.  The g3 values are the same
- * either way and the linewidths agree to FP64 rounding.
- * on = 1 (default) runs the lean epilogue kernel where it applies (fixed
- * Gaussian smearing, at most 8 bands per inner point; it also takes the
- * learned screen's slot masks), on = 2 the first epilogue kernel always;
- * both give the same linewidths.  on = 3 moves the electron rotation
+ * to PHX_FP64 and PHX_FP32 with nm <= 32, nw <= 16, an x mesh <= 64, at most
+ * 24 x-groups and room for the g3 rows; with the fused y-stage off, the learned
+ * screen or on = 3 only to PHX_FP32 with nm <= 16 and nm nw <= 192; elsewhere
+ * the fused kernel runs.  The g3 values are the same either way and the
+ * linewidths agree to FP64 rounding.  on = 2 is the same as on = 1 (the
+ * default).  on = 3 moves the electron rotation
  * g'(nu, b2) = sum_w2 conj(U2(w2, b2)) g3(nu, w2) (FP64, the epilogue's own
  * arithmetic on the same FP32 g3) into the x-stage kernel, which writes g'
  * (nb2 x nm complex FP64 per kept row, slot rows of nb2max x nm) instead of
- * g3, and the lean epilogue starts from g'; where the lean epilogue does not
- * apply it runs as on = 1.  The linewidths agree with on = 1 to FP64
- * rounding.  No counterpart in the reference. */
+ * g3, and the epilogue starts from g'; with adaptive smearing it runs as
+ * on = 1.  The linewidths agree with on = 1 to FP64 rounding.  No counterpart
+ * in the reference. */
 int phx_lw_set_split_last_stage(phx_lw* h, int on);
 /* Split last stage: run the epilogue kernel of each panel chunk on a second
  * stream of the handle, concurrently with the next chunk's transform stages
@@ -482,7 +481,7 @@ int phx_lw_set_split_last_stage(phx_lw* h, int on);
  * in turn.  The linewidths are the same either way.  Takes effect for batches
  * prepared after the call.  No counterpart in the reference. */
 int phx_lw_set_epilogue_overlap(phx_lw* h, int on);
-/* Split last stage, PHX_FP32 without the learned screen: run the y-stage of
+/* Split last stage without the learned screen: run the y-stage of
  * the separable transform inside the x-stage kernel (on = 1, the default),
  * so that the x-stage slabs T2 stay in LDS instead of going through device
  * memory, or as its own kernel (on = 0).  Not with split mode 3.  The g3

@@ -700,10 +700,9 @@ class ElectronLinewidths:
         _check(lib().phx_lw_set_panel_chunk(self._h, int(panels)))
 
     def set_split_last_stage(self, on=True):
-        """Separable last stage as two kernels (default) or the fused one;
-        on=2 runs the split stage with the first epilogue kernel, on=3 with
-        the electron rotation in the x-stage kernel (g' through device memory
-        instead of g3)."""
+        """Separable last stage as two kernels (default; on=2 is the same) or
+        the fused one; on=3 runs the split stage with the electron rotation in
+        the x-stage kernel (g' through device memory instead of g3)."""
         _check(lib().phx_lw_set_split_last_stage(self._h, on if on in (2, 3) else int(bool(on))))
 
     def set_epilogue_overlap(self, on=True):
@@ -713,7 +712,7 @@ class ElectronLinewidths:
         _check(lib().phx_lw_set_epilogue_overlap(self._h, int(bool(on))))
 
     def set_fused_y_stage(self, on=True):
-        """FP32 split stage: the y-stage inside the x-stage kernel (default) or its own kernel."""
+        """Split stage: the y-stage inside the x-stage kernel (default) or its own kernel."""
         _check(lib().phx_lw_set_fused_y_stage(self._h, int(bool(on))))
 
     def last_stage_fused_y(self):

@@ -62,12 +62,8 @@ void launch_scatter_ph(int nq, int nm, const int* iq, const double* w, const dou
 // coupling_f64.hip and coupling_f32.hip)
 extern template void launch_coupling<double>(const CoupParams&, bool, hipStream_t);
 extern template void launch_coupling<float>(const CoupParams&, bool, hipStream_t);
-extern template void launch_separable<double>(const SepParams&, const CoupParams&, bool, int, int,
-                                              hipStream_t);
-extern template void launch_separable<float>(const SepParams&, const CoupParams&, bool, int, int,
-                                             hipStream_t);
-extern template void launch_separable_zy<double>(const SepParams&, int, int, hipStream_t, bool);
-extern template void launch_separable_zy<float>(const SepParams&, int, int, hipStream_t, bool);
+extern template void launch_separable_zy<double>(const SepParams&, int, hipStream_t, bool);
+extern template void launch_separable_zy<float>(const SepParams&, int, hipStream_t, bool);
 extern template bool launch_separable_x<double>(const SepParams&, const CoupParams&, bool, hipStream_t, hipEvent_t,
                                                   const EpFork&);
 extern template bool launch_separable_x<float>(const SepParams&, const CoupParams&, bool, hipStream_t, hipEvent_t,
@@ -780,7 +776,11 @@ struct LwHandle {
   // separable mesh transform of the R_ph sum (transform == PHX_TRANSFORM_SEPARABLE)
   int transform = 0;
   int nLines = 0, nG0 = 0, maxLineE = 0, maxGrpE = 0;
-  DevBuf<int> lineStart, lineF2, lineRp, grpStart, grpF1, grpLine, g0val, meshToRow;
+  DevBuf<int> lineStart, lineF2, lineRp, g0val, meshToRow;
+  // y-stage: the x-groups' lines in quads, dealt to four waves (SepParams)
+  int nQuads = 0, waveQ[5] = {0, 0, 0, 0, 0};
+  DevBuf<int2> quadEnt;
+  DevBuf<int> quadEnd;
   DevBuf<double2> twx, twy, twz;
   DevBuf<double> T1d, T2d;
   DevBuf<float> T1f, T2f;
@@ -788,14 +788,14 @@ struct LwHandle {
   // batched together when the line holds at least lineMin of them (0 = off)
   int lineMin = 0;
   int panelChunk = 0;      // panels per separable-transform launch (bounds T1 / T2 / g3); 0 = automatic
-  int splitLast = 1;       // last stage as k_sep_xg + epilogue where they apply (2: the first epilogue,
-                           // k_sep_ep; 3: the electron rotation in k_sep_xg, g' rows through HBM)
+  int splitLast = 1;       // last stage as x-stage and epilogue kernels where they apply (2: the same;
+                           // 3: the electron rotation in k_sep_xg, g' rows through HBM)
   DevBuf<float2> G3f;      // their g3 rows of one panel chunk, (slot, jx, col), or g' rows (slot, jx, b2, nu)
   // the split stage's epilogue of chunk i on streamEp, overlapping chunk i + 1's
   // transform stages on `stream`: chunks alternate between two sets of g3 rows
   // and row masks; epEv holds two events per chunk (x-stage done, epilogue done)
   int epOverlap = 0;
-  // FP32 split stage: the y-stage inside the x-stage kernel (k_sep_yx), no T2 in HBM
+  // split stage: the y-stage inside the x-stage kernel (k_sep_yx), no T2 in HBM
   int fuseYX = 1;
   double yxT1Bytes = 0.;   // timed launches of k_sep_yx: T1 bytes they read
   long long yxLaunches = 0;
@@ -873,14 +873,34 @@ struct LwHandle {
   }
 };
 
+// Whether the x-stage of the split last stage runs with the y-stage inside it
+// (k_sep_yx: any width, FP32 and FP64): not with the learned screen's slot masks
+// or the rotating x-stage.
+static bool lw_fused_y(const LwHandle* L, const phx_problem& p) {
+  const bool learned = L->lsCollect || (L->lsMode && L->mlpTrained);
+  return L->fuseYX && !learned && L->splitLast != 3 && L->nG0 <= 24 &&
+         sep_yx_lds_bytes(L->precision == PHX_FP64 ? 8 : 4, L->nQuads, p.mesh[1], L->nG0, p.mesh[0]) <= 160 * 1024;
+}
+
 // Whether the separable transform's last stage runs split (x-stage and
-// epilogue as two kernels, g3 rows through HBM): FP32 data, nm, nw <= 16,
-// nm nw <= 192, row masks (x mesh <= 64); the launcher also needs <= 24
-// x-groups (and, with the learned screen, the lean epilogue), and falls back
-// to the fused kernel otherwise.
+// epilogue as two kernels, g3 rows through HBM): nw <= 16, row masks (x mesh <=
+// 64) and an x-stage kernel for the sizes: k_sep_yx, or k_sep_xg (FP32, nm <=
+// 16, nm nw <= 192).  The launcher falls back to the fused kernel where it
+// cannot run split.  Two kernels write and read g3 but hide their latency at 2
+// to 4 waves per SIMD, where the fused one runs at 1 or 2: with 18 modes x 16
+// bands in FP32 on a 32^3 mesh 7.2 against 21.8 ms per pass, 12 x 16 in FP64 on
+// a 27 x 28 x 29 mesh 6.3 against 21.2.
 static bool lw_split_last(const LwHandle* L, const phx_problem& p) {
-  return L->splitLast && L->transform == PHX_TRANSFORM_SEPARABLE && L->precision == PHX_FP32 && p.nm <= 16 &&
-         p.nw <= 16 && p.nm * p.nw <= 192 && p.mesh[0] <= 64;
+  const bool xg = L->precision == PHX_FP32 && p.nm <= 16 && p.nm * p.nw <= 192;
+  return L->splitLast && L->transform == PHX_TRANSFORM_SEPARABLE && L->precision != PHX_BF16X3 && p.nw <= 16 &&
+         p.mesh[0] <= 64 && (xg || lw_fused_y(L, p));
+}
+
+// float2 values per panel of a chunk's g3 rows: nm nw complex values of the
+// transform's precision per mesh point, or nb2max nm complex FP64 (g').
+static size_t lw_g3_per_panel(const LwHandle* L, const phx_problem& p, int nb2max) {
+  const size_t ncol = size_t(p.nm) * p.nw * (L->precision == PHX_FP64 ? 2 : 1);
+  return size_t(p.mesh[0]) * p.mesh[1] * p.mesh[2] * std::max(ncol, size_t(2) * nb2max * p.nm);
 }
 
 // Panels per separable-transform launch: the handle's setting, or (0) as many
@@ -890,9 +910,7 @@ static bool lw_split_last(const LwHandle* L, const phx_problem& p) {
 constexpr double kChunkG3Bytes = 24. * (1ull << 30);
 static int lw_panel_chunk(const LwHandle* L, const phx_problem& p, int nPanels, int nb2max) {
   if (L->panelChunk > 0) return std::min(nPanels, L->panelChunk);
-  const double ncol = double(p.nm) * p.nw;
-  const double perPanel =
-      double(p.mesh[1]) * p.mesh[2] * p.mesh[0] * std::max(ncol, 2. * nb2max * p.nm) * sizeof(float2);
+  const double perPanel = double(lw_g3_per_panel(L, p, nb2max)) * sizeof(float2);
   const int c = int(std::min(128., std::max(16., std::floor(kChunkG3Bytes / perPanel))));
   return std::max(1, std::min(nPanels, c));
 }
@@ -1278,7 +1296,7 @@ static void lw_setup(LwHandle* L, const phx_problem* P, int precision, int k1Bat
       }
       grpE[grpOf[f0]].push_back(int(l));
     }
-    std::vector<int> ls{0}, lf2, lrp, gs{0}, gf1, gl;
+    std::vector<int> ls{0}, lf2, lrp;
     for (auto& e : lineE) {
       for (int r : e) {
         lf2.push_back(f[3 * r + 2]);
@@ -1287,14 +1305,30 @@ static void lw_setup(LwHandle* L, const phx_problem* P, int precision, int k1Bat
       ls.push_back(int(lrp.size()));
       L->maxLineE = std::max(L->maxLineE, int(e.size()));
     }
-    for (auto& e : grpE) {
-      for (int l : e) {
-        gf1.push_back(lineKey[l] / m[0]);
-        gl.push_back(l);
-      }
-      gs.push_back(int(gl.size()));
-      L->maxGrpE = std::max(L->maxGrpE, int(e.size()));
+    for (auto& e : grpE) L->maxGrpE = std::max(L->maxGrpE, int(e.size()));
+    // the y-stage's quads: each group to the wave with the fewest quads so far,
+    // the largest groups first
+    std::vector<int> byGrp(grpE.size());
+    std::iota(byGrp.begin(), byGrp.end(), 0);
+    std::stable_sort(byGrp.begin(), byGrp.end(), [&](int x, int y) { return grpE[x].size() > grpE[y].size(); });
+    std::vector<int> waveGrp[4], waveN(4, 0);
+    for (int g : byGrp) {
+      const int w = int(std::min_element(waveN.begin(), waveN.end()) - waveN.begin());
+      waveGrp[w].push_back(g);
+      waveN[w] += ceil_div((long long)grpE[g].size(), 4);
     }
+    std::vector<int2> qent;
+    std::vector<int> qend;
+    for (int w = 0; w < 4; ++w) {
+      for (int g : waveGrp[w]) {
+        for (int l : grpE[g]) qent.push_back(make_int2(l, lineKey[l] / m[0]));
+        while (qent.size() % 4) qent.push_back(make_int2(-1, 0));
+        qend.resize(qent.size() / 4, -1);
+        qend.back() = g;
+      }
+      L->waveQ[w + 1] = int(qend.size());
+    }
+    L->nQuads = int(qend.size());
     L->nLines = int(lineE.size());
     L->nG0 = int(grpE.size());
     {
@@ -1312,9 +1346,8 @@ static void lw_setup(LwHandle* L, const phx_problem* P, int precision, int k1Bat
     h2d(L->lineStart, ls, s);
     h2d(L->lineF2, lf2, s);
     h2d(L->lineRp, lrp, s);
-    h2d(L->grpStart, gs, s);
-    h2d(L->grpF1, gf1, s);
-    h2d(L->grpLine, gl, s);
+    h2d(L->quadEnt, qent, s);
+    h2d(L->quadEnd, qend, s);
     h2d(L->g0val, g0v, s);
     auto tw = [&](DevBuf<double2>& d, int n) {
       std::vector<double2> v(n);
@@ -1691,9 +1724,14 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
       L->xminPart.reserve(size_t(chunk) * kXminBlocks);
     }
     if (lw_split_last(L, p)) {  // g3 (complex FP32) or g' (complex FP64, nb2max nm per row)
-      const size_t g3 = slots * p.mesh[0] * std::max(ncol, size_t(2) * b.nb2max * nm);
-      L->G3f.reserve(g3);
-      if (L->epOverlap && p.mesh[0] <= 64) {
+      const size_t g3 = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
+      try {
+        L->G3f.reserve(g3);
+      } catch (const Error&) {  // no room for the g3 rows: the fused kernel runs, which needs none
+        (void)hipGetLastError();
+        L->G3f.release();
+      }
+      if (L->epOverlap && L->G3f.p) {
         L->G3f2.reserve(g3);
         L->keepMask2.reserve(slots);
       }
@@ -1898,9 +1936,10 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     sp.twz = L->twz.p;
     sp.t1PanelStride = size_t(L->nLines) * mz * ncol * 2;
     sp.nG0 = L->nG0;
-    sp.grpStart = L->grpStart.p;
-    sp.grpF1 = L->grpF1.p;
-    sp.grpLine = L->grpLine.p;
+    sp.nQuads = L->nQuads;
+    std::copy(L->waveQ, L->waveQ + 5, sp.waveQ);
+    sp.quadEnt = L->quadEnt.p;
+    sp.quadEnd = L->quadEnd.p;
     sp.twy = L->twy.p;
     sp.t2PanelStride = size_t(L->nG0) * my * mz * ncol * 2;
     // rows are addressed by active index: no k2 offset, range through rowLo/rowHi
@@ -1928,7 +1967,6 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     if (p.mesh[0] <= 64) cq.keepMask = L->keepMask.p;
     if (lw_split_last(L, p)) {
       cq.G3 = L->G3f.p;
-      cq.epFirst = L->splitLast == 2;
       cq.epRot = L->splitLast == 3;
     }
     // panels in chunks: the stage buffers T1 / T2 hold one chunk
@@ -1948,13 +1986,11 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     // g3 / g' rows of one chunk (what the batch's preparation reserved, unless a
     // setting changed since: then the fused kernel runs, or the chunks run in turn)
     const size_t slotsC = size_t(chunk) * nMtiles;
-    const size_t g3Need = slotsC * mx * std::max(size_t(ncol), size_t(2) * b.nb2max * nm);
+    const size_t g3Need = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
     const bool splitOk = lw_split_last(L, p) && L->G3f.n >= g3Need;
     const bool overlap = L->epOverlap && !learned && splitOk && L->G3f2.n >= g3Need &&
                          L->keepMask2.n >= slotsC;
-    // the y-stage inside the x-stage kernel: FP32 split stage without slot masks
-    const bool yx = L->fuseYX && splitOk && !learned && L->precision == PHX_FP32 && L->splitLast != 3 &&
-                    L->nG0 <= 24 && sep_yx_lds_bytes(L->nLines, L->nG0, mx) <= 160 * 1024;
+    const bool yx = splitOk && lw_fused_y(L, p);  // the y-stage inside the x-stage kernel
     cq.fuseYX = yx;
     const int nChunks = (nPanels + chunk - 1) / chunk;
     if (overlap) {
@@ -2010,7 +2046,7 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
                                : launch_separable_x<float>(sp, c, true, s, mid, fork);
         const bool forked = split && fork.ep;
         if (L->timing && split && c.fuseYX) {
-          L->yxT1Bytes += double(sp.nPanels) * mz * L->nLines * ncol * 8.;
+          L->yxT1Bytes += double(sp.nPanels) * mz * L->nLines * ncol * (f64 ? 16. : 8.);
           L->yxLaunches += 1;
         }
         if (forked) {
@@ -2024,8 +2060,9 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
           L->xevSplit.push_back(split ? 1 : 0);
         }
       };
-      if (f64) launch_separable_zy<double>(sp, L->maxLineE, L->maxGrpE, s, true);
-      else launch_separable_zy<float>(sp, L->maxLineE, L->maxGrpE, s, !yx);
+      sp.modeFast = (f64 ? sep_runs_split<double>(sp, cq) : sep_runs_split<float>(sp, cq)) ? nm : 0;
+      if (f64) launch_separable_zy<double>(sp, L->maxLineE, s, !yx);
+      else launch_separable_zy<float>(sp, L->maxLineE, s, !yx);
       if (!learned) {
         // this chunk rewrites set `set`: the epilogue of chunk ci - 2 must have read it
         if (epPending[set]) PHX_HIP(hipStreamWaitEvent(s, L->epEv[2 * (ci - 2) + 1], 0));
@@ -3967,9 +4004,9 @@ int phx_lw_last_stage_split_bytes(phx_lw* h, double* out2) {
     if (h->xSlots.p) PHX_HIP(hipMemcpy(&slots, h->xSlots.p, sizeof(slots), hipMemcpyDeviceToHost));
     if (h->xKept.p) PHX_HIP(hipMemcpy(&rows, h->xKept.p, sizeof(rows), hipMemcpyDeviceToHost));
     if (h->xBands.p) PHX_HIP(hipMemcpy(&bands, h->xBands.p, sizeof(bands), hipMemcpyDeviceToHost));
-    // complex FP32: the x-stage reads nG0 x (nm nw) per slot and writes nm nw per kept row;
+    // complex values: the x-stage reads nG0 x (nm nw) per slot and writes nm nw per kept row;
     // with the y-stage inside (k_sep_yx) it reads T1 instead of the slabs (slots not counted)
-    const double row = 8. * h->nm * h->nw;
+    const double row = (h->precision == PHX_FP64 ? 16. : 8.) * h->nm * h->nw;
     out2[0] = double(slots) * h->nG0 * row + h->yxT1Bytes;
     out2[1] = h->splitLaunches > 0 ? double(rows) * row : 0.;
     if (h->splitLast == 3 && h->splitLaunches > 0) {

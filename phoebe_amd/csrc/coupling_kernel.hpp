@@ -56,7 +56,6 @@ struct CoupParams {
   const double* bose;                     // (q, nu, calc)
   int nCalc; double invSigma, deltaPref, norm, cutoff;
   int gsizeMax;                           // largest panelGSize of the launch (0: unknown, kGMax)
-  int epRows;                             // k_sep_ep: rows per pass, waves x (rows per wave), rows per wave <= 64 / nm
   double* partial;                        // (L = panel*nMtiles + mtile, kGMax, kCMax)
   int nb2max;
   // separable mesh transform
@@ -97,10 +96,9 @@ struct CoupParams {
   const double2* polarX;
   const double2* U1pool;
   const int* U1off;
-  // split last stage (k_sep_xg + k_sep_ep): g3 rows of the chunk, (slot, jx, col) complex T
+  // split last stage (k_sep_yx or k_sep_xg, then k_sep_ep2): g3 rows of the chunk, (slot, jx, col) complex T
   void* G3;
-  unsigned long long* keptBands;          // k_sep_ep: sum of nb2 over the rows it computed (null: off)
-  int epFirst;                            // split epilogue: 1 = k_sep_ep, 0 = k_sep_ep2 where it applies
+  unsigned long long* keptBands;          // k_sep_ep2: sum of nb2 over the rows it computed (null: off)
   int epRot;                              // k_sep_xg also does the electron rotation (g' to HBM, not g3)
   int fuseYX;                             // the y-stage runs inside the x-stage kernel (k_sep_yx; no T2 in HBM)
   unsigned long long* keptSlots;          // k_sep_xg: slots (panel, yz line) it computed (null: off)
@@ -677,15 +675,20 @@ void launch_coupling(const CoupParams& p, bool reduce, hipStream_t s) {
 struct SepParams {
   const void* B; size_t panelStride; int ldb;   // panels: C(Rp, col) in row 2 Rp
   int ncol, nPanels, mx, my, mz;
+  int modeFast;                                 // nm: columns of T1 / T2 / g3 as (w2, nu); 0: as the panels, (nu, w2)
   int nLines; const int* lineStart; const int* lineF2; const int* lineRp;
   const double2* twz;                           // e^{2 pi i t / mz}
   void* T1; size_t t1PanelStride;               // (panel, line, jz, col)
-  int nG0; const int* grpStart; const int* grpF1; const int* grpLine;
+  int nG0;
+  // the groups' entries in quads (the last one padded), the groups dealt to four waves: wave w sums
+  // quads waveQ[w] .. waveQ[w + 1] - 1; entry (line, f1), line -1 = padding; quadEnd: group that ends
+  // with the quad, or -1
+  int nQuads; int waveQ[5]; const int2* quadEnt; const int* quadEnd;
   const double2* twy;                           // e^{2 pi i t / my}
   void* T2; size_t t2PanelStride;               // (panel, group, jy, jz, col)
 };
 
-// Register-blocked short transform shared by k_sep_z and k_sep_y:
+// Register-blocked short transform of k_sep_z:
 // out(j, c) = sum_e W(e, j) X(e, c) for j < m, c < ncol, X (the data's
 // precision, converted to FP64 on reading) and W in LDS.
 // Thread (wave w, lane l) takes the columns c = l, l + 64, ... and the rows
@@ -729,9 +732,10 @@ __device__ __forceinline__ void sep_short_transform(const typename Vec2<T>::type
 // j < m.  The rows' offsets and the f(e) are staged first (off, fe: ne ints
 // each); every thread then keeps up to 8 row loads in flight before its LDS
 // stores, so a workgroup waits about one memory latency, not one per entry.
+// nm > 0: column c = nu (ncol / nm) + w2 goes to w2 nm + nu.
 template <typename T2v, typename Meta>
 __device__ __forceinline__ void sep_stage_entries(const T2v* base, T2v* X, double2* W, int* off, int* fe, int ne,
-                                                  int ncol, int m, const double2* tw, Meta meta) {
+                                                  int ncol, int m, int nm, const double2* tw, Meta meta) {
   const int t = threadIdx.x, bs = blockDim.x;
   for (int e = t; e < ne; e += bs) meta(e, off[e], fe[e]);
   __syncthreads();
@@ -749,7 +753,14 @@ __device__ __forceinline__ void sep_stage_entries(const T2v* base, T2v* X, doubl
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int i = i0 + bs * u;
-      if (i < n) X[i] = v[u];
+      if (i < n) {
+        int d = i;
+        if (nm > 0) {
+          const int e = i / ncol, c = i - e * ncol, nw = ncol / nm, nu = c / nw;
+          d = e * ncol + (c - nu * nw) * nm + nu;
+        }
+        X[d] = v[u];
+      }
     }
   }
   for (int i = t; i < ne * m; i += bs) {
@@ -759,7 +770,7 @@ __device__ __forceinline__ void sep_stage_entries(const T2v* base, T2v* X, doubl
   __syncthreads();
 }
 
-// LDS of k_sep_z / k_sep_y for ne entries: X (ne x ncol in the data's
+// LDS of k_sep_z for ne entries: X (ne x ncol in the data's
 // precision), W (ne x m complex FP64), the entries' row offsets and factors.
 inline size_t sep_stage_lds_bytes(int elem, int ne, int ncol, int m) {
   const size_t x = (size_t(ne) * ncol * 2 * elem + 15) / 16 * 16;
@@ -768,6 +779,9 @@ inline size_t sep_stage_lds_bytes(int elem, int ne, int ncol, int m) {
 
 // T1(line, jz, c) = sum_{(f2, Rp) in line} w_z^{jz f2} C(Rp, c).  The line's
 // entries and their twiddles w_z^{jz f2} (an entries x mz table) sit in LDS.
+// The panels' columns are (nu, w2); with modeFast the staging turns them into
+// (w2, nu) for the split last stage, whose epilogue reads them with the modes in
+// neighbouring lanes.
 template <typename T>
 __global__ void __launch_bounds__(256) k_sep_z(SepParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -781,7 +795,7 @@ __global__ void __launch_bounds__(256) k_sep_z(SepParams p) {
   int* fe = off + ne;
   // C(Rp, c): row 2 Rp of the panel, complex entries (re, im) at 2c, 2c + 1
   const T2v* B = reinterpret_cast<const T2v*>(static_cast<const T*>(p.B) + size_t(panel) * p.panelStride);
-  sep_stage_entries(B, X, W, off, fe, ne, ncol, mz, p.twz, [&](int e, int& o, int& f) {
+  sep_stage_entries(B, X, W, off, fe, ne, ncol, mz, p.modeFast, p.twz, [&](int e, int& o, int& f) {
     o = p.lineRp[e0 + e] * p.ldb;  // row 2 Rp: 2 Rp ldb elements of T = Rp ldb complex
     f = p.lineF2[e0 + e];
   });
@@ -792,28 +806,114 @@ __global__ void __launch_bounds__(256) k_sep_z(SepParams p) {
   });
 }
 
-// T2(group, jy, jz, c) = sum_{(f1, line) in group} w_y^{jy f1} T1(line, jz, c)
-// (entries and twiddles in LDS as in k_sep_z)
+// ------------------------------------------------------------------ y-stage on the matrix cores
+// T2(g, jy, c) = sum_{(f1, line) in group g} w_y^{jy f1} T1(line, jz, c) for 16
+// y coordinates and 16 columns at once on v_mfma_f64_16x16x4: M = jy, N =
+// columns, K = a quad of the group's entries, whose real and imaginary parts
+// take two products per accumulator (Re += Wr x, Re += (-Wi) y, Im += Wi x,
+// Im += Wr y).  The groups are dealt to the four waves by the host (waveQ), so
+// a group's sum stays in one wave's registers, in ascending order of its
+// entries; T1 goes from L2 straight to registers, four quads ahead.  FP64 sums
+// of the data's precision, rounded once on storing.
+// Shared by k_sep_y and k_sep_yx, which so give the same T2 bit for bit.
+struct SepYShared {
+  double2* tw;  // my: e^{2 pi i t / my}
+  int2* ent;    // 4 nQuads: (T1 row at jz: offset of its first column, or -1: padding; f1)
+  int* end;     // nQuads: group that ends with the quad, or -1
+};
+__host__ __device__ inline size_t sep_y_lds_bytes(int my, int nQuads) {
+  return size_t(my) * sizeof(double2) + size_t(4) * nQuads * sizeof(int2) +
+         (size_t(nQuads) * sizeof(int) + 15) / 16 * 16;
+}
+__device__ __forceinline__ SepYShared sep_y_stage(const SepParams& p, unsigned char* smem, int jz) {
+  SepYShared s;
+  s.tw = reinterpret_cast<double2*>(smem);
+  s.ent = reinterpret_cast<int2*>(s.tw + p.my);
+  s.end = reinterpret_cast<int*>(s.ent + 4 * p.nQuads);
+  for (int i = threadIdx.x; i < p.my; i += 256) s.tw[i] = p.twy[i];
+  for (int i = threadIdx.x; i < 4 * p.nQuads; i += 256) {
+    const int2 e = p.quadEnt[i];
+    s.ent[i] = make_int2(e.x < 0 ? -1 : (e.x * p.mz + jz) * p.ncol, e.y);
+  }
+  for (int i = threadIdx.x; i < p.nQuads; i += 256) s.end[i] = p.quadEnd[i];
+  return s;
+}
+// store(g, jj, re, im): column min(col0 + lane % 16, ncol - 1) of y coordinate jy0 + jj
+template <typename T, typename Store>
+__device__ __forceinline__ void sep_y_tile(const SepParams& p, const SepYShared& s,
+                                           const typename Vec2<T>::type* T1, int col0, int jy0, Store store) {
+  typedef typename Vec2<T>::type T2v;
+  constexpr int NQ = 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15,
+            lg = lane >> 4;
+  const int q0 = p.waveQ[wave], q1 = p.waveQ[wave + 1];
+  if (q0 == q1) return;
+  const T2v* src = T1 + min(col0 + lr, p.ncol - 1);
+  const int jy = jy0 + lr;
+  const float invMy = 1.f / float(p.my);
+  T2v x[NQ], xn[NQ];
+  int2 e[NQ], en[NQ];
+  auto load = [&](T2v(&v)[NQ], int2(&w)[NQ], int q) {
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      w[u] = s.ent[4 * min(q + u, q1 - 1) + lg];
+      v[u] = src[max(w[u].x, 0)];
+    }
+  };
+  d4_t re = {0., 0., 0., 0.}, im = {0., 0., 0., 0.};
+  load(x, e, q0);
+  for (int q = q0; q < q1; q += NQ) {
+    load(xn, en, q + NQ);
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      if (q + u < q1) {
+        // (jy f1) mod my: the quotient through a float is off by at most one
+        const int n = jy * e[u].y;
+        int r = n - int(float(n) * invMy) * p.my;
+        r += r < 0 ? p.my : 0;
+        r -= r >= p.my ? p.my : 0;
+        const bool on = e[u].x >= 0;
+        const double2 w = s.tw[r];
+        const double wr = on ? w.x : 0., wi = on ? w.y : 0.;
+        const double xr = on ? double(x[u].x) : 0., xi = on ? double(x[u].y) : 0.;
+        re = Mfma4<double>::mac(wr, xr, re);
+        im = Mfma4<double>::mac(wi, xr, im);
+        re = Mfma4<double>::mac(-wi, xi, re);
+        im = Mfma4<double>::mac(wr, xi, im);
+        const int g = __builtin_amdgcn_readfirstlane(s.end[q + u]);
+        if (g >= 0) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            store(g, Mfma4<double>::row(lg, i), re[i], im[i]);
+            re[i] = im[i] = 0.;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      x[u] = xn[u];
+      e[u] = en[u];
+    }
+  }
+}
+
+// The y-stage alone, T2 to device memory.  Grid (blocks of 16 columns, jz, panels).
 template <typename T>
 __global__ void __launch_bounds__(256) k_sep_y(SepParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   typedef typename Vec2<T>::type T2v;
-  const int grp = blockIdx.x, jz = blockIdx.y, panel = blockIdx.z;
-  const int e0 = p.grpStart[grp], ne = p.grpStart[grp + 1] - e0;
-  const int ncol = p.ncol, my = p.my;
-  T2v* X = reinterpret_cast<T2v*>(smem);  // (entries, ncol)
-  double2* W = reinterpret_cast<double2*>(smem + (size_t(ne) * ncol * sizeof(T2v) + 15) / 16 * 16);  // (entries, my)
-  int* off = reinterpret_cast<int*>(W + size_t(ne) * my);
-  int* fe = off + ne;
+  const int jz = blockIdx.y, panel = blockIdx.z, col0 = blockIdx.x * 16;
+  const int c = col0 + (threadIdx.x & 15);
+  const SepYShared s = sep_y_stage(p, smem, jz);
+  __syncthreads();
   const T2v* T1 = reinterpret_cast<const T2v*>(static_cast<const T*>(p.T1) + size_t(panel) * p.t1PanelStride);
-  sep_stage_entries(T1, X, W, off, fe, ne, ncol, my, p.twy, [&](int e, int& o, int& f) {
-    o = (p.grpLine[e0 + e] * p.mz + jz) * ncol;
-    f = p.grpF1[e0 + e];
-  });
-  T2v* out = reinterpret_cast<T2v*>(static_cast<T*>(p.T2) + size_t(panel) * p.t2PanelStride);
-  sep_short_transform<T>(X, W, ne, my, ncol, [&](int jy, int c, double2 v) {
-    out[((size_t(grp) * my + jy) * p.mz + jz) * ncol + c] = T2v{T(v.x), T(v.y)};
-  });
+  T2v* out = reinterpret_cast<T2v*>(static_cast<T*>(p.T2) + size_t(panel) * p.t2PanelStride) + c;
+  for (int jy0 = 0; jy0 < p.my; jy0 += 16)
+    sep_y_tile<T>(p, s, T1, col0, jy0, [&](int g, int jj, double re, double im) {
+      const int jy = jy0 + jj;
+      if (jy < p.my && c < p.ncol) out[((size_t(g) * p.my + jy) * p.mz + jz) * p.ncol] = T2v{T(re), T(im)};
+    });
 }
 
 // Last stage + epilogue for one (jy, jz) line of mesh points and one panel.
@@ -1349,98 +1449,6 @@ __device__ __forceinline__ void sep_epilogue_tail(const CoupParams& p, const Sep
   }
 }
 
-// Second half of an epilogue pass of k_sep_ep, with |g|^2 kept in LDS
-// rather than in registers: gsq holds the rpp rows' |g(nu, b2)|^2, (row, nu,
-// b2) at (r nm + nu) nb2max + b2; occupations at sf2[(c rpp + r) nb2max + b].  The phonon rotation, symmetrizeCoupling
-// along b2 (each thread its own entries) and then along nu (read on the fly
-// from the group's entries), and the Gaussian-delta weights into part.  The
-// sums run in the same order as sep_epilogue_tail's.  Wave-level ordering.
-template <typename T, int NMX, int CM, int GM>
-__device__ __forceinline__ void sep_epilogue_tail_lds(const CoupParams& p, const SepXmRow& ri, int r, int rl,
-                                                      int sub, int nb2, bool modeOn, double w3, const double2* gp,
-                                                      int gps, double* gsq, const double* se2, const int* sg3,
-                                                      const double* sf2, const double* se1,
-                                                      const typename Vec2<T>::type (&e3c)[NMX],
-                                                      const double (&n3)[CM], double (&part)[GM][CM],
-                                                      const double* e1, int gsize, double inv_g, int rpp) {
-  const int nm = p.nm, nCalc = p.nCalc, nb2max = p.nb2max;
-  const double scrW = p.screen > 0. ? screen_width(p, int(e1 - p.e1pool)) : 0.;
-  double* own = gsq + (size_t(r) * nm + sub) * nb2max;
-  // g(nu2, b2) = sum_nu e3(nu, nu2) g'(nu, b2), thread nu2 = sub
-  if (modeOn)
-    for (int b2 = 0; b2 < nb2; ++b2) {
-      double sx = 0., sy = 0.;
-#pragma unroll
-      for (int nu = 0; nu < NMX; ++nu)
-        if (nu < nm) {
-          const double2 x = gp[rl * gps + nu * nb2max + b2];
-          const double er = double(e3c[nu].x), ei = double(e3c[nu].y);
-          sx += x.x * er - x.y * ei;
-          sy += x.x * ei + x.y * er;
-        }
-      own[b2] = sx * sx + sy * sy;
-    }
-  // symmetrizeCoupling along b2 (scattering.cpp:1250-1284), own entries
-  if (modeOn) {
-    const double* e2r = se2 + r * nb2max;
-    for (int b = 0; b < nb2;) {
-      int deg = 0;
-      for (int i = b; i < nb2; ++i) {
-        if (fabs(e2r[b] - e2r[i]) < 1.0e-6) deg++;
-        else break;
-      }
-      if (deg > 1) {
-        double s2 = 0.;
-        for (int i = 0; i < deg; ++i) s2 += own[b + i] / double(float(deg));
-        for (int i = 0; i < deg; ++i) own[b + i] = s2;
-      }
-      b += deg;
-    }
-  }
-  wave_sync();
-  // ... along nu (scattering.cpp:1286-1316) and the Gaussian-delta weights
-  // (el_scattering.cpp:277-380)
-  if (!modeOn || w3 < p.cutoff) return;
-  const int grp = sg3[r * nm + sub];
-  const int mystart = grp & 0xff, mydeg = grp >> 8;
-  const double* g0 = gsq + (size_t(r) * nm + mystart) * nb2max;
-#pragma unroll 1
-  for (int b2 = 0; b2 < nb2; ++b2) {
-    double vb;
-    if (mydeg > 1) {
-      vb = 0.;
-      for (int i = 0; i < mydeg; ++i) vb += g0[size_t(i) * nb2max + b2] / double(float(mydeg));
-    } else {
-      vb = own[b2];
-    }
-    const double en2 = se2[r * nb2max + b2];
-    const double cpl = vb * inv_g;
-    const int is2 = ri.soff + b2;
-#pragma unroll
-    for (int gi = 0; gi < GM; ++gi) {
-      if (gi >= gsize) break;
-      double d1, d2;
-      if (p.adaptive) {
-        const AdaptiveWidth aw = adaptive_width(p, int(e1 - p.e1pool) + gi, is2);
-        d1 = adaptive_delta(se1[gi] - en2 + w3, aw);
-        d2 = adaptive_delta(se1[gi] - en2 - w3, aw);
-      } else {
-        const double x1 = se1[gi] - en2 + w3, x2 = se1[gi] - en2 - w3;
-        if (p.screen > 0. && fmin(fabs(x1), fabs(x2)) * p.invSigma >= scrW) continue;
-        d1 = gaussian_delta(x1, p.invSigma, p.deltaPref);
-        d2 = gaussian_delta(x2, p.invSigma, p.deltaPref);
-      }
-      if (d1 <= 0. && d2 <= 0.) continue;
-#pragma unroll
-      for (int c = 0; c < CM; ++c) {
-        if (c >= nCalc) break;
-        const double f2 = sf2[(c * rpp + r) * nb2max + b2];
-        part[gi][c] += cpl * ((f2 + n3[c]) * d1 + (1. - f2 + n3[c]) * d2) * p.norm / w3 * 3.14159265358979323846;
-      }
-    }
-  }
-}
-
 // BF3: the x-stage GEMMs in split-BF16x3 (hi*hi + hi*lo + lo*hi on
 // v_mfma_f32_16x16x32_bf16, FP32 accumulation); T must be float.
 // BREG: the B operands of all k-steps (at most 12, i.e. 24 x-groups) are loaded
@@ -1910,12 +1918,12 @@ __global__ void __launch_bounds__(256, 2) k_sep_xm(CoupParams p) {
 
 
 // ------------------------------------------------------------------ split last stage
-// The last stage as two kernels with small footprints, for FP32 data, nm, nw
-// <= 16, nm nw <= 192 and precomputed row masks: many more workgroups share a
-// CU than with the fused k_sep_xm (about 65 KB of LDS and 255 VGPRs), which
-// is bound by memory latency.  g3 rows go through HBM, (slot, jx, col), and
-// the epilogue is the same sequence of operations on the same values, so the
-// results equal the fused kernel's.
+// The last stage as two kernels with small footprints, for nw <= 16 and
+// precomputed row masks: many more workgroups share a CU than with the fused
+// k_sep_xm (about 65 KB of LDS and 255 VGPRs), which is bound by memory latency.
+// g3 rows go through HBM, (slot, jx, col) with col = w2 nm + nu, and the
+// epilogue (sep_epilogue.hpp) does the same operations on the same values, so
+// the results equal the fused kernel's.
 
 // x-stage: g3(row, (nu, w2)) = sum_g w_x^{jx n0(g)} T2(g; nu, w2) of every
 // row kept by the slot's mask, stored at G3 (slot, jx) as complex T.
@@ -2005,7 +2013,7 @@ __global__ void __launch_bounds__(256) k_sep_xg(CoupParams p) {
 #pragma unroll
   for (int j = 0; j < kXmNt; ++j) {
     const int c = (wave * kXmNt + j) * 16 + lr;
-    sgOff[j] = (c / nw) * gs + c % nw;
+    sgOff[j] = (c % nm) * gs + c / nm;  // T2's columns are (w2, nu)
   }
   for (int m0r = 0; m0r < nkeep; m0r += 16) {
     const int nr = min(16, nkeep - m0r);
@@ -2100,377 +2108,108 @@ inline size_t sep_xg_lds_bytes(int elem, int nG0, int m0, int nm = 0, int nw = 0
 }
 
 // The y-stage and the x-stage in one kernel, so that the x-stage slabs T2
-// never go through HBM.  Workgroup (block of 16 columns, jz, panel): the T1
-// entries of every line at (jz, the block's columns) are staged in LDS once;
-// then, per chunk of kYxJC y coordinates, the y-stage sums
-// T2(g, jy, c) = sum_{lines of group g} w_y^{jy f1} T1(line, jz, c) into LDS
-// (FP64, the group's lines in ascending order, as k_sep_y does) and wave w
-// runs the x-stage of slots (jy0 + w + 4i, jz) on v_mfma_f32_16x16x4f32 as
-// k_sep_xg does (A = the twiddles of the slot's kept rows, B = T2 read from
-// LDS), writing the kept rows' g3 for the block's columns (waves take the
-// chunk's slots in turn).  The same values
-// in the same order as k_sep_y + k_sep_xg, so the same g3; HBM sees T1 once
-// and the g3 rows, not T2 twice.
-constexpr int kYxJC = 4;  // y coordinates per chunk: one slot per wave (8: 47 KB of LDS, slower)
-constexpr int kYxRow = 17;  // LDS row of 16 columns, padded: rows of different groups in different banks
-
-inline size_t sep_yx_lds_bytes(int nLines, int nG0, int m0) {
-  size_t b = (size_t(nLines) * kYxRow * sizeof(float2) + 15) / 16 * 16;  // T1 of the block
-  b += size_t(nLines) * kYxJC * sizeof(double2);                         // y twiddles of a chunk
-  b += size_t(nG0) * kYxJC * kYxRow * sizeof(float2);                    // T2 of a chunk
-  b += size_t(m0) * (nG0 + 2) * sizeof(float2);                          // x twiddles of every row
-  b += size_t(2 * nLines + nG0 + 1 + 4 * 64) * sizeof(int);          // entries, groups, kept rows
-  return b + 64;
+// never go through HBM.  Workgroup (block of 16 columns, jz, panel): per tile
+// of 16 y coordinates the y-stage (sep_y_tile) leaves T2 of every group in LDS,
+// real and imaginary parts as rows k = 2g, 2g + 1, and the waves run the
+// x-stage of the tile's slots in turn: g3(jx, c) = sum_k A(jx, k) B(k, c) on
+// v_mfma_*_16x16x4 with A = the twiddles of the slot's kept rows, (Re w, Im w)
+// at k = 2g and (-Im w, Re w) at 2g + 1, and write the kept rows' g3 for the
+// block's columns.  The k order is that of k_sep_xg and k_sep_xm, so the g3
+// are the same.
+// Matrix cores and the g3 writes: cfg2's full launch (128 panels of 40^3 x 192
+// columns) is 31 GFLOP FP64 in y (40 of 48 rows used), 80 GFLOP FP32 in x and
+// 7 GB of traffic.  With the y sums as FMAs of four y coordinates per LDS read
+// of T1, in threads that owned whole groups of uneven size, it took 3.9 ms; on
+// the matrix cores 3.3.
+inline size_t sep_yx_lds_bytes(int elem, int nQuads, int my, int nG0, int m0) {
+  const int kp = (2 * nG0 + 3) / 4 * 4;
+  return sep_y_lds_bytes(my, nQuads) + size_t(m0) * (kp + 1) * 2 * elem + size_t(16) * (kp * 16 + 16) * elem +
+         size_t(4) * 64 * sizeof(int) + 64;
 }
 
-static __global__ void __launch_bounds__(256) k_sep_yx(SepParams sp, CoupParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  typedef typename Mfma4<float>::acc_t acc_t;
-  const int cb = blockIdx.x, jz = blockIdx.y, panel = blockIdx.z;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lr = lane & 15, lg = lane >> 4;
-  const int ncol = sp.ncol, my = sp.my, mz = sp.mz, m0 = p.m0, nG0 = sp.nG0, nL = sp.nLines;
-  const int nG0p = nG0 + 1, wxs = nG0 + 2;  // wxs: padded row of the x twiddles
-  float2* sT1 = reinterpret_cast<float2*>(smem);  // (entry in group order, kYxRow)
-  double2* sWy = reinterpret_cast<double2*>(smem + (size_t(nL) * kYxRow * sizeof(float2) + 15) / 16 * 16);  // (entry, jj)
-  float2* sT2 = reinterpret_cast<float2*>(sWy + size_t(nL) * kYxJC);  // (g, jj, kYxRow)
-  float2* sWx = sT2 + size_t(nG0) * kYxJC * kYxRow;                    // (jx, g), g < nG0p, row wxs
-  int* sOff = reinterpret_cast<int*>(sWx + size_t(m0) * wxs);          // T1 row of each entry
-  int* sF1 = sOff + nL;                                                // f1 of each entry
-  int* sGs = sF1 + nL;                                                 // group starts
-  int* sJx = sGs + nG0 + 1;                                            // kept rows, 64 per wave
-  const float2* T1 = reinterpret_cast<const float2*>(static_cast<const float*>(sp.T1) + size_t(panel) * sp.t1PanelStride);
-  for (int e = t; e < nL; e += 256) {
-    sOff[e] = (sp.grpLine[e] * mz + jz) * ncol;
-    sF1[e] = sp.grpF1[e];
-  }
-  for (int i = t; i <= nG0; i += 256) sGs[i] = sp.grpStart[i];
-  for (int i = t; i < m0 * nG0p; i += 256) {
-    const int jx = i / nG0p, g = i - jx * nG0p;
-    float2 w = make_float2(0.f, 0.f);
-    if (g < nG0) {
-      const double2 d = p.tw0[(jx * p.g0val[g]) % m0];
-      w = make_float2(float(d.x), float(d.y));
-    }
-    sWx[jx * wxs + g] = w;
-  }
-  __syncthreads();
-  // T1 of the block: up to 8 loads per thread in flight before their LDS stores
-  for (int i0 = t; i0 < nL * 16; i0 += 8 * 256) {
-    float2 v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = i0 + 256 * u, col = cb * 16 + (i & 15);
-      v[u] = make_float2(0.f, 0.f);
-      if (i < nL * 16 && col < ncol) v[u] = T1[size_t(sOff[i >> 4]) + col];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = i0 + 256 * u;
-      if (i < nL * 16) sT1[(i >> 4) * kYxRow + (i & 15)] = v[u];
-    }
-  }
-  const int nLinesYZ = p.m1 * p.m2;
-  const int KS = (2 * nG0 + 3) / 4;  // <= 12, checked by the launcher
-  const int c = cb * 16 + lr;
-  for (int jy0 = 0; jy0 < my; jy0 += kYxJC) {
-    const int nj = min(kYxJC, my - jy0);
-    for (int i = t; i < nL * kYxJC; i += 256) {
-      const int e = i / kYxJC, jj = i - e * kYxJC;
-      sWy[i] = jj < nj ? sp.twy[((jy0 + jj) * sF1[e]) % my] : make_double2(0., 0.);
-    }
-    __syncthreads();  // also: T1 staged (first chunk)
-    // thread (g, column): all kYxJC y coordinates of the chunk from one read of each T1 entry
-    for (int i = t; i < nG0 * 16; i += 256) {
-      const int cc = i & 15, g = i >> 4;
-      double2 acc[kYxJC];
-#pragma unroll
-      for (int jj = 0; jj < kYxJC; ++jj) acc[jj] = make_double2(0., 0.);
-      for (int e = sGs[g]; e < sGs[g + 1]; ++e) {
-        const float2 xv = sT1[e * kYxRow + cc];
-        const double2 x = make_double2(double(xv.x), double(xv.y));
-#pragma unroll
-        for (int jj = 0; jj < kYxJC; ++jj) {
-          const double2 ww = sWy[e * kYxJC + jj];
-          acc[jj].x += ww.x * x.x - ww.y * x.y;
-          acc[jj].y += ww.x * x.y + ww.y * x.x;
-        }
-      }
-#pragma unroll
-      for (int jj = 0; jj < kYxJC; ++jj)
-        sT2[(g * kYxJC + jj) * kYxRow + cc] = make_float2(float(acc[jj].x), float(acc[jj].y));
-    }
-    __syncthreads();
-    for (int jw = wave; jw < nj; jw += 4) {
-      const int slot = panel * nLinesYZ + jz * p.m1 + jy0 + jw;
-      const unsigned long long mask = p.keepMask[slot];
-      if (mask != 0ull) {
-        int* jxs = sJx + wave * 64;
-        wave_sync();  // the wave's previous slot has read its list
-        if (lane < m0 && ((mask >> lane) & 1ull)) jxs[__popcll(mask & ((1ull << lane) - 1ull))] = lane;
-        wave_sync();
-        const int nkeep = __popcll(mask);
-        float bq[12];
-#pragma unroll
-        for (int q = 0; q < 12; ++q) {
-          const int k = 4 * q + lg, g = k >> 1, kc = k & 1;
-          float b = 0.f;
-          if (q < KS && g < nG0) {
-            const float2 v = sT2[(g * kYxJC + jw) * kYxRow + lr];
-            b = kc ? v.y : v.x;
-          }
-          bq[q] = b;
-        }
-        float2* out = static_cast<float2*>(p.G3) + size_t(slot) * m0 * ncol + c;
-        for (int m0r = 0; m0r < nkeep; m0r += 16) {
-          const int nr = min(16, nkeep - m0r);
-          const bool rowOk = lr < nr;
-          const float2* wrow = sWx + (rowOk ? jxs[m0r + lr] : 0) * wxs;
-          acc_t accr, acci;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) accr[i] = acci[i] = 0.f;
-#pragma unroll
-          for (int q = 0; q < 12; ++q) {
-            if (q < KS) {
-              const int k = 4 * q + lg, g = k >> 1, kc = k & 1;
-              const bool gOk = g < nG0;
-              const float2 w = wrow[gOk ? g : nG0];
-              const bool on = rowOk && gOk;
-              const float a1 = on ? (kc ? -w.y : w.x) : 0.f;
-              const float a2 = on ? (kc ? w.x : w.y) : 0.f;
-              accr = Mfma4<float>::mac(a1, bq[q], accr);
-              acci = Mfma4<float>::mac(a2, bq[q], acci);
-            }
-          }
-          if (c < ncol) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int row = Mfma4<float>::row(lg, i);
-              if (row < nr) out[size_t(jxs[m0r + row]) * ncol] = make_float2(accr[i], acci[i]);
-            }
-          }
-        }
-      }
-    }
-    __syncthreads();  // the next chunk rewrites the twiddles, T2 and the kept-row lists
-  }
-}
-
-constexpr int kSepEpThreads = 64;  // k_sep_ep workgroup: one wave
-
-// Row data of an rpp-row pass of k_sep_ep into LDS: U2 (row r at sU2 + r u2s,
-// nw x nb2max), e2 (rpp x nb2max), omega and mode groups (rpp x nm) and the
-// occupations (nCalc x rpp x nb2max).  The loads of the e2, omega and U2
-// entries are issued before their LDS stores; rpp nm <= blockDim, rpp nb2max
-// <= 2 blockDim.
-__device__ inline void sep_ep_stage_rows(const CoupParams& p, const SepXmRow* rows, int m0r, int nr, int rpp,
-                                         int nw, int nm, int u2s, double2* sU2, double* se2, double* sw3,
-                                         int* sg3, double* sf2) {
-  const int t = threadIdx.x, nb2max = p.nb2max, bs = blockDim.x;
-  const int ne = rpp * nb2max, nwv = rpp * nm, nf = p.nCalc * ne;
-  double ev[2] = {0., 0.}, wv = 0.;
-  int gv = 0;
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int i = t + bs * u;
-    if (i < ne) {
-      const int r = i / nb2max, b = i % nb2max;
-      if (r < nr && b < rows[m0r + r].nb2) ev[u] = p.e2pool[rows[m0r + r].soff + b];
-    }
-  }
-  if (t < nwv) {
-    const int r = t / nm, nu = t % nm;
-    if (r < nr) {
-      wv = p.Wpool[size_t(rows[m0r + r].iq) * nm + nu];
-      gv = p.qModeGrp[size_t(rows[m0r + r].iq) * nm + nu];
-    }
-  }
-  const int per = nw * nb2max, nU = rpp * per;
-  for (int i0 = t; i0 < nU; i0 += 4 * bs) {
-    double2 v[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = i0 + bs * u;
-      v[u] = make_double2(0., 0.);
-      if (i < nU) {
-        const int r = i / per, o = i % per;
-        if (r < nr) {
-          const SepXmRow& rr = rows[m0r + r];
-          if (o < nw * rr.nb2) v[u] = p.U2pool[rr.u2off + o];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = i0 + bs * u;
-      if (i < nU) sU2[(i / per) * u2s + i % per] = v[u];
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-    if (t + bs * u < ne) se2[t + bs * u] = ev[u];
-  if (t < nwv) {
-    sw3[t] = wv;
-    sg3[t] = gv;
-  }
-  for (int i = t; i < nf; i += bs) {
-    const int c = i / ne, o = i % ne, r = o / nb2max, b = o % nb2max;
-    double f = 0.;
-    if (r < nr && b < rows[m0r + r].nb2) f = p.fermi[size_t(c) * p.numStates + rows[m0r + r].soff + b];
-    sf2[i] = f;
-  }
-}
-
-// epilogue of the rows k_sep_xg wrote: the electron rotation from each
-// thread's g3 slice (registers), then the phonon data and sep_epilogue_tail;
-// nm threads per row, passes of epRows rows (whole rows per wave, nm <= NMX
-// <= 16).  The slice and the eigenvector column are never live together.  CM calculations
-// and GM members of the b1 group are held per thread: every panel of the
-// launch has gsize <= GM (checked on the host).
-template <typename T, int CM, int NMX, int GM>
-__global__ void __launch_bounds__(kSepEpThreads, 2) k_sep_ep(CoupParams p) {
+template <typename T>
+__global__ void __launch_bounds__(256) k_sep_yx(SepParams sp, CoupParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   typedef typename Vec2<T>::type T2v;
-  constexpr int NWX = 16;
-  const int nLinesYZ = p.m1 * p.m2;
-  const int nTilesTot = p.nPanels * nLinesYZ;
-  const int bid = blockIdx.x;
-  const int perXcd = gridDim.x / 8;
-  const int Lx = (bid % 8) * perXcd + bid / 8;
-  if (Lx >= nTilesTot) return;
-  const int yz = Lx / p.nPanels, panel = Lx % p.nPanels;
-  const int slot = panel * nLinesYZ + yz;
-  const int jy = yz % p.m1, jz = yz / p.m1;
-  const int t = threadIdx.x;
-  const unsigned long long mask = p.keepMask[slot];
-  if (mask == 0ull) {
-    if (t < kGMax * kCMax) p.partial[size_t(slot) * kGMax * kCMax + t] = 0.;
-    return;
+  typedef typename Mfma4<T>::acc_t acc_t;
+  const int cb = blockIdx.x, jz = blockIdx.y, panel = blockIdx.z;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, lr = lane & 15,
+            lg = lane >> 4;
+  const int ncol = sp.ncol, my = sp.my, m0 = p.m0, nG0 = sp.nG0;
+  const int KS = (2 * nG0 + 3) / 4, kp = 4 * KS;  // KS <= 12, checked by the launcher
+  const int as = kp + 1, js = kp * 16 + 16;       // padded: rows in different banks
+  const SepYShared sy = sep_y_stage(sp, smem, jz);
+  T2v* sA = reinterpret_cast<T2v*>(smem + sep_y_lds_bytes(my, sp.nQuads));  // (jx, k): (a1, a2)
+  T* sT2 = reinterpret_cast<T*>(sA + size_t(m0) * as);                      // (jj, k, 16 columns)
+  int* sJx = reinterpret_cast<int*>(sT2 + size_t(16) * js) + wave * 64;     // kept rows of the wave's slot
+  for (int i = t; i < m0 * kp; i += 256) {
+    const int jx = i / kp, k = i - jx * kp, g = k >> 1;
+    T2v a = T2v{T(0), T(0)};
+    if (g < nG0) {
+      const double2 d = p.tw0[(jx * p.g0val[g]) % m0];
+      a = (k & 1) ? T2v{-T(d.y), T(d.x)} : T2v{T(d.x), T(d.y)};
+    }
+    sA[jx * as + k] = a;
   }
-  const int nm = p.nm, nw = p.nw, ncol = nm * nw;
-  const int kk = p.panelKK[panel];
-  const int b1p = p.panelB1[panel];
-  const int kkMesh = p.kkMesh[kk];
-  const int u2s = nw * p.nb2max + 1, gps = nm * p.nb2max + 1;
-  const int rpp = p.epRows, rpw = rpp / (kSepEpThreads / 64);
-  SepXmRow* rows = reinterpret_cast<SepXmRow*>(smem);                          // 64
-  double2* sU2 = reinterpret_cast<double2*>(smem + (64 * sizeof(SepXmRow) + 15) / 16 * 16);  // rpp x u2s
-  double2* gp = sU2 + size_t(rpp) * u2s;                                       // rpp x gps
-  double* se2 = reinterpret_cast<double*>(gp + size_t(rpp) * gps);             // rpp x nb2max
-  double* sw3 = se2 + size_t(rpp) * p.nb2max;                                  // rpp x nm
-  double* sf2 = sw3 + size_t(rpp) * nm;                                        // nCalc x rpp x nb2max
-  double* se1 = sf2 + size_t(p.nCalc) * rpp * p.nb2max;                        // kGMax
-  double* gsq = se1 + kGMax;                                                   // rpp x nm x nb2max
-  int* sg3 = reinterpret_cast<int*>(gsq + size_t(rpp) * nm * p.nb2max);        // rpp x nm
-  if (t < p.panelGSize[panel]) se1[t] = p.e1pool[p.kkStateOff[kk] + p.panelGStart[panel] + t];
-  const int nkeep = __popcll(mask);
-  if (t < p.m0 && ((mask >> t) & 1ull)) {
-    const int mesh = (jz * p.m1 + jy) * p.m0 + t;
-    const int4 mr = p.meshRow[mesh];
-    rows[__popcll(mask & ((1ull << t) - 1ull))] =
-        SepXmRow{t, mr.x, mesh_diff_index(mesh, kkMesh, p.m0, p.m1, p.m2), mr.y, mr.z, mr.w};
+  for (int i = t; i < 16 * (kp - 2 * nG0) * 16; i += 256) {  // the padding of the last k-step
+    const int r = i / 16, jj = r / (kp - 2 * nG0), k = 2 * nG0 + r % (kp - 2 * nG0);
+    sT2[jj * js + k * 16 + (i & 15)] = T(0);
   }
-  if (t == 0 && p.keptRows) atomicAdd(p.keptRows, (unsigned long long)nkeep);
   __syncthreads();
-  if (t == 0 && p.keptBands) {
-    unsigned long long nb = 0;
-    for (int i = 0; i < nkeep; ++i) nb += rows[i].nb2;
-    atomicAdd(p.keptBands, nb);
-  }
-  double part[GM][CM];
-#pragma unroll
-  for (int gi = 0; gi < GM; ++gi)
-#pragma unroll
-    for (int c = 0; c < CM; ++c) part[gi][c] = 0.;
-  const int gstart = p.panelGStart[panel], gsize = p.panelGSize[panel];
-  const double* e1 = p.e1pool + p.kkStateOff[kk] + gstart;
-  const double inv_g = 1. / double(float(gsize));
-  const T2v* G3 = static_cast<const T2v*>(p.G3) + size_t(slot) * p.m0 * ncol;
-  // rpw whole rows of nm threads in each wave; the lanes beyond them idle
-  const int wave = t >> 6, lane = t & 63;
-  const bool laneOn = lane < rpw * nm;
-  const int r = laneOn ? wave * rpw + lane / nm : rpp, sub = laneOn ? lane % nm : 0, rl = r;
-  for (int m0r = 0; m0r < nkeep; m0r += rpp) {
-    const int nr = min(rpp, nkeep - m0r);
-    const bool rowOn = r < nr;
-    const bool modeOn = rowOn && sub < nm;
-    // the thread's g3 slice (mode sub of its row), loads issued before the
-    // row staging's
-    T2v g[NWX];
-    if (modeOn) {
-      const T2v* src = G3 + size_t(rows[m0r + r].jx) * ncol + sub * nw;
-      if (sizeof(T) == 4 && nw == NWX) {
-        // full slice: 16-byte loads (src is a multiple of 16 elements from
-        // the table's start)
-        const float4* s4 = reinterpret_cast<const float4*>(src);
-#pragma unroll
-        for (int h = 0; h < NWX / 2; ++h) {
-          const float4 v = s4[h];
-          g[2 * h].x = v.x;
-          g[2 * h].y = v.y;
-          g[2 * h + 1].x = v.z;
-          g[2 * h + 1].y = v.w;
-        }
-      } else {
-#pragma unroll
-        for (int w2 = 0; w2 < NWX; ++w2)
-          if (w2 < nw) g[w2] = src[w2];
-      }
-    }
-    sep_ep_stage_rows(p, rows, m0r, nr, rpp, nw, nm, u2s, sU2, se2, sw3, sg3, sf2);
+  const T2v* T1 = reinterpret_cast<const T2v*>(static_cast<const T*>(sp.T1) + size_t(panel) * sp.t1PanelStride);
+  const int nLinesYZ = p.m1 * p.m2;
+  const int c = cb * 16 + lr;
+  for (int jy0 = 0; jy0 < my; jy0 += 16) {
+    const int nj = min(16, my - jy0);
+    sep_y_tile<T>(sp, sy, T1, cb * 16, jy0, [&](int g, int jj, double re, double im) {
+      sT2[jj * js + (2 * g) * 16 + lr] = T(re);
+      sT2[jj * js + (2 * g + 1) * 16 + lr] = T(im);
+    });
     __syncthreads();
-    const SepXmRow ri = rows[m0r + (rowOn ? r : 0)];
-    const int nb2 = rowOn ? ri.nb2 : 0;
-    const double w3 = modeOn ? sw3[r * nm + sub] : 0.;
-    // g'(nu, b2) = sum_w2 conj(U2(w2, b2)) g3(nu, w2), thread nu = sub
-    if (modeOn) {
-      for (int b2 = 0; b2 < nb2; ++b2) {
-        const double2* u = sU2 + size_t(r) * u2s + b2 * nw;
-        double sx = 0., sy = 0.;
+    for (int jj = wave; jj < nj; jj += 4) {
+      const int slot = panel * nLinesYZ + jz * p.m1 + jy0 + jj;
+      const unsigned long long mask = p.keepMask[slot];
+      if (mask == 0ull) continue;
+      wave_sync();  // the wave's previous slot has read its list
+      if (lane < m0 && ((mask >> lane) & 1ull)) sJx[__popcll(mask & ((1ull << lane) - 1ull))] = lane;
+      wave_sync();
+      const int nkeep = __popcll(mask);
+      T b[12];
 #pragma unroll
-        for (int w2 = 0; w2 < NWX; ++w2)
-          if (w2 < nw) {
-            const double xr = double(g[w2].x), xi = double(g[w2].y);
-            sx += u[w2].x * xr + u[w2].y * xi;
-            sy += u[w2].x * xi - u[w2].y * xr;
+      for (int q = 0; q < 12; ++q)
+        if (q < KS) b[q] = sT2[jj * js + (4 * q + lg) * 16 + lr];
+      T2v* out = static_cast<T2v*>(p.G3) + size_t(slot) * m0 * ncol + c;
+      for (int m0r = 0; m0r < nkeep; m0r += 16) {
+        const int nr = min(16, nkeep - m0r);
+        const T2v* arow = sA + sJx[min(m0r + lr, nkeep - 1)] * as + lg;
+        acc_t accr, acci;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) accr[i] = acci[i] = T(0);
+#pragma unroll
+        for (int q = 0; q < 12; ++q) {
+          if (q < KS) {
+            const T2v a = arow[4 * q];
+            accr = Mfma4<T>::mac(a.x, b[q], accr);
+            acci = Mfma4<T>::mac(a.y, b[q], acci);
           }
-        gp[rl * gps + sub * p.nb2max + b2] = make_double2(sx, sy);
+        }
+        if (c < ncol) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int row = Mfma4<T>::row(lg, i);
+            if (row < nr) out[size_t(sJx[m0r + row]) * ncol] = T2v{accr[i], acci[i]};
+          }
+        }
       }
     }
-    // phonon eigenvector column and Bose factors of (row, mode sub)
-    T2v e3c[NMX];
-    double n3[CM];
-#pragma unroll
-    for (int c = 0; c < CM; ++c) n3[c] = 0.;
-    if (modeOn) {
-      const T2v* e3 = static_cast<const T2v*>(p.E3T) + size_t(ri.iq) * nm * nm + sub;
-#pragma unroll
-      for (int nu = 0; nu < NMX; ++nu)
-        if (nu < nm) e3c[nu] = e3[nu * nm];
-#pragma unroll
-      for (int c = 0; c < CM; ++c)
-        if (c < p.nCalc) n3[c] = p.bose[(size_t(ri.iq) * nm + sub) * p.nCalc + c];
-    }
-    wave_sync();
-    sep_epilogue_tail_lds<T, NMX, CM, GM>(p, ri, r, rl, sub, nb2, modeOn, w3, gp, gps, gsq, se2, sg3, sf2, se1, e3c,
-                                      n3, part, e1, gsize, inv_g, rpp);
-    __syncthreads();  // the next tile rewrites the row data
+    __syncthreads();  // the next tile rewrites T2
   }
-  reduce_partials<CM, GM, kSepEpThreads / 64>(p, slot, smem, part);
 }
 
-inline size_t sep_ep_lds_bytes(int nw, int nm, int nb2max, int nCalc, int rpp) {
-  size_t b = (64 * sizeof(SepXmRow) + 15) / 16 * 16;
-  b += size_t(rpp) * (nw * nb2max + 1) * sizeof(double2) + size_t(rpp) * (nm * nb2max + 1) * sizeof(double2) +
-       size_t(rpp) * nb2max * sizeof(double) + size_t(rpp) * nm * sizeof(double) +
-       size_t(nCalc) * rpp * nb2max * sizeof(double) + size_t(kGMax) * sizeof(double) +
-       size_t(rpp) * nm * nb2max * sizeof(double) + size_t(rpp) * nm * sizeof(int);
-  return std::max(b, size_t(kGMax) * kCMax * 4 * sizeof(double)) + 64;
-}
-
-// ------------------------------------------------------------------ split epilogue, lean form
-// Only what the epilogue of the split last stage reads (fixed Gaussian
-// smearing).  A small block: the kernel keeps its scalars in SGPRs instead of
-// spilling the full CoupParams' into VGPR lanes.
+// ------------------------------------------------------------------ split epilogue
+// Only what the epilogue of the split last stage reads.  A small block: the
+// kernel keeps its scalars in SGPRs instead of spilling the full CoupParams'
+// into VGPR lanes.
 struct EpParams {
   const unsigned long long* keepMask;
   double* partial;  // (slot, kGMax, kCMax)
@@ -2488,7 +2227,7 @@ struct EpParams {
   const double* fermi;     // (calc, state)
   const double* bose;      // (q, nu, calc)
   const void* E3T;         // (q, nu, nu2) in the transform's precision
-  const void* G3;          // (slot, jx, (nu, w2)) in the transform's precision; with the
+  const void* G3;          // (slot, jx, (w2, nu)) in the transform's precision; with the
                            // rotation done by the x-stage, (slot, jx, b2, nu) complex FP64
   const double* screenOf;  // per outer state: screen width of the panel its b1 group starts (null: screen)
   unsigned long long* keptRows;
@@ -2500,350 +2239,18 @@ struct EpParams {
   int m0, m1, m2, nPanels, nm, nw, nCalc, numStates;
   int nb2max;              // g' rows of the rotating x-stage hold nb2max nm entries
   int rpw;                 // rows per pass: whole rows of nm lanes, rpw nm <= 64
+  // adaptive smearing: group velocities of the states and the scaled cell (CoupParams)
+  int adaptive;
+  const double* stateV;
+  double qT[9];
+  double minWidth;
 };
 
-// Epilogue of the rows k_sep_xg wrote, one wave per slot (panel, yz line),
-// passes of rpw rows with lane (row r, mode sub).  The same operations in the
-// same order as k_sep_ep (so the same linewidths), arranged so that little is
-// live at once:
-//   A  electron rotation g'(nu, b2) = sum_w2 conj(U2(w2, b2)) g3(nu, w2),
-//      nu = sub, each g3 value converted once (outer loop over w2, NB2
-//      accumulators), U2 of the pass in LDS;
-//   B  phonon rotation g(nu2, b2) = sum_nu e3(nu, nu2) g'(nu, b2), nu2 = sub,
-//      the eigenvector column in registers, then |g|^2 and symmetrizeCoupling
-//      along b2 (scattering.cpp:1250-1284) on the lane's own entries;
-//   C  symmetrizeCoupling along nu (:1286-1316) from the group's entries and
-//      the Gaussian-delta weights of el_scattering.cpp:277-380 into per-lane
-//      partial sums (CM calculations, GM members of the b1 group).
-// Phases A and B run the pass's largest band count for every row (uniform
-// branches; a row's U2 columns beyond its own count are zero).  NB2 >= nb2max
-// is the LDS stride of a row's bands, NMX >= nm the eigenvector column length.
-// Phase A of k_sep_ep2 for NB bands: g'(nu, b2) = sum_w2 conj(U2(w2, b2)) g3(nu, w2)
-// for the lane's mode, w2 in order.  No branches inside: entries beyond nw
-// are zero in g and in U2, so every term adds an exact zero.
-template <typename T2v, int NWX, int NB2, int NB>
-__device__ __forceinline__ void ep2_rot_el(const T2v (&g)[NWX], const double2* u, double2* out) {
-  double ar[NB], ai[NB];
-#pragma unroll
-  for (int b2 = 0; b2 < NB; ++b2) ar[b2] = ai[b2] = 0.;
-#pragma unroll
-  for (int w2 = 0; w2 < NWX; ++w2) {
-    const double xr = double(g[w2].x), xi = double(g[w2].y);
-#pragma unroll
-    for (int b2 = 0; b2 < NB; ++b2) {
-      const double2 c = u[b2 * NWX + w2];
-      ar[b2] += c.x * xr + c.y * xi;
-      ai[b2] += c.x * xi - c.y * xr;
-    }
-  }
-#pragma unroll
-  for (int b2 = 0; b2 < NB; ++b2) out[b2] = make_double2(ar[b2], ai[b2]);
-}
-
-// Phase B of k_sep_ep2 for NB bands: g(nu2, b2) = sum_nu e3(nu, nu2) g'(nu, b2)
-// for the lane's mode nu2, nu in order, and |g|^2 into own.  Modes beyond nm
-// have zero eigenvector entries and read the last mode's (finite) g'.
-template <typename T2v, int NMX, int NB2, int NB>
-__device__ __forceinline__ void ep2_rot_ph(const T2v (&e3c)[NMX], const double2* x, int nm, double* own) {
-  double gr[NB], gi[NB];
-#pragma unroll
-  for (int b2 = 0; b2 < NB; ++b2) gr[b2] = gi[b2] = 0.;
-#pragma unroll
-  for (int nu = 0; nu < NMX; ++nu) {
-    const double er = double(e3c[nu].x), ei = double(e3c[nu].y);
-    const double2* xn = x + min(nu, nm - 1) * NB2;
-#pragma unroll
-    for (int b2 = 0; b2 < NB; ++b2) {
-      const double2 v = xn[b2];
-      gr[b2] += v.x * er - v.y * ei;
-      gi[b2] += v.x * ei + v.y * er;
-    }
-  }
-#pragma unroll
-  for (int b2 = 0; b2 < NB; ++b2) own[b2] = gr[b2] * gr[b2] + gi[b2] * gi[b2];
-}
-
-template <typename T, int CM, int NMX, int GM, int NB2, bool PRE = false>
-__global__ void __launch_bounds__(64, 3) k_sep_ep2(EpParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  typedef typename Vec2<T>::type T2v;
-  constexpr int NWX = 16;
-  constexpr int U2S = NWX * NB2 + 1;  // double2 per row of the U2 table (odd: rows in different banks)
-  constexpr int RMX = NB2 <= 4 ? 5 : 4;           // rows per pass at most (the launcher's cap)
-  constexpr int UPL = (NWX * NB2 * RMX + 63) / 64;  // U2 entries per lane
-  const int nLinesYZ = p.m1 * p.m2;
-  const int nTilesTot = p.nPanels * nLinesYZ;
-  const int bid = blockIdx.x;
-  const int perXcd = gridDim.x / 8;
-  const int Lx = (bid % 8) * perXcd + bid / 8;
-  if (Lx >= nTilesTot) return;
-  const int yz = Lx / p.nPanels, panel = Lx % p.nPanels;
-  const int slot = panel * nLinesYZ + yz;
-  const int jy = yz % p.m1, jz = yz / p.m1;
-  const int t = threadIdx.x;
-  if (p.gate && *p.gate == 0) return;
-  if (p.slotOn && !p.slotOn[slot]) {
-    if (p.slotZero && t < kGMax * kCMax) p.partial[size_t(slot) * kGMax * kCMax + t] = 0.;
-    return;
-  }
-  const unsigned long long mask = p.keepMask[slot];
-  if (mask == 0ull) {
-    if (t < kGMax * kCMax) p.partial[size_t(slot) * kGMax * kCMax + t] = 0.;
-    return;
-  }
-  const int nm = p.nm, nw = p.nw, ncol = nm * nw, R = p.rpw;
-  const int kk = p.panelKK[panel];
-  const int gstart = p.panelGStart[panel], gsize = __builtin_amdgcn_readfirstlane(p.panelGSize[panel]);
-  const int is1 = p.kkStateOff[kk] + gstart;
-  const double scrW = p.screen > 0. ? (p.screenOf ? p.screenOf[is1] : p.screen) : 0.;
-  const double inv_g = 1. / double(float(gsize));
-  // LDS: rows (64) | U2 (R x U2S double2), later |g|^2 (R x nm x NB2) | g' (R x nm x NB2 + 1 per row)
-  //      | e2 (R x NB2) | occupations (CM x R x NB2) | e1 (kGMax)
-  SepXmRow* rows = reinterpret_cast<SepXmRow*>(smem);
-  double2* sU2 = reinterpret_cast<double2*>(smem + (64 * sizeof(SepXmRow) + 15) / 16 * 16);
-  double* gsq = reinterpret_cast<double*>(sU2);
-  const int gps = nm * NB2 + 1;
-  double2* gp = sU2 + size_t(R) * U2S;
-  double* se2 = reinterpret_cast<double*>(gp + size_t(R) * gps);
-  double* sf2 = se2 + R * NB2;
-  double* se1 = sf2 + CM * R * NB2;
-  if (t < gsize) se1[t] = p.e1pool[is1 + t];
-  const int nkeep = __popcll(mask);
-  {
-    const int kkMesh = p.kkMesh[kk];
-    if (t < p.m0 && ((mask >> t) & 1ull)) {
-      const int mesh = (jz * p.m1 + jy) * p.m0 + t;
-      const int4 mr = p.meshRow[mesh];
-      rows[__popcll(mask & ((1ull << t) - 1ull))] =
-          SepXmRow{t, mr.x, mesh_diff_index(mesh, kkMesh, p.m0, p.m1, p.m2), mr.y, mr.z, mr.w};
-    }
-  }
-  __syncthreads();
-  if (t == 0) {
-    if (p.keptRows) atomicAdd(p.keptRows, (unsigned long long)nkeep);
-    if (p.keptBands) {
-      unsigned long long nb = 0;
-      for (int i = 0; i < nkeep; ++i) nb += rows[i].nb2;
-      atomicAdd(p.keptBands, nb);
-    }
-  }
-  // lane (r, sub): r < R rows of a pass, whole rows of nm lanes; the rest idle
-  const bool laneOn = t < R * nm;
-  const int r = laneOn ? t / nm : 0, sub = laneOn ? t % nm : 0;
-  const T2v* G3 = static_cast<const T2v*>(p.G3) + size_t(slot) * p.m0 * ncol;
-  const int rowG = p.nb2max * nm;  // PRE: g' row length, (b2, nu)
-  const double2* GP = static_cast<const double2*>(p.G3) + size_t(slot) * p.m0 * rowG;
-  const T2v* E3T = static_cast<const T2v*>(p.E3T);
-  double part[GM][CM];
-#pragma unroll
-  for (int gi = 0; gi < GM; ++gi)
-#pragma unroll
-    for (int c = 0; c < CM; ++c) part[gi][c] = 0.;
-
-  // registers of one pass, loaded at its start
-  T2v g[NWX];         // g3(nu = sub, w2) of the lane's row
-  double2 gv[NB2];    // PRE: g'(nu = sub, b2) of the lane's row
-  T2v e3c[NMX];       // e3(nu, nu2 = sub) at the row's q
-  double2 u2v[UPL];   // U2 entries of the pass (lane-strided over R x NWX x NB2)
-  double e2v = 0., f2v[CM], w3 = 0., n3[CM];
-  int grp = 0;
-  auto load_pass = [&](int m0r) {
-    const int nr = min(R, nkeep - m0r);
-    const bool rowOn = laneOn && r < nr;
-    const SepXmRow ri = rows[m0r + (rowOn ? r : 0)];
-    if (rowOn) {
-      if (PRE) {
-#pragma unroll
-        for (int b2 = 0; b2 < NB2; ++b2)
-          gv[b2] = b2 < ri.nb2 ? GP[size_t(ri.jx) * rowG + b2 * nm + sub] : make_double2(0., 0.);
-      } else if (sizeof(T) == 4 && nw == NWX) {
-        const float4* s4 = reinterpret_cast<const float4*>(G3 + size_t(ri.jx) * ncol + sub * nw);
-#pragma unroll
-        for (int h = 0; h < NWX / 2; ++h) {
-          const float4 v = s4[h];
-          g[2 * h].x = v.x;
-          g[2 * h].y = v.y;
-          g[2 * h + 1].x = v.z;
-          g[2 * h + 1].y = v.w;
-        }
-      } else {
-        const T2v* src = G3 + size_t(ri.jx) * ncol + sub * nw;
-#pragma unroll
-        for (int w2 = 0; w2 < NWX; ++w2) g[w2] = w2 < nw ? src[w2] : T2v{T(0), T(0)};
-      }
-      const T2v* e3 = E3T + size_t(ri.iq) * nm * nm + sub;
-#pragma unroll
-      for (int nu = 0; nu < NMX; ++nu) e3c[nu] = nu < nm ? e3[nu * nm] : T2v{T(0), T(0)};
-      w3 = p.Wpool[size_t(ri.iq) * nm + sub];
-      grp = p.qModeGrp[size_t(ri.iq) * nm + sub];
-#pragma unroll
-      for (int c = 0; c < CM; ++c) n3[c] = c < p.nCalc ? p.bose[(size_t(ri.iq) * nm + sub) * p.nCalc + c] : 0.;
-    } else {
-      w3 = 0.;
-      grp = 0;
-    }
-    // U2 of the pass: entry i = (row, b2, w2), w2 fastest, NWX x NB2 per row
-#pragma unroll
-    for (int u = 0; u < (PRE ? 0 : UPL); ++u) {
-      const int i = t + 64 * u, rr = i / (NWX * NB2), o = i % (NWX * NB2), b2 = o / NWX, w2 = o % NWX;
-      double2 v = make_double2(0., 0.);
-      if (rr < nr) {
-        const SepXmRow& q = rows[m0r + rr];
-        if (b2 < q.nb2 && w2 < nw) v = p.U2pool[q.u2off + b2 * nw + w2];
-      }
-      u2v[u] = v;
-    }
-    // band energies and occupations: lane = (row, b2) for lanes < R NB2
-    e2v = 0.;
-#pragma unroll
-    for (int c = 0; c < CM; ++c) f2v[c] = 0.;
-    if (t < R * NB2) {
-      const int rr = t / NB2, b2 = t % NB2;
-      if (rr < nr && b2 < rows[m0r + rr].nb2) {
-        const int st = rows[m0r + rr].soff + b2;
-        e2v = p.e2pool[st];
-#pragma unroll
-        for (int c = 0; c < CM; ++c)
-          if (c < p.nCalc) f2v[c] = p.fermi[size_t(c) * p.numStates + st];
-      }
-    }
-  };
-  for (int m0r = 0; m0r < nkeep; m0r += R) {
-    load_pass(m0r);
-    const int nr = min(R, nkeep - m0r);
-    const bool rowOn = laneOn && r < nr;
-    const int nb2 = rowOn ? rows[m0r + r].nb2 : 0;
-    // largest band count of the pass's rows, uniform over the wave: phases A
-    // and B run that many bands for every row (a row's U2 columns beyond its
-    // own count are zero, so those entries come out zero and are never read)
-    int nbw = 0;
-    for (int i = 0; i < nr; ++i) nbw = max(nbw, rows[m0r + i].nb2);
-    nbw = __builtin_amdgcn_readfirstlane(nbw);
-    // row data of the pass into LDS
-#pragma unroll
-    for (int u = 0; u < (PRE ? 0 : UPL); ++u) {
-      const int i = t + 64 * u, rr = i / (NWX * NB2);
-      if (rr < R) sU2[rr * U2S + i % (NWX * NB2)] = u2v[u];  // R <= RMX
-    }
-    if (t < R * NB2) {
-      se2[t] = e2v;
-#pragma unroll
-      for (int c = 0; c < CM; ++c) sf2[c * R * NB2 + t] = f2v[c];
-    }
-    __syncthreads();
-    // A: electron rotation, thread nu = sub (PRE: done by the x-stage kernel)
-    if (PRE && rowOn) {
-      double2* out = gp + r * gps + sub * NB2;
-#pragma unroll
-      for (int b2 = 0; b2 < NB2; ++b2) out[b2] = gv[b2];
-    }
-    if (!PRE && rowOn) {
-      const double2* u = sU2 + r * U2S;
-      double2* out = gp + r * gps + sub * NB2;
-      switch (nbw) {
-        case 1: ep2_rot_el<T2v, NWX, NB2, 1>(g, u, out); break;
-        case 2: ep2_rot_el<T2v, NWX, NB2, 2>(g, u, out); break;
-        case 3: ep2_rot_el<T2v, NWX, NB2, 3>(g, u, out); break;
-        case 4: ep2_rot_el<T2v, NWX, NB2, 4>(g, u, out); break;
-        default:
-          if constexpr (NB2 > 4) ep2_rot_el<T2v, NWX, NB2, NB2>(g, u, out);
-      }
-    }
-    wave_sync();
-    // B: phonon rotation, thread nu2 = sub, then |g|^2 and the b2 groups
-    double* own = gsq + (size_t(r) * nm + sub) * NB2;
-    if (rowOn) {
-      const double2* x = gp + r * gps;
-      switch (nbw) {
-        case 1: ep2_rot_ph<T2v, NMX, NB2, 1>(e3c, x, nm, own); break;
-        case 2: ep2_rot_ph<T2v, NMX, NB2, 2>(e3c, x, nm, own); break;
-        case 3: ep2_rot_ph<T2v, NMX, NB2, 3>(e3c, x, nm, own); break;
-        case 4: ep2_rot_ph<T2v, NMX, NB2, 4>(e3c, x, nm, own); break;
-        default:
-          if constexpr (NB2 > 4) ep2_rot_ph<T2v, NMX, NB2, NB2>(e3c, x, nm, own);
-      }
-      const double* e2r = se2 + r * NB2;
-      for (int b = 0; b < nb2;) {
-        int deg = 0;
-        for (int i = b; i < nb2; ++i) {
-          if (fabs(e2r[b] - e2r[i]) < 1.0e-6) deg++;
-          else break;
-        }
-        if (deg > 1) {
-          double s2 = 0.;
-          for (int i = 0; i < deg; ++i) s2 += own[b + i] / double(float(deg));
-          for (int i = 0; i < deg; ++i) own[b + i] = s2;
-        }
-        b += deg;
-      }
-    }
-    wave_sync();
-    const double w3c = w3;
-    const int grpc = grp;
-    double n3c[CM];
-#pragma unroll
-    for (int c = 0; c < CM; ++c) n3c[c] = n3[c];
-    // C: the nu groups and the Gaussian weights
-    if (rowOn && w3c >= p.cutoff) {
-      const int mystart = grpc & 0xff, mydeg = grpc >> 8;
-      const double* g0 = gsq + (size_t(r) * nm + mystart) * NB2;
-      const double wfac = p.norm / w3c * 3.14159265358979323846;  // once per lane, not per term
-#pragma unroll 1
-      for (int b2 = 0; b2 < nb2; ++b2) {
-        double vb;
-        if (mydeg > 1) {
-          vb = 0.;
-          for (int i = 0; i < mydeg; ++i) vb += g0[size_t(i) * NB2 + b2] / double(float(mydeg));
-        } else {
-          vb = own[b2];
-        }
-        const double en2 = se2[r * NB2 + b2];
-        const double cpl = vb * inv_g;
-#pragma unroll
-        for (int gi = 0; gi < GM; ++gi) {
-          if (gi >= gsize) break;
-          const double x1 = se1[gi] - en2 + w3c, x2 = se1[gi] - en2 - w3c;
-          if (p.screen > 0. && fmin(fabs(x1), fabs(x2)) * p.invSigma >= scrW) continue;
-          const double d1 = gaussian_delta(x1, p.invSigma, p.deltaPref);
-          const double d2 = gaussian_delta(x2, p.invSigma, p.deltaPref);
-          if (d1 <= 0. && d2 <= 0.) continue;
-#pragma unroll
-          for (int c = 0; c < CM; ++c) {
-            if (c >= p.nCalc) break;
-            const double f2 = sf2[(c * R + r) * NB2 + b2];
-            part[gi][c] += cpl * ((f2 + n3c[c]) * d1 + (1. - f2 + n3c[c]) * d2) * wfac;
-          }
-        }
-      }
-    }
-    __syncthreads();  // the next pass rewrites the row data
-  }
-  // wave reduction of the partial linewidths into partial[slot]
-  double* red = reinterpret_cast<double*>(smem);
-  const int lane = t & 63;
-#pragma unroll
-  for (int gi = 0; gi < GM; ++gi)
-#pragma unroll
-    for (int c = 0; c < CM; ++c) {
-      double v = part[gi][c];
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-      if (lane == 0) red[gi * kCMax + c] = v;
-    }
-  __syncthreads();
-  if (t < kGMax * kCMax) {
-    const int c = t % kCMax, gi = t / kCMax;
-    p.partial[size_t(slot) * kGMax * kCMax + t] = (c < CM && gi < GM) ? red[t] : 0.;
-  }
-}
-
-inline size_t sep_ep2_lds_bytes(int nm, int nb2, int cm, int rpw) {
-  size_t b = (64 * sizeof(SepXmRow) + 15) / 16 * 16;
-  b += size_t(rpw) * (16 * nb2 + 1) * sizeof(double2);              // U2, later |g|^2
-  b += size_t(rpw) * (nm * nb2 + 1) * sizeof(double2);              // g'
-  b += size_t(rpw) * nb2 * sizeof(double) * (1 + cm);               // e2, occupations
-  b += size_t(kGMax) * sizeof(double);                              // e1
-  return std::max(b, size_t(kGMax) * kCMax * sizeof(double)) + 64;
-}
+// The epilogue kernel (sep_epilogue.hpp) of `grid` slots on stream s: rows per
+// pass and template instance by the mode count, band counts, b1 groups and
+// calculations of the launch.  pre: G3 holds g' (FP32 data only).
+template <typename T>
+void launch_ep2(EpParams q, int gsizeMax, int grid, bool pre, hipStream_t s);
 
 constexpr int kXminBlocks = 64;
 
@@ -2981,12 +2388,12 @@ inline size_t sep_xm_lds_bytes(int elem, int nG0, int m0, int nw, int nm, int nb
   return std::max(b, size_t(kGMax) * kCMax * 4 * sizeof(double)) + 64;
 }
 
-// maxLineE / maxGrpE: largest number of entries of a line / group (LDS sizing).
+// maxLineE: largest number of entries of a line (LDS sizing).
 template <typename T>
-void launch_separable_zy(const SepParams& sp, int maxLineE, int maxGrpE, hipStream_t s, bool yStage = true) {
+void launch_separable_zy(const SepParams& sp, int maxLineE, hipStream_t s, bool yStage = true) {
   if (sp.nPanels <= 0) return;
   const size_t ldsZ = sep_stage_lds_bytes(sizeof(T), maxLineE, sp.ncol, sp.mz);
-  const size_t ldsY = sep_stage_lds_bytes(sizeof(T), maxGrpE, sp.ncol, sp.my);
+  const size_t ldsY = sep_y_lds_bytes(sp.my, sp.nQuads);
   PHX_REQUIRE(ldsZ <= 160 * 1024 && ldsY <= 160 * 1024, "separable transform: LDS budget exceeded");
   PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sep_z<T>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, int(std::max<size_t>(ldsZ, 16))));
@@ -2995,7 +2402,7 @@ void launch_separable_zy(const SepParams& sp, int maxLineE, int maxGrpE, hipStre
   hipLaunchKernelGGL(k_sep_z<T>, dim3(sp.nLines, sp.nPanels), dim3(256), ldsZ, s, sp);
   PHX_HIP(hipGetLastError());
   if (!yStage) return;  // the x-stage kernel runs the y-stage itself (k_sep_yx)
-  hipLaunchKernelGGL(k_sep_y<T>, dim3(sp.nG0, sp.mz, sp.nPanels), dim3(256), ldsY, s, sp);
+  hipLaunchKernelGGL(k_sep_y<T>, dim3(ceil_div(sp.ncol, 16), sp.mz, sp.nPanels), dim3(256), ldsY, s, sp);
   PHX_HIP(hipGetLastError());
 }
 
@@ -3009,6 +2416,15 @@ struct EpFork {
   hipEvent_t xgStart = nullptr;  // timing: recorded on the launch's stream right before the x-stage kernel
 };
 
+// Whether the last stage runs split (x-stage and epilogue kernels, g3 through
+// HBM), which the z-stage has to know too: its columns are then (w2, nu).
+// k_sep_yx takes any width and both precisions; k_sep_xg FP32 and at most 192 columns.
+template <typename T>
+inline bool sep_runs_split(const SepParams& sp, const CoupParams& p) {
+  return p.G3 && !p.bf16x3 && p.keepMask && p.nw <= 16 && (2 * p.nG0 + 3) / 4 <= 12 && sp.ncol <= 4 * 6 * 16 &&
+         (p.fuseYX || (sizeof(T) == 4 && sp.ncol <= 4 * 3 * 16 && p.nm <= 16));
+}
+
 // mid (optional): recorded between the x-stage and the epilogue kernel when
 // the last stage runs split.  Returns whether it did (then the epilogue ran
 // on fork.ep when that is set).
@@ -3017,7 +2433,7 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
                         hipEvent_t mid, const EpFork& fork = EpFork{}) {
   PHX_REQUIRE(p.nm <= kSepNm && p.nb2max <= kSepNb2,
               "separable transform supports nm <= 32 and at most 8 bands per inner point");
-  PHX_REQUIRE(!p.fuseYX || (sizeof(T) == 4 && reduce), "separable transform: fused y/x-stage is FP32 only");
+  PHX_REQUIRE(!p.fuseYX || reduce, "separable transform: the fused y/x-stage belongs to the reduction");
   if (sp.nPanels <= 0) return false;
   const int tiles = sp.nPanels * sp.my * sp.mz;
   const int grid = ceil_div(tiles, 8) * 8;
@@ -3047,158 +2463,84 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
       hipLaunchKernelGGL(k_sep_screen, dim3(ceil_div(tiles, 256)), dim3(256), 0, s, p);
       PHX_HIP(hipGetLastError());
     }
-    if constexpr (sizeof(T) == 4) {
-      // the lean epilogue also takes slot masks and a gate (the learned screen's passes)
-      const bool ep2ok = !p.epFirst && !p.adaptive && p.nb2max <= 8;
-      const bool split = p.G3 && !bf3 && !wide && p.keepMask && (ep2ok || (!p.slotOn && !p.gate)) &&
-                         p.nm <= 16 && p.nw <= 16 && (2 * p.nG0 + 3) / 4 <= 12;
-      PHX_REQUIRE(split || !p.fuseYX, "separable transform: fused y/x-stage outside the split last stage");
-      if (split) {
-        // the electron rotation in the x-stage kernel: with the lean epilogue only
-        const bool rot = p.epRot && ep2ok;
+    const bool split = sep_runs_split<T>(sp, p);
+    PHX_REQUIRE(split == (sp.modeFast != 0), "separable transform: column order of the split last stage");
+    PHX_REQUIRE(split || !p.fuseYX, "separable transform: fused y/x-stage outside the split last stage");
+    if (split) {
+      if (fork.xgStart) PHX_HIP(hipEventRecord(fork.xgStart, s));
+      // the electron rotation in the x-stage kernel: FP32 and fixed smearing only
+      const bool rot = p.epRot && !p.adaptive && !p.fuseYX;
+      if (p.fuseYX) {
+        PHX_REQUIRE(!p.slotOn && !p.gate, "separable transform: fused y/x-stage without slot masks");
+        const size_t ldsYX = sep_yx_lds_bytes(sizeof(T), sp.nQuads, sp.my, sp.nG0, p.m0);
+        PHX_REQUIRE(ldsYX <= 160 * 1024, "separable transform: LDS budget exceeded");
+        PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sep_yx<T>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(ldsYX)));
+        hipLaunchKernelGGL(k_sep_yx<T>, dim3(ceil_div(sp.ncol, 16), sp.mz, sp.nPanels), dim3(256), ldsYX, s, sp, p);
+      } else if constexpr (sizeof(T) == 4) {
         const size_t ldsA = sep_xg_lds_bytes(sizeof(T), p.nG0, p.m0, p.nm, p.nw, rot, p.nb2max);
-        // whole rows of nm threads per wave, at most 8, fewer if the LDS
-        // budget needs it (4 rows per wave always fit what 16 x 16 threads did)
-        CoupParams pe = p;
-        int rpw = std::min(64 / p.nm, 8);
-        constexpr int nWaves = kSepEpThreads / 64;
-        while (rpw > 4 && sep_ep_lds_bytes(p.nw, p.nm, p.nb2max, p.nCalc, nWaves * rpw) > 160 * 1024) --rpw;
-        pe.epRows = nWaves * rpw;
-        const size_t ldsB = sep_ep_lds_bytes(p.nw, p.nm, p.nb2max, p.nCalc, pe.epRows);
-        PHX_REQUIRE(ldsA <= 160 * 1024 && ldsB <= 160 * 1024, "separable transform: LDS budget exceeded");
+        PHX_REQUIRE(ldsA <= 160 * 1024, "separable transform: LDS budget exceeded");
         auto xg = [&](auto kern) {
           PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(ldsA)));
           hipLaunchKernelGGL(kern, dim3(grid), dim3(256), ldsA, s, p);
         };
-        if (fork.xgStart) PHX_HIP(hipEventRecord(fork.xgStart, s));
-        if (p.fuseYX) {
-          if constexpr (sizeof(T) == 4) {
-            PHX_REQUIRE(!rot && !p.slotOn && !p.gate, "separable transform: fused y/x-stage without slot masks");
-            const size_t ldsYX = sep_yx_lds_bytes(sp.nLines, sp.nG0, p.m0);
-            PHX_REQUIRE(ldsYX <= 160 * 1024, "separable transform: LDS budget exceeded");
-            PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sep_yx),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(ldsYX)));
-            hipLaunchKernelGGL(k_sep_yx, dim3(ceil_div(sp.ncol, 16), sp.mz, sp.nPanels), dim3(256), ldsYX, s, sp,
-                               p);
-          }
-        } else if (rot) {
-          xg(k_sep_xg<T, 3, true>);
-        } else {
-          xg(k_sep_xg<T, 3, false>);
-        }
-        PHX_HIP(hipGetLastError());
-        if (mid) PHX_HIP(hipEventRecord(mid, s));
-        hipStream_t se = s;
-        if (fork.ep) {
-          PHX_HIP(hipEventRecord(fork.xgDone, s));
-          PHX_HIP(hipStreamWaitEvent(fork.ep, fork.xgDone, 0));
-          se = fork.ep;
-        }
-        if (fork.epStart) PHX_HIP(hipEventRecord(fork.epStart, se));
-        auto ep = [&](auto kern) {
-          PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(ldsB)));
-          hipLaunchKernelGGL(kern, dim3(grid), dim3(kSepEpThreads), ldsB, se, pe);
-        };
-        // partial sums held per thread: calculations x b1-group members of
-        // the launch, no more than the launch needs
-        const int gm = p.gsizeMax > 0 ? p.gsizeMax : kGMax;
-        PHX_REQUIRE(gm <= kGMax, "separable transform: b1 group larger than kGMax");
-        if (ep2ok) {
-          // lean epilogue: rows per pass capped by its U2 prefetch registers
-          const int nb2 = p.nb2max <= 4 ? 4 : 8;
-          const int rpw2 = std::min(64 / p.nm, nb2 <= 4 ? 5 : 4);
-          const int cm = one ? 1 : p.nCalc <= 2 ? 2 : kCMax;
-          const size_t lds2 = sep_ep2_lds_bytes(p.nm, nb2, cm, rpw2);
-          PHX_REQUIRE(lds2 <= 160 * 1024, "separable transform: LDS budget exceeded");
-          EpParams q{};
-          q.keepMask = p.keepMask;
-          q.partial = p.partial;
-          q.panelKK = p.panelKK;
-          q.panelGStart = p.panelGStart;
-          q.panelGSize = p.panelGSize;
-          q.kkMesh = p.kkMesh;
-          q.kkStateOff = p.kkStateOff;
-          q.meshRow = p.meshRow;
-          q.e1pool = p.e1pool;
-          q.e2pool = p.e2pool;
-          q.Wpool = p.Wpool;
-          q.qModeGrp = p.qModeGrp;
-          q.U2pool = p.U2pool;
-          q.fermi = p.fermi;
-          q.bose = p.bose;
-          q.E3T = p.E3T;
-          q.G3 = p.G3;
-          q.screenOf = p.screenOf;
-          q.keptRows = p.keptRows;
-          q.keptBands = p.keptBands;
-          q.slotOn = p.slotOn;
-          q.gate = p.gate;
-          q.slotZero = p.slotZero;
-          q.invSigma = p.invSigma;
-          q.deltaPref = p.deltaPref;
-          q.norm = p.norm;
-          q.cutoff = p.cutoff;
-          q.screen = p.screen;
-          q.m0 = p.m0;
-          q.m1 = p.m1;
-          q.m2 = p.m2;
-          q.nPanels = p.nPanels;
-          q.nm = p.nm;
-          q.nw = p.nw;
-          q.nCalc = p.nCalc;
-          q.numStates = p.numStates;
-          q.rpw = rpw2;
-          q.nb2max = p.nb2max;
-          auto ep2 = [&](auto kern) {
-            PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds2)));
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(64), lds2, se, q);
-          };
-          auto ep2f = [&](auto nmx, auto nb2c, auto fz) {
-            constexpr int NM = decltype(nmx)::value, NB = decltype(nb2c)::value;
-            constexpr bool F = decltype(fz)::value;
-            if (gm <= 4) {
-              if (one) ep2(k_sep_ep2<T, 1, NM, 4, NB, F>);
-              else if (p.nCalc <= 2) ep2(k_sep_ep2<T, 2, NM, 4, NB, F>);
-              else ep2(k_sep_ep2<T, kCMax, NM, 4, NB, F>);
-            } else {
-              if (one) ep2(k_sep_ep2<T, 1, NM, kGMax, NB, F>);
-              else if (p.nCalc <= 2) ep2(k_sep_ep2<T, 2, NM, kGMax, NB, F>);
-              else ep2(k_sep_ep2<T, kCMax, NM, kGMax, NB, F>);
-            }
-          };
-          auto ep2c = [&](auto nmx, auto nb2c) {
-            if (rot) ep2f(nmx, nb2c, std::true_type{});
-            else ep2f(nmx, nb2c, std::false_type{});
-          };
-          using I12 = std::integral_constant<int, 12>;
-          using I16 = std::integral_constant<int, 16>;
-          using B4 = std::integral_constant<int, 4>;
-          using B8 = std::integral_constant<int, 8>;
-          if (p.nm <= 12) nb2 <= 4 ? ep2c(I12{}, B4{}) : ep2c(I12{}, B8{});
-          else nb2 <= 4 ? ep2c(I16{}, B4{}) : ep2c(I16{}, B8{});
-          PHX_HIP(hipGetLastError());
-          return true;
-        }
-        auto epc = [&](auto nmx) {
-          constexpr int NM = decltype(nmx)::value;
-          if (gm <= 4) {
-            if (one) ep(k_sep_ep<T, 1, NM, 4>);
-            else if (p.nCalc <= 2) ep(k_sep_ep<T, 2, NM, 4>);
-            else ep(k_sep_ep<T, kCMax, NM, 4>);
-          } else {
-            if (one) ep(k_sep_ep<T, 1, NM, kGMax>);
-            else if (p.nCalc <= 2) ep(k_sep_ep<T, 2, NM, kGMax>);
-            else ep(k_sep_ep<T, kCMax, NM, kGMax>);
-          }
-        };
-        if (p.nm <= 12) epc(std::integral_constant<int, 12>{});
-        else epc(std::integral_constant<int, 16>{});
-        PHX_HIP(hipGetLastError());
-        return true;
+        if (rot) xg(k_sep_xg<T, 3, true>);
+        else xg(k_sep_xg<T, 3, false>);
       }
+      PHX_HIP(hipGetLastError());
+      if (mid) PHX_HIP(hipEventRecord(mid, s));
+      hipStream_t se = s;
+      if (fork.ep) {
+        PHX_HIP(hipEventRecord(fork.xgDone, s));
+        PHX_HIP(hipStreamWaitEvent(fork.ep, fork.xgDone, 0));
+        se = fork.ep;
+      }
+      if (fork.epStart) PHX_HIP(hipEventRecord(fork.epStart, se));
+      EpParams q{};
+      q.keepMask = p.keepMask;
+      q.partial = p.partial;
+      q.panelKK = p.panelKK;
+      q.panelGStart = p.panelGStart;
+      q.panelGSize = p.panelGSize;
+      q.kkMesh = p.kkMesh;
+      q.kkStateOff = p.kkStateOff;
+      q.meshRow = p.meshRow;
+      q.e1pool = p.e1pool;
+      q.e2pool = p.e2pool;
+      q.Wpool = p.Wpool;
+      q.qModeGrp = p.qModeGrp;
+      q.U2pool = p.U2pool;
+      q.fermi = p.fermi;
+      q.bose = p.bose;
+      q.E3T = p.E3T;
+      q.G3 = p.G3;
+      q.screenOf = p.screenOf;
+      q.keptRows = p.keptRows;
+      q.keptBands = p.keptBands;
+      q.slotOn = p.slotOn;
+      q.gate = p.gate;
+      q.slotZero = p.slotZero;
+      q.invSigma = p.invSigma;
+      q.deltaPref = p.deltaPref;
+      q.norm = p.norm;
+      q.cutoff = p.cutoff;
+      q.screen = p.screen;
+      q.m0 = p.m0;
+      q.m1 = p.m1;
+      q.m2 = p.m2;
+      q.nPanels = p.nPanels;
+      q.nm = p.nm;
+      q.nw = p.nw;
+      q.nCalc = p.nCalc;
+      q.numStates = p.numStates;
+      q.nb2max = p.nb2max;
+      q.adaptive = p.adaptive;
+      q.stateV = p.stateV;
+      for (int i = 0; i < 9; ++i) q.qT[i] = p.qT[i];
+      q.minWidth = p.minWidth;
+      launch_ep2<T>(q, p.gsizeMax, grid, rot, se);
+      return true;
     }
     auto go = [&](auto kern) {
       PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -3247,13 +2589,6 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
   }
   PHX_HIP(hipGetLastError());
   return false;
-}
-
-template <typename T>
-void launch_separable(const SepParams& sp, const CoupParams& p, bool reduce, int maxLineE,
-                      int maxGrpE, hipStream_t s) {
-  launch_separable_zy<T>(sp, maxLineE, maxGrpE, s);
-  launch_separable_x<T>(sp, p, reduce, s, nullptr);
 }
 
 }  // namespace phx
