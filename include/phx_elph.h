@@ -62,8 +62,9 @@ int phx_device_count(int* count);
  * (src/common_kokkos.h:49, common_kokkos.cpp:11-100).
  *   A  : M matrices N x N, column-major complex; on return the eigenvectors
  *        (columns), eigenvalues ascending in W (M x N).
- *   info (optional, M ints): Jacobi sweeps used, -1 if not converged.
- * N <= 44 (the matrix and its eigenvectors stay in one wavefront's LDS). */
+ *   info (optional, M ints): most iterations spent on an eigenvalue, -1 if not
+ *   converged.
+ * N <= 44. */
 int phx_zheev_batched(int M, int N, double* A, double* W, int* info);
 
 /* Same on device buffers, enqueued on a HIP stream (0 = default stream). */

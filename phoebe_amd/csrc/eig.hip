@@ -1,14 +1,14 @@
-// Batched Hermitian eigensolver: one matrix per wavefront, LDS resident.
+// Batched Hermitian eigensolver, LDS resident.
 //
 // Replaces kokkosZHEEV (common_kokkos.cpp:11-100): eigenvalues ascending,
 // eigenvectors written over the input as the columns of a column-major
 // matrix (each matrix contiguous, LayoutStride (N^2,1,N), common_kokkos.cpp:
-// 32-41; electron_h0_wannier.cpp:787-791).  The algorithm is a parallel
-// cyclic complex Jacobi method with round-robin pair ordering: all N/2
-// disjoint rotations of a round are applied at once by the 64 lanes, the
-// matrix and the accumulated eigenvectors stay in LDS for all sweeps.
+// 32-41; electron_h0_wannier.cpp:787-791).  Electrons: k_eig_ql.  Phonons: a
+// parallel cyclic complex Jacobi method with round-robin pair ordering: all N/2
+// disjoint rotations of a round are applied at once, the matrix and the
+// accumulated eigenvectors stay in LDS for all sweeps.
 //
-// The phonon variant fuses the steps either side of the eigensolve in
+// The phonon kernels fuse the steps either side of the eigensolve in
 // PhononH0::kokkosBatchedBuildBlochHamiltonian / DiagonalizeFromCoordinates
 // (phonon_h0_kokkos.cpp:150-170, 186-219): D <- (D + D^H)/2 / sqrt(M_m M_n)
 // before, omega = sign(l) sqrt|l| and e_m <- e_m / sqrt(M_m) after.
@@ -35,7 +35,6 @@ __device__ inline int rr_player(int pos, int round, int n) {
   return (round + pos - 1) % (n - 1) + 1;
 }
 
-template <bool PHONON>
 __global__ void __launch_bounds__(64) k_jacobi(int N, int M, double2* __restrict__ A,
                                                double* __restrict__ W, int* __restrict__ info,
                                                const double* __restrict__ masses, int maxSweeps) {
@@ -54,16 +53,10 @@ __global__ void __launch_bounds__(64) k_jacobi(int N, int M, double2* __restrict
   for (int e = lane; e < NN; e += 64) {
     int i = e % N, j = e / N;
     double2 x;
-    if (PHONON) {
-      double2 aij = Am[i + N * j], aji = Am[j + N * i];
-      x = make_double2(0.5 * (aij.x + aji.x), 0.5 * (aij.y - aji.y));
-      x.x /= sqrt(masses[i] * masses[j]);
-      x.y /= sqrt(masses[i] * masses[j]);
-    } else {
-      // lower triangle is the reference (uplo = L)
-      x = (i >= j) ? Am[i + N * j] : cconj(Am[j + N * i]);
-      if (i == j) x.y = 0.;
-    }
+    double2 aij = Am[i + N * j], aji = Am[j + N * i];
+    x = make_double2(0.5 * (aij.x + aji.x), 0.5 * (aij.y - aji.y));
+    x.x /= sqrt(masses[i] * masses[j]);
+    x.y /= sqrt(masses[i] * masses[j]);
     a[e] = x;
     v[e] = make_double2(i == j ? 1. : 0., 0.);
   }
@@ -169,15 +162,13 @@ __global__ void __launch_bounds__(64) k_jacobi(int N, int M, double2* __restrict
       rank += (dj < di) || (dj == di && j < i);
     }
     double lam = di;
-    if (PHONON) lam = lam > 0. ? sqrt(lam) : -sqrt(-lam);
+    lam = lam > 0. ? sqrt(lam) : -sqrt(-lam);
     W[size_t(mat) * N + rank] = lam;
     for (int k = 0; k < N; ++k) {
       double2 x = v[k + N * i];
-      if (PHONON) {
-        double s = sqrt(masses[k]);
-        x.x /= s;
-        x.y /= s;
-      }
+      double s = sqrt(masses[k]);
+      x.x /= s;
+      x.y /= s;
       Am[k + N * rank] = x;
     }
   }
@@ -188,7 +179,7 @@ size_t jacobi_lds_bytes(int N) {
   return size_t(2) * N * N * sizeof(double2) + 32 * sizeof(Rot) + 64 * sizeof(double);
 }
 
-// The same Jacobi method with the order N fixed at compile time and 64 / L
+// The Jacobi method with the order N fixed at compile time and 64 / L
 // matrices per wavefront, L >= N lanes each: every lane works on one matrix,
 // index arithmetic is by constants, and a wave issues its instructions for
 // several matrices at once.  Each matrix goes through the rotations of the
@@ -196,7 +187,7 @@ size_t jacobi_lds_bytes(int N) {
 // element; the wave runs sweeps until all its matrices have converged (a
 // converged matrix's rotations are skipped, so its result and sweep count
 // are its own).
-template <bool PHONON, int N, int L>
+template <int N, int L>
 __global__ void __launch_bounds__(64) k_jacobi_n(int M, double2* __restrict__ A, double* __restrict__ W,
                                                  int* __restrict__ info, const double* __restrict__ masses,
                                                  int maxSweeps) {
@@ -216,15 +207,10 @@ __global__ void __launch_bounds__(64) k_jacobi_n(int M, double2* __restrict__ A,
     const int i = e % N, j = e / N;
     double2 x = make_double2(0., 0.);
     if (on) {
-      if (PHONON) {
-        const double2 aij = Am[i + N * j], aji = Am[j + N * i];
-        x = make_double2(0.5 * (aij.x + aji.x), 0.5 * (aij.y - aji.y));
-        x.x /= sqrt(masses[i] * masses[j]);
-        x.y /= sqrt(masses[i] * masses[j]);
-      } else {
-        x = (i >= j) ? Am[i + N * j] : cconj(Am[j + N * i]);
-        if (i == j) x.y = 0.;
-      }
+      const double2 aij = Am[i + N * j], aji = Am[j + N * i];
+      x = make_double2(0.5 * (aij.x + aji.x), 0.5 * (aij.y - aji.y));
+      x.x /= sqrt(masses[i] * masses[j]);
+      x.y /= sqrt(masses[i] * masses[j]);
     }
     a[e] = x;
     v[e] = make_double2(i == j ? 1. : 0., 0.);
@@ -329,19 +315,301 @@ __global__ void __launch_bounds__(64) k_jacobi_n(int M, double2* __restrict__ A,
       rank += (dj < di) || (dj == di && j < i);
     }
     double lam = di;
-    if (PHONON) lam = lam > 0. ? sqrt(lam) : -sqrt(-lam);
+    lam = lam > 0. ? sqrt(lam) : -sqrt(-lam);
     W[size_t(mat) * N + rank] = lam;
     for (int k = 0; k < N; ++k) {
       double2 x = v[k + N * i];
-      if (PHONON) {
-        const double s = sqrt(masses[k]);
-        x.x /= s;
-        x.y /= s;
-      }
+      const double s = sqrt(masses[k]);
+      x.x /= s;
+      x.y /= s;
       Am[k + N * rank] = x;
     }
   }
   if (on && li == 0 && info) info[mat] = mySweeps >= 0 ? mySweeps : -1;
+}
+
+// ------------------------------------------------------------------ tridiagonal form and QL
+// Electron matrices, any order: Householder reduction to a real tridiagonal
+// matrix, the unitary factor formed in place, and implicit QL iterations with
+// Wilkinson's shift on it (Bowdler, Martin, Reinsch and Wilkinson, Numerische
+// Mathematik 11 (1968) 293-306), about a tenth of the operations of cyclic
+// Jacobi.  L lanes per matrix, L >= N the next of 8, 16, 32, 64, so 64 / L
+// matrices per wave; the matrix, then the factor, is the only array in LDS
+// (rows padded to an odd length, since both phases run through rows and through
+// columns).  A lane is a row in the reduction and in the rotations, a column
+// while the factor is formed; the scalar recurrences of QL are computed by all
+// lanes of a group alike, and the groups of a wave go through their (matrix,
+// eigenvalue, iteration) states in one loop, so a group never waits for
+// another's eigenvalue.
+// Bound by latency: the rotations' chain of dependent FP64 operations, at the
+// seven waves per CU whose matrices fit LDS.  32768 matrices of order 16: 3.85 ms
+// with one Jacobi matrix per wave (LDS-bound), 1.2 so.  The phonons keep Jacobi, which finds the small
+// eigenvalues of D(q), whose square roots are the acoustic frequencies, to better
+// than the norm's rounding.
+__device__ __forceinline__ void group_sync() {  // orders a wave's LDS accesses
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// v of the lane that a DPP control names (within rows of 16 lanes)
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  union { double d; int i[2]; } x{v};
+  x.i[0] = __builtin_amdgcn_update_dpp(0, x.i[0], CTRL, 0xf, 0xf, true);
+  x.i[1] = __builtin_amdgcn_update_dpp(0, x.i[1], CTRL, 0xf, 0xf, true);
+  return x.d;
+}
+
+// Sum over the L lanes of a group, the same in all of them: neighbours, quads
+// and halves of a row by DPP, rows by shuffles.
+template <int L>
+__device__ __forceinline__ double group_sum(double v) {
+  v += dpp_move<0xB1>(v);              // quad_perm [1, 0, 3, 2]
+  v += dpp_move<0x4E>(v);              // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0x141>(v);             // row_half_mirror: the other quad of 8
+  if (L >= 16) v += dpp_move<0x140>(v);  // row_mirror: the other 8 of 16
+#pragma unroll
+  for (int o = 16; o < L; o *= 2) v += __shfl_xor(v, o);
+  return v;
+}
+
+// 1 / sqrt(x), x normal: the hardware estimate and one third-order step.
+__device__ __forceinline__ double rsqrt_refined(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double h = fma(-x * y, y, 1.);
+  return fma(y * h, fma(0.375, h, 0.5), y);
+}
+
+inline size_t ql_lds_bytes(int N, int L) {
+  const size_t ld = N | 1;
+  return size_t(64 / L) * ((size_t(N) * ld + 2 * N) * sizeof(double2) + (size_t(2) * N + 2) * sizeof(double));
+}
+
+constexpr int kQlMaxIter = 60;  // QL iterations per eigenvalue (two or three are usual)
+
+template <int L>
+__global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict__ A, double* __restrict__ W,
+                                               int* __restrict__ info) {
+  extern __shared__ double2 lds[];
+  const int lane = threadIdx.x, sg = lane / L, li = lane % L;
+  const int mat = blockIdx.x * (64 / L) + sg;
+  const bool on = mat < M;
+  const int ld = N | 1;
+  double2* a = lds + size_t(sg) * (size_t(N) * ld + 2 * N);  // (row, column) at row + ld column
+  double2* sv = a + size_t(N) * ld;                          // Householder vector
+  double2* sw = sv + N;
+  double* d = reinterpret_cast<double*>(lds + size_t(64 / L) * (size_t(N) * ld + 2 * N)) + size_t(sg) * (2 * N + 2);
+  double* e = d + N;
+  double2* Am = A + size_t(on ? mat : 0) * N * N;
+  const bool row = li < N;
+
+  // the lower triangle is the reference (uplo = L); scaled by a power of two to
+  // a largest component near one, so that no square over- or underflows
+  double big = 0.;
+#pragma unroll 4
+  for (int j = 0; j < N; ++j) {
+    double2 x = make_double2(0., 0.);
+    if (row && on) {
+      x = li >= j ? Am[li + N * j] : cconj(Am[j + N * li]);
+      if (li == j) x.y = 0.;
+    }
+    if (row) a[li + ld * j] = x;
+    big = fmax(big, fmax(fabs(x.x), fabs(x.y)));
+  }
+#pragma unroll
+  for (int o = L / 2; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o));
+  const int ex = big > 0. && big < HUGE_VAL ? ilogb(big) : 0;
+  group_sync();
+  if (row)
+    for (int j = 0; j < N; ++j) {
+      const double2 x = a[li + ld * j];
+      a[li + ld * j] = make_double2(ldexp(x.x, -ex), ldexp(x.y, -ex));
+    }
+  group_sync();
+
+  // Householder: reflector k = I - tau v v^H, v(k + 1) = 1, maps column k below the
+  // diagonal to the real number beta; A <- H^H A H as A - v w^H - w v^H.
+  // v stays in column k (rows > k + 1), tau in sw's place at the end: kept in e's lanes
+  double2 tauK = make_double2(0., 0.);  // lane k holds tau of reflector k
+  for (int k = 0; k + 1 < N; ++k) {
+    const bool in = row && li > k;
+    const double2 x = in ? a[li + ld * k] : make_double2(0., 0.);
+    const double2 alpha = a[k + 1 + ld * k];
+    const double tail = group_sum<L>(li > k + 1 ? x.x * x.x + x.y * x.y : 0.);
+    double beta = alpha.x;
+    double2 tau = make_double2(0., 0.), v = make_double2(li == k + 1 ? 1. : 0., 0.);
+    if (tail > 0. || alpha.y != 0.) {
+      beta = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + tail);
+      if (alpha.x > 0.) beta = -beta;
+      tau = make_double2((beta - alpha.x) / beta, -alpha.y / beta);
+      // x / (alpha - beta)
+      const double ar = alpha.x - beta, ai = alpha.y, q = 1. / (ar * ar + ai * ai);
+      if (li > k + 1) v = make_double2((x.x * ar + x.y * ai) * q, (x.y * ar - x.x * ai) * q);
+    }
+    if (!in) v = make_double2(0., 0.);
+    if (li == k) tauK = tau;
+    if (li == 0) e[k] = beta;
+    if (in) sv[li] = v;
+    group_sync();
+    // p = tau A v
+    double2 p = make_double2(0., 0.);
+    if (in)
+#pragma unroll 4
+      for (int j = k + 1; j < N; ++j) {
+        const double2 aj = a[li + ld * j], vj = sv[j];
+        p.x += aj.x * vj.x - aj.y * vj.y;
+        p.y += aj.x * vj.y + aj.y * vj.x;
+      }
+    p = cmul(tau, p);
+    // w = p - (tau / 2) (p^H v) v, with tau p^H v = |tau|^2 v^H A v real
+    const double2 pv = make_double2(group_sum<L>(in ? p.x * v.x + p.y * v.y : 0.),
+                                    group_sum<L>(in ? p.x * v.y - p.y * v.x : 0.));
+    const double h = -0.5 * (tau.x * pv.x - tau.y * pv.y);
+    const double2 w = make_double2(p.x + h * v.x, p.y + h * v.y);
+    if (in) sw[li] = w;
+    group_sync();
+    if (in) {
+#pragma unroll 4
+      for (int j = k + 1; j < N; ++j) {
+        const double2 vj = sv[j], wj = sw[j];
+        double2 aj = a[li + ld * j];
+        aj.x -= v.x * wj.x + v.y * wj.y + w.x * vj.x + w.y * vj.y;
+        aj.y -= v.y * wj.x - v.x * wj.y + w.y * vj.x - w.x * vj.y;
+        a[li + ld * j] = aj;
+      }
+      if (li > k + 1) a[li + ld * k] = v;
+    }
+    group_sync();
+  }
+  if (row) d[li] = a[li + ld * li].x;
+  if (li == 0) e[N - 1] = 0.;
+
+  // Q = H_0 H_1 ... H_{N-2} in place: column k + 1 from reflector k (in column k), the
+  // columns beyond it (lane = column) by H_k
+  for (int k = N - 2; k >= 0; --k) {
+    const double2 tau = make_double2(__shfl(tauK.x, sg * L + k), __shfl(tauK.y, sg * L + k));
+    if (li > k + 1 && row) {
+      double2 y = make_double2(0., 0.);
+#pragma unroll 4
+      for (int i = k + 2; i < N; ++i) {
+        const double2 v = a[i + ld * k], q = a[i + ld * li];
+        y.x += v.x * q.x + v.y * q.y;
+        y.y += v.x * q.y - v.y * q.x;
+      }
+      y = cmul(tau, y);
+      a[k + 1 + ld * li] = make_double2(-y.x, -y.y);
+#pragma unroll 4
+      for (int i = k + 2; i < N; ++i) {
+        const double2 v = a[i + ld * k];
+        double2 q = a[i + ld * li];
+        q.x -= v.x * y.x - v.y * y.y;
+        q.y -= v.x * y.y + v.y * y.x;
+        a[i + ld * li] = q;
+      }
+    }
+    group_sync();
+    if (li > k && row) {  // lane = row
+      const double2 v = li == k + 1 ? make_double2(1., 0.) : a[li + ld * k];
+      const double2 t = cmul(tau, v);
+      a[li + ld * (k + 1)] = make_double2((li == k + 1 ? 1. : 0.) - t.x, -t.y);
+    }
+    group_sync();
+  }
+  if (row) {
+    a[li] = make_double2(li == 0 ? 1. : 0., 0.);
+    a[ld * li] = make_double2(li == 0 ? 1. : 0., 0.);
+  }
+  group_sync();
+
+  // implicit QL: eigenvalue l of the group, it iterations spent on it
+  int l = 0, it = 0, worst = 0;
+  bool bad = false;
+  while (__any(l < N && !bad)) {
+    if (l < N && !bad) {
+      // the first negligible off-diagonal from l on ends the block l .. m
+      bool small = false;
+      if (li >= l && li < N - 1) small = fabs(e[li]) <= 2.220446049250313e-16 * (fabs(d[li]) + fabs(d[li + 1]));
+      const unsigned long long ones = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
+      const unsigned long long hit = (__ballot(small) >> (sg * L)) & ones;
+      const int m = hit ? __ffsll(hit) - 1 : N - 1;
+      if (m == l) {
+        ++l;
+        it = 0;
+      } else if (it == kQlMaxIter) {
+        bad = true;
+      } else {
+        ++it;
+        worst = max(worst, it);
+        const double dl = d[l], el = e[l];
+        double g = (d[l + 1] - dl) / (2. * el);
+        g = d[m] - dl + el / (g + copysign(sqrt(g * g + 1.), g));
+        double s = 1., c = 1., p = 0.;
+        double2 f2 = row ? a[li + ld * m] : make_double2(0., 0.);  // column i + 1 of the lane's row
+        double dn = d[m];                                        // d(i + 1)
+        double di = d[m - 1], ei = e[m - 1];
+        double2 z = row ? a[li + ld * (m - 1)] : make_double2(0., 0.);
+        int i = m - 1;
+        bool cut = false;
+        for (; i >= l; --i) {
+          // the next rotation's operands, while this one's chain runs
+          const int in = max(i - 1, 0);
+          const double dnx = d[in], enx = e[in];
+          const double2 znx = row ? a[li + ld * in] : make_double2(0., 0.);
+          const double f = s * ei, b = c * ei;
+          const double r2 = f * f + g * g;
+          if (r2 < 1e-290) {  // zero next to the largest component, near one: the block splits at i + 1
+            if (li == 0) {
+              e[i + 1] = 0.;
+              d[i + 1] = dn - p;
+              e[m] = 0.;
+            }
+            cut = true;
+            break;
+          }
+          const double ri = rsqrt_refined(r2);
+          if (li == 0) e[i + 1] = r2 * ri;
+          s = f * ri;
+          c = g * ri;
+          g = dn - p;
+          const double t = (di - g) * s + 2. * c * b;
+          p = s * t;
+          if (li == 0) d[i + 1] = g + p;
+          g = c * t - b;
+          // columns i, i + 1 of the eigenvectors
+          if (row) a[li + ld * (i + 1)] = make_double2(s * z.x + c * f2.x, s * z.y + c * f2.y);
+          f2 = make_double2(c * z.x - s * f2.x, c * z.y - s * f2.y);
+          dn = di;
+          di = dnx;
+          ei = enx;
+          z = znx;
+        }
+        if (row) a[li + ld * (i + 1)] = f2;
+        if (!cut && li == 0) {
+          d[l] = dn - p;
+          e[l] = g;
+          e[m] = 0.;
+        }
+      }
+    }
+    group_sync();
+  }
+
+  // ascending order by rank (stable); lane = eigenvalue, then lane = row
+  int rank = 0;
+  if (row) {
+    const double di = d[li];
+    for (int j = 0; j < N; ++j) {
+      const double dj = d[j];
+      rank += (dj < di) || (dj == di && j < li);
+    }
+    if (on) W[size_t(mat) * N + rank] = ldexp(di, ex);
+  }
+  for (int j = 0; j < N; ++j) {
+    const int r = __shfl(rank, sg * L + j);
+    if (row && on) Am[li + N * r] = a[li + ld * j];
+  }
+  if (on && li == 0 && info) info[mat] = bad ? -1 : worst;
 }
 
 template <int N, int L>
@@ -353,35 +621,40 @@ static size_t jacobi_n_lds_bytes() {
 template <int N, int L>
 static void launch_jacobi_n(int M, double2* A, double* W, int* info, const double* masses, hipStream_t stream) {
   constexpr int G = 64 / L;
-  const size_t lds = jacobi_n_lds_bytes<N, L>();
-  const dim3 grid(ceil_div(M, G));
-  if (masses)
-    hipLaunchKernelGGL((k_jacobi_n<true, N, L>), grid, dim3(64), lds, stream, M, A, W, info, masses, 40);
-  else
-    hipLaunchKernelGGL((k_jacobi_n<false, N, L>), grid, dim3(64), lds, stream, M, A, W, info, nullptr, 40);
+  hipLaunchKernelGGL((k_jacobi_n<N, L>), dim3(ceil_div(M, G)), dim3(64), (jacobi_n_lds_bytes<N, L>()), stream, M, A, W,
+                     info, masses, 40);
 }
 
-// Launch the batched eigensolver on device buffers: the fixed-order kernel
-// for the orders of the path's matrices (6, 8, 12, 16 and 18: 2, 4 and 6
-// atoms, 8 and 16 Wannier functions), packed 8 or 4 matrices per wave up to
-// N = 12 and one per wave above (where 4 would hold 35 KB of LDS per
-// workgroup and leave one wave per SIMD), the runtime-order kernel otherwise.
+template <int L>
+static void launch_eig_ql(int N, int M, double2* A, double* W, int* info, hipStream_t stream) {
+  const size_t lds = ql_lds_bytes(N, L);
+  PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_eig_ql<L>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              int(lds)));
+  hipLaunchKernelGGL(k_eig_ql<L>, dim3(ceil_div(M, 64 / L)), dim3(64), lds, stream, N, M, A, W, info);
+}
+
+// Launch the batched eigensolver on device buffers.  Electrons (no masses):
+// the tridiagonal QL kernel, with the lanes per matrix that hold its rows.
+// Phonons: Jacobi, with the order fixed at compile time for 2, 4 and 6 atoms
+// (6, 12 and 18 modes), packed 8 or 4 matrices per wave up to N = 12 and one per
+// wave above (where 4 would hold 35 KB of LDS per workgroup and leave one wave
+// per SIMD), the runtime-order kernel otherwise.
 void launch_jacobi(int N, int M, double2* A, double* W, int* info, const double* masses,
                    hipStream_t stream) {
   PHX_REQUIRE(N >= 1 && N <= 64, "eigensolver supports 1 <= N <= 64");
   if (M <= 0) return;
-  switch (N) {
-    case 6: launch_jacobi_n<6, 8>(M, A, W, info, masses, stream); break;
-    case 8: launch_jacobi_n<8, 8>(M, A, W, info, masses, stream); break;
-    case 12: launch_jacobi_n<12, 16>(M, A, W, info, masses, stream); break;
-    case 16: launch_jacobi_n<16, 64>(M, A, W, info, masses, stream); break;
-    case 18: launch_jacobi_n<18, 64>(M, A, W, info, masses, stream); break;
-    default: {
-      const size_t lds = jacobi_lds_bytes(N);
-      if (masses)
-        hipLaunchKernelGGL(k_jacobi<true>, dim3(M), dim3(64), lds, stream, N, M, A, W, info, masses, 40);
-      else
-        hipLaunchKernelGGL(k_jacobi<false>, dim3(M), dim3(64), lds, stream, N, M, A, W, info, nullptr, 40);
+  if (!masses) {
+    if (N <= 8) launch_eig_ql<8>(N, M, A, W, info, stream);
+    else if (N <= 16) launch_eig_ql<16>(N, M, A, W, info, stream);
+    else if (N <= 32) launch_eig_ql<32>(N, M, A, W, info, stream);
+    else launch_eig_ql<64>(N, M, A, W, info, stream);
+  } else {
+    switch (N) {
+      case 6: launch_jacobi_n<6, 8>(M, A, W, info, masses, stream); break;
+      case 12: launch_jacobi_n<12, 16>(M, A, W, info, masses, stream); break;
+      case 18: launch_jacobi_n<18, 64>(M, A, W, info, masses, stream); break;
+      default:
+        hipLaunchKernelGGL(k_jacobi, dim3(M), dim3(64), jacobi_lds_bytes(N), stream, N, M, A, W, info, masses, 40);
     }
   }
   PHX_HIP(hipGetLastError());

@@ -1,0 +1,69 @@
+"""The electron eigensolver (Householder tridiagonalization + QL) over every
+lane layout (orders around 8, 16, 32) and over matrices it can trip on: block
+diagonal, diagonal, zero, rank one, graded, tiny and huge entries, exact
+degeneracies, many matrices per wave; the Bloch sums at few and many points."""
+import numpy as np
+import pytest
+
+import phoebe_amd as P
+from phoebe_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(A):
+    W, V = P.zheev_batched(A)
+    n = A.shape[1]
+    for i, H in enumerate(A):
+        low = np.tril(H, -1)
+        H = low + low.conj().T + np.diag(np.diag(H).real)  # uplo = L
+        wl = np.linalg.eigvalsh(H)
+        scale = max(np.abs(wl).max(), np.finfo(float).tiny)
+        # backward stable: a small multiple of n eps of the norm
+        tol = 8 * n * np.finfo(float).eps
+        assert np.abs(W[i] - wl).max() <= tol * scale, i
+        assert np.abs(V[i].conj().T @ V[i] - np.eye(n)).max() <= tol, i
+        assert np.abs((H / scale) @ V[i] - V[i] * (W[i] / scale)).max() <= tol, i
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 8, 9, 15, 16, 17, 23, 31, 32, 33, 44])
+def test_orders(n):
+    rng = np.random.default_rng(n)
+    cx = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)
+    X = cx(9, n, n)
+    A = X + X.conj().transpose(0, 2, 1)
+    A[1] = 0.0
+    A[2] = np.diag(rng.standard_normal(n))
+    u = cx(n)
+    A[3] = np.outer(u, u.conj())
+    A[4][: n // 2, n // 2:] = 0.0
+    A[4][n // 2:, : n // 2] = 0.0
+    g = 10.0 ** -np.arange(n)
+    A[5] = g[:, None] * A[5] * g[None, :]
+    A[6] *= 1e-180
+    A[7] *= 1e170
+    Q = np.linalg.qr(cx(n, n))[0]
+    lam = np.sort(rng.standard_normal(n))
+    lam[: max(1, n // 2)] = lam[0]
+    A[8] = (Q * lam) @ Q.conj().T
+    _check(A)
+
+
+@pytest.mark.parametrize("kind,n,nk", [("el", 3, 1), ("el", 8, 5), ("el", 9, 2100), ("el", 12, 700), ("el", 16, 8200),
+                                       ("el", 17, 33), ("ph", 6, 3), ("ph", 9, 2100), ("ph", 12, 8300), ("ph", 18, 40)])
+def test_bloch_sums(kind, n, nk):
+    f = synth.eig_family(kind, n, rgrid=3)
+    ks = (f["recip"] @ np.random.default_rng(n).uniform(0, 1, (3, nk))).T
+    if kind == "el":
+        E, _ = P.el_bloch_diag(ks, f["R"], f["weight"], f["coef"])
+    else:
+        E, _ = P.ph_bloch_diag(ks, f["R"], f["weight"], f["coef"], f["masses"])
+    pick = np.unique(np.concatenate([np.arange(min(nk, 4)), np.arange(max(0, nk - 4), nk)]))
+    for i in pick:
+        if kind == "el":
+            ref = np.linalg.eigvalsh(np.tensordot(np.exp(1j * (f["R"] @ ks[i])) / f["weight"], f["coef"], axes=(0, 0)))
+        else:
+            D = np.tensordot(np.exp(-1j * (f["R"] @ ks[i])) * f["weight"], f["coef"], axes=(0, 0))
+            lam = np.linalg.eigvalsh(0.5 * (D + D.conj().T) / np.sqrt(np.outer(f["masses"], f["masses"])))
+            ref = np.sign(lam) * np.sqrt(np.abs(lam))
+        assert np.abs(E[i] - ref).max() <= 1e-12 * np.abs(ref).max()
