@@ -10,32 +10,39 @@
 // Each workgroup owns TK wavevectors and a slice of the matrix entries; the
 // phases of a chunk of R vectors are generated once into LDS (FP64 sincos)
 // and every thread streams its entry's coefficient column with coalesced
-// loads, accumulating TK complex sums in registers.
+// loads, accumulating TK complex sums in registers.  Small matrices leave most
+// of 256 threads without an entry: with nE <= 64 (128) entries four (two) slices
+// of the threads share each chunk's R vectors, added up in LDS at the end.
+// Bound by FP64 FMAs at many wavevectors, by latency at few: TK is 16 where that
+// leaves at least 512 workgroups, else 4 or 1.  101 wavevectors, 8 x 8, 453 R:
+// 386 us with TK = 16 and one slice (7 workgroups of one busy wave), 21 us so.
 #include "phx_common.hpp"
 
 namespace phx {
 
-constexpr int kBlochTK = 16;
 constexpr int kBlochRC = 32;
 
-template <bool PHONON>
-__global__ void __launch_bounds__(256) k_bloch(int nk, int nE, int nR,
+template <bool PHONON, int TK>
+__global__ void __launch_bounds__(256) k_bloch(int nk, int nE, int nR, int slices,
                                                const double* __restrict__ kc,  // nk x 3
                                                const double* __restrict__ R,   // nR x 3
                                                const double* __restrict__ rw,  // nR (d or w)
                                                const void* __restrict__ coef,  // (nR, nE)
                                                double2* __restrict__ out,      // (nk, nE) col-major per k
                                                int nw) {
-  __shared__ double2 ph[kBlochTK][kBlochRC];
-  const int k0 = blockIdx.x * kBlochTK;
-  const int e = blockIdx.y * 256 + threadIdx.x;
-  double2 acc[kBlochTK];
+  constexpr int RC = kBlochRC * (TK < 16 ? 4 : 1);  // R vectors per chunk
+  __shared__ double2 ph[TK][RC];
+  __shared__ double2 red[256];
+  const int k0 = blockIdx.x * TK;
+  const int width = 256 / slices, slice = threadIdx.x / width;
+  const int e = blockIdx.y * width + threadIdx.x % width;
+  double2 acc[TK];
 #pragma unroll
-  for (int t = 0; t < kBlochTK; ++t) acc[t] = make_double2(0., 0.);
-  for (int r0 = 0; r0 < nR; r0 += kBlochRC) {
+  for (int t = 0; t < TK; ++t) acc[t] = make_double2(0., 0.);
+  for (int r0 = 0; r0 < nR; r0 += RC) {
     __syncthreads();
-    for (int i = threadIdx.x; i < kBlochTK * kBlochRC; i += 256) {
-      int t = i / kBlochRC, r = i % kBlochRC;
+    for (int i = threadIdx.x; i < TK * RC; i += 256) {
+      int t = i / RC, r = i % RC;
       int k = k0 + t, iR = r0 + r;
       double2 p = make_double2(0., 0.);
       if (k < nk && iR < nR) {
@@ -50,13 +57,14 @@ __global__ void __launch_bounds__(256) k_bloch(int nk, int nE, int nR,
     }
     __syncthreads();
     if (e < nE) {
-      const int rmax = min(kBlochRC, nR - r0);
-      for (int r = 0; r < rmax; ++r) {
+      const int rmax = min(RC, nR - r0);
+#pragma unroll 4
+      for (int r = slice; r < rmax; r += slices) {
         double2 h;
         if (PHONON) h = make_double2(static_cast<const double*>(coef)[size_t(r0 + r) * nE + e], 0.);
         else h = static_cast<const double2*>(coef)[size_t(r0 + r) * nE + e];
 #pragma unroll
-        for (int t = 0; t < kBlochTK; ++t) {
+        for (int t = 0; t < TK; ++t) {
           double2 p = ph[t][r];
           acc[t].x += p.x * h.x - p.y * h.y;
           acc[t].y += p.x * h.y + p.y * h.x;
@@ -64,11 +72,24 @@ __global__ void __launch_bounds__(256) k_bloch(int nk, int nE, int nR,
       }
     }
   }
-  if (e < nE) {
+  if (slices > 1) {
+#pragma unroll
+    for (int t = 0; t < TK; ++t) {
+      __syncthreads();
+      red[threadIdx.x] = acc[t];
+      __syncthreads();
+      if (slice == 0)
+        for (int j = 1; j < slices; ++j) {
+          acc[t].x += red[j * width + threadIdx.x].x;
+          acc[t].y += red[j * width + threadIdx.x].y;
+        }
+    }
+  }
+  if (e < nE && slice == 0) {
     // coefficient entry e = m*nw + n (row-major (m,n)); output column-major
     const int m = e / nw, n = e % nw;
 #pragma unroll
-    for (int t = 0; t < kBlochTK; ++t) {
+    for (int t = 0; t < TK; ++t) {
       int k = k0 + t;
       if (k < nk) out[size_t(k) * nE + m + size_t(nw) * n] = acc[t];
     }
@@ -169,11 +190,22 @@ void launch_bloch(bool phonon, int nk, int nw, int nR, const double* kc, const d
                   const double* rw, const void* coef, double2* out, hipStream_t stream) {
   if (nk <= 0) return;
   const int nE = nw * nw;
-  dim3 grid(ceil_div(nk, kBlochTK), ceil_div(nE, 256));
-  if (phonon)
-    hipLaunchKernelGGL(k_bloch<true>, grid, dim3(256), 0, stream, nk, nE, nR, kc, R, rw, coef, out, nw);
-  else
-    hipLaunchKernelGGL(k_bloch<false>, grid, dim3(256), 0, stream, nk, nE, nR, kc, R, rw, coef, out, nw);
+  const int slices = nE <= 64 ? 4 : nE <= 128 ? 2 : 1;
+  const int rows = ceil_div(nE, 256 / slices);
+  auto go = [&](auto kern, int tk) {
+    hipLaunchKernelGGL(kern, dim3(ceil_div(nk, tk), rows), dim3(256), 0, stream, nk, nE, nR, slices, kc, R, rw, coef,
+                       out, nw);
+  };
+  const int tk = ceil_div(nk, 16) * rows >= 512 ? 16 : ceil_div(nk, 4) * rows >= 512 ? 4 : 1;
+  if (phonon) {
+    if (tk == 16) go(k_bloch<true, 16>, tk);
+    else if (tk == 4) go(k_bloch<true, 4>, tk);
+    else go(k_bloch<true, 1>, tk);
+  } else {
+    if (tk == 16) go(k_bloch<false, 16>, tk);
+    else if (tk == 4) go(k_bloch<false, 4>, tk);
+    else go(k_bloch<false, 1>, tk);
+  }
   PHX_HIP(hipGetLastError());
 }
 
