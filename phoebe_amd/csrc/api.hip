@@ -48,9 +48,6 @@ void synth_gw_host(double* gW, size_t n, size_t blk, const double* decay, uint64
 template <typename T> void launch_fill(T* p, size_t n, T v, hipStream_t s);
 void launch_phase_table(int rows, int nR, const double* kc, const double* R, const double* scale,
                         double sign, double2* P, hipStream_t s);
-template <typename T>
-void launch_phase_rows(int nrows, int rowsPad, int nRp, int Kp, const double* kc, const double* R,
-                       T* A, hipStream_t s);
 void launch_gather_eig(int na, int nw, const int* ik, const int* lo, const int* nb, const int* off,
                        const double2* U, double2* pool, hipStream_t s);
 void launch_transpose_e3(int nk, int nm, const double2* ev, void* out, bool fp32, hipStream_t s);
@@ -68,7 +65,6 @@ extern template bool launch_separable_x<double>(const SepParams&, const CoupPara
                                                   const EpFork&);
 extern template bool launch_separable_x<float>(const SepParams&, const CoupParams&, bool, hipStream_t, hipEvent_t,
                                                   const EpFork&);
-int coupling_rows_per_tile_f64(int ldb);
 
 
 
@@ -500,7 +496,7 @@ struct ElphHandle {
   }
   // cached state of the last cacheElPh
   int nb1 = -1;
-  int Kp = 0, ldb = 0;
+  int ldb = 0;
   DevBuf<double> Bd;
   DevBuf<float> Bf;
   DevBuf<double2> U1;
@@ -539,7 +535,6 @@ static void elph_common_init(ElphHandle* H, int nw, int nm, int nRp, int nRe, co
   h2d(H->degE, elDeg, size_t(nRe), H->stream);
   h2d(H->Rp, phR, size_t(nRp) * 3, H->stream);
   h2d(H->degP, phDeg, size_t(nRp), H->stream);
-  H->Kp = int(round_up(2 * size_t(nRp), 16));
   H->ldb = int(round_up(2 * size_t(nm) * nw, 16));
 }
 
@@ -548,7 +543,7 @@ static void elph_common_init(ElphHandle* H, int nw, int nm, int nRp, int nRe, co
 static void elph_cache(ElphHandle* H, const double* U1, int nb1, const double* k1) {
   PHX_REQUIRE(nb1 >= 1 && nb1 <= H->nw, "cacheElPh: bad nb1");
   hipStream_t s = H->stream;
-  const size_t pstride = size_t(H->Kp) * H->ldb;
+  const size_t pstride = size_t(H->nRp) * H->ldb;
   if (nb1 > H->nb1 || H->nb1 < 0) {
     if (H->precision == PHX_FP64) {
       H->Bd.alloc(pstride * nb1);
@@ -587,9 +582,9 @@ static void elph_cache(ElphHandle* H, const double* U1, int nb1, const double* k
     }
     H->sPhE.reserve(cache_phase_size(H->nRe));
     if (H->precision == PHX_FP64)
-      launch_phase_cols<double>(1, H->nRe, H->sK.p, H->Re.p, H->invE.p, H->sPhE.p, s);
+      launch_phase_cols<double>(1, cache_phase_cols(1), H->nRe, H->sK.p, H->Re.p, H->invE.p, H->sPhE.p, s);
     else
-      launch_phase_cols<float>(1, H->nRe, H->sK.p, H->Re.p, H->invE.p, H->sPhE.p, s);
+      launch_phase_cols<float>(1, cache_phase_cols(1), H->nRe, H->sK.p, H->Re.p, H->invE.p, H->sPhE.p, s);
     CacheParams cp{};
     cp.nRe = H->nRe;
     cp.nRp = H->nRp;
@@ -623,9 +618,6 @@ static void elph_coupling_sq(ElphHandle* H, int nq, const double* U2s, const int
   if (nq <= 0) return;
   hipStream_t s = H->stream;
   const int nw = H->nw, nm = H->nm, nb1 = H->nb1;
-  const int rows = coupling_rows_per_tile_f64(H->ldb);
-  const int nMtiles = ceil_div(nq, rows);
-  const int rowsPad = nMtiles * rows;
   std::vector<int> u2off(nq), nb2v(nq), e3idx(nq);
   std::vector<long long> outoff(nq);
   long long totU2 = 0, totOut = 0;
@@ -653,15 +645,16 @@ static void elph_coupling_sq(ElphHandle* H, int nq, const double* U2s, const int
     launch_fill<double>(H->W0.p, H->W0.n, 0., s);
   }
   CoupParams p{};
-  p.lda = H->Kp;
-  p.Kp = H->Kp;
+  const bool f64 = H->precision == PHX_FP64;
+  p.lda = size_t(nq);
+  p.nRp = H->nRp;
   p.ldb = H->ldb;
-  p.panelStride = size_t(H->Kp) * H->ldb;
+  p.panelStride = size_t(H->nRp) * H->ldb;
   p.M = nq;
   p.nm = nm;
   p.nw = nw;
   p.nPanels = nb1;
-  p.nMtiles = nMtiles;
+  p.nMtiles = ceil_div(nq, coupling_tiling(f64, nm, nw, nb2max).rows);
   p.panelKK = H->meta.p + 4;
   p.panelB1 = H->meta.p + 4 + nb1;
   p.U2pool = H->sU2.p;
@@ -690,15 +683,15 @@ static void elph_coupling_sq(ElphHandle* H, int nq, const double* U2s, const int
     p.U1pool = H->U1.p;
     p.U1off = H->meta.p + 0;
   }
-  if (H->precision == PHX_FP64) {
-    H->sA.reserve(size_t(rowsPad) * H->Kp);
-    launch_phase_rows<double>(nq, rowsPad, H->nRp, H->Kp, H->sQ.p, H->Rp.p, H->sA.p, s);
+  if (f64) {
+    H->sA.reserve(2 * phase_cols_size(H->nRp, nq));
+    launch_phase_cols<double>(nq, nq, H->nRp, H->sQ.p, H->Rp.p, nullptr, H->sA.p, s);
     p.A = H->sA.p;
     p.B = H->Bd.p;
     launch_coupling<double>(p, false, s);
   } else {
-    H->sAf.reserve(size_t(rowsPad) * H->Kp);
-    launch_phase_rows<float>(nq, rowsPad, H->nRp, H->Kp, H->sQ.p, H->Rp.p, H->sAf.p, s);
+    H->sAf.reserve(2 * phase_cols_size(H->nRp, nq));
+    launch_phase_cols<float>(nq, nq, H->nRp, H->sQ.p, H->Rp.p, nullptr, H->sAf.p, s);
     p.A = H->sAf.p;
     p.B = H->Bf.p;
     launch_coupling<float>(p, false, s);
@@ -760,7 +753,7 @@ struct LwHandle {
   DevBuf<double2> E3Td;        // ... or FP64
   DevBuf<int> rowMesh, rowNb2, rowU2off, rowStateOff, gStartD, gSizeD;
   DevBuf<double> kcartActive;  // na x 3
-  int Kp = 0, ldb = 0, rows = 32, rowsPad = 0;
+  int ldb = 0;
   DevBuf<double> Ad;
   DevBuf<float> Af;
   // per-batch
@@ -1254,17 +1247,14 @@ static void lw_setup(LwHandle* L, const phx_problem* P, int precision, int k1Bat
   }
 
   // ---- GEMM A operand: e^{ik2.Rp} rows for every active point
-  L->Kp = int(round_up(2 * size_t(p.nRp), 16));
   L->ldb = int(round_up(2 * size_t(nm) * nw, 16));
-  L->rows = coupling_rows_per_tile_f64(L->ldb);
-  L->rowsPad = int(round_up(size_t(na), L->rows)) + L->rows;
   if (L->transform == PHX_TRANSFORM_DIRECT) {
     if (precision == PHX_FP64) {
-      L->Ad.alloc(size_t(L->rowsPad) * L->Kp);
-      launch_phase_rows<double>(na, L->rowsPad, p.nRp, L->Kp, L->kcartActive.p, L->Rp.p, L->Ad.p, s);
+      L->Ad.alloc(2 * phase_cols_size(p.nRp, na));
+      launch_phase_cols<double>(na, na, p.nRp, L->kcartActive.p, L->Rp.p, nullptr, L->Ad.p, s);
     } else {
-      L->Af.alloc(size_t(L->rowsPad) * L->Kp);
-      launch_phase_rows<float>(na, L->rowsPad, p.nRp, L->Kp, L->kcartActive.p, L->Rp.p, L->Af.p, s);
+      L->Af.alloc(2 * phase_cols_size(p.nRp, na));
+      launch_phase_cols<float>(na, na, p.nRp, L->kcartActive.p, L->Rp.p, nullptr, L->Af.p, s);
     }
   } else {
     // ---- separable transform: integer coordinates n_d = b_d.R / 2pi of every R_ph,
@@ -1562,7 +1552,7 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
   // panels of this batch
   int nPanels = 0;
   for (int i = 0; i < nkk; ++i) nPanels += L->nb[k1s[i]];
-  const size_t pstride = size_t(L->Kp) * L->ldb;
+  const size_t pstride = size_t(L->nRp) * L->ldb;
   if (nPanels > L->maxPanels) {
     L->maxPanels = std::max(nPanels, L->k1Batch * nw);
     if (L->precision == PHX_FP64) {
@@ -1574,8 +1564,12 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
     }
   }
   const int M = k2e - k2b;
-  const int nMtiles = L->transform == PHX_TRANSFORM_DIRECT ? ceil_div(M, L->rows)
-                                                         : p.mesh[1] * p.mesh[2];
+  b.nb2max = 1;
+  for (int a = k2b; a < k2e; ++a) b.nb2max = std::max(b.nb2max, L->nb[a]);
+  const int nMtiles =
+      L->transform == PHX_TRANSFORM_DIRECT
+          ? ceil_div(M, coupling_tiling(L->precision == PHX_FP64, nm, nw, b.nb2max).rows)
+          : p.mesh[1] * p.mesh[2];
   b.nkk = nkk;
   b.nPanels = nPanels;
   b.nMtiles = nMtiles;
@@ -1698,8 +1692,6 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
   }
   b.nLinesB = nLinesB;
   L->phP.reserve(size_t(nkk) * L->nRp);
-  b.nb2max = 1;
-  for (int a = k2b; a < k2e; ++a) b.nb2max = std::max(b.nb2max, L->nb[a]);
   b.nb1Max = 0;
   for (int i = 0; i < nkk; ++i) b.nb1Max = std::max(b.nb1Max, L->nb[k1s[i]]);
   // scratch of the separable transform: one panel chunk of stage buffers, row masks,
@@ -1777,7 +1769,7 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
   const int nkk = b.nkk, nPanels = b.nPanels, nMtiles = b.nMtiles, M = b.M, k2b = b.k2b, k2e = b.k2e;
   const int nLinesB = b.nLinesB;
   const bool line = b.line;
-  const size_t pstride = size_t(L->Kp) * L->ldb;
+  const size_t pstride = size_t(L->nRp) * L->ldb;
   const int* dm = b.meta.p;
   const int* dU1off = dm;
   const int* dNb1 = dm + nkk;
@@ -1791,9 +1783,9 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
   // phases: e^{ik1.Re}/de (GEMM form), e^{-ik1.Rp}/dp
   if (!line) {
     if (L->precision == PHX_FP64)
-      launch_phase_cols<double>(nkk, L->nRe, b.k1.p, L->Re.p, L->invDegE.p, L->phE.p, s);
+      launch_phase_cols<double>(nkk, cache_phase_cols(nkk), L->nRe, b.k1.p, L->Re.p, L->invDegE.p, L->phE.p, s);
     else
-      launch_phase_cols<float>(nkk, L->nRe, b.k1.p, L->Re.p, L->invDegE.p, L->phE.p, s);
+      launch_phase_cols<float>(nkk, cache_phase_cols(nkk), L->nRe, b.k1.p, L->Re.p, L->invDegE.p, L->phE.p, s);
   }
   launch_phase_table(nkk, L->nRp, b.k1.p, L->Rp.p, L->invDegP.p, -1.0, L->phP.p, s);
   if (L->timing) PHX_HIP(hipEventRecord(L->ev[0], s));
@@ -1811,7 +1803,6 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
   cp.U1off = dU1off;
   cp.nb1 = dNb1;
   cp.nb1Max = b.nb1Max;
-  cp.evenRows = L->transform == PHX_TRANSFORM_SEPARABLE;
   cp.panelBase = dPbase;
   cp.panelStride = pstride;
   cp.ldb = L->ldb;
@@ -1861,8 +1852,8 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
   if (L->timing) PHX_HIP(hipEventRecord(L->ev[1], s));
   // coupling + fused reduction
   CoupParams cq{};
-  cq.lda = L->Kp;
-  cq.Kp = L->Kp;
+  cq.lda = size_t(L->na);
+  cq.nRp = L->nRp;
   cq.ldb = L->ldb;
   cq.panelStride = pstride;
   cq.M = M;
@@ -1911,11 +1902,11 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
   }
   if (L->transform == PHX_TRANSFORM_DIRECT) {
     if (L->precision == PHX_FP64) {
-      cq.A = L->Ad.p + size_t(k2b) * L->Kp;
+      cq.A = L->Ad.p + 2 * size_t(k2b);
       cq.B = L->Bd.p;
       launch_coupling<double>(cq, true, s);
     } else {
-      cq.A = L->Af.p + size_t(k2b) * L->Kp;
+      cq.A = L->Af.p + 2 * size_t(k2b);
       cq.B = L->Bf.p;
       launch_coupling<float>(cq, true, s);
     }
@@ -2263,7 +2254,6 @@ struct PhelHandle {
   DevBuf<float> Af, Bf;   // FP32 ones
   DevBuf<int> info, fail, rowU2off, rowNb2, rowE3, e2off, cmeta, pmeta;
   DevBuf<long long> rowOutOff;
-  int rowsPad = 0;
   size_t pstride = 0, g2Stride = 0;
   long long pairs = 0;
   // kernel timing: 2 events for the batch's cacheElPh + 3 per outer point
@@ -2420,15 +2410,13 @@ static void phel_setup(PhelHandle* P, const phx_problem& p, ElphHandle* H, const
     PHX_HIP(hipMemcpyAsync(P->omega.data(), P->W3.p, P->W3.bytes(), hipMemcpyDeviceToHost, s));
     PHX_HIP(hipStreamSynchronize(s));
     for (int i = 0; i < P->nq; ++i) PHX_REQUIRE(qi[i] >= 0, "phonon eigensolve did not converge");
-    // phase rows e^{iq3.Rp} (explicit-q mode of the coupling kernel)
-    const int rows = coupling_rows_per_tile_f64(H->ldb);
-    P->rowsPad = ceil_div(P->nq, rows) * rows;
+    // phases e^{iq3.Rp} (explicit-q mode of the coupling kernel)
     if (H->precision == PHX_FP64) {
-      P->A.alloc(size_t(P->rowsPad) * H->Kp);
-      launch_phase_rows<double>(P->nq, P->rowsPad, H->nRp, H->Kp, dq.p, H->Rp.p, P->A.p, s);
+      P->A.alloc(2 * phase_cols_size(H->nRp, P->nq));
+      launch_phase_cols<double>(P->nq, P->nq, H->nRp, dq.p, H->Rp.p, nullptr, P->A.p, s);
     } else {
-      P->Af.alloc(size_t(P->rowsPad) * H->Kp);
-      launch_phase_rows<float>(P->nq, P->rowsPad, H->nRp, H->Kp, dq.p, H->Rp.p, P->Af.p, s);
+      P->Af.alloc(2 * phase_cols_size(H->nRp, P->nq));
+      launch_phase_cols<float>(P->nq, P->nq, H->nRp, dq.p, H->Rp.p, nullptr, P->Af.p, s);
     }
   }
   // ---- batched cacheElPh: e^{ik1.Re}/de per outer point, 1/dp (the e^{iq3.Rp}
@@ -2449,7 +2437,7 @@ static void phel_setup(PhelHandle* P, const phx_problem& p, ElphHandle* H, const
     P->kb.alloc(3 * size_t(kCacheNKK));
     P->cmeta.alloc(3 * size_t(kCacheNKK));
     P->pmeta.alloc(size_t(kCacheNKK) * (1 + 2 * P->nb1max));
-    P->pstride = size_t(H->Kp) * H->ldb;
+    P->pstride = size_t(H->nRp) * H->ldb;
     const size_t nPanels = size_t(kCacheNKK) * P->nb1max;
     if (H->precision == PHX_FP64) {
       P->Bd.alloc(P->pstride * nPanels);
@@ -2539,8 +2527,8 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
   PHX_HIP(hipMemcpyAsync(P->pmeta.p, pm.data(), pm.size() * sizeof(int), hipMemcpyHostToDevice, s));
   PHX_HIP(hipMemcpyAsync(P->F1.p, F.data(), F.size() * sizeof(double), hipMemcpyHostToDevice, s));
   rec(0);
-  if (f64) launch_phase_cols<double>(n, H->nRe, P->kb.p, H->Re.p, P->invE.p, P->phE.p, s);
-  else launch_phase_cols<float>(n, H->nRe, P->kb.p, H->Re.p, P->invE.p, P->phE.p, s);
+  if (f64) launch_phase_cols<double>(n, cache_phase_cols(n), H->nRe, P->kb.p, H->Re.p, P->invE.p, P->phE.p, s);
+  else launch_phase_cols<float>(n, cache_phase_cols(n), H->nRe, P->kb.p, H->Re.p, P->invE.p, P->phE.p, s);
   CacheParams cp{};
   cp.nRe = H->nRe;
   cp.nRp = H->nRp;
@@ -2615,15 +2603,15 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
     // calcCouplingSquared, store mode, every q3 in one launch
     const int* pmk = P->pmeta.p + size_t(i) * blk;
     CoupParams c{};
-    c.lda = H->Kp;
-    c.Kp = H->Kp;
+    c.lda = size_t(nq);
+    c.nRp = H->nRp;
     c.ldb = H->ldb;
     c.panelStride = P->pstride;
     c.M = nq;
     c.nm = nm;
     c.nw = nw;
     c.nPanels = nb1;
-    c.nMtiles = P->rowsPad / coupling_rows_per_tile_f64(H->ldb);
+    c.nMtiles = ceil_div(nq, coupling_tiling(f64, nm, nw, nw).rows);
     c.panelKK = pmk + 1;
     c.panelB1 = pmk + 1 + P->nb1max;
     c.kkNb1 = pmk;

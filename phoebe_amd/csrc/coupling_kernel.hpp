@@ -1,6 +1,6 @@
 // Coupling kernels for one batch of outer points k1 (panels = (k1, b1) pairs):
 //
-//  * k_coupling  : direct R_ph transform, g3 = A B' with A(row, .) = e^{ik2.Rp}
+//  * k_coupling  : direct R_ph transform, g3(row, c) = sum_Rp e^{ik2.Rp} C(Rp, c)
 //                  (or e^{iq.Rp} for explicit q) on v_mfma_{f64,f32}_16x16x4,
 //                  followed by the shared epilogue;
 //  * k_sep_*     : the same g3 for k2 on the Gamma-centred mesh as three short
@@ -31,13 +31,12 @@ typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kNmMax = 36;
-constexpr int kKC = 16;   // K chunk staged in LDS
 
 struct CoupParams {
   // direct transform operands
-  const void* A; int lda;                 // rows (padded to the row tile) x lda
-  const void* B; size_t panelStride; int ldb;
-  int M, Kp, nm, nw, nPanels, nMtiles;
+  const void* A; size_t lda;              // (R_p rounded up to quads, rows): e^{ik2.Rp} complex, zero beyond R_p; row length lda
+  const void* B; size_t panelStride; int ldb;  // panels (R_p, col) complex, ldb reals per R_p
+  int M, nRp, nm, nw, nPanels, nMtiles;
   const int* panelKK;
   const int* panelB1;
   // rows
@@ -48,6 +47,8 @@ struct CoupParams {
   const int* rowE3; const int* rowMesh; const int* kkMesh; int m0, m1, m2;
   // store mode (calcCouplingSquared): out(q)(b1 + nb1 (b2 + nb2 nu))
   double* out; const long long* rowOutOff; const int* kkNb1;
+  // several outer points per launch with rows of their own: added per kk to rowU2off and out
+  long long rowKKStride, outKKStride;
   // reduce mode
   const double* e2pool; const int* rowStateOff;
   const double* e1pool; const int* kkStateOff;
@@ -76,7 +77,6 @@ struct CoupParams {
   int slotZero;                           // off slots: 1 = write zero partials, 0 = leave untouched
   const int* gate;                        // run only when *gate != 0 (null: always)
   unsigned long long* keptRows;           // rows computed by the last stage are added here (null: off)
-  int wideCols;                           // k_coupling_wide: real columns per mode window (multiple of 16)
   // precomputed row lists of the last stage (m0 <= 64)
   unsigned long long* keepMask;           // per slot: bit jx set = row jx kept (null: screen in k_sep_xm)
   const int4* meshRow;                    // per mesh point: (row, nb2, u2off, stateOff), row -1 if inactive
@@ -175,11 +175,6 @@ template <> struct Mfma4<float> {
   __device__ static int row(int lk, int i) { return 4 * lk + i; }
 };
 
-// LDS bytes of the shared epilogue (g3 tile, g', |g|^2 per row).
-inline size_t epilogue_lds_bytes(int elem, int ldb, int nm, int nb2max) {
-  return size_t(16) * ldb * elem + size_t(16) * nm * nb2max * (sizeof(double2) + sizeof(double));
-}
-
 // Electron rotation of the modes nuLo .. nuHi-1 for the 16 rows whose g3
 // blocks are in LDS (row r at g3 + r*PWp, (re, im) of column (nu, w2) at
 // 2((nu - nuLo)*nw + w2)) into g'(nu, b2) in scratch.  Thread t serves row t/16.
@@ -197,6 +192,7 @@ __device__ void epilogue16_u2(const CoupParams& p, const T* g3, int PWp, unsigne
   for (int o = sub; o < (nuHi - nuLo) * nb2; o += 16) {
     const int nl = o / nb2, b2 = o % nb2;
     double2 s = make_double2(0., 0.);
+#pragma unroll 8
     for (int w2 = 0; w2 < nw; ++w2) {
       const double2 u = U2[w2 + nw * b2];
       const double xr = double(g[2 * (nl * nw + w2)]), xi = double(g[2 * (nl * nw + w2) + 1]);
@@ -209,9 +205,11 @@ __device__ void epilogue16_u2(const CoupParams& p, const T* g3, int PWp, unsigne
 
 // Rest of the epilogue once g'(nu, b2) of every mode is in scratch: phonon
 // rotation, |g|^2, then the store or the symmetrization and the weights.
-// Must be called by all 256 threads.
+// Must be called by all 256 threads.  stage (null: none): LDS of 16 (nm +
+// nb2max) doubles for the rows' frequencies and band energies, which the search
+// for degenerate groups would else read from memory one after the other.
 template <bool REDUCE>
-__device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, int panel, int kk, int b1p,
+__device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, double* stage, int panel, int kk, int b1p,
                                 int myRow, int myIq, double (&part)[kGMax][kCMax]) {
   const int t = threadIdx.x, r = t >> 4, sub = t & 15;
   const int nm = p.nm;
@@ -223,9 +221,18 @@ __device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, int
   const int nb2 = valid ? p.rowNb2[myRow] : 0;
   const double2* e3 = p.E3pool + size_t(myIq) * nm * nm;
   const bool polar = p.polarX != nullptr && valid;
+  const double* const w3g = p.Wpool + size_t(myIq) * nm;
+  const double* const e2g = p.e2pool + (valid ? p.rowStateOff[myRow] : 0);
+  double* const w3s = stage ? stage + r * nm : nullptr;
+  double* const e2s = stage ? stage + 16 * nm + r * p.nb2max : nullptr;
+  if (REDUCE && stage && valid) {
+    for (int i = sub; i < nm; i += 16) w3s[i] = w3g[i];
+    for (int i = sub; i < nb2; i += 16) e2s[i] = e2g[i];
+  }
   for (int o = sub; o < nm * nb2; o += 16) {
     const int nu2 = o / nb2, b2 = o % nb2;
     double2 s = make_double2(0., 0.);
+#pragma unroll 6
     for (int nu = 0; nu < nm; ++nu) {
       const double2 e = e3[nu + nm * nu2], x = gp[nu * nb2 + b2];
       s.x += x.x * e.x - x.y * e.y;
@@ -257,14 +264,14 @@ __device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, int
   if (!REDUCE) return;
   __syncthreads();
 
-  const double* w3 = p.Wpool + size_t(myIq) * nm;
-  const double* e2 = p.e2pool + (valid ? p.rowStateOff[myRow] : 0);
+  auto w3 = [&](int i) { return stage ? w3s[i] : w3g[i]; };
+  auto e2 = [&](int i) { return stage ? e2s[i] : e2g[i]; };
   // symmetrizeCoupling (scattering.cpp:1209-1318) along b2, then nu
   for (int nu = sub; nu < nm && valid; nu += 16) {
     for (int b = 0; b < nb2; ++b) {
       int deg = 0;
       for (int i = b; i < nb2; ++i) {
-        if (fabs(e2[b] - e2[i]) < 1.0e-6) deg++;
+        if (fabs(e2(b) - e2(i)) < 1.0e-6) deg++;
         else break;
       }
       if (deg > 1) {
@@ -280,7 +287,7 @@ __device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, int
     for (int nu = 0; nu < nm; ++nu) {
       int deg = 0;
       for (int i = nu; i < nm; ++i) {
-        if (fabs(w3[nu] - w3[i]) < 1.0e-6) deg++;
+        if (fabs(w3(nu) - w3(i)) < 1.0e-6) deg++;
         else break;
       }
       if (deg > 1) {
@@ -300,10 +307,10 @@ __device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, int
   const double inv_g = 1. / double(float(gsize));
   for (int o = sub; o < nm * nb2; o += 16) {
     const int nu = o / nb2, b2 = o % nb2;
-    const double en3 = w3[nu];
+    const double en3 = w3(nu);
     if (en3 < p.cutoff) continue;
     const double cpl = gs[nu * nb2 + b2] * inv_g;
-    const double en2 = e2[b2];
+    const double en2 = e2(b2);
     const int is2 = p.rowStateOff[myRow] + b2;
 #pragma unroll
     for (int gi = 0; gi < kGMax; ++gi) {
@@ -328,18 +335,6 @@ __device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, int
       }
     }
   }
-}
-
-// Epilogue for the 16 rows whose full g3 rows are in LDS (row r at g3 + r*PWp,
-// (re, im) of column (nu, w2) at 2(nu*nw + w2)).  Thread t serves row t/16;
-// myRow < 0 marks an empty slot.  Must be called by all 256 threads.
-template <typename T, bool REDUCE>
-__device__ void epilogue16(const CoupParams& p, const T* g3, int PWp, unsigned char* scratch,
-                           int panel, int kk, int b1p, int myRow, int myIq,
-                           double (&part)[kGMax][kCMax]) {
-  epilogue16_u2<T>(p, g3, PWp, scratch, myRow, 0, p.nm);
-  __syncthreads();
-  epilogue16_tail<REDUCE>(p, scratch, panel, kk, b1p, myRow, myIq, part);
 }
 
 // Block reduction of the per-thread partial linewidths into partial[L]
@@ -371,309 +366,26 @@ __device__ inline void reduce_partials(const CoupParams& p, int L, unsigned char
 }
 
 // ------------------------------------------------------------------ direct transform
-template <typename T, int MT, int NTW, bool REDUCE>
-__global__ void __launch_bounds__(256, 2) k_coupling(CoupParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int ROWS = 16 * MT;
-  const int nTilesTot = p.nPanels * p.nMtiles;
-  const int bid = blockIdx.x;
-  const int perXcd = gridDim.x / 8;
-  const int L = (bid % 8) * perXcd + bid / 8;  // XCD-contiguous logical index
-  if (L >= nTilesTot) return;
-  const int panel = L / p.nMtiles, mtile = L % p.nMtiles;
-  const int row0 = mtile * ROWS;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int PWp = p.ldb;
-  const int ntiles = PWp / 16;
+// (coupling_direct.hpp, instantiated in coupling_direct_f64.hip and coupling_direct_f32.hip)
 
-  typedef typename Mfma4<T>::acc_t acc_t;
-  acc_t acc[MT][NTW];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int j = 0; j < NTW; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[m][j][i] = 0;
-
-  // A tile (ROWS x kKC) double-buffered in LDS; B fragments, which belong to
-  // one wave only, go straight to registers one K chunk ahead of their use.
-  constexpr int LDA = kKC + 1;
-  constexpr int KS = kKC / 4;              // MFMA k-steps per chunk
-  constexpr int AE = ROWS * kKC / 256;     // A elements loaded per thread per chunk
-  T* As0 = reinterpret_cast<T*>(smem);
-  T* As1 = As0 + ROWS * LDA;
-  const T* A = static_cast<const T*>(p.A) + size_t(row0) * p.lda;
-  const T* B = static_cast<const T*>(p.B) + size_t(panel) * p.panelStride;
-  const int lr = lane & 15, lk = lane >> 4;
-  T areg[AE];
-  T b0[KS][NTW], b1[KS][NTW];
-
-  auto load_a = [&](int kc) {
-#pragma unroll
-    for (int e = 0; e < AE; ++e) {
-      const int i = t + 256 * e, r = i / kKC, k = i % kKC;
-      areg[e] = A[size_t(r) * p.lda + kc + k];
-    }
-  };
-  auto store_a = [&](T* As) {
-#pragma unroll
-    for (int e = 0; e < AE; ++e) {
-      const int i = t + 256 * e, r = i / kKC, k = i % kKC;
-      As[r * LDA + k] = areg[e];
-    }
-  };
-  auto load_b = [&](T(&b)[KS][NTW], int kc) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const T* Bk = B + size_t(kc + ks * 4 + lk) * PWp + lr;
-#pragma unroll
-      for (int j = 0; j < NTW; ++j)
-        if (wave + 4 * j < ntiles) b[ks][j] = Bk[(wave + 4 * j) * 16];
-    }
-  };
-  auto compute = [&](const T* As, const T(&b)[KS][NTW]) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      T a[MT];
-#pragma unroll
-      for (int m = 0; m < MT; ++m) a[m] = As[(16 * m + lr) * LDA + ks * 4 + lk];
-#pragma unroll
-      for (int j = 0; j < NTW; ++j)
-        if (wave + 4 * j < ntiles) {
-#pragma unroll
-          for (int m = 0; m < MT; ++m) acc[m][j] = Mfma4<T>::mac(a[m], b[ks][j], acc[m][j]);
-        }
-    }
-  };
-
-  const int nch = p.Kp / kKC;
-  load_a(0);
-  load_b(b0, 0);
-  store_a(As0);
-  __syncthreads();
-  for (int c = 0; c < nch; c += 2) {
-    if (c + 1 < nch) {
-      load_a((c + 1) * kKC);
-      load_b(b1, (c + 1) * kKC);
-    }
-    compute(As0, b0);
-    if (c + 1 < nch) store_a(As1);
-    __syncthreads();
-    if (c + 1 >= nch) break;
-    if (c + 2 < nch) {
-      load_a((c + 2) * kKC);
-      load_b(b0, (c + 2) * kKC);
-    }
-    compute(As1, b1);
-    if (c + 2 < nch) store_a(As0);
-    __syncthreads();
-  }
-
-  const int kk = p.panelKK[panel];
-  const int b1p = p.panelB1[panel];
-  T* g3 = reinterpret_cast<T*>(smem);
-  unsigned char* scratch = smem + size_t(16) * PWp * sizeof(T);
-  double part[kGMax][kCMax];
-#pragma unroll
-  for (int gi = 0; gi < kGMax; ++gi)
-#pragma unroll
-    for (int c = 0; c < kCMax; ++c) part[gi][c] = 0.;
-#pragma unroll
-  for (int h = 0; h < MT; ++h) {
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) {
-      const int tile = wave + 4 * j;
-      if (tile < ntiles) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) g3[Mfma4<T>::row(lk, i) * PWp + tile * 16 + lr] = acc[h][j][i];
-      }
-    }
-    __syncthreads();
-    const int row = row0 + 16 * h + (t >> 4);
-    const int myRow = row < p.M ? row : -1;
-    int myIq = 0;
-    if (myRow >= 0)
-      myIq = p.qmode ? mesh_diff_index(p.rowMesh[myRow], p.kkMesh[kk], p.m0, p.m1, p.m2) : p.rowE3[myRow];
-    epilogue16<T, REDUCE>(p, g3, PWp, scratch, panel, kk, b1p, myRow, myIq, part);
-  }
-  if (REDUCE) reduce_partials<kCMax>(p, L, smem, part);
-}
-
-// Wide panels (2 nm nw > 576): 16-row tiles, the panel columns in windows of
-// whole modes (<= 384 real columns), each window's MFMA product rotated by U2
-// into g'(nu, b2) before the next; the phonon rotation and the weights run once
-// all modes are in.
-constexpr int kWideNtw = 6;
-template <typename T, bool REDUCE>
-__global__ void __launch_bounds__(256, 1) k_coupling_wide(CoupParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NTW = kWideNtw;
-  const int WCOL = p.wideCols;  // <= 4 * NTW * 16
-  const int nTilesTot = p.nPanels * p.nMtiles;
-  const int bid = blockIdx.x;
-  const int perXcd = gridDim.x / 8;
-  const int L = (bid % 8) * perXcd + bid / 8;
-  if (L >= nTilesTot) return;
-  const int panel = L / p.nMtiles, mtile = L % p.nMtiles;
-  const int row0 = mtile * 16;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lr = lane & 15, lk = lane >> 4;
-  typedef typename Mfma4<T>::acc_t acc_t;
-  constexpr int LDA = kKC + 1, KS = kKC / 4, AE = 16 * kKC / 256;
-  T* As = reinterpret_cast<T*>(smem);                                    // 16 x LDA
-  T* g3 = As + 16 * LDA;                                                 // 16 x WCOL
-  unsigned char* scratch = reinterpret_cast<unsigned char*>(g3 + 16 * WCOL);
-  scratch = smem + (size_t(scratch - smem) + 15) / 16 * 16;
-  const T* A = static_cast<const T*>(p.A) + size_t(row0) * p.lda;
-  const T* B = static_cast<const T*>(p.B) + size_t(panel) * p.panelStride;
-  const int kk = p.panelKK[panel];
-  const int b1p = p.panelB1[panel];
-  const int row = row0 + (t >> 4);
-  const int myRow = row < p.M ? row : -1;
-  const int nuPerWin = max(1, (WCOL / 2) / p.nw);  // WCOL >= 2 nw
-  for (int nu0 = 0; nu0 < p.nm; nu0 += nuPerWin) {
-    const int nu1 = min(p.nm, nu0 + nuPerWin);
-    const int c0 = 2 * nu0 * p.nw, width = 2 * (nu1 - nu0) * p.nw;
-    const int ntiles = (width + 15) / 16;
-    acc_t acc[NTW];
-#pragma unroll
-    for (int j = 0; j < NTW; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[j][i] = 0;
-    for (int kc = 0; kc < p.Kp; kc += kKC) {
-      __syncthreads();
-#pragma unroll
-      for (int e = 0; e < AE; ++e) {
-        const int i = t + 256 * e, r = i / kKC, k = i % kKC;
-        As[r * LDA + k] = A[size_t(r) * p.lda + kc + k];
-      }
-      T b[KS][NTW];
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const T* Bk = B + size_t(kc + ks * 4 + lk) * p.ldb + c0 + lr;
-#pragma unroll
-        for (int j = 0; j < NTW; ++j) {
-          const int col = (wave + 4 * j) * 16 + lr;
-          b[ks][j] = (wave + 4 * j < ntiles && col < width) ? Bk[(wave + 4 * j) * 16] : T(0);
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const T a = As[lr * LDA + ks * 4 + lk];
-#pragma unroll
-        for (int j = 0; j < NTW; ++j)
-          if (wave + 4 * j < ntiles) acc[j] = Mfma4<T>::mac(a, b[ks][j], acc[j]);
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) {
-      const int tile = wave + 4 * j;
-      if (tile < ntiles)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) g3[Mfma4<T>::row(lk, i) * WCOL + tile * 16 + lr] = acc[j][i];
-    }
-    __syncthreads();
-    epilogue16_u2<T>(p, g3, WCOL, scratch, myRow, nu0, nu1);
-  }
-  __syncthreads();
-  int myIq = 0;
-  if (myRow >= 0)
-    myIq = p.qmode ? mesh_diff_index(p.rowMesh[myRow], p.kkMesh[kk], p.m0, p.m1, p.m2) : p.rowE3[myRow];
-  double part[kGMax][kCMax];
-#pragma unroll
-  for (int gi = 0; gi < kGMax; ++gi)
-#pragma unroll
-    for (int c = 0; c < kCMax; ++c) part[gi][c] = 0.;
-  epilogue16_tail<REDUCE>(p, scratch, panel, kk, b1p, myRow, myIq, part);
-  if (REDUCE) reduce_partials<kCMax>(p, L, smem, part);
-}
-
-inline size_t coupling_wide_lds_bytes(int elem, int nm, int nb2max, int wcol) {
-  const size_t a = (size_t(16) * (kKC + 1) + size_t(16) * wcol) * elem;
-  return std::max((a + 15) / 16 * 16 + size_t(16) * nm * nb2max * (sizeof(double2) + sizeof(double)),
-                  size_t(kGMax) * kCMax * 4 * sizeof(double));
-}
-
-inline size_t coupling_lds_bytes(int elem, int MT, int ldb, int nm, int nb2max, bool reduce) {
-  (void)reduce;
-  const int ROWS = 16 * MT;
-  size_t a = 2 * size_t(ROWS) * (kKC + 1) * elem;
-  size_t e = epilogue_lds_bytes(elem, ldb, nm, nb2max);
-  size_t r = size_t(kGMax) * kCMax * 4 * sizeof(double);
-  return std::max(std::max(a, e), r);
-}
-
-template <typename T, int MT, int NTW, bool REDUCE>
-static void launch_coupling_t(const CoupParams& p, int grid, size_t lds, hipStream_t s) {
-  auto kern = k_coupling<T, MT, NTW, REDUCE>;
-  PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, s, p);
-  PHX_HIP(hipGetLastError());
-}
-
-// Panels up to 384 real columns (at most 6 column tiles per wave) use 32-row
-// tiles, wider panels 16-row tiles, so that accumulators stay in registers.
-template <typename T, bool REDUCE>
-static void dispatch_ntw(int ntw, const CoupParams& p, int grid, size_t lds, hipStream_t s) {
-  switch (ntw) {
-#define PHX_NTW(mt, n) case n: launch_coupling_t<T, mt, n, REDUCE>(p, grid, lds, s); break;
-    PHX_NTW(2, 1) PHX_NTW(2, 2) PHX_NTW(2, 3) PHX_NTW(2, 4) PHX_NTW(2, 5) PHX_NTW(2, 6)
-    PHX_NTW(1, 7) PHX_NTW(1, 8) PHX_NTW(1, 9)
-#undef PHX_NTW
-    default: throw Error(-1, "coupling kernel: panel too wide");
-  }
-}
-
-inline int coupling_rows_per_tile(int ldb) { return ldb <= 384 ? 32 : 16; }  // wide panels: 16
-
+// How the direct transform cuts its work: workgroups of `rows` inner points,
+// 4 / wc waves of mt 16-row tiles by wc waves of nt 16-column tiles, the panel
+// columns in windows of `modes` whole modes.
+struct CoupTiling {
+  int mt, nt, wc, rows, modes;
+  int stage;  // the g3 tile's LDS holds the rows' frequencies and energies once g3 has been used
+  size_t lds;
+};
+CoupTiling coupling_tiling(bool f64, int nm, int nw, int nb2max);
 template <typename T>
-void launch_coupling(const CoupParams& p, bool reduce, hipStream_t s) {
-  PHX_REQUIRE(p.nm <= kNmMax, "coupling kernel supports nm <= 36");
-  PHX_REQUIRE(p.ldb % 16 == 0 && p.Kp % kKC == 0, "coupling kernel: bad padding");
-  if (p.ldb > 9 * 64) {  // wider than one pass of the tiled kernel
-    PHX_REQUIRE(p.nMtiles * 16 >= p.M, "coupling kernel: wide panels use 16-row tiles");
-    const int tiles = p.nPanels * p.nMtiles;
-    if (tiles <= 0) return;
-    // widest mode window (whole modes, <= 384 real columns) that fits the LDS budget
-    CoupParams q = p;
-    q.wideCols = 0;
-    size_t lds = 0;
-    for (int nuw = std::max(1, 192 / p.nw); nuw >= 1; --nuw) {
-      q.wideCols = int(round_up(size_t(2) * nuw * p.nw, 16));
-      lds = coupling_wide_lds_bytes(sizeof(T), p.nm, p.nb2max, q.wideCols);
-      if (lds <= 160 * 1024) break;
-    }
-    PHX_REQUIRE(lds <= 160 * 1024, "coupling kernel: nm x bands per inner point too large for LDS");
-    auto go = [&](auto kern) {
-      PHX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-      hipLaunchKernelGGL(kern, dim3(ceil_div(tiles, 8) * 8), dim3(256), lds, s, q);
-    };
-    if (reduce) go(k_coupling_wide<T, true>);
-    else go(k_coupling_wide<T, false>);
-    PHX_HIP(hipGetLastError());
-    return;
-  }
-  const int MT = coupling_rows_per_tile(p.ldb) / 16;
-  const int ntw = ceil_div(p.ldb / 16, 4);
-  const int tiles = p.nPanels * p.nMtiles;
-  if (tiles <= 0) return;
-  const int grid = ceil_div(tiles, 8) * 8;
-  const size_t lds = coupling_lds_bytes(sizeof(T), MT, p.ldb, p.nm, p.nb2max, reduce);
-  PHX_REQUIRE(lds <= 160 * 1024, "coupling kernel: LDS budget exceeded");
-  if (reduce) dispatch_ntw<T, true>(ntw, p, grid, lds, s);
-  else dispatch_ntw<T, false>(ntw, p, grid, lds, s);
-}
+void launch_coupling(const CoupParams& p, bool reduce, hipStream_t s);
 
 // ------------------------------------------------------------------ separable transform
 // Integer layout of the R_ph set folded on the mesh:
 //   lines  = distinct (f0, f1), entries (f2, Rp)          (stage z)
 //   groups = distinct f0,       entries (f1, line)        (stage y)
 struct SepParams {
-  const void* B; size_t panelStride; int ldb;   // panels: C(Rp, col) in row 2 Rp
+  const void* B; size_t panelStride; int ldb;   // panels: C(Rp, col), ldb reals per Rp
   int ncol, nPanels, mx, my, mz;
   int modeFast;                                 // nm: columns of T1 / T2 / g3 as (w2, nu); 0: as the panels, (nu, w2)
   int nLines; const int* lineStart; const int* lineF2; const int* lineRp;
@@ -793,10 +505,9 @@ __global__ void __launch_bounds__(256) k_sep_z(SepParams p) {
   double2* W = reinterpret_cast<double2*>(smem + (size_t(ne) * ncol * sizeof(T2v) + 15) / 16 * 16);  // (entries, mz)
   int* off = reinterpret_cast<int*>(W + size_t(ne) * mz);
   int* fe = off + ne;
-  // C(Rp, c): row 2 Rp of the panel, complex entries (re, im) at 2c, 2c + 1
   const T2v* B = reinterpret_cast<const T2v*>(static_cast<const T*>(p.B) + size_t(panel) * p.panelStride);
   sep_stage_entries(B, X, W, off, fe, ne, ncol, mz, p.modeFast, p.twz, [&](int e, int& o, int& f) {
-    o = p.lineRp[e0 + e] * p.ldb;  // row 2 Rp: 2 Rp ldb elements of T = Rp ldb complex
+    o = p.lineRp[e0 + e] * (p.ldb / 2);
     f = p.lineF2[e0 + e];
   });
   T2v* out = reinterpret_cast<T2v*>(static_cast<T*>(p.T1) + size_t(panel) * p.t1PanelStride) +

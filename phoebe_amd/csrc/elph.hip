@@ -9,11 +9,10 @@
 //            gW element is read once per batch and used for every k1]
 //            C(Rp,nu,b1,w2) = sum_w1 g1 U1(w1,b1) * s(k1,Rp)               [fused epilogue]
 //            with s = e^{-ik1.Rp}/dp (mesh mode) or 1/dp (explicit-q mode), written
-//            as real "panels" B'(k, c), one panel per (k1, b1): rows 2Rp, 2Rp+1 hold
-//            C and i*C interleaved, so that a complex product becomes a real GEMM.
+//            as complex panels (Rp, (nu, w2)), one panel per (k1, b1).
 //  k_coupling  rows = outer-product partners (k2 or explicit q):
-//            g3(row, nu, w2) = sum_Rp A(row, Rp) C(Rp, nu, b1, w2)            [real GEMM on MFMA,
-//            A(row, .) = e^{ik2.Rp} interleaved, so e^{iq.Rp} = e^{ik2.Rp} e^{-ik1.Rp}]
+//            g3(row, nu, w2) = sum_Rp A(row, Rp) C(Rp, nu, b1, w2)            [MFMA,
+//            A(row, .) = e^{ik2.Rp}, so e^{iq.Rp} = e^{ik2.Rp} e^{-ik1.Rp}]
 //            epilogue in LDS: g4 = e3^T g3 (phonon rotation, e3 not conjugated),
 //            g = U2^H g4, |g|^2, then either store |g|^2 (calcCouplingSquared) or
 //            symmetrize over degenerate b2 / nu groups and contract with the
@@ -136,67 +135,39 @@ void launch_phase_table(int rows, int nR, const double* kc, const double* R, con
   PHX_HIP(hipGetLastError());
 }
 
-// The same table transposed for k_cache, in the GEMM's precision: out(r, i) with
-// `cols` points per row (points beyond `rows` zero) and nR rounded up to whole
-// quads (rows beyond nR zero).
+// The same table transposed for the GEMMs of k_cache and k_coupling, in their
+// precision: out(r, i) with `cols` >= rows points per row (points beyond `rows`
+// zero) and nR rounded up to whole quads (rows beyond nR zero).
 template <typename T>
 __global__ void k_phase_cols(int rows, int cols, int nR, const double* __restrict__ kc,
                              const double* __restrict__ R, const double* __restrict__ scale, T* __restrict__ out) {
-  const int n = (nR + 3) / 4 * 4 * cols;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
-    const int r = t / cols, i = t - r * cols;
+  const size_t n = size_t(nR + 3) / 4 * 4 * cols;
+  for (size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x; t < n; t += size_t(gridDim.x) * blockDim.x) {
+    const int r = int(t / cols), i = int(t - size_t(r) * cols);
     double s = 0., c = 0.;
     if (r < nR && i < rows) {
       sincos(kc[3 * i] * R[3 * r] + kc[3 * i + 1] * R[3 * r + 1] + kc[3 * i + 2] * R[3 * r + 2], &s, &c);
-      s *= scale[r];
-      c *= scale[r];
+      if (scale) {
+        s *= scale[r];
+        c *= scale[r];
+      }
     }
-    out[2 * size_t(t)] = T(c);
-    out[2 * size_t(t) + 1] = T(s);
+    out[2 * t] = T(c);
+    out[2 * t + 1] = T(s);
   }
 }
 
 template <typename T>
-void launch_phase_cols(int rows, int nR, const double* kc, const double* R, const double* scale, void* out,
+void launch_phase_cols(int rows, int cols, int nR, const double* kc, const double* R, const double* scale, void* out,
                        hipStream_t s) {
   if (rows <= 0) return;
-  const int cols = cache_phase_cols(rows);
-  hipLaunchKernelGGL(k_phase_cols<T>, dim3(ceil_div(ceil_div(nR, 4) * 4 * cols, 256)), dim3(256), 0, s, rows, cols,
-                     nR, kc, R, scale, static_cast<T*>(out));
+  const size_t n = phase_cols_size(nR, cols);
+  hipLaunchKernelGGL(k_phase_cols<T>, dim3(unsigned(std::min<size_t>((n + 255) / 256, 16384))), dim3(256), 0, s, rows,
+                     cols, nR, kc, R, scale, static_cast<T*>(out));
   PHX_HIP(hipGetLastError());
 }
-template void launch_phase_cols<double>(int, int, const double*, const double*, const double*, void*, hipStream_t);
-template void launch_phase_cols<float>(int, int, const double*, const double*, const double*, void*, hipStream_t);
-
-// GEMM A operand: rows of e^{ik.Rp} (no degeneracy factor), interleaved (re, im)
-// over Kp >= 2 nRp columns (zero padded), for rowsPad rows (rows >= nrows zero).
-template <typename T>
-__global__ void k_phase_rows(int nrows, int rowsPad, int nRp, int Kp, const double* __restrict__ kc,
-                             const double* __restrict__ R, T* __restrict__ A) {
-  size_t n = size_t(rowsPad) * (Kp / 2);
-  for (size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x; t < n;
-       t += size_t(gridDim.x) * blockDim.x) {
-    int i = int(t / (Kp / 2)), r = int(t % (Kp / 2));
-    double c = 0., s = 0.;
-    if (i < nrows && r < nRp) {
-      double arg = kc[3 * i] * R[3 * r] + kc[3 * i + 1] * R[3 * r + 1] + kc[3 * i + 2] * R[3 * r + 2];
-      sincos(arg, &s, &c);
-    }
-    A[size_t(i) * Kp + 2 * r] = T(c);
-    A[size_t(i) * Kp + 2 * r + 1] = T(s);
-  }
-}
-
-template <typename T>
-void launch_phase_rows(int nrows, int rowsPad, int nRp, int Kp, const double* kc, const double* R,
-                       T* A, hipStream_t s) {
-  hipLaunchKernelGGL(k_phase_rows<T>, dim3(4096), dim3(256), 0, s, nrows, rowsPad, nRp, Kp, kc, R, A);
-  PHX_HIP(hipGetLastError());
-}
-template void launch_phase_rows<double>(int, int, int, int, const double*, const double*, double*,
-                                        hipStream_t);
-template void launch_phase_rows<float>(int, int, int, int, const double*, const double*, float*,
-                                       hipStream_t);
+template void launch_phase_cols<double>(int, int, int, const double*, const double*, const double*, void*, hipStream_t);
+template void launch_phase_cols<float>(int, int, int, const double*, const double*, const double*, void*, hipStream_t);
 
 // Gather windowed eigenvector columns: pool(off_a + w + nw*b) = U(ik_a)(w, lo_a + b).
 __global__ void k_gather_eig(int na, int nw, const int* __restrict__ ik, const int* __restrict__ lo,
@@ -321,17 +292,10 @@ __device__ __forceinline__ void cache_panel_epilogue(const CacheParams& p, const
       v.y += ar * u.y + ai * u.x;
     }
     const double2 c = make_double2(v.x * s.x - v.y * s.y, v.x * s.y + v.y * s.x);
-    // rows 2 rp (C) and 2 rp + 1 (i C) of the panel, whose rows are whole 16-element blocks
-    O2* row = reinterpret_cast<O2*>(static_cast<OutT*>(p.B) + size_t(pan0 + e) * p.panelStride +
-                                    size_t(2 * rp) * p.ldb) + size_t(nu) * nw + w2;
-    O2* rowI = row + p.ldb / 2;
-    if (w1lo == 0) {
-      row[0] = O2{OutT(c.x), OutT(c.y)};
-      if (!p.evenRows) rowI[0] = O2{OutT(-c.y), OutT(c.x)};
-    } else {  // later column passes add their w1 range
-      row[0] = O2{row[0].x + OutT(c.x), row[0].y + OutT(c.y)};
-      if (!p.evenRows) rowI[0] = O2{rowI[0].x + OutT(-c.y), rowI[0].y + OutT(c.x)};
-    }
+    O2* out = reinterpret_cast<O2*>(static_cast<OutT*>(p.B) + size_t(pan0 + e) * p.panelStride + size_t(rp) * p.ldb) +
+              size_t(nu) * nw + w2;
+    if (w1lo == 0) out[0] = O2{OutT(c.x), OutT(c.y)};
+    else out[0] = O2{out[0].x + OutT(c.x), out[0].y + OutT(c.y)};  // later column passes add their w1 range
   }
 }
 

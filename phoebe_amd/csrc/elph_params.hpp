@@ -24,11 +24,13 @@ inline int line_count_padded(int n) {
 // Outer points per row of the GEMM form's phase table: the batch rounded up to
 // k_cache's 16-point tiles.
 inline int cache_phase_cols(int nkk) { return nkk <= 16 ? 16 : kCacheNKK; }
+// Complex values of a transposed phase table of nR vectors and cols points.
+inline size_t phase_cols_size(int nR, int cols) { return size_t(nR + 3) / 4 * 4 * cols; }
 // Complex FP64 values that hold the table of any batch, in either precision.
-inline size_t cache_phase_size(int nRe) { return size_t(kCacheNKK) * ((nRe + 3) / 4 * 4); }
+inline size_t cache_phase_size(int nRe) { return phase_cols_size(nRe, kCacheNKK); }
 
 // g1(k1; Rp,nu,w1,w2) = sum_Re e^{ik1.Re}/de gW(Re,Rp,nu,w1,w2), rotated by U1
-// and scaled by s(k1, Rp) into one real panel per (k1, b1).
+// and scaled by s(k1, Rp) into one complex panel per (k1, b1).
 struct CacheParams {
   int nRe, nRp, nm, nw, nkk;
   const void* gW;         // (nRe, nRp, nm, nw, nw) complex, element type T
@@ -43,8 +45,7 @@ struct CacheParams {
   const int* panelBase;   // first panel of kk; the panels of consecutive points follow each other
   void* B;                // panels
   size_t panelStride;     // elements
-  int ldb;                // elements per panel row (a multiple of 16)
-  int evenRows;           // write the panels' rows 2 Rp (C) only: the mesh-separable transform reads no others
+  int ldb;                // elements per panel row, one row per Rp (a multiple of 16)
   // outer points on one mesh line (k_cache_line_a / k_cache_line_b)
   size_t N;               // gW columns: nRp * nm * nw^2
   int nGe;                // R_e groups: distinct n0(R_e) mod m0
@@ -77,7 +78,7 @@ struct CollectParams {
 
 template <typename T, typename OutT> void launch_cache(const CacheParams& p, hipStream_t s);
 template <typename T>
-void launch_phase_cols(int rows, int nR, const double* kc, const double* R, const double* scale, void* out,
+void launch_phase_cols(int rows, int cols, int nR, const double* kc, const double* R, const double* scale, void* out,
                        hipStream_t s);
 template <typename T, typename OutT> void launch_cache_line(const CacheParams& p, hipStream_t s);
 void launch_collect(const CollectParams& p, hipStream_t s);
