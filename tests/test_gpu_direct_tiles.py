@@ -1,0 +1,34 @@
+"""The direct coupling transform over its tilings: one, two and four column
+waves, one and two row tiles per wave, panels in windows of modes, R_p counts
+that are not whole quads, and point counts around the row tiles."""
+import numpy as np
+import pytest
+
+import phoebe_amd as P
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("nw,nm,nRp,nq", [(2, 3, 1, 1), (8, 6, 5, 65), (7, 9, 4, 33), (5, 15, 3, 16), (8, 18, 6, 31),
+                                          (16, 12, 7, 33), (23, 15, 9, 17), (16, 24, 2, 15), (17, 24, 5, 18),
+                                          (32, 12, 3, 2), (30, 27, 2, 16)])
+def test_store_mode_against_direct_sum(nw, nm, nRp, nq, precision):
+    rng = np.random.default_rng(7 * nw + nm)
+    cx = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)
+    gW = cx(2, nRp, nm, nw, nw)
+    Re, Rp = rng.integers(-3, 4, (2, 3)) * 1.3, rng.integers(-3, 4, (nRp, 3)) * 1.3
+    dE, dP = np.ones(2), rng.integers(1, 4, nRp).astype(float)
+    U1 = np.linalg.qr(cx(nw, nw))[0][:, :2]
+    U2 = [np.linalg.qr(cx(nw, nw))[0][:, :min(1 + i % 4, nw)] for i in range(nq)]
+    e3 = [cx(nm, nm) for _ in range(nq)]
+    k1, q3 = rng.standard_normal(3), rng.standard_normal((nq, 3))
+    inter = P.InteractionElPhWan(gW, Re, dE, Rp, dP, precision)
+    inter.cacheElPh(U1, k1)
+    inter.calcCouplingSquared(U1, U2, e3, q3)
+    g1 = np.einsum("e,epvab,ac->pvcb", np.exp(1j * Re @ k1) / dE, gW, U1)
+    tol = 1e-12 if precision == "fp64" else 2e-6
+    for i in range(nq):
+        g3 = np.tensordot(np.exp(1j * Rp @ q3[i]) / dP, g1, axes=(0, 0))  # (nu, b1, w2)
+        ref = np.abs(np.einsum("vcb,bd,vm->cdm", g3, U2[i].conj(), e3[i], optimize=True)) ** 2
+        assert np.abs(inter.getCouplingSquared(i) - ref).max() <= tol * ref.max()
