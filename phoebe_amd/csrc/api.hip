@@ -2255,8 +2255,9 @@ struct PhelHandle {
   DevBuf<int> info, fail, rowU2off, rowNb2, rowE3, e2off, cmeta, pmeta;
   DevBuf<long long> rowOutOff;
   size_t pstride = 0, g2Stride = 0;
+  int points = 1;           // outer points per coupling launch
   long long pairs = 0;
-  // kernel timing: 2 events for the batch's cacheElPh + 3 per outer point
+  // kernel timing: 2 events for the batch's cacheElPh + 3 per coupling launch
   bool timing = false;
   std::vector<hipEvent_t> tev;
   double cacheMs = 0., coupMs = 0., redMs = 0., coupFlops = 0.;
@@ -2436,7 +2437,7 @@ static void phel_setup(PhelHandle* P, const phx_problem& p, ElphHandle* H, const
     P->phE.alloc(cache_phase_size(H->nRe));
     P->kb.alloc(3 * size_t(kCacheNKK));
     P->cmeta.alloc(3 * size_t(kCacheNKK));
-    P->pmeta.alloc(size_t(kCacheNKK) * (1 + 2 * P->nb1max));
+    P->pmeta.alloc(size_t(kCacheNKK) * (2 + 2 * P->nb1max));
     P->pstride = size_t(H->nRp) * H->ldb;
     const size_t nPanels = size_t(kCacheNKK) * P->nb1max;
     if (H->precision == PHX_FP64) {
@@ -2449,6 +2450,15 @@ static void phel_setup(PhelHandle* P, const phx_problem& p, ElphHandle* H, const
   }
   // ---- coupling rows (one per q3) and the reduction's buffers
   P->g2Stride = size_t(P->nb1max) * nw * nm;
+  // outer points per coupling launch: with the k-mesh eigenpairs as many as keep
+  // their |g|^2 within 2 GiB (a point of a small q mesh alone does not fill the
+  // chip: 32 points of 16^3 wavevectors, 12 bands and 9 modes one by one 2.3 ms, in
+  // one launch 1.1); unfolded points have k2 eigenpairs of their own, computed
+  // one by one
+  P->points = 1;
+  if (P->folded)
+    P->points = int(std::max<size_t>(
+        1, std::min<size_t>(kCacheNKK, (size_t(2) << 30) / (size_t(P->nq) * P->g2Stride * sizeof(double)))));
   std::vector<int> u2off(P->nq), nb2(P->nq, nw), e3i(P->nq), e2o(P->nq);
   std::vector<long long> oo(P->nq);
   for (int q = 0; q < P->nq; ++q) {
@@ -2468,7 +2478,18 @@ static void phel_setup(PhelHandle* P, const phx_problem& p, ElphHandle* H, const
     P->k2.alloc(size_t(P->nq) * 3);
     P->info.alloc(P->nq);
   }
-  P->g2.alloc(size_t(P->nq) * P->g2Stride);
+  try {
+    P->g2.alloc(size_t(P->points) * P->nq * P->g2Stride);
+  } catch (const Error&) {  // no room for several points' couplings: one at a time
+    if (P->points == 1) throw;
+    (void)hipGetLastError();
+    P->points = 1;
+    P->g2.alloc(size_t(P->nq) * P->g2Stride);
+  }
+  if (P->folded) {
+    P->rowU2off.alloc(size_t(kCacheNKK) * P->nq);
+    P->e2off.alloc(size_t(kCacheNKK) * P->nq);
+  }
   P->F1.alloc(size_t(kCacheNKK) * kCMax * nw);
   P->W0.alloc(size_t(nm));
   launch_fill<double>(P->W0.p, P->W0.n, 0., s);
@@ -2501,7 +2522,8 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
   };
   // ---- batched cacheElPh
   std::vector<double> kb(3 * size_t(n));
-  std::vector<int> cm(3 * size_t(K), 0), pm(size_t(K) * blk, 0);
+  // pm: bands per point (K), per panel its point within the coupling launch and its band, mesh index per point (K)
+  std::vector<int> cm(3 * size_t(K), 0), pm(size_t(K) * (blk + 1), 0);
   std::vector<double> F(size_t(K) * kCMax * nw, 0.);
   int pb = 0;
   for (int i = 0; i < n; ++i) {
@@ -2510,10 +2532,12 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
     cm[i] = int(P->u1Off[a]);
     cm[K + i] = nb1;
     cm[2 * K + i] = pb;
-    pb += nb1;
-    int* m = &pm[size_t(i) * blk];  // kkNb1, panelKK (all 0), panelB1
-    m[0] = nb1;
-    for (int b = 0; b < nb1; ++b) m[1 + P->nb1max + b] = b;
+    pm[i] = nb1;
+    pm[size_t(K) * blk + i] = P->active[a];
+    for (int b = 0; b < nb1; ++b, ++pb) {
+      pm[size_t(K) + pb] = i % P->points;
+      pm[size_t(K) + size_t(K) * P->nb1max + pb] = b;
+    }
     const double* e1 = &P->stateE[P->stateOff[a]];
     for (int c = 0; c < P->nCalc; ++c)
       for (int b = 0; b < nb1; ++b) {
@@ -2553,31 +2577,16 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
     launch_cache<float, float>(cp, s);
   }
   rec(1);
-  // ---- every outer point against all q3
-  std::vector<double> k2(3 * size_t(nq));
-  std::vector<int> u2off, e2o;
-  for (int i = 0; i < n; ++i) {
-    const int a = as[i], nb1 = P->nb[a], ik = P->active[a];
-    const double* k1 = &P->kcart[3 * size_t(ik)];
-    if (P->folded) {
-      // k2 = k1 + q3 on the k mesh (first index fastest)
-      u2off.resize(nq);
-      e2o.resize(nq);
-      const int* m = P->kmesh;
-      const int j0 = ik % m[0], j1 = (ik / m[0]) % m[1], j2 = ik / (m[0] * m[1]);
-      for (int q = 0; q < nq; ++q) {
-        const int* mq = P->qmesh;
-        const int q0 = q % mq[0], q1 = (q / mq[0]) % mq[1], q2 = q / (mq[0] * mq[1]);
-        const int x = (j0 + q0 * (m[0] / mq[0])) % m[0], y = (j1 + q1 * (m[1] / mq[1])) % m[1],
-                  z = (j2 + q2 * (m[2] / mq[2])) % m[2];
-        const int k = (z * m[1] + y) * m[0] + x;
-        u2off[q] = k * nw * nw;
-        e2o[q] = k * nw;
-      }
-      PHX_HIP(hipMemcpyAsync(P->rowU2off.p, u2off.data(), nq * sizeof(int), hipMemcpyHostToDevice, s));
-      PHX_HIP(hipMemcpyAsync(P->e2off.p, e2o.data(), nq * sizeof(int), hipMemcpyHostToDevice, s));
-    } else {
+  // ---- groups of outer points against all q3
+  if (P->folded)
+    launch_phel_rows(n, nq, nw, P->kmesh, P->qmesh, P->pmeta.p + size_t(K) * blk, P->rowU2off.p, P->e2off.p, s);
+  std::vector<double> k2(P->folded ? 0 : 3 * size_t(nq));
+  int launches = 0;
+  for (int i0 = 0; i0 < n; i0 += P->points) {
+    const int np = std::min(P->points, n - i0);
+    if (!P->folded) {
       // k2 = k1 + q3, not folded, all bands (electronH0.populate, phel_scattering.cpp:225-243)
+      const double* k1 = &P->kcart[3 * size_t(P->active[as[i0]])];
       for (int q = 0; q < nq; ++q)
         for (int d = 0; d < 3; ++d) k2[3 * size_t(q) + d] = P->qcart[3 * size_t(q) + d] + k1[d];
       if (P->adaptive) {
@@ -2600,8 +2609,7 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
         launch_phel_flag_failures(nq, P->info.p, P->fail.p, s);
       }
     }
-    // calcCouplingSquared, store mode, every q3 in one launch
-    const int* pmk = P->pmeta.p + size_t(i) * blk;
+    // calcCouplingSquared, store mode, every q3 of the group's points in one launch
     CoupParams c{};
     c.lda = size_t(nq);
     c.nRp = H->nRp;
@@ -2610,23 +2618,27 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
     c.M = nq;
     c.nm = nm;
     c.nw = nw;
-    c.nPanels = nb1;
     c.nMtiles = ceil_div(nq, coupling_tiling(f64, nm, nw, nw).rows);
-    c.panelKK = pmk + 1;
-    c.panelB1 = pmk + 1 + P->nb1max;
-    c.kkNb1 = pmk;
+    const int pan0 = cm[2 * K + i0];
+    c.nPanels = (i0 + np < n ? cm[2 * K + i0 + np] : pb) - pan0;
+    // panels of the batch: point (relative to the group's first) and band
+    c.panelKK = P->pmeta.p + K + pan0;
+    c.panelB1 = P->pmeta.p + K + size_t(K) * P->nb1max + pan0;
+    c.kkNb1 = P->pmeta.p + i0;
     c.U2pool = P->U2.p;
-    c.rowU2off = P->rowU2off.p;
+    c.rowU2off = P->rowU2off.p + (P->folded ? size_t(i0) * nq : 0);
+    c.rowKKStride = nq;
     c.rowNb2 = P->rowNb2.p;
     c.E3pool = P->E3.p;
     c.Wpool = P->W0.p;
     c.qmode = 0;
     c.rowE3 = P->rowE3.p;
     c.out = P->g2.p;
+    c.outKKStride = (long long)nq * (long long)P->g2Stride;
     c.rowOutOff = P->rowOutOff.p;
     c.nb2max = nw;
-    const size_t panel0 = size_t(cm[2 * K + i]) * P->pstride;
-    rec(2 + 3 * i);
+    const size_t panel0 = size_t(pan0) * P->pstride;
+    rec(2 + 3 * launches);
     if (f64) {
       c.A = P->A.p;
       c.B = P->Bd.p + panel0;
@@ -2636,20 +2648,25 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
       c.B = P->Bf.p + panel0;
       launch_coupling<float>(c, false, s);
     }
-    rec(3 + 3 * i);
+    rec(3 + 3 * launches);
     PhelParams r{};
     r.nq = nq;
-    r.nb1 = nb1;
+    r.np = np;
     r.nb2 = nw;
     r.nm = nm;
     r.nCalc = P->nCalc;
+    for (int j = 0; j < np; ++j) {
+      r.nb1[j] = P->nb[as[i0 + j]];
+      r.e1[j] = int(P->stateOff[as[i0 + j]]);
+    }
     r.g2 = P->g2.p;
     r.g2Stride = P->g2Stride;
-    r.e1 = P->stateEd.p + P->stateOff[a];
+    r.E1 = P->stateEd.p;
     r.E2 = P->E2.p;
-    r.e2off = P->e2off.p;
+    r.e2off = P->e2off.p + (P->folded ? size_t(i0) * nq : 0);
     r.W3 = P->W3.p;
-    r.F1 = P->F1.p + size_t(i) * kCMax * nw;
+    r.F1 = P->F1.p + size_t(i0) * kCMax * nw;
+    r.f1Stride = size_t(kCMax) * nw;
     r.invT = P->invT.p;
     r.norm = P->norm;
     r.cutoff = phonon_cutoff();
@@ -2657,18 +2674,19 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
     r.deltaPref = P->deltaPref;
     r.adaptive = P->adaptive;
     if (P->adaptive) {
-      r.v1 = P->v1d.p + 3 * P->stateOff[a];
+      r.v1 = P->v1d.p;
       r.V2 = P->V2.p;
       for (int d = 0; d < 9; ++d) r.qT[d] = P->qT[d];
       r.minWidth = 0.0001 / units::energyRyToEv;
     }
     r.lw = P->lw.p;
     launch_phel_reduce(r, s);
-    rec(4 + 3 * i);
-    P->pairs += nq;
+    rec(4 + 3 * launches);
+    ++launches;
+    P->pairs += (long long)np * nq;
   }
   if (P->timing) {
-    PHX_HIP(hipEventSynchronize(P->tev[1 + 3 * size_t(n)]));
+    PHX_HIP(hipEventSynchronize(P->tev[1 + 3 * size_t(launches)]));
     auto ms = [&](int a, int b) {
       float t = 0.f;
       PHX_HIP(hipEventElapsedTime(&t, P->tev[a], P->tev[b]));
@@ -2676,13 +2694,13 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
     };
     P->cacheMs += ms(0, 1);
     P->cacheLaunches += 1;
-    for (int i = 0; i < n; ++i) {
+    for (int i = 0; i < launches; ++i) {
       P->coupMs += ms(2 + 3 * i, 3 + 3 * i);
       P->redMs += ms(3 + 3 * i, 4 + 3 * i);
-      // R_ph transform of the coupling: real GEMM nq x 2 nRp x 2 nm nw per panel
-      P->coupFlops += 8. * nq * H->nRp * nm * nw * P->nb[as[i]];
     }
-    P->coupLaunches += n;
+    // R_ph transform of the coupling: real GEMM nq x 2 nRp x 2 nm nw per panel
+    for (int i = 0; i < n; ++i) P->coupFlops += 8. * nq * H->nRp * nm * nw * P->nb[as[i]];
+    P->coupLaunches += launches;
   }
 }
 
