@@ -32,8 +32,10 @@ struct EpRow {
 // after B), so part of its latency passes behind the other phases; the loads
 // are unconditional (rows beyond the slot's read its last one), because a load
 // under a branch makes the compiler wait for every load in flight.  cfg2's full
-// launch (128 panels, 4 million rows of 12 modes, 16 bands x 1.7): 2.4 ms, and
-// 2.5 with w2 fastest in g3 and all loads at a pass's start.  With k_sep_yx
+// launch (128 panels, 4 million rows of 12 modes, 16 bands x 1.7): 2.37 ms; 2.43
+// with the rows in mesh order and column length rounded up to 16 modes (an exact
+// one drops a quarter of phase B there), 2.5 with w2 fastest in g3 and all loads
+// at a pass's start.  With k_sep_yx
 // against the fused k_sep_xm and its y-stage, ms per pass: FP64, 12 modes x 16
 // bands, 6 lines of a 27 x 28 x 29 mesh 6.3 against 21.2; FP32, 18 x 16, 4 lines
 // of a 32^3 mesh 7.2 against 21.8.
@@ -87,6 +89,10 @@ __device__ __forceinline__ void ep2_rot_ph(const T2v (&e3c)[NMX], const double2*
   for (int b2 = 0; b2 < NB; ++b2) own[b2] = gr[b2] * gr[b2] + gi[b2] * gi[b2];
 }
 
+// Instances that serve one mode count only (1 to 6 atoms): the modes' offsets are
+// then constants of the load instructions.
+constexpr bool ep2_exact(int nmx) { return nmx <= 18; }
+
 // Rows per pass at most: whole rows of nm lanes for the least nm served with
 // NMX, and no more than five.  Ten rows of 6 modes fill the wave but hold twice
 // the U2 entries in registers, and spill: 52 us against 37 per launch of 128
@@ -121,7 +127,7 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams
     if (t < kGMax * kCMax) p.partial[size_t(slot) * kGMax * kCMax + t] = 0.;
     return;
   }
-  const int nm = p.nm, nw = p.nw, ncol = nm * nw, R = p.rpw;
+  const int nm = ep2_exact(NMX) ? NMX : p.nm, nw = p.nw, ncol = nm * nw, R = p.rpw;
   const int kk = p.panelKK[panel];
   const int gstart = p.panelGStart[panel], gsize = __builtin_amdgcn_readfirstlane(p.panelGSize[panel]);
   const int is1 = p.kkStateOff[kk] + gstart;
@@ -142,13 +148,24 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams
   for (int i = t; i < R * GPS; i += 64) gp[i] = make_double2(0., 0.);
   const int nkeep = __popcll(mask);
   {
-    const int kkMesh = p.kkMesh[kk];
-    if (t < p.m0 && ((mask >> t) & 1ull)) {
-      const int mesh = (jz * p.m1 + jy) * p.m0 + t;
-      const int4 mr = p.meshRow[mesh];
-      rows[__popcll(mask & ((1ull << t) - 1ull))] =
-          EpRow{t | mr.y << 8, mesh_diff_index(mesh, kkMesh, p.m0, p.m1, p.m2), mr.z, mr.w};
+    // q = k2 - k1 folded: its y and z are the slot's, x the row's
+    int x1, y1, z1;
+    mesh_coords(__builtin_amdgcn_readfirstlane(p.kkMesh[kk]), p.m0, p.m1, x1, y1, z1);
+    const int dy = jy - y1 + (jy < y1 ? p.m1 : 0), dz = jz - z1 + (jz < z1 ? p.m2 : 0);
+    const bool keep = t < p.m0 && ((mask >> t) & 1ull);
+    int4 mr = make_int4(0, 0, 0, 0);
+    if (keep) mr = p.meshRow[(jz * p.m1 + jy) * p.m0 + t];
+    // the rows in order of their band counts, most first: a pass runs its largest
+    // count for all of its rows, so rows of like counts share passes
+    const unsigned long long below = (1ull << t) - 1ull;
+    int pos = 0;
+#pragma unroll
+    for (int n = NB2; n >= 1; --n) {
+      const unsigned long long same = __ballot(keep && mr.y == n);
+      if (mr.y == n) pos += __popcll(same & below);
+      else if (mr.y < n) pos += __popcll(same);
     }
+    if (keep) rows[pos] = EpRow{t | mr.y << 8, (dz * p.m1 + dy) * p.m0 + t - x1 + (t < x1 ? p.m0 : 0), mr.z, mr.w};
   }
   __syncthreads();
   if (t == 0) {
@@ -187,12 +204,12 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams
       for (int b2 = 0; b2 < NB2; ++b2) gv[b2] = GP[size_t(jx) * rowG + min(b2, (ri.jxnb >> 8) - 1) * nm + sub];
     } else {
       // a row's modes are neighbours, so one load's lanes fall into a few lines
-      // (with w2 fastest every lane was in a line of its own)
-      const T2v* src = G3 + size_t(jx) * ncol + sub;
-      int st = nm;
-      asm volatile("" : "+s"(st));
+      // (with w2 fastest every lane was in a line of its own); the w2 offset is
+      // uniform, the lane's 32-bit offset the same for all of them
+      const unsigned off = unsigned(jx * ncol + sub) * unsigned(sizeof(T2v));
 #pragma unroll
-      for (int w2 = 0; w2 < NWX; ++w2) g[w2] = src[min(w2, nw - 1) * st];
+      for (int w2 = 0; w2 < NWX; ++w2)
+        g[w2] = *reinterpret_cast<const T2v*>(reinterpret_cast<const char*>(G3 + min(w2, nw - 1) * nm) + off);
     }
   };
   // U2 of the pass: entry i = (row, b2, w2), w2 fastest, NWX x NB2 per row; and the band
@@ -202,8 +219,10 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams
 #pragma unroll
       for (int u = 0; u < UPL; ++u) {  // NWX NB2 is one or two waves of entries: a row per load
         const EpRow q = row_of(m0r, min(64 * u / (NWX * NB2), R - 1));
-        const int b2 = (t + 64 * u) % (NWX * NB2) / NWX;
-        u2v[u] = p.U2pool[q.u2off + min(b2, (q.jxnb >> 8) - 1) * nw + min(t % NWX, nw - 1)];
+        const int b2 = (t + 64 * u) % (NWX * NB2) / NWX, nb = __builtin_amdgcn_readfirstlane(q.jxnb >> 8);
+        const double2* src = p.U2pool + __builtin_amdgcn_readfirstlane(q.u2off);
+        const unsigned off = unsigned(min(b2, nb - 1) * nw + min(t % NWX, nw - 1)) * unsigned(sizeof(double2));
+        u2v[u] = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(src) + off);
       }
     }
     const EpRow q = row_of(m0r, min(t / NB2, R - 1));
@@ -220,7 +239,7 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams
     asm volatile("" : "+s"(st));
     const T2v* e3 = E3T + size_t(iq) * nm * nm + sub;
 #pragma unroll
-    for (int nu = 0; nu < NMX; ++nu) e3c[nu] = e3[min(nu, st - 1) * st];
+    for (int nu = 0; nu < NMX; ++nu) e3c[nu] = ep2_exact(NMX) ? e3[nu * NMX] : e3[min(nu, st - 1) * st];
     w3 = p.Wpool[size_t(iq) * nm + sub];
     grp = p.qModeGrp[size_t(iq) * nm + sub];
 #pragma unroll
@@ -279,7 +298,9 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams
       }
     } else if (rowOn) {
       const double2* u = sU2 + r * U2S;
-      for (int b = 0; b < nbw; b += 2) ep2_rot_el<T2v, NWX, 2>(g, u + b * NWX, out + b);
+      int b = 0;
+      for (; b + 1 < nbw; b += 2) ep2_rot_el<T2v, NWX, 2>(g, u + b * NWX, out + b);
+      if (b < nbw) ep2_rot_el<T2v, NWX, 1>(g, u + b * NWX, out + b);
     }
     load_g(m0r + R);
     load_u2(m0r + R);
@@ -288,7 +309,9 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams
     double* gq = gsq + (r * NMX + sub) * NB2;
     if (rowOn) {
       const double2* x = gp + r * GPS;
-      for (int b = 0; b < nbw; b += 2) ep2_rot_ph<T2v, NMX, NB2, 2>(e3c, x + b, gq + b);
+      int b = 0;
+      for (; b + 1 < nbw; b += 2) ep2_rot_ph<T2v, NMX, NB2, 2>(e3c, x + b, gq + b);
+      if (b < nbw) ep2_rot_ph<T2v, NMX, NB2, 1>(e3c, x + b, gq + b);
     }
     const double w3c = w3;
     const int grpc = grp;
@@ -390,7 +413,7 @@ void launch_ep2(EpParams q, int gsizeMax, int grid, bool pre, hipStream_t s) {
   const int gm = gsizeMax > 0 ? gsizeMax : kGMax;
   PHX_REQUIRE(gm <= kGMax && q.nb2max <= kSepNb2 && q.nm <= kSepNm && q.nCalc <= kCMax,
               "separable transform: epilogue sizes");
-  PHX_REQUIRE(!pre || (sizeof(T) == 4 && q.nm <= 18 && !q.adaptive), "separable transform: rotated x-stage is FP32 only");
+  PHX_REQUIRE(!pre || (sizeof(T) == 4 && q.nm <= 24 && !q.adaptive), "separable transform: rotated x-stage is FP32 only");
   auto go = [&](auto nmx, auto small, auto cmx, auto prec) {
     constexpr int NM = decltype(nmx)::value, NB = decltype(small)::value ? 4 : 8, CM = decltype(cmx)::value;
     constexpr bool PRE = decltype(prec)::value == 1, ADAPT = decltype(prec)::value == 2;
@@ -414,17 +437,22 @@ void launch_ep2(EpParams q, int gsizeMax, int grid, bool pre, hipStream_t s) {
     small ? calcs(nmx, std::true_type{}, kind) : calcs(nmx, std::false_type{}, kind);
   };
   auto sizes = [&](auto nmx) {
-    if constexpr (sizeof(T) == 4 && decltype(nmx)::value <= 18) {
+    if constexpr (sizeof(T) == 4 && decltype(nmx)::value <= 24) {
       if (pre) return kinds(nmx, std::integral_constant<int, 1>{});
     }
     q.adaptive ? kinds(nmx, std::integral_constant<int, 2>{}) : kinds(nmx, std::integral_constant<int, 0>{});
   };
-  if (q.nm <= 6) sizes(std::integral_constant<int, 6>{});
-  else if (q.nm <= 9) sizes(std::integral_constant<int, 9>{});
-  else if (q.nm <= 12) sizes(std::integral_constant<int, 12>{});
-  else if (q.nm <= 18) sizes(std::integral_constant<int, 18>{});
-  else if (q.nm <= 24) sizes(std::integral_constant<int, 24>{});
-  else sizes(std::integral_constant<int, kSepNm>{});
+  switch (q.nm) {
+    case 3: sizes(std::integral_constant<int, 3>{}); break;
+    case 6: sizes(std::integral_constant<int, 6>{}); break;
+    case 9: sizes(std::integral_constant<int, 9>{}); break;
+    case 12: sizes(std::integral_constant<int, 12>{}); break;
+    case 15: sizes(std::integral_constant<int, 15>{}); break;
+    case 18: sizes(std::integral_constant<int, 18>{}); break;
+    default:
+      if (q.nm <= 24) sizes(std::integral_constant<int, 24>{});
+      else sizes(std::integral_constant<int, kSepNm>{});
+  }
   PHX_HIP(hipGetLastError());
 }
 
