@@ -1976,42 +1976,58 @@ constexpr int kXminBlocks = 64;
 // pair, so once the block has found a pair closer than n the skipped rows
 // cannot hold its minimum.  Otherwise it evaluates every row.  One partial
 // minimum (energy units, HUGE_VAL when there is no pair) per block.
+// Bound by the frequencies' loads: a wave lists its rows in LDS and then takes
+// them (row, mode) by lane, so that a load's lanes read neighbouring modes.  With
+// a row per lane each load touched 64 lines: 313 us against 199 for 128 panels of
+// a 40^3 mesh of 12 modes, 12.7 against 10.3 for a line of a 9 x 8 x 7 mesh of 9.
 static __global__ void __launch_bounds__(256) k_sep_xmin(CoupParams p) {
-  const int panel = blockIdx.y, t = threadIdx.x;
+  const int panel = blockIdx.y, t = threadIdx.x, lane = t & 63;
   const int kk = p.panelKK[panel];
   const int kmesh = p.kkMesh[kk];
   const double* e1 = p.e1pool + p.kkStateOff[kk] + p.panelGStart[panel];
   const int gsz = p.panelGSize[panel];
   const double lim = p.screen / p.invSigma;
-  const int nmesh = p.m0 * p.m1 * p.m2;
+  const int nmesh = p.m0 * p.m1 * p.m2, nm = p.nm;
   __shared__ double red[256];
+  __shared__ int4 list[256];  // per wave 64 rows: (q, first state, bands)
+  int4* mine = list + (t & ~63);
+  const float invNm = 1.f / float(nm);
   double best = HUGE_VAL, bmin = HUGE_VAL;
   for (int pass = 0; pass < 2; ++pass) {
-    for (int mesh = blockIdx.x * 256 + t; mesh < nmesh; mesh += 256 * kXminBlocks) {
-      const int row = p.meshToRow[mesh];
-      if (row < p.rowLo || row >= p.rowHi) continue;
-      const int iq = mesh_diff_index(mesh, kmesh, p.m0, p.m1, p.m2);
-      const double wlo = p.qWlo[iq], whi = p.qWhi[iq];
-      if (whi < wlo) continue;  // no mode above the cutoff
-      if (pass == 0) {
-        const double2 er = p.rowE2range[row];
-        bool keep = false;
-        for (int gi = 0; gi < gsz; ++gi) {
-          const double a_lo = e1[gi] - er.y + wlo, a_hi = e1[gi] - er.x + whi;
-          const double b_lo = e1[gi] - er.y - whi, b_hi = e1[gi] - er.x - wlo;
-          keep |= (a_hi > -lim && a_lo < lim) || (b_hi > -lim && b_lo < lim);
+    for (int m0 = blockIdx.x * 256 + (t & ~63); m0 < nmesh; m0 += 256 * kXminBlocks) {
+      const int mesh = m0 + lane;
+      int4 mr = make_int4(-1, 0, 0, 0);
+      if (mesh < nmesh) mr = p.meshRow[mesh];
+      bool keep = mr.x >= p.rowLo && mr.x < p.rowHi;
+      int iq = 0;
+      if (keep) {
+        iq = mesh_diff_index(mesh, kmesh, p.m0, p.m1, p.m2);
+        const double wlo = p.qWlo[iq], whi = p.qWhi[iq];
+        keep = whi >= wlo;  // a mode above the cutoff
+        if (keep && pass == 0) {
+          const double2 er = p.rowE2range[mr.x];
+          keep = false;
+          for (int gi = 0; gi < gsz; ++gi) {
+            const double a_lo = e1[gi] - er.y + wlo, a_hi = e1[gi] - er.x + whi;
+            const double b_lo = e1[gi] - er.y - whi, b_hi = e1[gi] - er.x - wlo;
+            keep |= (a_hi > -lim && a_lo < lim) || (b_hi > -lim && b_lo < lim);
+          }
         }
-        if (!keep) continue;
       }
-      const double* w = p.Wpool + size_t(iq) * p.nm;
-      const int soff = p.rowStateOff[row], nb2 = p.rowNb2[row];
-      for (int b2 = 0; b2 < nb2; ++b2) {
-        const double e2 = p.e2pool[soff + b2];
-        for (int gi = 0; gi < gsz; ++gi) {
-          const double d = e1[gi] - e2;
-          for (int nu = 0; nu < p.nm; ++nu) {
-            const double om = w[nu];
-            if (om < p.cutoff) continue;
+      const unsigned long long kept = __ballot(keep);
+      wave_sync();  // the wave has read its previous list
+      if (keep) mine[__popcll(kept & ((1ull << lane) - 1ull))] = make_int4(iq, mr.w, mr.y, 0);
+      wave_sync();
+      const int items = __popcll(kept) * nm;
+      for (int i = lane; i < items; i += 64) {
+        int r = int((float(i) + 0.5f) * invNm);  // i / nm, exact up to 64 rows
+        const int4 row = mine[r];
+        const double om = p.Wpool[size_t(row.x) * nm + (i - r * nm)];
+        if (om < p.cutoff) continue;
+        for (int b2 = 0; b2 < row.z; ++b2) {
+          const double e2 = p.e2pool[row.y + b2];
+          for (int gi = 0; gi < gsz; ++gi) {
+            const double d = e1[gi] - e2;
             // only pairs the one-sided Gaussian can weigh (x <= 6, delta_function.cpp:43)
             const double a = d + om, b = d - om;
             if (a * p.invSigma <= 6.) best = fmin(best, fabs(a));
@@ -2033,44 +2049,55 @@ static __global__ void __launch_bounds__(256) k_sep_xmin(CoupParams p) {
   if (t == 0) p.xminPart[size_t(panel) * kXminBlocks + blockIdx.x] = bmin;
 }
 
-// Screen width of each panel: sqrt(xmin^2 + n^2) sigma, with xmin its closest
+// Screen width of a panel: sqrt(xmin^2 + n^2) sigma, with xmin its closest
 // approach to resonance in units of sigma.  A pair that the screen drops then
 // weighs at most exp(-n^2) of the panel's most resonant weighed pair, whatever
 // the panel's distance to resonance (a panel whose pairs all lie in the
-// Gaussian tails keeps its closest rows).  One thread per panel.
-static __global__ void __launch_bounds__(64) k_sep_xmin_fin(CoupParams p) {
-  const int panel = blockIdx.x * 64 + threadIdx.x;
-  if (panel >= p.nPanels) return;
+// Gaussian tails keeps its closest rows).  For a whole wave; the same value in
+// every lane.
+__device__ inline double sep_panel_width(const CoupParams& p, int panel) {
   double m = HUGE_VAL;
-  for (int b = 0; b < kXminBlocks; ++b) m = fmin(m, p.xminPart[size_t(panel) * kXminBlocks + b]);
+  for (int b = threadIdx.x & 63; b < kXminBlocks; b += 64) m = fmin(m, p.xminPart[size_t(panel) * kXminBlocks + b]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o));
   const double x = m * p.invSigma;
-  const int is1 = p.kkStateOff[p.panelKK[panel]] + p.panelGStart[panel];
-  p.screenOf[is1] = x < HUGE_VAL ? sqrt(x * x + p.screen * p.screen) : p.screen;
+  return x < HUGE_VAL ? sqrt(x * x + p.screen * p.screen) : p.screen;
+}
+
+// The widths alone (where no row masks are made).  One wave per panel.
+static __global__ void __launch_bounds__(64) k_sep_xmin_fin(CoupParams p) {
+  const int panel = blockIdx.x;
+  const double w = sep_panel_width(p, panel);
+  if (threadIdx.x == 0) p.screenOf[p.kkStateOff[p.panelKK[panel]] + p.panelGStart[panel]] = w;
 }
 
 // Row lists of the last stage: for every (panel, yz) slot, bit jx of
 // keepMask[slot] is set when mesh point (jx, jy, jz) is an inner point of the
 // range and passes the energy screen (same interval test as k_sep_x; every
-// valid row when the screen is off).  One thread per slot, m0 <= 64.
-static __global__ void __launch_bounds__(256) k_sep_screen(CoupParams p) {
-  const int nLinesYZ = p.m1 * p.m2;
-  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= p.nPanels * nLinesYZ) return;
-  const int panel = slot / nLinesYZ, yz = slot % nLinesYZ;
-  const int jy = yz % p.m1, jz = yz / p.m1;
+// valid row when the screen is off), m0 <= 64.  A row per lane, 64, 32 or 16 lanes
+// per slot; grid (slots of a panel, panels).  With widths per panel each wave
+// works its panel's out, and the first stores it for the epilogue.  A slot per
+// thread reads its rows one after the other from lines of its own: 144 us for 128
+// panels of a 40^3 mesh against 101, and 14 against 5 for 128 panels of a 12^3 one.
+template <int L>
+__global__ void __launch_bounds__(256) k_sep_screen(CoupParams p) {
+  const int nLinesYZ = p.m1 * p.m2, panel = blockIdx.y, t = threadIdx.x, jx = t % L;
+  const int yz = blockIdx.x * (256 / L) + t / L;
   const int kk = p.panelKK[panel];
-  const int kmesh = p.kkMesh[kk];
-  const double* e1 = p.e1pool + p.kkStateOff[kk] + p.panelGStart[panel];
-  const int gsz = p.panelGSize[panel];
-  const double lim = screen_width(p, int(e1 - p.e1pool)) / p.invSigma;
-  unsigned long long mask = 0ull;
-  for (int jx = 0; jx < p.m0; ++jx) {
-    const int mesh = (jz * p.m1 + jy) * p.m0 + jx;
-    const int row = p.meshRow[mesh].x;
-    if (row < p.rowLo || row >= p.rowHi) continue;
-    bool keep = true;
-    if (p.screen > 0.) {
-      const int iq = mesh_diff_index(mesh, kmesh, p.m0, p.m1, p.m2);
+  const int gstart = p.panelGStart[panel], gsz = p.panelGSize[panel];
+  const double* e1 = p.e1pool + p.kkStateOff[kk] + gstart;
+  double lim = 0.;
+  if (p.screen > 0.) {
+    lim = p.screenOf ? sep_panel_width(p, panel) : p.screen;
+    if (p.screenOf && t == 0 && blockIdx.x == 0) p.screenOf[p.kkStateOff[kk] + gstart] = lim;
+    lim /= p.invSigma;
+  }
+  bool keep = false;
+  if (yz < nLinesYZ && jx < p.m0) {
+    const int mesh = yz * p.m0 + jx, row = p.meshRow[mesh].x;
+    keep = row >= p.rowLo && row < p.rowHi;
+    if (keep && p.screen > 0.) {
+      const int iq = mesh_diff_index(mesh, p.kkMesh[kk], p.m0, p.m1, p.m2);
       const double wlo = p.qWlo[iq], whi = p.qWhi[iq];
       const double2 er = p.rowE2range[row];
       keep = false;
@@ -2081,9 +2108,9 @@ static __global__ void __launch_bounds__(256) k_sep_screen(CoupParams p) {
           keep |= (a_hi > -lim && a_lo < lim) || (b_hi > -lim && b_lo < lim);
         }
     }
-    if (keep) mask |= 1ull << jx;
   }
-  p.keepMask[slot] = mask;
+  const unsigned long long all = __ballot(keep), ones = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
+  if (jx == 0 && yz < nLinesYZ) p.keepMask[size_t(panel) * nLinesYZ + yz] = (all >> ((t & 63) / L * L)) & ones;
 }
 
 inline size_t sep_xm_lds_bytes(int elem, int nG0, int m0, int nw, int nm, int nb2max, int rpp, int nCalc) {
@@ -2157,11 +2184,13 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
   PHX_REQUIRE(!bf3 || (bf3t && reduce && sp.ncol <= 4 * 6 * 16),
               "split-BF16x3: FP32 data, the linewidth reduction and nm nw <= 384");
   if (reduce && p.screen > 0. && p.screenOf) {
-    PHX_REQUIRE(p.xminPart && p.meshToRow, "energy screen: closest-approach buffers missing");
+    PHX_REQUIRE(p.xminPart && p.meshRow, "energy screen: closest-approach buffers missing");
     hipLaunchKernelGGL(k_sep_xmin, dim3(kXminBlocks, sp.nPanels), dim3(256), 0, s, p);
     PHX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_sep_xmin_fin, dim3(ceil_div(sp.nPanels, 64)), dim3(64), 0, s, p);
-    PHX_HIP(hipGetLastError());
+    if (!(p.keepMask && sp.ncol <= 4 * 6 * 16)) {  // else the row masks' kernel stores the widths
+      hipLaunchKernelGGL(k_sep_xmin_fin, dim3(sp.nPanels), dim3(64), 0, s, p);
+      PHX_HIP(hipGetLastError());
+    }
   }
   if (reduce && sp.ncol <= 4 * 6 * 16) {
     const bool wide = sp.ncol > 4 * 3 * 16;
@@ -2171,7 +2200,11 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
     PHX_REQUIRE(p.qModeGrp && p.E3T, "separable transform: mode-group or eigenvector table missing");
     if (p.keepMask) {
       PHX_REQUIRE(p.m0 <= 64 && p.meshRow, "separable transform: row masks need m0 <= 64");
-      hipLaunchKernelGGL(k_sep_screen, dim3(ceil_div(tiles, 256)), dim3(256), 0, s, p);
+      const int lines = sp.my * sp.mz;
+      if (p.m0 <= 16) hipLaunchKernelGGL(k_sep_screen<16>, dim3(ceil_div(lines, 16), sp.nPanels), dim3(256), 0, s, p);
+      else if (p.m0 <= 32)
+        hipLaunchKernelGGL(k_sep_screen<32>, dim3(ceil_div(lines, 8), sp.nPanels), dim3(256), 0, s, p);
+      else hipLaunchKernelGGL(k_sep_screen<64>, dim3(ceil_div(lines, 4), sp.nPanels), dim3(256), 0, s, p);
       PHX_HIP(hipGetLastError());
     }
     const bool split = sep_runs_split<T>(sp, p);
