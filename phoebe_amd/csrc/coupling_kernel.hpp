@@ -519,18 +519,23 @@ __global__ void __launch_bounds__(256) k_sep_z(SepParams p) {
 
 // ------------------------------------------------------------------ y-stage on the matrix cores
 // T2(g, jy, c) = sum_{(f1, line) in group g} w_y^{jy f1} T1(line, jz, c) for 16
-// y coordinates and 16 columns at once on v_mfma_f64_16x16x4: M = jy, N =
-// columns, K = a quad of the group's entries, whose real and imaginary parts
-// take two products per accumulator (Re += Wr x, Re += (-Wi) y, Im += Wi x,
-// Im += Wr y).  The groups are dealt to the four waves by the host (waveQ), so
+// y coordinates and 16 columns at once on v_mfma_f64_16x16x4, N = columns, K = a
+// quad of the group's entries.  The coordinates go in pairs jy, my - jy, whose
+// twiddles are conjugate: with C = sum cos x and S = sum sin x over the entries,
+// T2(jy) = (Re C - Im S, Im C + Re S) and T2(my - jy) = (Re C + Im S, Im C - Re S).
+// Rows 0..7 of M are the cosines of eight pairs and rows 8..15 their sines, so that
+// a pair's C and S are registers of the same lane, and a quad takes two products
+// (x's real and imaginary parts) where one coordinate per row took four.  The pair
+// of jy = 0 has no sines; for even my its S rows hold w^{f1 my / 2} = (-1)^f1, and
+// S is T2(my / 2).  The groups are dealt to the four waves by the host (waveQ), so
 // a group's sum stays in one wave's registers, in ascending order of its
 // entries; T1 goes from L2 straight to registers, four quads ahead.  FP64 sums
 // of the data's precision, rounded once on storing.
 // Shared by k_sep_y and k_sep_yx, which so give the same T2 bit for bit.
 struct SepYShared {
-  double2* tw;  // my: e^{2 pi i t / my}
-  int2* ent;    // 4 nQuads: (T1 row at jz: offset of its first column, or -1: padding; f1)
-  int* end;     // nQuads: group that ends with the quad, or -1
+  double* tw;  // my: cos(2 pi t / my), then my: sin
+  int2* ent;   // 4 nQuads: (T1 row at jz: offset of its first column, or -1: padding; f1)
+  int* end;    // nQuads: group that ends with the quad, or -1
 };
 __host__ __device__ inline size_t sep_y_lds_bytes(int my, int nQuads) {
   return size_t(my) * sizeof(double2) + size_t(4) * nQuads * sizeof(int2) +
@@ -538,10 +543,14 @@ __host__ __device__ inline size_t sep_y_lds_bytes(int my, int nQuads) {
 }
 __device__ __forceinline__ SepYShared sep_y_stage(const SepParams& p, unsigned char* smem, int jz) {
   SepYShared s;
-  s.tw = reinterpret_cast<double2*>(smem);
-  s.ent = reinterpret_cast<int2*>(s.tw + p.my);
+  s.tw = reinterpret_cast<double*>(smem);
+  s.ent = reinterpret_cast<int2*>(s.tw + 2 * p.my);
   s.end = reinterpret_cast<int*>(s.ent + 4 * p.nQuads);
-  for (int i = threadIdx.x; i < p.my; i += 256) s.tw[i] = p.twy[i];
+  for (int i = threadIdx.x; i < p.my; i += 256) {
+    const double2 w = p.twy[i];
+    s.tw[i] = w.x;
+    s.tw[p.my + i] = w.y;
+  }
   for (int i = threadIdx.x; i < 4 * p.nQuads; i += 256) {
     const int2 e = p.quadEnt[i];
     s.ent[i] = make_int2(e.x < 0 ? -1 : (e.x * p.mz + jz) * p.ncol, e.y);
@@ -549,10 +558,20 @@ __device__ __forceinline__ SepYShared sep_y_stage(const SepParams& p, unsigned c
   for (int i = threadIdx.x; i < p.nQuads; i += 256) s.end[i] = p.quadEnd[i];
   return s;
 }
-// store(g, jj, re, im): column min(col0 + lane % 16, ncol - 1) of y coordinate jy0 + jj
+// The pairs of a y mesh, and the coordinate of a tile's place jj (pairs r0 .. r0 + 7:
+// places 0..7 their first coordinates, 8..15 their second ones), or -1.
+__host__ __device__ inline int sep_y_pairs(int my) { return (my + 1) / 2; }
+__device__ __forceinline__ int sep_y_coord(int my, int r0, int jj) {
+  const int r = r0 + (jj & 7);
+  if (r >= sep_y_pairs(my)) return -1;
+  if (jj < 8) return r;
+  return r > 0 ? my - r : my % 2 == 0 ? my / 2 : -1;
+}
+// store(g, jj, re, im): column min(col0 + lane % 16, ncol - 1) of place jj's y coordinate
+// (for places without one, of no meaning)
 template <typename T, typename Store>
 __device__ __forceinline__ void sep_y_tile(const SepParams& p, const SepYShared& s,
-                                           const typename Vec2<T>::type* T1, int col0, int jy0, Store store) {
+                                           const typename Vec2<T>::type* T1, int col0, int r0, Store store) {
   typedef typename Vec2<T>::type T2v;
   constexpr int NQ = 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15,
@@ -560,7 +579,10 @@ __device__ __forceinline__ void sep_y_tile(const SepParams& p, const SepYShared&
   const int q0 = p.waveQ[wave], q1 = p.waveQ[wave + 1];
   if (q0 == q1) return;
   const T2v* src = T1 + min(col0 + lr, p.ncol - 1);
-  const int jy = jy0 + lr;
+  // the lane's twiddles: cosines of coordinate r0 + lr, or sines of r0 + lr - 8
+  const bool half = r0 == 0 && lr == 8;  // S row of jy = 0: cosines of my / 2
+  const int jy = half ? p.my / 2 : r0 + (lr & 7);
+  const double* tw = s.tw + (lr < 8 || half ? 0 : p.my);
   const float invMy = 1.f / float(p.my);
   T2v x[NQ], xn[NQ];
   int2 e[NQ], en[NQ];
@@ -584,20 +606,20 @@ __device__ __forceinline__ void sep_y_tile(const SepParams& p, const SepYShared&
         r += r < 0 ? p.my : 0;
         r -= r >= p.my ? p.my : 0;
         const bool on = e[u].x >= 0;
-        const double2 w = s.tw[r];
-        const double wr = on ? w.x : 0., wi = on ? w.y : 0.;
-        const double xr = on ? double(x[u].x) : 0., xi = on ? double(x[u].y) : 0.;
-        re = Mfma4<double>::mac(wr, xr, re);
-        im = Mfma4<double>::mac(wi, xr, im);
-        re = Mfma4<double>::mac(-wi, xi, re);
-        im = Mfma4<double>::mac(wr, xi, im);
+        const double w = tw[r];
+        re = Mfma4<double>::mac(w, on ? double(x[u].x) : 0., re);
+        im = Mfma4<double>::mac(w, on ? double(x[u].y) : 0., im);
         const int g = __builtin_amdgcn_readfirstlane(s.end[q + u]);
         if (g >= 0) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            store(g, Mfma4<double>::row(lg, i), re[i], im[i]);
-            re[i] = im[i] = 0.;
+          for (int i = 0; i < 2; ++i) {
+            const int r = Mfma4<double>::row(lg, i);  // < 8; its sines are row(lg, i + 2) = r + 8
+            const bool zero = r0 + r == 0;
+            store(g, r, zero ? re[i] : re[i] - im[i + 2], zero ? im[i] : im[i] + re[i + 2]);
+            store(g, r + 8, zero ? re[i + 2] : re[i] + im[i + 2], zero ? im[i + 2] : im[i] - re[i + 2]);
           }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) re[i] = im[i] = 0.;
         }
       }
     }
@@ -620,10 +642,10 @@ __global__ void __launch_bounds__(256) k_sep_y(SepParams p) {
   __syncthreads();
   const T2v* T1 = reinterpret_cast<const T2v*>(static_cast<const T*>(p.T1) + size_t(panel) * p.t1PanelStride);
   T2v* out = reinterpret_cast<T2v*>(static_cast<T*>(p.T2) + size_t(panel) * p.t2PanelStride) + c;
-  for (int jy0 = 0; jy0 < p.my; jy0 += 16)
-    sep_y_tile<T>(p, s, T1, col0, jy0, [&](int g, int jj, double re, double im) {
-      const int jy = jy0 + jj;
-      if (jy < p.my && c < p.ncol) out[((size_t(g) * p.my + jy) * p.mz + jz) * p.ncol] = T2v{T(re), T(im)};
+  for (int r0 = 0; r0 < sep_y_pairs(p.my); r0 += 8)
+    sep_y_tile<T>(p, s, T1, col0, r0, [&](int g, int jj, double re, double im) {
+      const int jy = sep_y_coord(p.my, r0, jj);
+      if (jy >= 0 && c < p.ncol) out[((size_t(g) * p.my + jy) * p.mz + jz) * p.ncol] = T2v{T(re), T(im)};
     });
 }
 
@@ -1828,10 +1850,12 @@ inline size_t sep_xg_lds_bytes(int elem, int nG0, int m0, int nm = 0, int nw = 0
 // block's columns.  The k order is that of k_sep_xg and k_sep_xm, so the g3
 // are the same.
 // Matrix cores and the g3 writes: cfg2's full launch (128 panels of 40^3 x 192
-// columns) is 31 GFLOP FP64 in y (40 of 48 rows used), 80 GFLOP FP32 in x and
-// 7 GB of traffic.  With the y sums as FMAs of four y coordinates per LDS read
+// columns) is 16 GFLOP FP64 in y (20 of 24 pair rows used), 80 GFLOP FP32 in x and
+// 9 GB of traffic.  With the y sums as FMAs of four y coordinates per LDS read
 // of T1, in threads that owned whole groups of uneven size, it took 3.9 ms; on
-// the matrix cores 3.3.
+// the matrix cores 3.3 with a coordinate per row, 3.1 with conjugate pairs (FP64,
+// 27 x 28 x 29: 1.94 and 1.88 ms).  Non-temporal g3 stores and the slots' masks in
+// LDS measured the same.
 inline size_t sep_yx_lds_bytes(int elem, int nQuads, int my, int nG0, int m0) {
   const int kp = (2 * nG0 + 3) / 4 * 4;
   return sep_y_lds_bytes(my, nQuads) + size_t(m0) * (kp + 1) * 2 * elem + size_t(16) * (kp * 16 + 16) * elem +
@@ -1870,15 +1894,17 @@ __global__ void __launch_bounds__(256) k_sep_yx(SepParams sp, CoupParams p) {
   const T2v* T1 = reinterpret_cast<const T2v*>(static_cast<const T*>(sp.T1) + size_t(panel) * sp.t1PanelStride);
   const int nLinesYZ = p.m1 * p.m2;
   const int c = cb * 16 + lr;
-  for (int jy0 = 0; jy0 < my; jy0 += 16) {
-    const int nj = min(16, my - jy0);
-    sep_y_tile<T>(sp, sy, T1, cb * 16, jy0, [&](int g, int jj, double re, double im) {
+  for (int r0 = 0; r0 < sep_y_pairs(my); r0 += 8) {
+    sep_y_tile<T>(sp, sy, T1, cb * 16, r0, [&](int g, int jj, double re, double im) {
       sT2[jj * js + (2 * g) * 16 + lr] = T(re);
       sT2[jj * js + (2 * g + 1) * 16 + lr] = T(im);
     });
     __syncthreads();
-    for (int jj = wave; jj < nj; jj += 4) {
-      const int slot = panel * nLinesYZ + jz * p.m1 + jy0 + jj;
+    const int np = min(8, sep_y_pairs(my) - r0);
+    for (int i = wave; i < 2 * np; i += 4) {  // only the tile's pairs, so that the waves share them evenly
+      const int jj = i < np ? i : 8 + i - np, jy = sep_y_coord(my, r0, jj);
+      if (jy < 0) continue;
+      const int slot = panel * nLinesYZ + jz * p.m1 + jy;
       const unsigned long long mask = p.keepMask[slot];
       if (mask == 0ull) continue;
       wave_sync();  // the wave's previous slot has read its list
