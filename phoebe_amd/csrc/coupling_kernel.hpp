@@ -1050,138 +1050,6 @@ __device__ inline void bf16_split8(const float (&x)[8], bf16x8_t& hi, bf16x8_t& 
   lo = __builtin_bit_cast(bf16x8_t, l8);
 }
 
-// Second half of an epilogue pass of k_sep_ep (k_sep_xm keeps the same steps
-// inline, where the compiler allocates them without spills).  Once the
-// wave's g'(nu, b2) rows are in gp (row rl at gp + rl * gps, (nu, b2) at
-// nu * nb2max + b2): the phonon rotation, |g|^2, symmetrizeCoupling along b2
-// and nu, and the Gaussian-delta weights into part (or the store of |g|^2).
-// The thread serves row r (rl within the pass) and mode sub; the row data
-// (e2, mode groups, occupations) of the 16-row tile and the b1 group's
-// energies se1 are in LDS.  Wave-level ordering only.
-template <typename T, bool REDUCE, int NMX, int CM>
-__device__ __forceinline__ void sep_epilogue_tail(const CoupParams& p, const SepXmRow& ri, int r, int rl, int sub,
-                                                  int nb2, bool modeOn, double w3, double2* gp, int gps,
-                                                  const double* se2, const int* sg3, const double* sf2,
-                                                  const double* se1, const typename Vec2<T>::type (&e3c)[NMX],
-                                                  const double (&n3)[CM], double (&part)[kGMax][CM],
-                                                  const double* e1, int kk, int b1p, int gsize, double inv_g) {
-  const int nm = p.nm, nCalc = p.nCalc;
-  const double scrW = p.screen > 0. ? screen_width(p, int(e1 - p.e1pool)) : 0.;
-  // g(nu2, b2) = sum_nu e3(nu, nu2) g'(nu, b2), thread nu2 = sub; |g|^2 in registers
-  double v[kSepNb2];
-#pragma unroll
-  for (int b = 0; b < kSepNb2; ++b) v[b] = 0.;
-  if (modeOn) {
-#pragma unroll
-    for (int b2 = 0; b2 < kSepNb2; ++b2) {
-      if (b2 < nb2) {
-        double sx = 0., sy = 0.;
-#pragma unroll
-        for (int nu = 0; nu < NMX; ++nu)
-          if (nu < nm) {
-            const double2 x = gp[rl * gps + nu * p.nb2max + b2];
-            const double er = double(e3c[nu].x), ei = double(e3c[nu].y);
-            sx += x.x * er - x.y * ei;
-            sy += x.x * ei + x.y * er;
-          }
-        v[b2] = sx * sx + sy * sy;
-      }
-    }
-    if (!REDUCE) {
-      const int nb1 = p.kkNb1[kk];
-      for (int b2 = 0; b2 < nb2; ++b2)
-        p.out[p.rowOutOff[ri.row] + b1p + size_t(nb1) * (b2 + size_t(nb2) * sub)] = v[b2];
-    }
-  }
-  if (REDUCE) {
-    // symmetrizeCoupling along b2 (scattering.cpp:1250-1284), in registers
-    if (modeOn) {
-      const double* e2r = se2 + r * p.nb2max;
-      for (int b = 0; b < nb2;) {
-        int deg = 0;
-        for (int i = b; i < nb2; ++i) {
-          if (fabs(e2r[b] - e2r[i]) < 1.0e-6) deg++;
-          else break;
-        }
-        if (deg > 1) {
-          double s2 = 0.;
-#pragma unroll
-          for (int i = 0; i < kSepNb2; ++i)
-            if (i >= b && i < b + deg) s2 += v[i] / double(float(deg));
-#pragma unroll
-          for (int i = 0; i < kSepNb2; ++i)
-            if (i >= b && i < b + deg) v[i] = s2;
-        }
-        b += deg;
-      }
-    }
-    // ... and along nu (scattering.cpp:1286-1316), through LDS when modes are degenerate
-    // the mode's degenerate group (consecutive modes within 1e-6 of the
-    // group's first), tabulated per q at set-up
-    int mydeg = 1, mystart = sub;
-    if (modeOn) {
-      const int grp = sg3[r * nm + sub];
-      mystart = grp & 0xff;
-      mydeg = grp >> 8;
-    }
-    if (__any(mydeg > 1)) {  // g' of the row is dead here: its slots hold |g|^2
-      double* gs = reinterpret_cast<double*>(gp);
-      wave_sync();
-      if (modeOn)
-        for (int b2 = 0; b2 < nb2; ++b2) gs[2 * (rl * gps + sub * p.nb2max + b2)] = v[b2];
-      wave_sync();
-      if (modeOn && mydeg > 1)
-        for (int b2 = 0; b2 < nb2; ++b2) {
-          double s2 = 0.;
-          for (int i = 0; i < mydeg; ++i)
-            s2 += gs[2 * (rl * gps + (mystart + i) * p.nb2max + b2)] / double(float(mydeg));
-#pragma unroll
-          for (int b = 0; b < kSepNb2; ++b)
-            if (b == b2) v[b] = s2;
-        }
-    }
-    // Gaussian-delta weights (el_scattering.cpp:277-380); b2 loop kept rolled
-    if (modeOn && w3 >= p.cutoff) {
-#pragma unroll 1
-      for (int b2 = 0; b2 < nb2; ++b2) {
-        double vb = 0.;
-#pragma unroll
-        for (int b = 0; b < kSepNb2; ++b)
-          if (b == b2) vb = v[b];
-        const double en2 = se2[r * p.nb2max + b2];
-        const double cpl = vb * inv_g;
-        const int is2 = ri.soff + b2;
-#pragma unroll
-        for (int gi = 0; gi < kGMax; ++gi) {
-          if (gi >= gsize) break;
-          double d1, d2;
-          if (p.adaptive) {
-            const AdaptiveWidth aw = adaptive_width(p, int(e1 - p.e1pool) + gi, is2);
-            d1 = adaptive_delta(se1[gi] - en2 + w3, aw);
-            d2 = adaptive_delta(se1[gi] - en2 - w3, aw);
-          } else {
-            const double x1 = se1[gi] - en2 + w3, x2 = se1[gi] - en2 - w3;
-            // with the energy screen on, a pair whose both weights are below
-            // exp(-screen^2) of the peak is skipped, as whole rows are
-            if (p.screen > 0. && fmin(fabs(x1), fabs(x2)) * p.invSigma >= scrW)
-              continue;
-            d1 = gaussian_delta(x1, p.invSigma, p.deltaPref);
-            d2 = gaussian_delta(x2, p.invSigma, p.deltaPref);
-          }
-          if (d1 <= 0. && d2 <= 0.) continue;
-#pragma unroll
-          for (int c = 0; c < CM; ++c) {
-            if (c >= nCalc) break;
-            const double f2 = sf2[(c * 16 + r) * p.nb2max + b2];
-            part[gi][c] += cpl * ((f2 + n3[c]) * d1 + (1. - f2 + n3[c]) * d2) * p.norm / w3 *
-                           3.14159265358979323846;
-          }
-        }
-      }
-    }
-  }
-}
-
 // BF3: the x-stage GEMMs in split-BF16x3 (hi*hi + hi*lo + lo*hi on
 // v_mfma_f32_16x16x32_bf16, FP32 accumulation); T must be float.
 // BREG: the B operands of all k-steps (at most 12, i.e. 24 x-groups) are loaded

@@ -46,7 +46,7 @@ struct CacheParams {
   void* B;                // panels
   size_t panelStride;     // elements
   int ldb;                // elements per panel row, one row per Rp (a multiple of 16)
-  // outer points on one mesh line (k_cache_line_a / k_cache_line_b)
+  // outer points on one mesh line (k_cache_line_a or k_cache_line_am, then k_cache's jobs)
   size_t N;               // gW columns: nRp * nm * nw^2
   int nGe;                // R_e groups: distinct n0(R_e) mod m0
   const int* reOrder;     // nRe: native index of the i-th R_e in group order
