@@ -243,7 +243,7 @@ def eig_main(args):
            "config": {"workload": f"cfg1: {args.points} random points per family, H(k) 8x8 and 16x16, "
                                   "D(q) 6x6 and 18x18, R on WS(8^3)"},
            "families": fams,
-           "roofline": {"bound": "mfma", "kernel": "k_jacobi", "achieved": round(ach, 4),
+           "roofline": {"bound": "mfma", "kernel": "k_eig_ql / k_jacobi", "achieved": round(ach, 4),
                         "peak": PEAK_TFLOPS["fp64"], "unit": "TFLOP/s",
                         "frac": round(ach / PEAK_TFLOPS["fp64"], 5), "traffic": None,
                         "flop_model": "23 N^3 per matrix (Householder tridiagonalization, back-transform, QL)"}}
