@@ -461,8 +461,8 @@ int phx_lw_set_panel_chunk(phx_lw* h, int panels);
  * to device memory, (panel chunk) x (y, z lines) x m0 x nm nw complex,
  * and an epilogue kernel reads them; both use far fewer registers and LDS
  * than the fused kernel, so more workgroups hide the memory latency.  Applies
- * to PHX_FP64 and PHX_FP32 with nm <= 32, nw <= 16, an x mesh <= 64, at most
- * 24 x-groups and room for the g3 rows; with the fused y-stage off, the learned
+ * to PHX_FP64 and PHX_FP32 with nm <= 32, nw <= 16, nm nw <= 384, an x mesh
+ * <= 64, at most 24 x-groups and room for the g3 rows; with the fused y-stage off, the learned
  * screen or on = 3 only to PHX_FP32 with nm <= 16 and nm nw <= 192; elsewhere
  * the fused kernel runs.  The g3 values are the same either way and the
  * linewidths agree to FP64 rounding.  on = 2 is the same as on = 1 (the

@@ -866,27 +866,14 @@ struct LwHandle {
   }
 };
 
-// Whether the x-stage of the split last stage runs with the y-stage inside it
-// (k_sep_yx: any width, FP32 and FP64): not with the learned screen's slot masks
-// or the rotating x-stage.
-static bool lw_fused_y(const LwHandle* L, const phx_problem& p) {
+// The kernels of the separable transform's last stage under the handle's present
+// settings (the batch's buffers may still rule the split stage out).
+static LastStage lw_last_stage(const LwHandle* L, const phx_problem& p) {
+  if (L->transform != PHX_TRANSFORM_SEPARABLE) return kStageFused;
   const bool learned = L->lsCollect || (L->lsMode && L->mlpTrained);
-  return L->fuseYX && !learned && L->splitLast != 3 && L->nG0 <= 24 &&
-         sep_yx_lds_bytes(L->precision == PHX_FP64 ? 8 : 4, L->nQuads, p.mesh[1], L->nG0, p.mesh[0]) <= 160 * 1024;
-}
-
-// Whether the separable transform's last stage runs split (x-stage and
-// epilogue as two kernels, g3 rows through HBM): nw <= 16, row masks (x mesh <=
-// 64) and an x-stage kernel for the sizes: k_sep_yx, or k_sep_xg (FP32, nm <=
-// 16, nm nw <= 192).  The launcher falls back to the fused kernel where it
-// cannot run split.  Two kernels write and read g3 but hide their latency at 2
-// to 4 waves per SIMD, where the fused one runs at 1 or 2: with 18 modes x 16
-// bands in FP32 on a 32^3 mesh 7.2 against 21.8 ms per pass, 12 x 16 in FP64 on
-// a 27 x 28 x 29 mesh 6.3 against 21.2.
-static bool lw_split_last(const LwHandle* L, const phx_problem& p) {
-  const bool xg = L->precision == PHX_FP32 && p.nm <= 16 && p.nm * p.nw <= 192;
-  return L->splitLast && L->transform == PHX_TRANSFORM_SEPARABLE && L->precision != PHX_BF16X3 && p.nw <= 16 &&
-         p.mesh[0] <= 64 && (xg || lw_fused_y(L, p));
+  const LastStageSizes z{L->precision == PHX_FP64, L->precision == PHX_BF16X3, p.nm, p.nw, p.mesh[0], p.mesh[1],
+                         L->nG0, L->nQuads, L->adaptive};
+  return last_stage(z, L->splitLast, L->fuseYX != 0, learned);
 }
 
 // float2 values per panel of a chunk's g3 rows: nm nw complex values of the
@@ -1715,7 +1702,7 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
       L->screenOf.reserve(size_t(L->numStates));
       L->xminPart.reserve(size_t(chunk) * kXminBlocks);
     }
-    if (lw_split_last(L, p)) {  // g3 (complex FP32) or g' (complex FP64, nb2max nm per row)
+    if (lw_last_stage(L, p) != kStageFused) {  // g3 (complex T) or g' (complex FP64, nb2max nm per row)
       const size_t g3 = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
       try {
         L->G3f.reserve(g3);
@@ -1956,10 +1943,6 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     cq.bf16x3 = L->precision == PHX_BF16X3;
     cq.meshRow = L->meshRow.p;
     if (p.mesh[0] <= 64) cq.keepMask = L->keepMask.p;
-    if (lw_split_last(L, p)) {
-      cq.G3 = L->G3f.p;
-      cq.epRot = L->splitLast == 3;
-    }
     // panels in chunks: the stage buffers T1 / T2 hold one chunk
     const int chunk = lw_panel_chunk(L, p, nPanels, b.nb2max);
     if (L->precision == PHX_FP64) {
@@ -1978,11 +1961,10 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     // setting changed since: then the fused kernel runs, or the chunks run in turn)
     const size_t slotsC = size_t(chunk) * nMtiles;
     const size_t g3Need = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
-    const bool splitOk = lw_split_last(L, p) && L->G3f.n >= g3Need;
-    const bool overlap = L->epOverlap && !learned && splitOk && L->G3f2.n >= g3Need &&
-                         L->keepMask2.n >= slotsC;
-    const bool yx = splitOk && lw_fused_y(L, p);  // the y-stage inside the x-stage kernel
-    cq.fuseYX = yx;
+    cq.stage = L->G3f.n >= g3Need ? lw_last_stage(L, p) : kStageFused;
+    const bool split = cq.stage != kStageFused, yx = cq.stage == kStageYx;
+    const bool overlap = L->epOverlap && !learned && split && L->G3f2.n >= g3Need && L->keepMask2.n >= slotsC;
+    sp.modeFast = split ? nm : 0;
     const int nChunks = (nPanels + chunk - 1) / chunk;
     if (overlap) {
       if (!L->streamEp) PHX_HIP(hipStreamCreateWithFlags(&L->streamEp, hipStreamNonBlocking));
@@ -1997,7 +1979,7 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     for (int p0 = 0, ci = 0; p0 < nPanels; p0 += chunk, ++ci) {
       const int n = std::min(chunk, nPanels - p0);
       const int set = overlap ? (ci & 1) : 0;
-      cq.G3 = splitOk ? (set ? L->G3f2.p : L->G3f.p) : nullptr;
+      cq.G3 = split ? (set ? L->G3f2.p : L->G3f.p) : nullptr;
       if (p.mesh[0] <= 64) cq.keepMask = set ? L->keepMask2.p : L->keepMask.p;
       sp.nPanels = n;
       cq.nPanels = n;
@@ -2033,10 +2015,10 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
           fork.epStart = L->xev[L->xevUsed + 3];
           PHX_HIP(hipEventRecord(L->xev[L->xevUsed], s));
         }
-        const bool split = f64 ? launch_separable_x<double>(sp, c, true, s, mid, fork)
-                               : launch_separable_x<float>(sp, c, true, s, mid, fork);
-        const bool forked = split && fork.ep;
-        if (L->timing && split && c.fuseYX) {
+        const bool ran = f64 ? launch_separable_x<double>(sp, c, true, s, mid, fork)
+                             : launch_separable_x<float>(sp, c, true, s, mid, fork);
+        const bool forked = ran && fork.ep;
+        if (L->timing && ran && yx) {
           L->yxT1Bytes += double(sp.nPanels) * mz * L->nLines * ncol * (f64 ? 16. : 8.);
           L->yxLaunches += 1;
         }
@@ -2048,10 +2030,9 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
         if (L->timing) {
           PHX_HIP(hipEventRecord(L->xev[L->xevUsed + 4], forked ? L->streamEp : s));
           L->xevUsed += 5;
-          L->xevSplit.push_back(split ? 1 : 0);
+          L->xevSplit.push_back(ran ? 1 : 0);
         }
       };
-      sp.modeFast = (f64 ? sep_runs_split<double>(sp, cq) : sep_runs_split<float>(sp, cq)) ? nm : 0;
       if (f64) launch_separable_zy<double>(sp, L->maxLineE, s, !yx);
       else launch_separable_zy<float>(sp, L->maxLineE, s, !yx);
       if (!learned) {

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "elph_params.hpp"
+#include "last_stage.hpp"
 #include "phx_common.hpp"
 
 namespace phx {
@@ -99,8 +100,7 @@ struct CoupParams {
   // split last stage (k_sep_yx or k_sep_xg, then k_sep_ep2): g3 rows of the chunk, (slot, jx, col) complex T
   void* G3;
   unsigned long long* keptBands;          // k_sep_ep2: sum of nb2 over the rows it computed (null: off)
-  int epRot;                              // k_sep_xg also does the electron rotation (g' to HBM, not g3)
-  int fuseYX;                             // the y-stage runs inside the x-stage kernel (k_sep_yx; no T2 in HBM)
+  int stage;                              // kernels of the last stage (LastStage)
   unsigned long long* keptSlots;          // k_sep_xg: slots (panel, yz line) it computed (null: off)
 };
 
@@ -537,10 +537,6 @@ struct SepYShared {
   int2* ent;   // 4 nQuads: (T1 row at jz: offset of its first column, or -1: padding; f1)
   int* end;    // nQuads: group that ends with the quad, or -1
 };
-__host__ __device__ inline size_t sep_y_lds_bytes(int my, int nQuads) {
-  return size_t(my) * sizeof(double2) + size_t(4) * nQuads * sizeof(int2) +
-         (size_t(nQuads) * sizeof(int) + 15) / 16 * 16;
-}
 __device__ __forceinline__ SepYShared sep_y_stage(const SepParams& p, unsigned char* smem, int jz) {
   SepYShared s;
   s.tw = reinterpret_cast<double*>(smem);
@@ -1724,12 +1720,6 @@ inline size_t sep_xg_lds_bytes(int elem, int nG0, int m0, int nm = 0, int nw = 0
 // the matrix cores 3.3 with a coordinate per row, 3.1 with conjugate pairs (FP64,
 // 27 x 28 x 29: 1.94 and 1.88 ms).  Non-temporal g3 stores and the slots' masks in
 // LDS measured the same.
-inline size_t sep_yx_lds_bytes(int elem, int nQuads, int my, int nG0, int m0) {
-  const int kp = (2 * nG0 + 3) / 4 * 4;
-  return sep_y_lds_bytes(my, nQuads) + size_t(m0) * (kp + 1) * 2 * elem + size_t(16) * (kp * 16 + 16) * elem +
-         size_t(4) * 64 * sizeof(int) + 64;
-}
-
 template <typename T>
 __global__ void __launch_bounds__(256) k_sep_yx(SepParams sp, CoupParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -2048,15 +2038,6 @@ struct EpFork {
   hipEvent_t xgStart = nullptr;  // timing: recorded on the launch's stream right before the x-stage kernel
 };
 
-// Whether the last stage runs split (x-stage and epilogue kernels, g3 through
-// HBM), which the z-stage has to know too: its columns are then (w2, nu).
-// k_sep_yx takes any width and both precisions; k_sep_xg FP32 and at most 192 columns.
-template <typename T>
-inline bool sep_runs_split(const SepParams& sp, const CoupParams& p) {
-  return p.G3 && !p.bf16x3 && p.keepMask && p.nw <= 16 && (2 * p.nG0 + 3) / 4 <= 12 && sp.ncol <= 4 * 6 * 16 &&
-         (p.fuseYX || (sizeof(T) == 4 && sp.ncol <= 4 * 3 * 16 && p.nm <= 16));
-}
-
 // mid (optional): recorded between the x-stage and the epilogue kernel when
 // the last stage runs split.  Returns whether it did (then the epilogue ran
 // on fork.ep when that is set).
@@ -2065,7 +2046,12 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
                         hipEvent_t mid, const EpFork& fork = EpFork{}) {
   PHX_REQUIRE(p.nm <= kSepNm && p.nb2max <= kSepNb2,
               "separable transform supports nm <= 32 and at most 8 bands per inner point");
-  PHX_REQUIRE(!p.fuseYX || reduce, "separable transform: the fused y/x-stage belongs to the reduction");
+  // what the host chose (last_stage), whose stages before this one and buffers depend on it
+  const bool split = p.stage != kStageFused;
+  PHX_REQUIRE(split == (sp.modeFast != 0), "separable transform: column order of the split last stage");
+  PHX_REQUIRE(!split || (reduce && p.G3 && p.keepMask && p.nw <= 16 && p.nG0 <= kSplitGroups && sp.ncol <= kSplitCols),
+              "separable transform: the split last stage does not take these sizes");
+  PHX_REQUIRE(p.stage == kStageYx || p.T2, "separable transform: x-stage without the y-stage's output");
   if (sp.nPanels <= 0) return false;
   const int tiles = sp.nPanels * sp.my * sp.mz;
   const int grid = ceil_div(tiles, 8) * 8;
@@ -2075,19 +2061,19 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
   const bool bf3 = p.bf16x3 != 0;
   constexpr bool bregt = sizeof(T) == 4;  // B in registers for the whole item: FP32, <= 24 x-groups
   const bool breg = bregt && (2 * p.nG0 + 3) / 4 <= 12;
-  PHX_REQUIRE(!bf3 || (bf3t && reduce && sp.ncol <= 4 * 6 * 16),
+  PHX_REQUIRE(!bf3 || (bf3t && reduce && sp.ncol <= kSplitCols),
               "split-BF16x3: FP32 data, the linewidth reduction and nm nw <= 384");
   if (reduce && p.screen > 0. && p.screenOf) {
     PHX_REQUIRE(p.xminPart && p.meshRow, "energy screen: closest-approach buffers missing");
     hipLaunchKernelGGL(k_sep_xmin, dim3(kXminBlocks, sp.nPanels), dim3(256), 0, s, p);
     PHX_HIP(hipGetLastError());
-    if (!(p.keepMask && sp.ncol <= 4 * 6 * 16)) {  // else the row masks' kernel stores the widths
+    if (!(p.keepMask && sp.ncol <= kSplitCols)) {  // else the row masks' kernel stores the widths
       hipLaunchKernelGGL(k_sep_xmin_fin, dim3(sp.nPanels), dim3(64), 0, s, p);
       PHX_HIP(hipGetLastError());
     }
   }
-  if (reduce && sp.ncol <= 4 * 6 * 16) {
-    const bool wide = sp.ncol > 4 * 3 * 16;
+  if (reduce && sp.ncol <= kSplitCols) {
+    const bool wide = sp.ncol > kXgCols;
     const size_t ldsXm = sep_xm_lds_bytes(sizeof(T), p.nG0, p.m0, p.nw, p.nm, p.nb2max, nmb <= 16 ? 16 : 8,
                                              p.nCalc);
     PHX_REQUIRE(ldsXm <= 160 * 1024, "separable transform: LDS budget exceeded");
@@ -2101,14 +2087,12 @@ bool launch_separable_x(const SepParams& sp, const CoupParams& p, bool reduce, h
       else hipLaunchKernelGGL(k_sep_screen<64>, dim3(ceil_div(lines, 4), sp.nPanels), dim3(256), 0, s, p);
       PHX_HIP(hipGetLastError());
     }
-    const bool split = sep_runs_split<T>(sp, p);
-    PHX_REQUIRE(split == (sp.modeFast != 0), "separable transform: column order of the split last stage");
-    PHX_REQUIRE(split || !p.fuseYX, "separable transform: fused y/x-stage outside the split last stage");
     if (split) {
       if (fork.xgStart) PHX_HIP(hipEventRecord(fork.xgStart, s));
-      // the electron rotation in the x-stage kernel: FP32 and fixed smearing only
-      const bool rot = p.epRot && !p.adaptive && !p.fuseYX;
-      if (p.fuseYX) {
+      const bool rot = p.stage == kStageRot;
+      PHX_REQUIRE(p.stage == kStageYx || (sizeof(T) == 4 && sp.ncol <= kXgCols && p.nm <= 16 && !(rot && p.adaptive)),
+                  "separable transform: the x-stage kernel does not take these sizes");
+      if (p.stage == kStageYx) {
         PHX_REQUIRE(!p.slotOn && !p.gate, "separable transform: fused y/x-stage without slot masks");
         const size_t ldsYX = sep_yx_lds_bytes(sizeof(T), sp.nQuads, sp.my, sp.nG0, p.m0);
         PHX_REQUIRE(ldsYX <= 160 * 1024, "separable transform: LDS budget exceeded");

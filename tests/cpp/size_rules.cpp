@@ -1,0 +1,22 @@
+// The kernels' size rules, evaluated on the host: one form per line of stdin.
+//   stage f64 bf16x3 nm nw m0 my nG0 nQuads adaptive mode fuseY learned -> LastStage
+#include <iostream>
+#include <string>
+
+#include "../../phoebe_amd/csrc/last_stage.hpp"
+
+int main() {
+  std::string kind;
+  while (std::cin >> kind) {
+    if (kind == "stage") {
+      phx::LastStageSizes z{};
+      int mode, fuseY, learned;
+      std::cin >> z.f64 >> z.bf16x3 >> z.nm >> z.nw >> z.m0 >> z.my >> z.nG0 >> z.nQuads >> z.adaptive >> mode >>
+          fuseY >> learned;
+      std::cout << int(phx::last_stage(z, mode, fuseY != 0, learned != 0)) << "\n";
+    } else {
+      return 1;
+    }
+    if (!std::cin) return 1;
+  }
+}

@@ -1,0 +1,45 @@
+"""The rules that choose kernels by size, on the host: which kernels run the
+mesh-separable last stage, over every combination of its limits."""
+import itertools
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+FUSED, XG, ROT, YX = range(4)
+
+
+@pytest.fixture(scope="session")
+def rules(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rules") / "size_rules")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-o", exe, os.path.join(HERE, "cpp", "size_rules.cpp")],
+                   check=True)
+
+    def ask(kind, forms, timeout=60):
+        text = "\n".join(kind + " " + " ".join(str(int(x)) for x in f) for f in forms) + "\n"
+        r = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=timeout)
+        return [tuple(int(x) for x in line.split()) for line in r.stdout.splitlines()]
+
+    return ask
+
+
+def test_last_stage(rules):
+    sizes = [(3, 4), (12, 16), (15, 13), (16, 12), (16, 13), (18, 16), (24, 16), (25, 16), (27, 15), (27, 16), (30, 16),
+             (32, 12), (32, 13), (32, 16), (12, 17), (6, 32)]
+    forms = [(f64, bf, nm, nw, m0, my, nG0, nQ, ad, mode, fy, ls)
+             for (nm, nw), f64, bf, (m0, my), (nG0, nQ), ad, mode, fy, ls in
+             itertools.product(sizes, (0, 1), (0, 1), ((1, 1), (64, 64), (65, 5)), ((1, 1), (24, 100), (25, 100), (24, 4000)),
+                               (0, 1), (0, 1, 2, 3), (0, 1), (0, 1)) if not (f64 and bf)]
+    got = rules("stage", forms)
+    assert len(got) == len(forms)
+    for (f64, bf, nm, nw, m0, my, nG0, nQ, ad, mode, fy, ls), (g,) in zip(forms, got):
+        if mode == 0 or bf or nw > 16 or m0 > 64 or nG0 > 24 or nm * nw > 384:
+            want = FUSED
+        elif fy and not ls and mode != 3 and nQ < 4000:  # 4000 quads: 144 KB of entries, beyond LDS with the rest
+            want = YX
+        elif f64 or nm > 16 or nm * nw > 192:
+            want = FUSED
+        else:
+            want = ROT if mode == 3 and not ad else XG
+        assert g == want, (f64, bf, nm, nw, m0, my, nG0, nQ, ad, mode, fy, ls)
