@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "coupling_tiling.hpp"
 #include "elph_params.hpp"
 #include "last_stage.hpp"
 #include "phx_common.hpp"
@@ -368,15 +369,7 @@ __device__ inline void reduce_partials(const CoupParams& p, int L, unsigned char
 // ------------------------------------------------------------------ direct transform
 // (coupling_direct.hpp, instantiated in coupling_direct_f64.hip and coupling_direct_f32.hip)
 
-// How the direct transform cuts its work: workgroups of `rows` inner points,
-// 4 / wc waves of mt 16-row tiles by wc waves of nt 16-column tiles, the panel
-// columns in windows of `modes` whole modes.
-struct CoupTiling {
-  int mt, nt, wc, rows, modes;
-  int stage;  // the g3 tile's LDS holds the rows' frequencies and energies once g3 has been used
-  size_t lds;
-};
-CoupTiling coupling_tiling(bool f64, int nm, int nw, int nb2max);
+static_assert(kCoupReduceLds == size_t(kGMax) * kCMax * 4 * sizeof(double), "LDS of reduce_partials");
 template <typename T>
 void launch_coupling(const CoupParams& p, bool reduce, hipStream_t s);
 

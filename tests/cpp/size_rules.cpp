@@ -1,8 +1,10 @@
 // The kernels' size rules, evaluated on the host: one form per line of stdin.
 //   stage f64 bf16x3 nm nw m0 my nG0 nQuads adaptive mode fuseY learned -> LastStage
+//   tiling f64 nm nw nb2max -> mt nt wc rows modes stage lds
 #include <iostream>
 #include <string>
 
+#include "../../phoebe_amd/csrc/coupling_tiling.hpp"
 #include "../../phoebe_amd/csrc/last_stage.hpp"
 
 int main() {
@@ -14,6 +16,12 @@ int main() {
       std::cin >> z.f64 >> z.bf16x3 >> z.nm >> z.nw >> z.m0 >> z.my >> z.nG0 >> z.nQuads >> z.adaptive >> mode >>
           fuseY >> learned;
       std::cout << int(phx::last_stage(z, mode, fuseY != 0, learned != 0)) << "\n";
+    } else if (kind == "tiling") {
+      int f64, nm, nw, nb2max;
+      std::cin >> f64 >> nm >> nw >> nb2max;
+      const phx::CoupTiling c = phx::coupling_tiling(f64 != 0, nm, nw, nb2max);
+      std::cout << c.mt << " " << c.nt << " " << c.wc << " " << c.rows << " " << c.modes << " " << c.stage << " "
+                << c.lds << "\n";
     } else {
       return 1;
     }

@@ -32,3 +32,32 @@ def test_store_mode_against_direct_sum(nw, nm, nRp, nq, precision):
         g3 = np.tensordot(np.exp(1j * Rp @ q3[i]) / dP, g1, axes=(0, 0))  # (nu, b1, w2)
         ref = np.abs(np.einsum("vcb,bd,vm->cdm", g3, U2[i].conj(), e3[i], optimize=True)) ** 2
         assert np.abs(inter.getCouplingSquared(i) - ref).max() <= tol * ref.max()
+
+
+def _call(nw, nm, nb2, nq, precision, seed):
+    rng = np.random.default_rng(seed)
+    cx = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)
+    gW = cx(1, 2, nm, nw, nw)
+    U1, U2 = np.linalg.qr(cx(nw, nw))[0][:, :1], [np.linalg.qr(cx(nw, nw))[0][:, :nb2] for _ in range(nq)]
+    e3, Rp, q3 = [cx(nm, nm) for _ in range(nq)], rng.integers(-3, 4, (2, 3)) * 1.3, rng.standard_normal((nq, 3))
+    inter = P.InteractionElPhWan(gW, np.zeros((1, 3)), np.ones(1), Rp, np.ones(2), precision)
+    inter.cacheElPh(U1, np.zeros(3))
+    inter.calcCouplingSquared(U1, U2, e3, q3)
+    g1 = np.einsum("epvab,ac->pvcb", gW, U1)
+    for i in range(nq):
+        g3 = np.tensordot(np.exp(1j * Rp @ q3[i]), g1, axes=(0, 0))
+        ref = np.abs(np.einsum("vcb,bd,vm->cdm", g3, U2[i].conj(), e3[i], optimize=True)) ** 2
+        assert np.abs(inter.getCouplingSquared(i) - ref).max() <= (1e-12 if precision == "fp64" else 2e-6) * ref.max()
+
+
+@pytest.mark.parametrize("nw,nm,nb2,precision", [(31, 12, 31, "fp64"), (32, 36, 11, "fp64"), (31, 13, 31, "fp32"),
+                                                 (29, 14, 29, "fp32")])
+def test_windows_narrowed_by_many_bands(nw, nm, nb2, precision):
+    """g' of the inner points' bands leaves LDS to a few modes per window."""
+    _call(nw, nm, nb2, 2, precision, 5)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_too_many_bands_are_refused(precision):
+    with pytest.raises(P.PhxError):
+        _call(20, 24, 20, 1, precision, 6)

@@ -1,5 +1,6 @@
 """The rules that choose kernels by size, on the host: which kernels run the
-mesh-separable last stage, over every combination of its limits."""
+mesh-separable last stage, over every combination of its limits; how the direct
+transform cuts a panel, over every size."""
 import itertools
 import os
 import subprocess
@@ -43,3 +44,31 @@ def test_last_stage(rules):
         else:
             want = ROT if mode == 3 and not ad else XG
         assert g == want, (f64, bf, nm, nw, m0, my, nG0, nQ, ad, mode, fy, ls)
+
+
+# the instances of k_coupling, by precision
+INSTANCES = {1: {(1, 1), (1, 2), (1, 3), (1, 4), (2, 3)},
+             0: {(1, 1), (1, 2), (1, 3), (1, 4), (1, 5), (1, 6), (2, 3), (2, 4), (2, 5), (2, 6)}}
+
+
+@pytest.mark.parametrize("f64", [1, 0])
+def test_coupling_tiling(rules, f64):
+    """Every size ends (some windows once never got smaller), the tiles cover the
+    window's columns with an instance that exists, and a size is refused only when
+    not even one mode at a time fits LDS."""
+    forms = [(f64, nm, nw, nb) for nm in range(1, 37) for nw in range(1, 33) for nb in range(1, nw + 1)]
+    got = rules("tiling", forms, timeout=120)
+    assert len(got) == len(forms)
+    elem, most = (16, 192) if f64 else (8, 384)
+    seen = set()
+    for (_, nm, nw, nb), (mt, nt, wc, rows, modes, stage, lds) in zip(forms, got):
+        at = (nm, nw, nb)
+        scratch = 16 * nm * nb * 24
+        assert 1 <= modes <= nm and (modes * nw <= most or modes == 1), at
+        assert lds == max(16 * modes * nw * elem + scratch, 1024), at
+        assert (lds <= 160 * 1024) == (16 * nw * elem + scratch <= 160 * 1024), at
+        assert wc * nt * 16 >= modes * nw > wc * (nt - 1) * 16 * (nt > 1) and wc in (1, 2, 4), at
+        assert rows == (16 if modes < nm else 16 * mt * (4 // wc)) and (modes == nm or (mt, wc) == (1, 4)), at
+        assert stage == (16 * modes * nw * elem >= 16 * (nm + nb) * 8), at
+        seen.add((mt, nt))
+    assert seen == INSTANCES[f64]
