@@ -386,6 +386,9 @@ inline size_t ql_lds_bytes(int N, int L) {
   return size_t(64 / L) * ((size_t(N) * ld + 2 * N) * sizeof(double2) + (size_t(2) * N + 2) * sizeof(double));
 }
 
+// Below this an element next to a largest component near one counts as zero: far
+// below the norm's rounding, and its square is a normal number.
+constexpr double kQlTiny = 1e-140;
 constexpr int kQlMaxIter = 60;  // QL iterations per eigenvalue (two or three are usual)
 
 template <int L>
@@ -405,7 +408,8 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
   const bool row = li < N;
 
   // the lower triangle is the reference (uplo = L); scaled by a power of two to
-  // a largest component near one, so that no square over- or underflows
+  // a largest component near one, so that no square overflows; what a square that
+  // underflows can lose is below kQlTiny
   double big = 0.;
 #pragma unroll 4
   for (int j = 0; j < N; ++j) {
@@ -437,10 +441,13 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
     const double2 x = in ? a[li + ld * k] : make_double2(0., 0.);
     const double2 alpha = a[k + 1 + ld * k];
     const double tail = group_sum<L>(li > k + 1 ? x.x * x.x + x.y * x.y : 0.);
+    const double norm2 = alpha.x * alpha.x + alpha.y * alpha.y + tail;
     double beta = alpha.x;
     double2 tau = make_double2(0., 0.), v = make_double2(li == k + 1 ? 1. : 0., 0.);
-    if (tail > 0. || alpha.y != 0.) {
-      beta = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + tail);
+    if (norm2 < kQlTiny * kQlTiny) {  // the column counts as zero: its square is no longer exact, nor is 1 / square finite
+      beta = 0.;
+    } else if (tail > 0. || alpha.y != 0.) {
+      beta = sqrt(norm2);
       if (alpha.x > 0.) beta = -beta;
       tau = make_double2((beta - alpha.x) / beta, -alpha.y / beta);
       // x / (alpha - beta)

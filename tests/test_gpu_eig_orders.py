@@ -49,6 +49,25 @@ def test_orders(n):
     _check(A)
 
 
+@pytest.mark.parametrize("n", [2, 4, 8, 9, 17, 40])
+@pytest.mark.parametrize("phase", [1.0, 1j, np.exp(0.7j)])
+def test_columns_whose_squares_underflow(n, phase):
+    """A column below the diagonal of 1e-130 to 1e-320 of the norm, as a whole or its
+    first or second element alone (zero counts: the pairing is exact)."""
+    rng = np.random.default_rng(n)
+    A = []
+    for tiny in (1e-130, 1e-139, 1e-141, 1e-150, 1e-154, 1e-156, 1e-160, 1e-162, 1e-170, 1e-200, 1e-310, 1e-320):
+        for where in (slice(1, None), slice(1, 2), slice(2, 3)):
+            X = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+            H = 0.15 * (X + X.conj().T) + np.diag(1.0 + np.arange(n))
+            col = np.zeros(n, complex)
+            col[where] = phase * tiny * rng.uniform(0.5, 1.0, n)[where]
+            col[0] = 1.0
+            H[:, 0], H[0, :] = col, col.conj()
+            A.append(H)
+    _check(np.array(A))
+
+
 @pytest.mark.parametrize("kind,n,nk", [("el", 3, 1), ("el", 8, 5), ("el", 9, 2100), ("el", 12, 700), ("el", 16, 8200),
                                        ("el", 17, 33), ("ph", 6, 3), ("ph", 9, 2100), ("ph", 12, 8300), ("ph", 18, 40)])
 def test_bloch_sums(kind, n, nk):
