@@ -389,7 +389,9 @@ inline size_t ql_lds_bytes(int N, int L) {
 // Below this an element next to a largest component near one counts as zero: far
 // below the norm's rounding, and its square is a normal number.
 constexpr double kQlTiny = 1e-140;
-constexpr int kQlMaxIter = 60;  // QL iterations per eigenvalue (two or three are usual)
+// QL iterations of a matrix of order N: at most 30 N, as two or three per eigenvalue
+// are usual but one alone can take about N (rank one with structured phases).
+constexpr int kQlMaxIter = 30;
 
 template <int L>
 __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict__ A, double* __restrict__ W,
@@ -530,23 +532,25 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
   group_sync();
 
   // implicit QL: eigenvalue l of the group, it iterations spent on it
-  int l = 0, it = 0, worst = 0;
+  int l = 0, it = 0, total = 0, worst = 0;
   bool bad = false;
   while (__any(l < N && !bad)) {
     if (l < N && !bad) {
       // the first negligible off-diagonal from l on ends the block l .. m
       bool small = false;
-      if (li >= l && li < N - 1) small = fabs(e[li]) <= 2.220446049250313e-16 * (fabs(d[li]) + fabs(d[li + 1]));
+      if (li >= l && li < N - 1)
+        small = fabs(e[li]) <= fmax(kQlTiny, 2.220446049250313e-16 * (fabs(d[li]) + fabs(d[li + 1])));
       const unsigned long long ones = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
       const unsigned long long hit = (__ballot(small) >> (sg * L)) & ones;
       const int m = hit ? __ffsll(hit) - 1 : N - 1;
       if (m == l) {
         ++l;
         it = 0;
-      } else if (it == kQlMaxIter) {
+      } else if (total == kQlMaxIter * N) {
         bad = true;
       } else {
         ++it;
+        ++total;
         worst = max(worst, it);
         const double dl = d[l], el = e[l];
         double g = (d[l + 1] - dl) / (2. * el);
@@ -565,7 +569,9 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
           const double2 znx = row ? a[li + ld * in] : make_double2(0., 0.);
           const double f = s * ei, b = c * ei;
           const double r2 = f * f + g * g;
-          if (r2 < 1e-290) {  // zero next to the largest component, near one: the block splits at i + 1
+          // zero next to the largest component, near one: the block splits at i + 1.  Never the first
+          // rotation, where f = e(m - 1) > kQlTiny, so every iteration changes the matrix
+          if (r2 < 1e-290) {
             if (li == 0) {
               e[i + 1] = 0.;
               d[i + 1] = dn - p;

@@ -68,6 +68,33 @@ def test_columns_whose_squares_underflow(n, phase):
     _check(np.array(A))
 
 
+@pytest.mark.parametrize("n", [3, 5, 8, 9, 17, 40])
+def test_tiny_couplings_between_equal_levels(n):
+    """Nothing relative to compare a coupling of 1e-130 to 1e-170 with: zero, or
+    equal and opposite, diagonal elements."""
+    rng = np.random.default_rng(n)
+    A = []
+    for tiny in (1e-130, 1e-139, 1e-141, 1e-145, 1e-150, 1e-160, 1e-170):
+        for i in range(n - 1):
+            H = np.zeros((n, n), complex)
+            H[0, 0] = 1.0
+            H[i + 1, i] = H[i, i + 1] = tiny
+            A.append(H)
+        H = np.diag(np.r_[1.0, np.zeros(n - 1)]).astype(complex)
+        H[1:, 1:] = tiny * np.triu(rng.standard_normal((n - 1, n - 1)))
+        A.append(np.triu(H).conj().T)
+    _check(np.array(A))
+
+
+@pytest.mark.parametrize("n", [6, 8, 16, 31, 32, 33, 44])
+def test_rank_one_with_structured_phases(n):
+    """All but one eigenvalue equal, where one can take many iterations."""
+    j = np.arange(n)
+    u = np.array([np.exp(2j * np.pi * j * j * s / n) * (1.0 + j) ** p
+                  for s in (0.25, 0.5, 1.0, np.sqrt(2)) for p in (0.0, 0.5, -0.5)] + [np.exp(1j * j)])
+    _check(u[:, :, None] * u[:, None, :].conj())
+
+
 @pytest.mark.parametrize("kind,n,nk", [("el", 3, 1), ("el", 8, 5), ("el", 9, 2100), ("el", 12, 700), ("el", 16, 8200),
                                        ("el", 17, 33), ("ph", 6, 3), ("ph", 9, 2100), ("ph", 12, 8300), ("ph", 18, 40)])
 def test_bloch_sums(kind, n, nk):
