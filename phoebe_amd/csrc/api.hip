@@ -765,6 +765,7 @@ struct LwHandle {
   BatchMeta cur;                    // the batch being run by phx_lw_run
   std::vector<BatchMeta> plan;      // a prepared sweep (phx_lw_plan)
   hipGraphExec_t graphExec = nullptr;
+  std::vector<const void*> graphBuffers;  // lw_shared_buffers when it was captured
   long long planPairs = 0;
   // separable mesh transform of the R_ph sum (transform == PHX_TRANSFORM_SEPARABLE)
   int transform = 0;
@@ -1528,6 +1529,93 @@ static void learned_screen_chunk(LwHandle* L, const CoupParams& cq, XStage&& xst
   launch_fail_fold(L->lsFail.p, L->lsCounts.p + 3, s);
 }
 
+// Every scratch buffer that a batch's launch needs under the handle's present
+// settings, grown where it is too small.
+static void lw_scratch(LwHandle* L, const BatchMeta& b) {
+  const phx_problem& p = L->prob;
+  hipStream_t s = L->stream;
+  const int nw = L->nw, nm = L->nm;
+  const size_t pstride = size_t(L->nRp) * L->ldb;
+  if (b.nPanels > L->maxPanels) {
+    const int most = std::max(b.nPanels, L->k1Batch * nw);
+    L->maxPanels = 0;  // while there are none, should the allocation fail
+    if (L->precision == PHX_FP64) {
+      L->Bd.alloc(pstride * most);
+      launch_fill<double>(L->Bd.p, L->Bd.n, 0., s);
+    } else {
+      L->Bf.alloc(pstride * most);
+      launch_fill<float>(L->Bf.p, L->Bf.n, 0.f, s);
+    }
+    L->maxPanels = most;
+  }
+  L->partial.reserve(size_t(L->maxPanels) * std::max(b.nMtiles, 1) * kGMax * kCMax);
+  if (b.line) {
+    const size_t Tg = size_t(line_count_padded(b.nLinesB)) * L->nGe * L->nRp * nm * nw * nw;
+    if (L->precision == PHX_FP64) L->TgD.reserve(Tg);
+    else L->TgF.reserve(Tg);
+  } else {
+    L->phE.reserve(cache_phase_size(L->nRe));
+  }
+  L->phP.reserve(size_t(b.nkk) * L->nRp);
+  // scratch of the separable transform: one panel chunk of stage buffers, row masks,
+  // and the learned screen's per-block arrays
+  if (L->transform == PHX_TRANSFORM_SEPARABLE && b.M > 0) {
+    // sized for the handle's full chunk, not this batch's panel count, so that a
+    // later, larger batch does not reallocate them
+    const int chunk = lw_panel_chunk(L, p, std::numeric_limits<int>::max(), b.nb2max);
+    const size_t ncol = size_t(nm) * nw;
+    const size_t t1 = size_t(L->nLines) * p.mesh[2] * ncol * 2, t2 = size_t(L->nG0) * p.mesh[1] * p.mesh[2] * ncol * 2;
+    if (L->precision == PHX_FP64) {
+      L->T1d.reserve(t1 * chunk);
+      L->T2d.reserve(t2 * chunk);
+    } else {
+      L->T1f.reserve(t1 * chunk);
+      L->T2f.reserve(t2 * chunk);
+    }
+    const size_t slots = size_t(chunk) * b.nMtiles;
+    if (p.mesh[0] <= 64) L->keepMask.reserve(slots);
+    if (L->screen > 0.) {
+      L->screenOf.reserve(size_t(L->numStates));
+      L->xminPart.reserve(size_t(chunk) * kXminBlocks);
+    }
+    if (lw_last_stage(L, p) != kStageFused) {  // g3 (complex T) or g' (complex FP64, nb2max nm per row)
+      const size_t g3 = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
+      try {
+        L->G3f.reserve(g3);
+      } catch (const Error&) {  // no room for the g3 rows: the fused kernel runs, which needs none
+        (void)hipGetLastError();
+        L->G3f.release();
+      }
+      if (L->epOverlap && L->G3f.p) {
+        L->G3f2.reserve(g3);
+        L->keepMask2.reserve(slots);
+      }
+    }
+    if (L->lsMode && L->mlpTrained) {
+      L->lsFeat.reserve(slots * kMlpIn);
+      L->lsNscr.reserve(slots);
+      L->lsMaskC.reserve(slots);
+      L->lsMaskA.reserve(slots);
+      L->lsMaskS.reserve(slots);
+      L->lsPred.reserve(slots);
+      L->mlpScratch.reserve(mlp_scratch_floats(int(slots)));
+      L->lsThrAbs.reserve(chunk);
+      L->lsPanelStats.reserve(2 * size_t(chunk));
+      L->partialAudit.reserve(slots * kGMax * kCMax);
+    }
+  }
+}
+
+// The buffers a launch uses that other calls may replace (runs of larger batches,
+// settings): a captured sweep is valid while they are the same.
+static std::vector<const void*> lw_shared_buffers(const LwHandle* L) {
+  return {L->Bd.p,         L->Bf.p,      L->partial.p,   L->TgD.p,    L->TgF.p,     L->phE.p,      L->phP.p,
+          L->T1d.p,        L->T1f.p,     L->T2d.p,       L->T2f.p,    L->G3f.p,     L->G3f2.p,     L->keepMask.p,
+          L->keepMask2.p,  L->screenOf.p, L->xminPart.p, L->polX.p,   L->lsFeat.p,  L->lsNscr.p,   L->lsMaskC.p,
+          L->lsMaskA.p,    L->lsMaskS.p, L->lsPred.p,    L->mlpP.p,   L->mlpScratch.p, L->lsThrAbs.p, L->lsPanelStats.p,
+          L->partialAudit.p, L->lsFail.p, L->lsCounts.p, L->lsStats.p};
+}
+
 // Host side of one batch of outer points: metadata and line tables into b
 // (uploaded on the handle's stream), every scratch buffer the launch needs
 // sized.  line: the outer points lie on at most kLinesPerBatch mesh lines and
@@ -1536,20 +1624,8 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
   const phx_problem& p = L->prob;
   hipStream_t s = L->stream;
   const int nw = L->nw, nm = L->nm;
-  // panels of this batch
   int nPanels = 0;
   for (int i = 0; i < nkk; ++i) nPanels += L->nb[k1s[i]];
-  const size_t pstride = size_t(L->nRp) * L->ldb;
-  if (nPanels > L->maxPanels) {
-    L->maxPanels = std::max(nPanels, L->k1Batch * nw);
-    if (L->precision == PHX_FP64) {
-      L->Bd.alloc(pstride * L->maxPanels);
-      launch_fill<double>(L->Bd.p, L->Bd.n, 0., s);
-    } else {
-      L->Bf.alloc(pstride * L->maxPanels);
-      launch_fill<float>(L->Bf.p, L->Bf.n, 0.f, s);
-    }
-  }
   const int M = k2e - k2b;
   b.nb2max = 1;
   for (int a = k2b; a < k2e; ++a) b.nb2max = std::max(b.nb2max, L->nb[a]);
@@ -1564,7 +1640,6 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
   b.k2b = k2b;
   b.k2e = k2e;
   b.line = line;
-  L->partial.reserve(size_t(L->maxPanels) * std::max(nMtiles, 1) * kGMax * kCMax);
   // metadata: [U1off nkk][nb1 nkk][panelBase nkk][kkMesh nkk][kkStateOff nkk]
   //           [panelKK P][panelB1 P][panelGStart P][panelGSize P]
   std::vector<int>& m = b.hmeta;
@@ -1670,64 +1745,11 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
       PHX_HIP(hipMemcpyAsync(b.phLineF.p, b.hphLineF.data(), nph * sizeof(float2),
                              hipMemcpyHostToDevice, s));
     }
-    const size_t N = size_t(L->nRp) * nm * nw * nw;
-    const size_t nA = size_t(line_count_padded(nLinesB));
-    if (L->precision == PHX_FP64) L->TgD.reserve(nA * L->nGe * N);
-    else L->TgF.reserve(nA * L->nGe * N);
-  } else {
-    L->phE.reserve(cache_phase_size(L->nRe));
   }
   b.nLinesB = nLinesB;
-  L->phP.reserve(size_t(nkk) * L->nRp);
   b.nb1Max = 0;
   for (int i = 0; i < nkk; ++i) b.nb1Max = std::max(b.nb1Max, L->nb[k1s[i]]);
-  // scratch of the separable transform: one panel chunk of stage buffers, row masks,
-  // and the learned screen's per-block arrays
-  if (L->transform == PHX_TRANSFORM_SEPARABLE && M > 0) {
-    // sized for the handle's full chunk, not this batch's panel count, so that a
-    // later, larger batch does not reallocate them
-    const int chunk = lw_panel_chunk(L, p, std::numeric_limits<int>::max(), b.nb2max);
-    const size_t ncol = size_t(nm) * nw;
-    const size_t t1 = size_t(L->nLines) * p.mesh[2] * ncol * 2, t2 = size_t(L->nG0) * p.mesh[1] * p.mesh[2] * ncol * 2;
-    if (L->precision == PHX_FP64) {
-      L->T1d.reserve(t1 * chunk);
-      L->T2d.reserve(t2 * chunk);
-    } else {
-      L->T1f.reserve(t1 * chunk);
-      L->T2f.reserve(t2 * chunk);
-    }
-    const size_t slots = size_t(chunk) * nMtiles;
-    if (p.mesh[0] <= 64) L->keepMask.reserve(slots);
-    if (L->screen > 0.) {
-      L->screenOf.reserve(size_t(L->numStates));
-      L->xminPart.reserve(size_t(chunk) * kXminBlocks);
-    }
-    if (lw_last_stage(L, p) != kStageFused) {  // g3 (complex T) or g' (complex FP64, nb2max nm per row)
-      const size_t g3 = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
-      try {
-        L->G3f.reserve(g3);
-      } catch (const Error&) {  // no room for the g3 rows: the fused kernel runs, which needs none
-        (void)hipGetLastError();
-        L->G3f.release();
-      }
-      if (L->epOverlap && L->G3f.p) {
-        L->G3f2.reserve(g3);
-        L->keepMask2.reserve(slots);
-      }
-    }
-    if (L->lsMode && L->mlpTrained) {
-      L->lsFeat.reserve(slots * kMlpIn);
-      L->lsNscr.reserve(slots);
-      L->lsMaskC.reserve(slots);
-      L->lsMaskA.reserve(slots);
-      L->lsMaskS.reserve(slots);
-      L->lsPred.reserve(slots);
-      L->mlpScratch.reserve(mlp_scratch_floats(int(slots)));
-      L->lsThrAbs.reserve(chunk);
-      L->lsPanelStats.reserve(2 * size_t(chunk));
-      L->partialAudit.reserve(slots * kGMax * kCMax);
-    }
-  }
+  lw_scratch(L, b);
   // algorithmic FLOPs of the coupling stage (per (pair, b1): transform, rotations, |g|^2)
   double f = 0.;
   if (L->transform == PHX_TRANSFORM_DIRECT) {
@@ -2162,11 +2184,11 @@ static void lw_plan(LwHandle* L, int nk1, const int* k1list, int k2b, int k2e) {
   if (k2e < 0) k2e = L->na;
   PHX_REQUIRE(k2b >= 0 && k2b <= k2e && k2e <= L->na, "phx_lw_plan: bad k2 range");
   PHX_REQUIRE(!L->lsCollect, "phx_lw_plan: not while collecting screen samples");
+  PHX_HIP(hipStreamSynchronize(L->stream));
   if (L->graphExec) {
     PHX_HIP(hipGraphExecDestroy(L->graphExec));
     L->graphExec = nullptr;
   }
-  PHX_HIP(hipStreamSynchronize(L->stream));
   L->plan.clear();
   L->planPairs = 0;
   const std::vector<BatchSpec> specs = lw_batches(L, nk1, k1list);
@@ -2182,6 +2204,15 @@ static void lw_plan(LwHandle* L, int nk1, const int* k1list, int k2b, int k2e) {
 // first use and replayed as one graph launch.  Asynchronous on the handle's stream.
 static long long lw_plan_run(LwHandle* L, int graph) {
   PHX_REQUIRE(!L->plan.empty() || L->planPairs == 0, "phx_lw_plan_run: no plan");
+  if (L->graphExec && L->graphBuffers != lw_shared_buffers(L)) {
+    PHX_HIP(hipStreamSynchronize(L->stream));
+    PHX_HIP(hipGraphExecDestroy(L->graphExec));
+    L->graphExec = nullptr;
+  }
+  // settings may have changed since the plan was made; none of its batches may replace
+  // a buffer once another one is on its way
+  if (!graph || !L->graphExec)
+    for (const BatchMeta& b : L->plan) lw_scratch(L, b);
   if (!graph) {
     for (const BatchMeta& b : L->plan) lw_launch(L, b);
     return L->planPairs;
@@ -2204,6 +2235,7 @@ static long long lw_plan_run(LwHandle* L, int graph) {
     hipError_t e = hipGraphInstantiate(&L->graphExec, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     PHX_HIP(e);
+    L->graphBuffers = lw_shared_buffers(L);
   }
   PHX_HIP(hipGraphLaunch(L->graphExec, L->stream));
   return L->planPairs;

@@ -72,6 +72,42 @@ def test_graph_sweeps_and_concurrent_materials_match_sequential_runs():
     assert np.array_equal(lw.linewidths(average=False), seq[0])
 
 
+@pytest.mark.parametrize("precision,transform", [("fp64", "direct"), ("fp32", "separable")])
+def test_plan_outlives_larger_runs(precision, transform):
+    """A captured sweep after runs of larger batches, which replace the buffers it was
+    captured with, and a plan run after settings that need other buffers."""
+    p = synth.make_problem(2, 6, 3, 3, 8, seed=33, name="plan")
+    lw = P.ElectronLinewidths(p, gW=p.gw_host(), precision=precision, transform=transform, k1_batch=1)
+    k1 = np.arange(3, dtype=np.int32)
+    lw.run(k1_list=k1)
+    want = lw.linewidths(average=False)
+    lw.plan(k1)
+
+    def check(graph, tol=0.0):
+        lw.reset()
+        lw.plan_run(graph=graph)
+        lw.sync()
+        got = lw.linewidths(average=False)
+        assert np.array_equal(got != 0, want != 0)
+        assert np.abs(got - want).max() <= tol * np.abs(want).max()
+
+    check(True)
+    lw.set_batching(k1_batch=32)
+    lw.set_line_batching(1)
+    lw.run()  # line batches of many points: larger panel, partial-sum and phase buffers
+    check(True)
+    check(True)
+    check(False)
+    if transform == "separable":
+        # rounding: the screen drops nothing above exp(-36), other kernels take the same values
+        for setting in (lambda: lw.set_screen(6.0), lambda: lw.set_epilogue_overlap(True),
+                        lambda: lw.set_fused_y_stage(False), lambda: lw.set_split_last_stage(3),
+                        lambda: lw.set_split_last_stage(0), lambda: lw.set_panel_chunk(1),
+                        lambda: lw.set_panel_chunk(200)):
+            setting()
+            check(False, 1e-12)
+
+
 def test_autotuner_keeps_results():
     p = synth.make_problem(2, 6, 3, 3, 8, seed=91, name="tune")
     lw = P.ElectronLinewidths(p, gW=p.gw_host(), precision="fp64", transform="separable")
