@@ -1587,8 +1587,13 @@ static void lw_scratch(LwHandle* L, const BatchMeta& b) {
         L->G3f.release();
       }
       if (L->epOverlap && L->G3f.p) {
-        L->G3f2.reserve(g3);
-        L->keepMask2.reserve(slots);
+        try {
+          L->G3f2.reserve(g3);
+          L->keepMask2.reserve(slots);
+        } catch (const Error&) {  // nor for a second set: the chunks run in turn
+          (void)hipGetLastError();
+          L->G3f2.release();
+        }
       }
     }
     if (L->lsMode && L->mlpTrained) {
