@@ -784,6 +784,7 @@ struct LwHandle {
   int panelChunk = 0;      // panels per separable-transform launch (bounds T1 / T2 / g3); 0 = automatic
   int splitLast = 1;       // last stage as x-stage and epilogue kernels where they apply (2: the same;
                            // 3: the electron rotation in k_sep_xg, g' rows through HBM)
+  double g3Room = kG3RoomMax;  // bytes a chunk's g3 rows may take (automatic chunks)
   DevBuf<float2> G3f;      // their g3 rows of one panel chunk, (slot, jx, col), or g' rows (slot, jx, b2, nu)
   // the split stage's epilogue of chunk i on streamEp, overlapping chunk i + 1's
   // transform stages on `stream`: chunks alternate between two sets of g3 rows
@@ -885,15 +886,14 @@ static size_t lw_g3_per_panel(const LwHandle* L, const phx_problem& p, int nb2ma
 }
 
 // Panels per separable-transform launch: the handle's setting, or (0) as many
-// as keep one chunk's g3 rows of the split last stage within kChunkG3Bytes,
-// between 16 and 128: fewer, larger launches have shorter tails (cfg2: 128
-// panels, 12.6 GB of g3; a 60^3 mesh with 18 modes: 51).
-constexpr double kChunkG3Bytes = 24. * (1ull << 30);
+// as panel_chunk gives g3 rows of the split last stage (cfg2: 128 panels,
+// 12.6 GB of g3 in FP32; a 60^3 mesh with 18 modes: 51).  Where the fused kernel runs,
+// the same count as for FP32 rows.
 static int lw_panel_chunk(const LwHandle* L, const phx_problem& p, int nPanels, int nb2max) {
   if (L->panelChunk > 0) return std::min(nPanels, L->panelChunk);
-  const double perPanel = double(lw_g3_per_panel(L, p, nb2max)) * sizeof(float2);
-  const int c = int(std::min(128., std::max(16., std::floor(kChunkG3Bytes / perPanel))));
-  return std::max(1, std::min(nPanels, c));
+  double perPanel = double(lw_g3_per_panel(L, p, nb2max)) * sizeof(float2);
+  if (L->precision == PHX_FP64 && lw_last_stage(L, p) == kStageFused) perPanel /= 2;
+  return std::max(1, std::min(nPanels, panel_chunk(perPanel, L->g3Room)));
 }
 
 // Fold the events of the last timed batch into kernelMs (stream must be idle).
@@ -1562,29 +1562,38 @@ static void lw_scratch(LwHandle* L, const BatchMeta& b) {
   if (L->transform == PHX_TRANSFORM_SEPARABLE && b.M > 0) {
     // sized for the handle's full chunk, not this batch's panel count, so that a
     // later, larger batch does not reallocate them
-    const int chunk = lw_panel_chunk(L, p, std::numeric_limits<int>::max(), b.nb2max);
+    const int all = std::numeric_limits<int>::max();
+    const LastStage stage = lw_last_stage(L, p);
+    const size_t perG3 = lw_g3_per_panel(L, p, b.nb2max);
+    // g3 rows about to be made leave most of the card to other handles and callers
+    if (stage != kStageFused && !L->panelChunk && L->G3f.n < perG3 * lw_panel_chunk(L, p, all, b.nb2max)) {
+      size_t avail = 0, total = 0;
+      PHX_HIP(hipMemGetInfo(&avail, &total));
+      avail += L->G3f.bytes() + L->G3f2.bytes();
+      L->g3Room = std::min(L->g3Room, double(avail) * kG3Share / (L->epOverlap ? 2 : 1));
+    }
+    const int chunk = lw_panel_chunk(L, p, all, b.nb2max);
     const size_t ncol = size_t(nm) * nw;
     const size_t t1 = size_t(L->nLines) * p.mesh[2] * ncol * 2, t2 = size_t(L->nG0) * p.mesh[1] * p.mesh[2] * ncol * 2;
-    if (L->precision == PHX_FP64) {
-      L->T1d.reserve(t1 * chunk);
-      L->T2d.reserve(t2 * chunk);
-    } else {
-      L->T1f.reserve(t1 * chunk);
-      L->T2f.reserve(t2 * chunk);
-    }
+    // k_sep_yx keeps T2 in LDS
+    auto reserve_t2 = [&] { L->precision == PHX_FP64 ? L->T2d.reserve(t2 * chunk) : L->T2f.reserve(t2 * chunk); };
+    if (L->precision == PHX_FP64) L->T1d.reserve(t1 * chunk);
+    else L->T1f.reserve(t1 * chunk);
+    if (stage != kStageYx) reserve_t2();
     const size_t slots = size_t(chunk) * b.nMtiles;
     if (p.mesh[0] <= 64) L->keepMask.reserve(slots);
     if (L->screen > 0.) {
       L->screenOf.reserve(size_t(L->numStates));
       L->xminPart.reserve(size_t(chunk) * kXminBlocks);
     }
-    if (lw_last_stage(L, p) != kStageFused) {  // g3 (complex T) or g' (complex FP64, nb2max nm per row)
-      const size_t g3 = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
+    if (stage != kStageFused) {  // g3 (complex T) or g' (complex FP64, nb2max nm per row)
+      const size_t g3 = size_t(chunk) * perG3;
       try {
         L->G3f.reserve(g3);
       } catch (const Error&) {  // no room for the g3 rows: the fused kernel runs, which needs none
         (void)hipGetLastError();
         L->G3f.release();
+        reserve_t2();
       }
       if (L->epOverlap && L->G3f.p) {
         try {
@@ -1990,6 +1999,9 @@ static long long lw_launch(LwHandle* L, const BatchMeta& b) {
     const size_t g3Need = size_t(chunk) * lw_g3_per_panel(L, p, b.nb2max);
     cq.stage = L->G3f.n >= g3Need ? lw_last_stage(L, p) : kStageFused;
     const bool split = cq.stage != kStageFused, yx = cq.stage == kStageYx;
+    PHX_REQUIRE(std::max(L->T1d.n, L->T1f.n) >= sp.t1PanelStride * chunk &&
+                    (yx || std::max(L->T2d.n, L->T2f.n) >= sp.t2PanelStride * chunk),
+                "separable transform: stage buffers smaller than a chunk");
     const bool overlap = L->epOverlap && !learned && split && L->G3f2.n >= g3Need && L->keepMask2.n >= slotsC;
     sp.modeFast = split ? nm : 0;
     const int nChunks = (nPanels + chunk - 1) / chunk;

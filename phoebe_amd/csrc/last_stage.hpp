@@ -55,4 +55,13 @@ constexpr LastStage last_stage(const LastStageSizes& z, int mode, bool fuseY, bo
   return mode == 3 && !z.adaptive ? kStageRot : kStageXg;
 }
 
+// Panels per launch of the split last stage when its g3 rows may take `room` bytes:
+// between 16 and 128, as fewer, larger launches have shorter tails.
+constexpr double kG3RoomMax = 24. * (1ull << 30);
+constexpr double kG3Share = 0.25;  // of the memory that is free when the rows are made
+constexpr int panel_chunk(double bytesPerPanel, double room) {
+  const double n = room / bytesPerPanel;
+  return n < 16. ? 16 : n > 128. ? 128 : int(n);
+}
+
 }  // namespace phx

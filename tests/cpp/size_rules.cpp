@@ -1,6 +1,7 @@
 // The kernels' size rules, evaluated on the host: one form per line of stdin.
 //   stage f64 bf16x3 nm nw m0 my nG0 nQuads adaptive mode fuseY learned -> LastStage
 //   tiling f64 nm nw nb2max -> mt nt wc rows modes stage lds
+//   chunk bytesPerPanel room -> panels
 #include <iostream>
 #include <string>
 
@@ -22,6 +23,10 @@ int main() {
       const phx::CoupTiling c = phx::coupling_tiling(f64 != 0, nm, nw, nb2max);
       std::cout << c.mt << " " << c.nt << " " << c.wc << " " << c.rows << " " << c.modes << " " << c.stage << " "
                 << c.lds << "\n";
+    } else if (kind == "chunk") {
+      double per, room;
+      std::cin >> per >> room;
+      std::cout << phx::panel_chunk(per, std::min(room, phx::kG3RoomMax)) << "\n";
     } else {
       return 1;
     }

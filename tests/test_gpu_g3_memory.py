@@ -1,4 +1,5 @@
-"""Device memory of the split last stage: what it does without when the g3 rows,
+"""Device memory of the split last stage: no x-stage slabs (T2) beside the fused
+y-stage, and what it does without when the g3 rows,
 or the second set of them that the epilogue overlap takes, find no room.  Chunks
 of more panels than fit are asked for; every other buffer of the problem is
 small (one mesh line of R_ph)."""
@@ -46,3 +47,23 @@ def test_no_room(share, overlap, split):
     assert np.array_equal(got != 0, want != 0)
     nz = want != 0
     assert np.abs(got[nz] / want[nz] - 1).max() < 1e-12
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_fused_y_stage_holds_no_slabs(precision):
+    def used(fused, chunk):
+        lw = _handle(precision)
+        lw.set_panel_chunk(chunk)
+        lw.set_fused_y_stage(fused)
+        lw.sync()
+        free = torch.cuda.mem_get_info()[0]
+        lw.run(k1_list=np.arange(4, dtype=np.int32))
+        lw.sync()
+        return free - torch.cuda.mem_get_info()[0]
+
+    # FP32: k_sep_xg's slabs; FP64: the fused last stage's, which has no g3 rows
+    elem = 8 if precision == "fp32" else 16
+    slabs, rows = 8000 * 16 * 16 * 12 * elem, 0 if precision == "fp32" else 8000 * int(np.prod(MESH)) * 12 * elem
+    used(True, 4), used(False, 4)  # the runtime's own memory for these kernels
+    a, b = used(True, 8000), used(False, 8000)
+    assert abs((b - a) - (slabs - rows)) < 0.2 * slabs, (a, b, slabs, rows)

@@ -72,3 +72,11 @@ def test_coupling_tiling(rules, f64):
         assert stage == (16 * modes * nw * elem >= 16 * (nm + nb) * 8), at
         seen.add((mt, nt))
     assert seen == INSTANCES[f64]
+
+
+def test_panel_chunk(rules):
+    """At most 24 GiB of g3 rows, 16 to 128 panels."""
+    G = 1 << 30
+    forms = [(100 << 20, 100 * G), (100 << 20, 24 * G), (100 << 20, 10 * G), (100 << 20, G), (100 << 20, 0), (G, 100 * G),
+             (4 * G, 100 * G), (1, 100 * G)]
+    assert [c for c, in rules("chunk", forms)] == [128, 128, 102, 16, 16, 24, 16, 128]
