@@ -223,7 +223,7 @@ __device__ void epilogue16_tail(const CoupParams& p, unsigned char* scratch, dou
   const double2* e3 = p.E3pool + size_t(myIq) * nm * nm;
   const bool polar = p.polarX != nullptr && valid;
   const double* const w3g = p.Wpool + size_t(myIq) * nm;
-  const double* const e2g = p.e2pool + (valid ? p.rowStateOff[myRow] : 0);
+  const double* const e2g = REDUCE ? p.e2pool + (valid ? p.rowStateOff[myRow] : 0) : nullptr;  // no states in store mode
   double* const w3s = stage ? stage + r * nm : nullptr;
   double* const e2s = stage ? stage + 16 * nm + r * p.nb2max : nullptr;
   if (REDUCE && stage && valid) {
