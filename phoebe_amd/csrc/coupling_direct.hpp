@@ -156,36 +156,28 @@ void launch_coupling(const CoupParams& p, bool reduce, hipStream_t s) {
                                 int(c.lds)));
     hipLaunchKernelGGL(kern, dim3(ceil_div(tiles, 8) * 8), dim3(256), c.lds, s, p, c);
   };
+  // the tiles per wave that coupling_tiling gives: FP64 at most 4 columns (3 with two row tiles)
   auto red = [&](auto mt, auto nt) {
     constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value;
-    if (reduce) go(k_coupling<T, MT, NT, true>);
-    else go(k_coupling<T, MT, NT, false>);
+    if constexpr (MT == 1 ? NT <= (sizeof(T) == 8 ? 4 : 6) : NT >= 3 && NT <= (sizeof(T) == 8 ? 3 : 6)) {
+      if (reduce) go(k_coupling<T, MT, NT, true>);
+      else go(k_coupling<T, MT, NT, false>);
+    } else {
+      PHX_REQUIRE(false, "coupling kernel: no instance for these tiles");
+    }
   };
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
-  using I4 = std::integral_constant<int, 4>;
-  using I5 = std::integral_constant<int, 5>;
-  using I6 = std::integral_constant<int, 6>;
-  if (c.mt == 1) {
+  auto nts = [&](auto mt) {
     switch (c.nt) {
-      case 1: red(I1{}, I1{}); break;
-      case 2: red(I1{}, I2{}); break;
-      case 3: red(I1{}, I3{}); break;
-      case 4: red(I1{}, I4{}); break;
-      case 5: red(I1{}, I5{}); break;
-      default: red(I1{}, I6{});
+      case 1: red(mt, std::integral_constant<int, 1>{}); break;
+      case 2: red(mt, std::integral_constant<int, 2>{}); break;
+      case 3: red(mt, std::integral_constant<int, 3>{}); break;
+      case 4: red(mt, std::integral_constant<int, 4>{}); break;
+      case 5: red(mt, std::integral_constant<int, 5>{}); break;
+      default: red(mt, std::integral_constant<int, 6>{});
     }
-  } else {
-    switch (c.nt) {
-      case 1: red(I2{}, I1{}); break;
-      case 2: red(I2{}, I2{}); break;
-      case 3: red(I2{}, I3{}); break;
-      case 4: red(I2{}, I4{}); break;
-      case 5: red(I2{}, I5{}); break;
-      default: red(I2{}, I6{});
-    }
-  }
+  };
+  if (c.mt == 1) nts(std::integral_constant<int, 1>{});
+  else nts(std::integral_constant<int, 2>{});
   PHX_HIP(hipGetLastError());
 }
 

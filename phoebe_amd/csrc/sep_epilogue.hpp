@@ -413,7 +413,7 @@ void launch_ep2(EpParams q, int gsizeMax, int grid, bool pre, hipStream_t s) {
   const int gm = gsizeMax > 0 ? gsizeMax : kGMax;
   PHX_REQUIRE(gm <= kGMax && q.nb2max <= kSepNb2 && q.nm <= kSepNm && q.nCalc <= kCMax,
               "separable transform: epilogue sizes");
-  PHX_REQUIRE(!pre || (sizeof(T) == 4 && q.nm <= 24 && !q.adaptive), "separable transform: rotated x-stage is FP32 only");
+  PHX_REQUIRE(!pre || (sizeof(T) == 4 && q.nm <= 16 && !q.adaptive), "separable transform: rotated x-stage is FP32 only");
   auto go = [&](auto nmx, auto small, auto cmx, auto prec) {
     constexpr int NM = decltype(nmx)::value, NB = decltype(small)::value ? 4 : 8, CM = decltype(cmx)::value;
     constexpr bool PRE = decltype(prec)::value == 1, ADAPT = decltype(prec)::value == 2;
@@ -437,7 +437,7 @@ void launch_ep2(EpParams q, int gsizeMax, int grid, bool pre, hipStream_t s) {
     small ? calcs(nmx, std::true_type{}, kind) : calcs(nmx, std::false_type{}, kind);
   };
   auto sizes = [&](auto nmx) {
-    if constexpr (sizeof(T) == 4 && decltype(nmx)::value <= 24) {
+    if constexpr (sizeof(T) == 4 && decltype(nmx)::value <= 24 && decltype(nmx)::value != 18) {  // up to 16 modes
       if (pre) return kinds(nmx, std::integral_constant<int, 1>{});
     }
     q.adaptive ? kinds(nmx, std::integral_constant<int, 2>{}) : kinds(nmx, std::integral_constant<int, 0>{});
