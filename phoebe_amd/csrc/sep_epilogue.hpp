@@ -93,19 +93,34 @@ __device__ __forceinline__ void ep2_rot_ph(const T2v (&e3c)[NMX], const double2*
 // then constants of the load instructions.
 constexpr bool ep2_exact(int nmx) { return nmx <= 18; }
 
+// FP32 rows of more than 4 bands whose U2 goes through registers: twice the U2
+// entries and |g|^2, so 256 registers at two waves per SIMD (at 168 they spill 36
+// to 183, which also cost more than the third wave gives).
+constexpr bool ep2_wide(int elem, int nb2, bool pre) { return elem == 4 && nb2 > 4 && !pre; }
+constexpr int ep2_waves(int elem, int nb2, bool pre) { return elem == 4 && !ep2_wide(elem, nb2, pre) ? 3 : 2; }
+
 // Rows per pass at most: whole rows of nm lanes for the least nm served with
-// NMX, and no more than five.  Ten rows of 6 modes fill the wave but hold twice
-// the U2 entries in registers, and spill: 52 us against 37 per launch of 128
-// panels on a 12^3 mesh.
-constexpr int ep2_rows_max(int nmx) { return nmx <= 12 ? 5 : nmx <= 18 ? 4 : nmx <= 24 ? 3 : 2; }
+// NMX, and no more than five, or with up to 9 modes in the wide form 8, 6 or 7,
+// as many as pay.  Ten rows of 6 modes fill the wave but hold twice the U2 entries
+// in registers, and spill: 52 us against 37 per launch of 128 panels on a 12^3
+// mesh.  Wide form, 8 bands, 200 points against a 16 x 17 x 16 mesh, adaptive, one and
+// four calculations (three waves and five rows; two waves; the epilogue of one
+// thread per row and mode that adaptive widths had before), ms: 3 modes 12.0 and
+// 15.5; 9.3 and 9.7; 9.7 and 11.1.  6 modes 14.7 and 18.7; 11.6 and 12.1; 11.5 and
+// 12.9.  9 modes (14^3) 11.1 and 15.0; 9.5 and 10.0; 9.5 and 12.3.  12 modes 21.6
+// and 28.2; 19.2 and 19.8; 20.7 and 24.7.
+constexpr int ep2_rows_max(int nmx, bool wide) {
+  if (wide && nmx <= 9) return nmx <= 3 ? 8 : nmx <= 6 ? 6 : 7;
+  return nmx <= 12 ? 5 : nmx <= 18 ? 4 : nmx <= 24 ? 3 : 2;
+}
 
 template <typename T, int CM, int NMX, int GM, int NB2, bool PRE, bool ADAPT>
-__global__ void __launch_bounds__(64, sizeof(T) == 4 ? 3 : 2) k_sep_ep2(EpParams p) {
+__global__ void __launch_bounds__(64, ep2_waves(sizeof(T), NB2, PRE)) k_sep_ep2(EpParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   typedef typename Vec2<T>::type T2v;
   constexpr int NWX = 16;
   constexpr int U2S = NWX * NB2 + 1;  // double2 per row of the U2 table (odd: rows in different banks)
-  constexpr int RMX = ep2_rows_max(NMX);
+  constexpr int RMX = ep2_rows_max(NMX, ep2_wide(sizeof(T), NB2, PRE));
   constexpr int UPL = PRE ? 1 : (NWX * NB2 * RMX + 63) / 64;  // U2 entries per lane
   const int nLinesYZ = p.m1 * p.m2;
   const int nTilesTot = p.nPanels * nLinesYZ;
@@ -418,7 +433,7 @@ void launch_ep2(EpParams q, int gsizeMax, int grid, bool pre, hipStream_t s) {
     constexpr int NM = decltype(nmx)::value, NB = decltype(small)::value ? 4 : 8, CM = decltype(cmx)::value;
     constexpr bool PRE = decltype(prec)::value == 1, ADAPT = decltype(prec)::value == 2;
     constexpr int GM = NB == 4 ? 4 : kGMax;
-    q.rpw = std::min(64 / q.nm, ep2_rows_max(NM));
+    q.rpw = std::min(64 / q.nm, ep2_rows_max(NM, ep2_wide(sizeof(T), NB, PRE)));
     const size_t lds = sep_ep2_lds_bytes(NM, NB, CM, gm, q.rpw, PRE, ADAPT);
     PHX_REQUIRE(lds <= 160 * 1024, "separable transform: LDS budget exceeded");
     auto kern = k_sep_ep2<T, CM, NM, GM, NB, PRE, ADAPT>;

@@ -10,6 +10,7 @@ import pytest
 
 import phoebe_amd as P
 from oracle import oracle as O
+from phoebe_amd import synth
 from tests.helpers import rel_err, tiny_problem
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +45,28 @@ def test_split_equals_fused_and_oracle(precision, natoms, nw, mesh, rg_p, nt, sm
     # adaptive widths: central differences summed in another order
     tol = 1e-6 if precision == "fp32" else 1e-7 if smearing else 1e-10
     assert rel_err(lw.linewidths(), ref).max() < tol
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("natoms,nw", [(1, 8), (2, 7), (3, 5), (4, 8), (5, 6), (8, 8)])
+@pytest.mark.parametrize("nt,smearing", [(1, 1), (4, 1), (1, 0)])
+def test_many_bands_per_point(precision, natoms, nw, nt, smearing):
+    """Five to eight bands at every inner point: the epilogue's wide form, whose passes
+    hold other numbers of rows (mesh lines of 13 points: whole passes and a remainder)."""
+    p = synth.make_problem(natoms, nw, 3, 2, (13, 4, 3), seed=52, window_ev=30.0)
+    p.temperatures = p.temperatures[:1] * np.arange(1, nt + 1)
+    p.chem_pots = p.chem_pots[:1].repeat(nt)
+    p.smearing = smearing
+    out = []
+    for split in (0, 1):
+        lw = P.ElectronLinewidths(p, precision=precision, transform="separable")
+        assert int((lw.band_hi - lw.band_lo).max()) + 1 == nw
+        lw.set_split_last_stage(split)
+        lw.set_timing(True)
+        lw.run(k1_list=np.arange(0, lw.num_active, 11, dtype=np.int32))
+        lw.sync()
+        assert (lw.split_times()["launches"] > 0) == bool(split)
+        out.append(lw.linewidths(average=False))
+    nz = out[0] != 0
+    assert nz.any() and np.array_equal(out[1] != 0, nz)
+    assert np.abs(out[1][nz] / out[0][nz] - 1).max() < 1e-12
