@@ -654,7 +654,7 @@ static void elph_coupling_sq(ElphHandle* H, int nq, const double* U2s, const int
   p.nm = nm;
   p.nw = nw;
   p.nPanels = nb1;
-  p.nMtiles = ceil_div(nq, coupling_tiling(f64, nm, nw, nb2max).rows);
+  p.nMtiles = ceil_div(nq, coupling_tiling(f64, nm, nw, nb2max, nq, nb1).rows);
   p.panelKK = H->meta.p + 4;
   p.panelB1 = H->meta.p + 4 + nb1;
   p.U2pool = H->sU2.p;
@@ -1549,7 +1549,11 @@ static void lw_scratch(LwHandle* L, const BatchMeta& b) {
     }
     L->maxPanels = most;
   }
-  L->partial.reserve(size_t(L->maxPanels) * std::max(b.nMtiles, 1) * kGMax * kCMax);
+  // partial sums of the batch, and of one of maxPanels panels (whose row tiles may be larger)
+  const int full = L->transform == PHX_TRANSFORM_DIRECT
+                       ? ceil_div(b.M, coupling_tiling(L->precision == PHX_FP64, nm, nw, b.nb2max, b.M, L->maxPanels).rows)
+                       : b.nMtiles;
+  L->partial.reserve(std::max({size_t(1), size_t(b.nPanels) * b.nMtiles, size_t(L->maxPanels) * full}) * kGMax * kCMax);
   if (b.line) {
     const size_t Tg = size_t(line_count_padded(b.nLinesB)) * L->nGe * L->nRp * nm * nw * nw;
     if (L->precision == PHX_FP64) L->TgD.reserve(Tg);
@@ -1646,7 +1650,7 @@ static void lw_prepare(LwHandle* L, const int* k1s, int nkk, int k2b, int k2e, b
   for (int a = k2b; a < k2e; ++a) b.nb2max = std::max(b.nb2max, L->nb[a]);
   const int nMtiles =
       L->transform == PHX_TRANSFORM_DIRECT
-          ? ceil_div(M, coupling_tiling(L->precision == PHX_FP64, nm, nw, b.nb2max).rows)
+          ? ceil_div(M, coupling_tiling(L->precision == PHX_FP64, nm, nw, b.nb2max, M, nPanels).rows)
           : p.mesh[1] * p.mesh[2];
   b.nkk = nkk;
   b.nPanels = nPanels;
@@ -2649,9 +2653,9 @@ static void phel_batch(PhelHandle* P, const int* as, int n) {
     c.M = nq;
     c.nm = nm;
     c.nw = nw;
-    c.nMtiles = ceil_div(nq, coupling_tiling(f64, nm, nw, nw).rows);
     const int pan0 = cm[2 * K + i0];
     c.nPanels = (i0 + np < n ? cm[2 * K + i0 + np] : pb) - pan0;
+    c.nMtiles = ceil_div(nq, coupling_tiling(f64, nm, nw, nw, nq, c.nPanels).rows);
     // panels of the batch: point (relative to the group's first) and band
     c.panelKK = P->pmeta.p + K + pan0;
     c.panelB1 = P->pmeta.p + K + size_t(K) * P->nb1max + pan0;

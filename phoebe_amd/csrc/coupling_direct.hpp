@@ -146,7 +146,7 @@ template <typename T>
 void launch_coupling(const CoupParams& p, bool reduce, hipStream_t s) {
   PHX_REQUIRE(p.nm <= kNmMax, "coupling kernel supports nm <= 36");
   PHX_REQUIRE(p.ldb % 2 == 0 && p.nRp >= 1 && p.lda >= size_t(std::max(p.M, 1)), "coupling kernel: bad operand shapes");
-  const CoupTiling c = coupling_tiling(sizeof(T) == 8, p.nm, p.nw, p.nb2max);
+  const CoupTiling c = coupling_tiling(sizeof(T) == 8, p.nm, p.nw, p.nb2max, p.M, p.nPanels);
   PHX_REQUIRE(c.lds <= 160 * 1024, "coupling kernel: nm x bands per inner point too large for LDS");
   PHX_REQUIRE(p.nMtiles == ceil_div(p.M, c.rows), "coupling kernel: row tiles");
   const int tiles = p.nPanels * p.nMtiles;

@@ -1,6 +1,6 @@
 // The kernels' size rules, evaluated on the host: one form per line of stdin.
 //   stage f64 bf16x3 nm nw m0 my nG0 nQuads adaptive mode fuseY learned -> LastStage
-//   tiling f64 nm nw nb2max -> mt nt wc rows modes stage lds
+//   tiling f64 nm nw nb2max points panels -> mt nt wc rows modes stage lds
 //   chunk bytesPerPanel room -> panels
 #include <iostream>
 #include <string>
@@ -18,9 +18,9 @@ int main() {
           fuseY >> learned;
       std::cout << int(phx::last_stage(z, mode, fuseY != 0, learned != 0)) << "\n";
     } else if (kind == "tiling") {
-      int f64, nm, nw, nb2max;
-      std::cin >> f64 >> nm >> nw >> nb2max;
-      const phx::CoupTiling c = phx::coupling_tiling(f64 != 0, nm, nw, nb2max);
+      int f64, nm, nw, nb2max, points, panels;
+      std::cin >> f64 >> nm >> nw >> nb2max >> points >> panels;
+      const phx::CoupTiling c = phx::coupling_tiling(f64 != 0, nm, nw, nb2max, points, panels);
       std::cout << c.mt << " " << c.nt << " " << c.wc << " " << c.rows << " " << c.modes << " " << c.stage << " "
                 << c.lds << "\n";
     } else if (kind == "chunk") {

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import phoebe_amd as P
+from phoebe_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +62,25 @@ def test_windows_narrowed_by_many_bands(nw, nm, nb2, precision):
 def test_too_many_bands_are_refused(precision):
     with pytest.raises(P.PhxError):
         _call(20, 24, 20, 1, precision, 6)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("fp32", 2e-6)])
+@pytest.mark.parametrize("natoms,nw", [(3, 16), (6, 16)])
+def test_row_tiles_by_the_number_of_workgroups(natoms, nw, precision, tol):
+    """A point alone takes 16 rows per workgroup, a batch of points 32, and runs of
+    either may follow the other; the linewidths of the points are the same."""
+    p = synth.make_problem(natoms, nw, 2, 3, (9, 8, 9), seed=23, window_ev=3.0)
+    lw = P.ElectronLinewidths(p, precision=precision, transform="direct", k1_batch=32)
+    k1 = np.arange(40, 72, dtype=np.int32)
+    panels = int((lw.band_hi - lw.band_lo + 1)[k1].sum())
+    assert -(-lw.num_active // 32) * panels > 256 >= -(-lw.num_active // 32) * int((lw.band_hi - lw.band_lo + 1).max())
+    out = []
+    for batch in (1, 32, 1, 32):
+        lw.reset()
+        lw.set_batching(k1_batch=batch)
+        lw.run(k1_list=k1)
+        out.append(lw.linewidths(average=False))
+    nz = out[0] != 0
+    assert nz.any()
+    for o in out[1:]:
+        assert np.array_equal(o != 0, nz) and np.abs(o[nz] / out[0][nz] - 1).max() <= tol

@@ -56,13 +56,15 @@ def test_coupling_tiling(rules, f64):
     """Every size ends (some windows once never got smaller), the tiles cover the
     window's columns with an instance that exists, and a size is refused only when
     not even one mode at a time fits LDS."""
-    forms = [(f64, nm, nw, nb) for nm in range(1, 37) for nw in range(1, 33) for nb in range(1, nw + 1)]
+    forms = [(f64, nm, nw, nb, points, panels) for nm in range(1, 37) for nw in range(1, 33) for nb in range(1, nw + 1)
+             for points, panels in ((8192, 1), (8193, 1), (33, 128), (33, 129), (0, 5))]
     got = rules("tiling", forms, timeout=120)
     assert len(got) == len(forms)
     elem, most = (16, 192) if f64 else (8, 384)
     seen = set()
-    for (_, nm, nw, nb), (mt, nt, wc, rows, modes, stage, lds) in zip(forms, got):
-        at = (nm, nw, nb)
+    for (_, nm, nw, nb, points, panels), (mt, nt, wc, rows, modes, stage, lds) in zip(forms, got):
+        at = (nm, nw, nb, points, panels)
+        assert mt == (2 if modes == nm and wc == 4 and -(-points // 32) * panels > 256 else 1), at
         scratch = 16 * nm * nb * 24
         assert 1 <= modes <= nm and (modes * nw <= most or modes == 1), at
         assert lds == max(16 * modes * nw * elem + scratch, 1024), at
