@@ -434,14 +434,14 @@ long long phx_lw_plan_run(phx_lw* h, int graph);
  * M tile is 2 x k1_batch) and mesh lines per line batch (1..16). */
 int phx_lw_set_batching(phx_lw* h, int k1_batch, int lines_per_batch);
 /* Autotuner: times full runs over the sample k1_list for k1 batches {8, 16,
- * 32}, lines per batch {1, 2, 4} (line batching on) and panels per separable
+ * 32}, lines per batch {1, 2, 4, 8, 16} (line batching on) and panels per separable
  * launch {16, 48, 128}, one knob at a time, keeps the fastest; the
  * linewidths are restored.  out4 = {k1_batch, lines_per_batch, panel_chunk,
  * best seconds}.  No counterpart in the reference. */
 int phx_lw_autotune(phx_lw* h, int nk1, const int* k1_list, double* out4);
 /* Mesh-line batching of the outer points: the points of a phx_lw_run call
  * that share a mesh line (equal j1, j2 of k1 = sum_d j_d/m_d b_d) are
- * processed together, up to 64 per batch, when the line holds at least
+ * processed together, up to 1024 per batch, when the line holds at least
  * min_points of them; cacheElPh then streams gW once per line and factors
  * e^{ik1.Re} = e^{2 pi i j0 n0/m0} e^{2 pi i (j1 n1/m1 + j2 n2/m2)} over the
  * lattice coordinates n_d of R_e.  The remaining points keep the k1-batched
@@ -489,8 +489,10 @@ int phx_lw_set_epilogue_overlap(phx_lw* h, int on);
  * the separable transform inside the x-stage kernel (on = 1, the default),
  * so that the x-stage slabs T2 stay in LDS instead of going through device
  * memory, or as its own kernel (on = 0).  Not with split mode 3.  The g3
- * values, and so the linewidths, are the same either way.  No counterpart
- * in the reference. */
+ * values, and so the linewidths, are the same either way where the x-stage has
+ * a kernel of its own (PHX_FP32, nm <= 16, nm nw <= 192); elsewhere on = 0 runs
+ * the fused last stage, whose linewidths agree to rounding.  No counterpart in
+ * the reference. */
 int phx_lw_set_fused_y_stage(phx_lw* h, int on);
 /* With timing on: *on = 1 when every timed split launch ran the y-stage inside
  * the x-stage kernel (the x-stage times and bytes then cover both stages).
@@ -502,12 +504,12 @@ int phx_lw_last_stage_fused_y(phx_lw* h, int* on);
 int phx_lw_last_stage_split_times(phx_lw* h, double* out4);
 /* With timing on and the last stage split: out2 = {bytes the x-stage kernel
  * moved, bytes of its output the epilogue read}.  The x-stage kernel reads
- * the x-stage slabs (slots computed x x-groups x nm nw complex FP32) and
- * writes g3 (kept rows x nm nw complex FP32); with the rotation in the
- * x-stage (split mode 3) it writes g' instead (kept bands x nm complex FP64)
- * and reads U2 (kept bands x nw complex FP64); with the y-stage inside it
- * reads the y-stage input T1 (panels x lines x mz x nm nw complex FP32)
- * instead of the slabs.  No counterpart in the
+ * the x-stage slabs (slots computed x x-groups x nm nw complex values of the
+ * handle's precision) and writes g3 (kept rows x nm nw of them); with the
+ * rotation in the x-stage (split mode 3) it writes g' instead (kept bands x nm
+ * complex FP64) and reads U2 (kept bands x nw complex FP64); with the y-stage
+ * inside it reads the y-stage input T1 (panels x lines x mz x nm nw complex
+ * values) instead of the slabs.  No counterpart in the
  * reference (a measurement call). */
 int phx_lw_last_stage_split_bytes(phx_lw* h, double* out2);
 /* ---- Learned q-block screen (separable transform with the energy screen on).

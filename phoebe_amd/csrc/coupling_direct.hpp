@@ -15,7 +15,10 @@ namespace phx {
 // row tile.  The matrix cores bound it where nm nw fills the tiles; with C as a
 // real [C; iC] panel and A staged in LDS between barriers one 4- or 8-byte load
 // fed one product per row tile, and wide panels were bound by those loads.
-// What is left is the epilogue's latency.  Per launch: 48 columns, 251 R_p, 1700
+// What is left is the epilogue's latency, and spills: the reduction's partial sums
+// (64 registers) live through the main loop, so two row tiles spill 32, 71 and 102
+// registers with 4, 5 and 6 column tiles in FP32 and 79 with 3 in FP64 (1 x 4: 8).
+// Per launch: 48 columns, 251 R_p, 1700
 // points, 32 outer points in FP64 0.23 -> 0.17 ms; 345 columns, 79 R_p in FP32
 // 3.0 -> 2.2 ms.
 template <typename T, int MT, int NT, bool REDUCE>
