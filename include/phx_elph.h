@@ -427,7 +427,8 @@ int phx_lw_set_polar(phx_lw* h, const phx_polar* polar);
 long long phx_lw_plan(phx_lw* h, int nk1, const int* k1_list, int k2_begin, int k2_end);
 /* Enqueue the prepared sweep on the handle's stream without host
  * synchronization; graph != 0 captures it into a hipGraph on first use and
- * replays that graph.  Handles run concurrently on their own streams.
+ * replays that graph (captured again when a buffer it uses has been replaced by
+ * another run or setting of the handle).  Handles run concurrently on their own streams.
  * Returns the (k1, k2) pair count. */
 long long phx_lw_plan_run(phx_lw* h, int graph);
 /* Batch shapes: outer points per GEMM-form batch (1..32, the cacheElPh GEMM

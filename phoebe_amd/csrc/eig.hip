@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
         p.x += aj.x * vj.x - aj.y * vj.y;
         p.y += aj.x * vj.y + aj.y * vj.x;
       }
-    p = cmul(tau, p);
+    p = tau.x != 0. || tau.y != 0. ? cmul(tau, p) : make_double2(0., 0.);  // identity: infinities stay where they are
     // w = p - (tau / 2) (p^H v) v, with tau p^H v = |tau|^2 v^H A v real
     const double2 pv = make_double2(group_sum<L>(in ? p.x * v.x + p.y * v.y : 0.),
                                     group_sum<L>(in ? p.x * v.y - p.y * v.x : 0.));
@@ -531,6 +531,7 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
   }
   group_sync();
 
+  const unsigned long long ones = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;  // a group's lanes in a ballot
   // implicit QL: eigenvalue l of the group, it iterations spent on it
   int l = 0, it = 0, total = 0, worst = 0;
   bool bad = false;
@@ -540,7 +541,6 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
       bool small = false;
       if (li >= l && li < N - 1)
         small = fabs(e[li]) <= fmax(kQlTiny, 2.220446049250313e-16 * (fabs(d[li]) + fabs(d[li + 1])));
-      const unsigned long long ones = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
       const unsigned long long hit = (__ballot(small) >> (sg * L)) & ones;
       const int m = hit ? __ffsll(hit) - 1 : N - 1;
       if (m == l) {
@@ -607,6 +607,9 @@ __global__ void __launch_bounds__(64) k_eig_ql(int N, int M, double2* __restrict
     }
     group_sync();
   }
+
+  // a NaN on the diagonal alone passes every test above
+  bad = bad || ((__ballot(row && d[li] != d[li]) >> (sg * L)) & ones) != 0ull;
 
   // ascending order by rank (stable); lane = eigenvalue, then lane = row
   int rank = 0;

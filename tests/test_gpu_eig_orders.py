@@ -95,6 +95,26 @@ def test_rank_one_with_structured_phases(n):
     _check(u[:, :, None] * u[:, None, :].conj())
 
 
+@pytest.mark.parametrize("n", [1, 2, 5, 8, 9, 17, 44])
+def test_not_a_number_is_reported(n):
+    """Wherever it is, and only for its own matrix; an infinite level without
+    couplings is one."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    good = X + X.conj().T
+    for i, j, H in [(0, 0, good), (n - 1, n - 1, good), (n - 1, 0, good), (n // 2, n // 2, np.diag(np.arange(n) + 0j))]:
+        A = np.stack([good] * 9)
+        A[4] = H
+        A[4][i, j] = np.nan
+        with pytest.raises(P.PhxError, match="matrix 4 "):
+            P.zheev_batched(A)
+    d = np.arange(n, dtype=float)
+    d[n // 2] = np.inf
+    order = np.r_[np.delete(np.arange(n), n // 2), n // 2]
+    W, V = P.zheev_batched(np.stack([good, np.diag(d) + 0j]))
+    assert np.array_equal(W[1], d[order]) and np.array_equal(V[1], np.eye(n)[:, order])
+
+
 @pytest.mark.parametrize("kind,n,nk", [("el", 3, 1), ("el", 8, 5), ("el", 9, 2100), ("el", 12, 700), ("el", 16, 8200),
                                        ("el", 17, 33), ("ph", 6, 3), ("ph", 9, 2100), ("ph", 12, 8300), ("ph", 18, 40)])
 def test_bloch_sums(kind, n, nk):
