@@ -19,15 +19,20 @@ constexpr size_t kCoupReduceLds = 1024;  // of reduce_partials
 
 // As few windows as fit: whole panels of up to 24 column tiles (FP32) or 12
 // (FP64, whose tiles take twice the registers and LDS), and fewer modes per window
-// where g' and |g|^2 of a row tile leave less LDS to g3.  One column wave up to 3
-// tiles, two up to 8, four beyond; the other waves take rows.  Several windows
-// leave a row tile's g' in LDS between them, so they run 16 rows per workgroup.
-// Four column waves take two row tiles each, which serve both from one load of the
-// panel, when more than 256 workgroups of 32 points do not fit the card at once as
-// twice as many of 16 points do.  18 modes x 16 bands in FP32, us per launch with
-// 32 and 16 points: 108 workgroups of 32 points 81 and 55, 256 83 and 64, 432 114
-// and 120, 3348 644 and 730; 12 x 16 in FP64 64 and 40, 67 and 52, 91 and 93, 513
-// and 542.
+// where g' and |g|^2 of a row tile leave less LDS to g3.  Several windows leave a row
+// tile's g' in LDS between them, so they run 16 rows per workgroup.
+// Whole panels take 16, 32 or 64 rows: more rows share a load of the panel, but
+// their epilogues follow each other, and two workgroups per CU, 512 in all, run at
+// once.  16 rows on four column waves while 32 would not even give every CU a
+// workgroup.  Else, up to 8 column tiles, 64 rows where the waves of 512 workgroups
+// they take, at 12/7 the time of 32 rows, are no longer: on one column wave up to
+// 6 tiles (FP64, whose accumulators take twice the registers: 4), in FP32 on two with
+// two row tiles each beyond.  More tiles: two row tiles on four column waves.
+// us per launch with 16, 32 and 64 rows in FP32; 5 column tiles: 28 workgroups of 32
+// rows 35, 52 and 63, 756 -, 108 and 97, 1022 -, 135 and 141, 12298 -, 1468 and 1230; 3
+// tiles, 28: 27, 41 and 63; 8 tiles, 15738: -, 2389 and 2112.  18 tiles with 16
+// and 32 rows: 108 workgroups of 32 rows 55 and 81, 256 64 and 83, 432 120 and 114,
+// 3348 730 and 644.
 inline CoupTiling coupling_tiling(bool f64, int nm, int nw, int nb2max, int points, int nPanels) {
   auto ceil = [](int a, int b) { return (a + b - 1) / b; };
   CoupTiling c{};
@@ -45,10 +50,20 @@ inline CoupTiling coupling_tiling(bool f64, int nm, int nw, int nb2max, int poin
     c.modes = std::min(c.modes - 1, ceil(nm, windows + 1));
   }
   const int tiles = ceil(c.modes * nw, 16);
-  c.wc = windows > 1 ? 4 : tiles <= 3 ? 1 : tiles <= 8 ? 2 : 4;
+  auto wgs = [&](int rows) { return (long long)ceil(points, rows) * nPanels; };
+  auto waves = [&](int rows) { return (wgs(rows) + 511) / 512; };
+  c.mt = 1;
+  if (windows > 1 || wgs(32) <= 256) {
+    c.wc = 4;
+  } else if (tiles > 8) {
+    c.wc = 4;
+    c.mt = 2;
+  } else {
+    const bool tall = 12 * waves(64) <= 7 * waves(32);
+    c.wc = tall && tiles <= (f64 ? 4 : 6) ? 1 : 2;
+    c.mt = tall && !f64 && tiles > 6 ? 2 : 1;
+  }
   c.nt = ceil(tiles, c.wc);
-  const bool many = (long long)ceil(points, 32) * nPanels > 256;
-  c.mt = windows == 1 && c.wc == 4 && many ? 2 : 1;
   c.rows = windows > 1 ? 16 : 16 * c.mt * (4 / c.wc);
   return c;
 }

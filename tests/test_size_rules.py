@@ -57,20 +57,30 @@ def test_coupling_tiling(rules, f64):
     window's columns with an instance that exists, and a size is refused only when
     not even one mode at a time fits LDS."""
     forms = [(f64, nm, nw, nb, points, panels) for nm in range(1, 37) for nw in range(1, 33) for nb in range(1, nw + 1)
-             for points, panels in ((8192, 1), (8193, 1), (33, 128), (33, 129), (0, 5))]
+             for points, panels in ((8192, 1), (8193, 1), (33, 128), (33, 129), (0, 5), (64, 512), (65, 512), (1000000, 3))]
     got = rules("tiling", forms, timeout=120)
     assert len(got) == len(forms)
     elem, most = (16, 192) if f64 else (8, 384)
     seen = set()
     for (_, nm, nw, nb, points, panels), (mt, nt, wc, rows, modes, stage, lds) in zip(forms, got):
         at = (nm, nw, nb, points, panels)
-        assert mt == (2 if modes == nm and wc == 4 and -(-points // 32) * panels > 256 else 1), at
+        n64, n32, tiles = -(-points // 64) * panels, -(-points // 32) * panels, -(-modes * nw // 16)
+        tall = 12 * -(-n64 // 512) <= 7 * -(-n32 // 512)
+        if modes < nm or n32 <= 256:
+            want = (1, 4)
+        elif tiles > 8:
+            want = (2, 4)
+        elif not tall:
+            want = (1, 2)
+        else:
+            want = (1, 1) if tiles <= (4 if f64 else 6) else (1, 2) if f64 else (2, 2)
+        assert (mt, wc) == want, at
         scratch = 16 * nm * nb * 24
         assert 1 <= modes <= nm and (modes * nw <= most or modes == 1), at
         assert lds == max(16 * modes * nw * elem + scratch, 1024), at
         assert (lds <= 160 * 1024) == (16 * nw * elem + scratch <= 160 * 1024), at
-        assert wc * nt * 16 >= modes * nw > wc * (nt - 1) * 16 * (nt > 1) and wc in (1, 2, 4), at
-        assert rows == (16 if modes < nm else 16 * mt * (4 // wc)) and (modes == nm or (mt, wc) == (1, 4)), at
+        assert nt == -(-tiles // wc), at
+        assert rows == (16 if modes < nm else 16 * mt * (4 // wc)), at
         assert stage == (16 * modes * nw * elem >= 16 * (nm + nb) * 8), at
         seen.add((mt, nt))
     assert seen == INSTANCES[f64]
