@@ -24,8 +24,10 @@ constexpr size_t kCoupReduceLds = 1024;  // of reduce_partials
 // Whole panels take 16, 32 or 64 rows: more rows share a load of the panel, but
 // their epilogues follow each other, and two workgroups per CU, 512 in all, run at
 // once.  16 rows on four column waves while 32 would not even give every CU a
-// workgroup.  Else, up to 8 column tiles, 64 rows where the waves of 512 workgroups
-// they take, at 12/7 the time of 32 rows, are no longer: on one column wave up to
+// workgroup.  Else, up to 8 column tiles, 64 rows where they take less time than
+// 32: a workgroup of 64 takes 1.6 times as long as one of 32 (6 to 8 tiles 1.75), a
+// launch as long as its workgroups of 512 at once, at least one such wave, two beyond
+// 512 of 32 rows, and 0.3 waves for the tail of 64.  They run on one column wave up to
 // 6 tiles (FP64, whose accumulators take twice the registers: 4), in FP32 on two with
 // two row tiles each beyond.  More tiles: two row tiles on four column waves.
 // us per launch with 16, 32 and 64 rows in FP32; 5 column tiles: 28 workgroups of 32
@@ -51,7 +53,6 @@ inline CoupTiling coupling_tiling(bool f64, int nm, int nw, int nb2max, int poin
   }
   const int tiles = ceil(c.modes * nw, 16);
   auto wgs = [&](int rows) { return (long long)ceil(points, rows) * nPanels; };
-  auto waves = [&](int rows) { return (wgs(rows) + 511) / 512; };
   c.mt = 1;
   if (windows > 1 || wgs(32) <= 256) {
     c.wc = 4;
@@ -59,7 +60,9 @@ inline CoupTiling coupling_tiling(bool f64, int nm, int nw, int nb2max, int poin
     c.wc = 4;
     c.mt = 2;
   } else {
-    const bool tall = 12 * waves(64) <= 7 * waves(32);
+    const long long t64 = wgs(64) <= 512 ? 512 : wgs(64) + 154;
+    const long long t32 = wgs(32) <= 512 ? 512 : std::max(wgs(32), 1024ll);
+    const bool tall = tiles <= 5 ? 8 * t64 <= 5 * t32 : 7 * t64 <= 4 * t32;
     c.wc = tall && tiles <= (f64 ? 4 : 6) ? 1 : 2;
     c.mt = tall && !f64 && tiles > 6 ? 2 : 1;
   }

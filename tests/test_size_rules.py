@@ -65,7 +65,8 @@ def test_coupling_tiling(rules, f64):
     for (_, nm, nw, nb, points, panels), (mt, nt, wc, rows, modes, stage, lds) in zip(forms, got):
         at = (nm, nw, nb, points, panels)
         n64, n32, tiles = -(-points // 64) * panels, -(-points // 32) * panels, -(-modes * nw // 16)
-        tall = 12 * -(-n64 // 512) <= 7 * -(-n32 // 512)
+        t64, t32 = 512 if n64 <= 512 else n64 + 154, 512 if n32 <= 512 else max(n32, 1024)
+        tall = 8 * t64 <= 5 * t32 if tiles <= 5 else 7 * t64 <= 4 * t32
         if modes < nm or n32 <= 256:
             want = (1, 4)
         elif tiles > 8:
