@@ -19,8 +19,11 @@ constexpr size_t kCoupReduceLds = 1024;  // of reduce_partials
 
 // As few windows as fit: whole panels of up to 24 column tiles (FP32) or 12
 // (FP64, whose tiles take twice the registers and LDS), and fewer modes per window
-// where g' and |g|^2 of a row tile leave less LDS to g3.  Several windows leave a row
-// tile's g' in LDS between them, so they run 16 rows per workgroup.
+// where g' and |g|^2 of a row tile leave less LDS to g3: half of the LDS, for two
+// workgroups per CU, where there are more than 256 and a window keeps a quarter of
+// its modes (27 modes x 19 bands in FP32, 4 bands per point, 1888 workgroups of 32
+// points: 1490 us with one workgroup per CU, 946 with two).  Several windows leave a
+// row tile's g' in LDS between them, so they run 16 rows per workgroup.
 // Whole panels take 16, 32 or 64 rows: more rows share a load of the panel, but
 // their epilogues follow each other, and two workgroups per CU, 512 in all, run at
 // once.  16 rows on four column waves while 32 would not even give every CU a
@@ -40,19 +43,22 @@ inline CoupTiling coupling_tiling(bool f64, int nm, int nw, int nb2max, int poin
   CoupTiling c{};
   const size_t scratch = size_t(16) * nm * nb2max * (16 + 8);
   const int most = f64 ? 192 : 384;
-  int windows = ceil(nm, std::max(1, most / nw));
-  c.modes = ceil(nm, windows);
-  for (;;) {
-    windows = ceil(nm, c.modes);
-    const size_t g3 = (size_t(16) * c.modes * nw * (f64 ? 16 : 8) + 15) / 16 * 16;
-    c.stage = g3 >= size_t(16) * (nm + nb2max) * 8;
-    c.lds = std::max(g3 + scratch, kCoupReduceLds);
-    if (c.lds <= 160 * 1024 || c.modes == 1) break;
-    // even windows, and at least one mode less: ceil(nm / (windows + 1)) can be the same number of modes
-    c.modes = std::min(c.modes - 1, ceil(nm, windows + 1));
-  }
-  const int tiles = ceil(c.modes * nw, 16);
+  const int whole = ceil(nm, ceil(nm, std::max(1, most / nw)));
   auto wgs = [&](int rows) { return (long long)ceil(points, rows) * nPanels; };
+  auto tile = [&](int modes) { return (size_t(16) * modes * nw * (f64 ? 16 : 8) + 15) / 16 * 16; };
+  auto lds = [&](int modes) { return std::max(tile(modes) + scratch, kCoupReduceLds); };
+  auto fit = [&](size_t room) {
+    int modes = whole;
+    // even windows, and at least one mode less: ceil(nm / (windows + 1)) can be the same number of modes
+    while (modes > 1 && lds(modes) > room) modes = std::min(modes - 1, ceil(nm, ceil(nm, modes) + 1));
+    return modes;
+  };
+  c.modes = fit(80 * 1024);
+  if (wgs(16) <= 256 || lds(c.modes) > 80 * 1024 || 4 * c.modes < whole) c.modes = fit(160 * 1024);
+  const int windows = ceil(nm, c.modes);
+  c.stage = tile(c.modes) >= size_t(16) * (nm + nb2max) * 8;
+  c.lds = lds(c.modes);
+  const int tiles = ceil(c.modes * nw, 16);
   c.mt = 1;
   if (windows > 1 || wgs(32) <= 256) {
     c.wc = 4;

@@ -65,7 +65,7 @@ def test_too_many_bands_are_refused(precision):
 
 
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("fp32", 2e-6)])
-@pytest.mark.parametrize("natoms,nw", [(2, 8), (3, 8), (3, 12), (3, 16), (6, 16)])
+@pytest.mark.parametrize("natoms,nw", [(2, 8), (3, 8), (3, 12), (3, 16), (6, 16), (9, 17)])
 def test_row_tiles_by_the_number_of_workgroups(natoms, nw, precision, tol):
     """A point alone takes 16 rows per workgroup, a batch of points 32 or 64, and runs
     of either may follow the other; the linewidths of the points are the same."""

@@ -77,6 +77,19 @@ def test_coupling_tiling(rules, f64):
             want = (1, 1) if tiles <= (4 if f64 else 6) else (1, 2) if f64 else (2, 2)
         assert (mt, wc) == want, at
         scratch = 16 * nm * nb * 24
+        up = lambda a, b: -(-a // b)
+        whole = up(nm, up(nm, max(1, most // nw)))
+
+        def fit(room):
+            m = whole
+            while m > 1 and max(16 * m * nw * elem + scratch, 1024) > room:
+                m = min(m - 1, up(nm, up(nm, m) + 1))
+            return m
+
+        half = fit(80 * 1024)
+        if up(points, 16) * panels <= 256 or 16 * half * nw * elem + scratch > 80 * 1024 or 4 * half < whole:
+            half = fit(160 * 1024)
+        assert modes == half, at
         assert 1 <= modes <= nm and (modes * nw <= most or modes == 1), at
         assert lds == max(16 * modes * nw * elem + scratch, 1024), at
         assert (lds <= 160 * 1024) == (16 * nw * elem + scratch <= 160 * 1024), at
